@@ -17,243 +17,575 @@
 // flat there).  The reference dW kernel keeps at most 16 coefficients in
 // registers; here K goes up to kMaxK.
 //
-// Both kernels contract over one axis against an operand with KP = K +
-// has_base "slots" per feature (slot 0 = SiLU when has_base):
-//   * k_cheby_bwd_dw: output tile 64 o x 16 features x KP slots, contraction
-//     over the batch.  Per chunk of 16 rows the workgroup evaluates the slots
-//     of its 16 x 16 (row, feature) pairs once into LDS; lane o of wave w
-//     accumulates features 4w..4w+3 (the slot reads are LDS broadcasts).  The
-//     workgroups of the first feature tile also reduce dbias.
-//   * k_cheby_bwd_dx: output tile 64 rows x 16 features, contraction over
-//     D_out in chunks of 16 against W / W_base tiles in LDS; the epilogue
-//     multiplies the per-slot sums by T'_k / SiLU' and adds them up.
+// T_0 = 1 and T'_0 = 0 for every input, so the k = 0 coefficients need no
+// contraction: dW[o, i*K] = dbias[o] for every i, and they add nothing to dX.
+// The NS = K - 1 + has_base "slots" left are SiLU (when has_base) and
+// T_1 .. T_{K-1}.
+//
+// Both gradients are matrix products on the bf16 matrix cores with every fp32
+// operand split into three bf16 terms (kans_split.h: six MFMAs per product
+// tile, fp32 accumulation, no operand rounded):
+//   * k_cheby_bwd_dw: M = outputs, N = (slot, feature), contraction over the
+//     batch; A = dY^T, B = the slot values of x, evaluated in the kernel.
+//   * k_cheby_bwd_dx: M = batch rows, N = (slot, feature), contraction over
+//     D_out; A = dY, B = the slot weights.  The epilogue multiplies the slot
+//     sums of one (row, feature) -- all in one lane -- by T'_k / SiLU' and adds
+//     them up.
+//
+// One workgroup = 8 waves = 4 (M) x 2 (32 features).  A wave owns MB x SG tiles
+// of 32 x 32 (MB row blocks, SG slots; MB * SG <= 10 tiles, 160 accumulators).
+// Per step of 16 contraction indices every operand tile of the workgroup is
+// loaded from global memory, split once by one wave and written to one of two
+// LDS stages in MFMA fragment order (3 KB per tile, lane-contiguous 16-byte
+// accesses); all waves read their fragments from there.  The two waves of a
+// SIMD take turns: one splits the next step's operands (VALU) while the other
+// multiplies (MFMA), then they swap, with one barrier per step.  That is
+// MB * SG * 6 MFMAs (1536 to 1920 cycles) per wave and step against 150 to 250
+// VALU instructions.
+//
+// The bound is the matrix pipe at 6 x 2 * B * D_in * D_out * NS operations: at
+// 8192 x 1024 -> 1024, K = 4 with the base branch, dW takes 350 us and dX 341 us
+// (1.18 and 1.21 PFLOP/s of bf16 MFMA, the rate a large bf16 matrix product
+// reaches on the same card), where the fp32 VALU kernels this replaces took 3203
+// and 2753 us.  Without the waves' turns 364 and 346 us.
+// Grids that leave CUs idle split the contraction (choose_splits) into partial
+// sums that a second kernel adds in order: 64 workgroups of dW at that shape
+// become 256, and the sums cost 27 us.
 #include "kans_common.h"
 #include "kans_api_internal.h"
+#include "kans_split.h"
+#include "kans_tile.h"
 #include <algorithm>
 
 namespace kans {
 namespace {
 
-constexpr int kBwdThreads = 256;
-constexpr int kBwdO = 64;    // output rows (dW) / batch rows (dX) per workgroup
-constexpr int kBwdF = 16;    // features per workgroup
-constexpr int kBwdC = 16;    // contraction chunk (batch rows for dW, outputs for dX)
+constexpr int kBwdThreads = 512;
+constexpr int kBwdF = 64;      // features per workgroup
+constexpr int kBwdStep = 16;   // contraction indices per step (one MFMA)
+constexpr int kBwdMaxSG = 10;  // slots per workgroup
+
+struct BwdArgs {
+  const float *dY, *X, *W, *Wb;
+  float *dW, *dWb, *db, *dX;
+  float* part;   // split partial sums (null: one split, results written directly)
+  float* dbp;    // split partial sums of dbias
+  int B, D_in, D_out, K, has_base, NS;
+  int m_tiles, f_tiles, groups;
+  int steps, steps_per_split;
+  int vec;       // dX: rows of dY readable with 16-byte loads
+};
 
 __device__ __forceinline__ float silu_deriv_f32(float x) {
   const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * kLog2e));
   return s * (1.0f + x * (1.0f - s));
 }
 
-// Slot values of one input: v[0] = SiLU(x) when has_base, then T_0..T_{K-1}(clamp x),
-// zero past the last slot.  Indices stay compile-time (the array lives in registers).
-template <int KPM>
-__device__ __forceinline__ void slot_values(float x, int K, int has_base, float* v) {
-  const float t = fminf(fmaxf(x, -1.0f), 1.0f);
-  const float sx = has_base ? silu_f32(x) : 0.0f;
-  float a = 1.0f, b = t;  // T_{k-2}, T_{k-1} once k >= 2
+// One operand tile (32 x 16) of a stage: three terms of 64 lanes x 16 bytes.
+__device__ __forceinline__ void put_tile(uint4* stage, int tile, int lane, const float* v) {
+  const Split8 s = split8(v);
 #pragma unroll
-  for (int s = 0; s < KPM; ++s) {
-    const int k = s - has_base;
-    float val;
-    if (k < 0) {
-      val = sx;
-    } else if (k == 0) {
-      val = 1.0f;
-    } else if (k == 1) {
-      val = t;
+  for (int q = 0; q < 3; ++q) stage[(tile * 3 + q) * 64 + lane] = s.t[q];
+}
+
+__device__ __forceinline__ void get_tile(const uint4* stage, int tile, int lane, bf16x8 (&f)[3]) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const uint4 u = stage[(tile * 3 + q) * 64 + lane];
+    f[q] = *reinterpret_cast<const bf16x8*>(&u);
+  }
+}
+
+// One step of the wave's MB x SG tiles from a stage (A tiles first, then the
+// 2 x SG B tiles).
+template <int SG, int MB>
+__device__ __forceinline__ void multiply(const uint4* stage, int wm, int wf, int lane, floatx16 (&acc)[MB][SG]) {
+  bf16x8 a[MB][3], b[2][3];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) get_tile(stage, wm * MB + mb, lane, a[mb]);
+  get_tile(stage, 4 * MB + wf * SG, lane, b[0]);
+#pragma unroll
+  for (int s = 0; s < SG; ++s) {
+    if (s + 1 < SG) get_tile(stage, 4 * MB + wf * SG + s + 1, lane, b[(s + 1) & 1]);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[mb][s] = mma_split(a[mb], b[s & 1], acc[mb][s]);
+  }
+}
+
+template <int SG, int MB>
+__device__ __forceinline__ void clear(floatx16 (&acc)[MB][SG]) {
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int s = 0; s < SG; ++s)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mb][s][r] = 0.0f;
+}
+
+template <int SG, int MB>
+__global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
+  constexpr int NA = 4 * MB;
+  __shared__ uint4 stage[2][(NA + 2 * SG) * 3 * 64];
+  __shared__ float dbs[NA * 32];
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 3, wf = wave >> 2;
+
+  const int tiles = P.m_tiles * P.f_tiles;
+  const int lin = xcd_remap(blockIdx.x, tiles * P.groups);
+  const int g = lin / tiles;
+  int m_tile, f_tile;
+  tile_of(lin - g * tiles, P.m_tiles, P.f_tiles, m_tile, f_tile);
+  const int o0 = m_tile * (NA * 32), i0 = f_tile * kBwdF, s0 = g * SG;
+  const int split = blockIdx.y;
+  const int t0 = split * P.steps_per_split;
+  const int nk = min(P.steps - t0, P.steps_per_split);
+
+  // A tiles (dY^T): with MB = 2 one per wave, with MB = 1 one for the waves
+  // that evaluate fewer slots
+  const bool do_a = MB == 2 || wm >= 2;
+  const int a_tile = MB == 2 ? wave : wf * 2 + wm - 2;
+  // lanes past D_out / D_in repeat the last one: their sums are not stored
+  const int ocol = min(o0 + a_tile * 32 + (lane & 31), P.D_out - 1);
+  const int icol = min(i0 + wf * 32 + (lane & 31), P.D_in - 1);
+  float ra[8], rx[8];
+  auto load = [&](int t) {
+    const int b0 = (t0 + t) * kBwdStep + 8 * half;
+    const float* pa = P.dY + (long)b0 * P.D_out + ocol;
+    const float* px = P.X + (long)b0 * P.D_in + icol;
+    if ((t0 + t + 1) * kBwdStep <= P.B) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (do_a) ra[j] = pa[(long)j * P.D_out];
+        rx[j] = px[(long)j * P.D_in];
+      }
     } else {
-      val = __builtin_fmaf(2.0f * t, b, -a);
-      a = b;
-      b = val;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const bool ok = b0 + j < P.B;
+        if (do_a) ra[j] = ok ? pa[(long)j * P.D_out] : 0.0f;
+        rx[j] = ok ? px[(long)j * P.D_in] : 0.0f;
+      }
     }
-    v[s] = k < K ? val : 0.0f;
-  }
-}
-
-template <int KPM>
-__global__ void __launch_bounds__(kBwdThreads)
-k_cheby_bwd_dw(const float* __restrict__ dY, const float* __restrict__ X, float* __restrict__ dW,
-               float* __restrict__ dWb, float* __restrict__ db, int B, int D_in, int D_out, int K,
-               int has_base) {
-  __shared__ float dys[kBwdC][kBwdO];
-  __shared__ __attribute__((aligned(16))) float phis[kBwdC][kBwdF][KPM];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int o0 = blockIdx.x * kBwdO, i0 = blockIdx.y * kBwdF;
-  const int KP = K + has_base;
-  const int o = o0 + lane;
-  const bool do_bias = db != nullptr && blockIdx.y == 0 && wave == 0;
-
-  float acc[4][KPM];
-#pragma unroll
-  for (int f = 0; f < 4; ++f)
-#pragma unroll
-    for (int s = 0; s < KPM; ++s) acc[f][s] = 0.0f;
-  float bsum = 0.0f;
-
-  for (int b0 = 0; b0 < B; b0 += kBwdC) {
-    // dY rows b0.. (columns o0..o0+63), zero past B / D_out
-#pragma unroll
-    for (int r = 0; r < kBwdC / 4; ++r) {
-      const int bb = wave * (kBwdC / 4) + r, b = b0 + bb;
-      dys[bb][lane] = (b < B && o < D_out) ? dY[(long)b * D_out + o] : 0.0f;
+  };
+  float bsum = 0.0f;  // this lane's share of dbias[ocol]
+  const bool base0 = P.has_base != 0 && s0 == 0;
+  const int k_first = s0 + 1 - P.has_base;  // T index of the group's first slot (g > 0)
+  auto produce = [&](uint4* st) {
+    if (do_a) {
+      put_tile(st, a_tile, lane, ra);
+      bsum += ((ra[0] + ra[1]) + (ra[2] + ra[3])) + ((ra[4] + ra[5]) + (ra[6] + ra[7]));
     }
-    // slots of the 16 x 16 (row, feature) pairs, one pair per thread
-    {
-      const int bb = tid / kBwdF, ff = tid % kBwdF, b = b0 + bb, i = i0 + ff;
-      float v[KPM];
+    float tw[8], c[8], p[8];  // 2t, T_k, T_{k-1}
 #pragma unroll
-      for (int s = 0; s < KPM; ++s) v[s] = 0.0f;
-      if (b < B && i < D_in) slot_values<KPM>(X[(long)b * D_in + i], K, has_base, v);
+    for (int j = 0; j < 8; ++j) {
+      const float t = fminf(fmaxf(rx[j], -1.0f), 1.0f);
+      tw[j] = t + t;
+      c[j] = t;
+      p[j] = 1.0f;
+    }
+    auto advance = [&]() {
 #pragma unroll
-      for (int s = 0; s < KPM; ++s) phis[bb][ff][s] = v[s];
+      for (int j = 0; j < 8; ++j) {
+        const float n = __builtin_fmaf(tw[j], c[j], -p[j]);
+        p[j] = c[j];
+        c[j] = n;
+      }
+    };
+    for (int k = 1; k < k_first; ++k) advance();
+#pragma unroll
+    for (int s = 0; s < SG; ++s) {
+      const bool mine = (s & 3) == wm;
+      if (s == 0 && base0) {
+        if (mine) {
+          float v[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = silu_f32(rx[j]);
+          put_tile(st, NA + wf * SG + s, lane, v);
+        }
+      } else {
+        if (mine) put_tile(st, NA + wf * SG + s, lane, c);
+        if (s + 1 < SG) advance();
+      }
+    }
+  };
+
+  floatx16 acc[MB][SG];
+  clear<SG, MB>(acc);
+  load(0);
+  produce(stage[0]);
+  if (nk > 1) load(1);
+  __syncthreads();
+  for (int t = 0; t < nk; ++t) {
+    const uint4* cur = stage[t & 1];
+    uint4* nxt = stage[(t + 1) & 1];
+    const bool more = t + 1 < nk;
+    if (wf == 0 && more) {
+      produce(nxt);
+      if (t + 2 < nk) load(t + 2);
+    }
+    multiply<SG, MB>(cur, wm, wf, lane, acc);
+    if (wf != 0 && more) {
+      produce(nxt);
+      if (t + 2 < nk) load(t + 2);
     }
     __syncthreads();
-    for (int bb = 0; bb < kBwdC; ++bb) {
-      const float dy = dys[bb][lane];
-      bsum += dy;
+  }
+
+  bsum += __shfl_xor(bsum, 32);
+  if (do_a && half == 0) dbs[a_tile * 32 + lane] = bsum;
+  __syncthreads();
+  const int tid = threadIdx.x;
+  if (f_tile == 0 && g == 0 && tid < NA * 32 && o0 + tid < P.D_out) {
+    if (P.part != nullptr) P.dbp[(long)split * P.D_out + o0 + tid] = dbs[tid];
+    else if (P.db != nullptr) P.db[o0 + tid] = dbs[tid];
+  }
+  // acc register r of lane l holds output 8*(r/4) + 4*(l/32) + r%4, feature l%32
+  const int i = i0 + wf * 32 + (lane & 31);
+  if (i >= P.D_in) return;
+  const long Kd = (long)P.D_in * P.K;
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        const float4* p = reinterpret_cast<const float4*>(&phis[bb][wave * 4 + f][0]);
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int q = 0; q < KPM / 4; ++q) {
-          const float4 u = p[q];
-          acc[f][4 * q + 0] = __builtin_fmaf(dy, u.x, acc[f][4 * q + 0]);
-          acc[f][4 * q + 1] = __builtin_fmaf(dy, u.y, acc[f][4 * q + 1]);
-          acc[f][4 * q + 2] = __builtin_fmaf(dy, u.z, acc[f][4 * q + 2]);
-          acc[f][4 * q + 3] = __builtin_fmaf(dy, u.w, acc[f][4 * q + 3]);
+    for (int r = 0; r < 16; ++r) {
+      const int ol = (wm * MB + mb) * 32 + 8 * (r >> 2) + 4 * half + (r & 3), o = o0 + ol;
+      if (o >= P.D_out) continue;
+      if (P.part != nullptr) {
+        float* out = P.part + (((long)split * P.D_out + o) * P.NS + s0) * P.D_in + i;
+#pragma unroll
+        for (int s = 0; s < SG; ++s)
+          if (s0 + s < P.NS) out[(long)s * P.D_in] = acc[mb][s][r];
+      } else {
+        float* out = P.dW + (long)o * Kd + (long)i * P.K;
+        if (g == 0) out[0] = dbs[ol];
+#pragma unroll
+        for (int s = 0; s < SG; ++s) {
+          if (s == 0 && base0) P.dWb[(long)o * P.D_in + i] = acc[mb][s][r];
+          else if (s0 + s < P.NS) out[s0 + s + 1 - P.has_base] = acc[mb][s][r];
         }
       }
     }
-    __syncthreads();
-  }
-
-  if (o >= D_out) return;
-  if (do_bias) db[o] = bsum;
-  const long Kd = (long)D_in * K;
-#pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    const int i = i0 + wave * 4 + f;
-    if (i >= D_in) continue;
-    if (has_base) dWb[(long)o * D_in + i] = acc[f][0];
-#pragma unroll
-    for (int s = 0; s < KPM; ++s) {
-      const int k = s - has_base;
-      if (k >= 0 && k < K) dW[(long)o * Kd + (long)i * K + k] = acc[f][s];
-    }
-  }
-  (void)KP;
 }
 
-template <int KPM>
-__global__ void __launch_bounds__(kBwdThreads)
-k_cheby_bwd_dx(const float* __restrict__ dY, const float* __restrict__ X, const float* __restrict__ W,
-               const float* __restrict__ Wb, float* __restrict__ dX, int B, int D_in, int D_out, int K,
-               int has_base) {
-  __shared__ float dys[kBwdC][kBwdO];
-  __shared__ __attribute__((aligned(16))) float ws[kBwdC][kBwdF][KPM];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int b0 = blockIdx.x * kBwdO, i0 = blockIdx.y * kBwdF;
-  const int b = b0 + lane;
-  const int KP = K + has_base;
-  const long Kd = (long)D_in * K;
-
-  float acc[4][KPM];
+// Sum of the splits' partial sums, in split order, into dW / dW_base / dbias.
+// One thread per (output, slot, feature); slot 0's threads also write the
+// k = 0 coefficient, which is dbias.
+__global__ void k_cheby_bwd_dw_reduce(BwdArgs P, int splits) {
+  const long n = (long)P.D_out * P.NS * P.D_in;
+  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += (long)gridDim.x * blockDim.x) {
+    const long row = idx / P.D_in;
+    const int i = (int)(idx - row * P.D_in), o = (int)(row / P.NS), sl = (int)(row - (long)o * P.NS);
+    float s = 0.0f;
+    for (int k0 = 0; k0 < splits; k0 += 8) {
+      float v[8];
 #pragma unroll
-  for (int f = 0; f < 4; ++f)
+      for (int u = 0; u < 8; ++u) v[u] = k0 + u < splits ? P.part[(long)(k0 + u) * n + idx] : 0.0f;
 #pragma unroll
-    for (int s = 0; s < KPM; ++s) acc[f][s] = 0.0f;
-
-  for (int oc = 0; oc < D_out; oc += kBwdC) {
-    // dY[b0.., oc..oc+15] transposed into dys[o][b]
-#pragma unroll
-    for (int r = 0; r < (kBwdC * kBwdO) / kBwdThreads; ++r) {
-      const int e = r * kBwdThreads + tid, bb = e / kBwdC, oo = e % kBwdC;
-      const int bq = b0 + bb, o = oc + oo;
-      dys[oo][bb] = (bq < B && o < D_out) ? dY[(long)bq * D_out + o] : 0.0f;
+      for (int u = 0; u < 8; ++u) s += v[u];
     }
-    // slot weights of outputs oc.. for features i0..i0+15: ws[o][f][s]
-    for (int e = tid; e < kBwdC * kBwdF * KPM; e += kBwdThreads) {
-      const int oo = e / (kBwdF * KPM), rem = e % (kBwdF * KPM), ff = rem / KPM, s = rem % KPM;
-      const int o = oc + oo, i = i0 + ff, k = s - has_base;
-      float w = 0.0f;
-      if (o < D_out && i < D_in && s < KP) w = k < 0 ? Wb[(long)o * D_in + i] : W[(long)o * Kd + (long)i * K + k];
-      ws[oo][ff][s] = w;
+    float* out = P.dW + ((long)o * P.D_in + i) * P.K;
+    if (sl == 0) {
+      float d = 0.0f;
+      for (int k = 0; k < splits; ++k) d += P.dbp[(long)k * P.D_out + o];
+      out[0] = d;
+      if (i == 0 && P.db != nullptr) P.db[o] = d;
     }
-    __syncthreads();
-    for (int oo = 0; oo < kBwdC; ++oo) {
-      const float dy = dys[oo][lane];
-#pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        const float4* p = reinterpret_cast<const float4*>(&ws[oo][wave * 4 + f][0]);
-#pragma unroll
-        for (int q = 0; q < KPM / 4; ++q) {
-          const float4 u = p[q];
-          acc[f][4 * q + 0] = __builtin_fmaf(dy, u.x, acc[f][4 * q + 0]);
-          acc[f][4 * q + 1] = __builtin_fmaf(dy, u.y, acc[f][4 * q + 1]);
-          acc[f][4 * q + 2] = __builtin_fmaf(dy, u.z, acc[f][4 * q + 2]);
-          acc[f][4 * q + 3] = __builtin_fmaf(dy, u.w, acc[f][4 * q + 3]);
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  if (b >= B) return;
-#pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    const int i = i0 + wave * 4 + f;
-    if (i >= D_in) continue;
-    const float x = X[(long)b * D_in + i];
-    float dx = has_base ? acc[f][0] * silu_deriv_f32(x) : 0.0f;
-    if (x >= -1.0f && x <= 1.0f) {
-      // T'_0 = 0, T'_1 = 1, T'_k = 2 T_{k-1} + 2x T'_{k-1} - T'_{k-2}
-      float Tm2 = 1.0f, Tm1 = x, dm2 = 0.0f, dm1 = 1.0f;
-#pragma unroll
-      for (int s = 0; s < KPM; ++s) {
-        const int k = s - has_base;
-        if (k == 1 && k < K) dx += acc[f][s];
-        if (k >= 2 && k < K) {
-          const float T = __builtin_fmaf(2.0f * x, Tm1, -Tm2);
-          const float d = __builtin_fmaf(2.0f * x, dm1, __builtin_fmaf(2.0f, Tm1, -dm2));
-          dx = __builtin_fmaf(acc[f][s], d, dx);
-          Tm2 = Tm1;
-          Tm1 = T;
-          dm2 = dm1;
-          dm1 = d;
-        }
-      }
-    }
-    dX[(long)b * D_in + i] = dx;
+    if (sl == 0 && P.has_base) P.dWb[(long)o * P.D_in + i] = s;
+    else out[sl + 1 - P.has_base] = s;
   }
 }
 
-template <int KPM>
-hipError_t launch_bwd(const float* dY, const float* X, const float* W, const float* Wb, float* dW, float* dWb,
-                      float* db, float* dX, int B, int D_in, int D_out, int K, int has_base, hipStream_t st) {
-  const dim3 gw((D_out + kBwdO - 1) / kBwdO, (D_in + kBwdF - 1) / kBwdF);
-  hipLaunchKernelGGL((k_cheby_bwd_dw<KPM>), gw, dim3(kBwdThreads), 0, st, dY, X, dW, dWb, db, B, D_in, D_out, K,
-                     has_base);
+template <int SG, int MB>
+__global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
+  constexpr int NA = 4 * MB, NT = NA + 2 * SG;
+  constexpr int R = (NT + 7) / 8;  // operand tiles a wave loads and splits per step
+  __shared__ uint4 stage[2][NT * 3 * 64];
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 3, wf = wave >> 2;
+
+  int m_tile, f_tile;
+  tile_of(xcd_remap(blockIdx.x, P.m_tiles * P.f_tiles), P.m_tiles, P.f_tiles, m_tile, f_tile);
+  const int b0 = m_tile * (NA * 32), i0 = f_tile * kBwdF;
+  const int split = blockIdx.y;
+  const int t0 = split * P.steps_per_split;
+  const int nk = min(P.steps - t0, P.steps_per_split);
+  const long Kd = (long)P.D_in * P.K;
+  float* const out = P.part != nullptr ? P.part + (long)split * P.B * P.D_in : P.dX;
+  const int i = i0 + wf * 32 + (lane & 31);
+
+  for (int g = 0; g < P.groups; ++g) {
+    const int s0 = g * SG;
+    // operand tile r * 8 + wave: A (dY rows, contiguous outputs) below NA, else
+    // slot weights; lanes past B / D_in and slots past NS repeat the last one
+    // (src: the wave's first address, lane_off: this lane's bytes from it)
+    const float* src[R];
+    unsigned lane_off[R];
+    long stride[R];
+    float raw[R][8];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int id = r * 8 + wave;
+      const long o = (long)t0 * kBwdStep;
+      if (id < NA) {
+        src[r] = P.dY + (long)b0 * P.D_out + o;
+        lane_off[r] = 4u * ((unsigned)(min(b0 + id * 32 + (lane & 31), P.B - 1) - b0) * P.D_out + 8 * half);
+        stride[r] = 1;
+      } else {
+        const int q = min(id, NT - 1) - NA, f = q / SG;
+        const int ic = min(i0 + f * 32 + (lane & 31), P.D_in - 1);
+        const int sl = min(s0 + q - f * SG, P.NS - 1), k = sl + 1 - P.has_base;
+        const bool base = P.has_base != 0 && sl == 0;
+        stride[r] = base ? P.D_in : Kd;
+        src[r] = (base ? P.Wb : P.W + k) + o * stride[r];
+        lane_off[r] = 4u * (8u * half * (unsigned)stride[r] + (unsigned)ic * (base ? 1 : P.K));
+      }
+    }
+    auto load = [&](int t) {
+      const bool full = (t0 + t + 1) * kBwdStep <= P.D_out;
+      const int left = P.D_out - (t0 + t) * kBwdStep - 8 * half;  // outputs from this lane's first on
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int id = r * 8 + wave;
+        if (id >= NT) continue;
+        const float* p = src[r] + (long)t * kBwdStep * stride[r];
+        auto at = [&](int j) { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(p + j * stride[r]) + lane_off[r]); };
+        if (full && id < NA && P.vec) {
+          const float4 u = *reinterpret_cast<const float4*>(at(0)), w = *reinterpret_cast<const float4*>(at(4));
+          raw[r][0] = u.x; raw[r][1] = u.y; raw[r][2] = u.z; raw[r][3] = u.w;
+          raw[r][4] = w.x; raw[r][5] = w.y; raw[r][6] = w.z; raw[r][7] = w.w;
+        } else if (full) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) raw[r][j] = *at(j);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) raw[r][j] = j < left ? *at(j) : 0.0f;
+        }
+      }
+    };
+    auto produce = [&](uint4* st) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (r * 8 + wave < NT) put_tile(st, r * 8 + wave, lane, raw[r]);
+    };
+
+    floatx16 acc[MB][SG];
+    clear<SG, MB>(acc);
+    load(0);
+    produce(stage[0]);
+    if (nk > 1) load(1);
+    __syncthreads();
+    for (int t = 0; t < nk; ++t) {
+      const uint4* cur = stage[t & 1];
+      uint4* nxt = stage[(t + 1) & 1];
+      const bool more = t + 1 < nk;
+      if (wf == 0 && more) {
+        produce(nxt);
+        if (t + 2 < nk) load(t + 2);
+      }
+      multiply<SG, MB>(cur, wm, wf, lane, acc);
+      if (wf != 0 && more) {
+        produce(nxt);
+        if (t + 2 < nk) load(t + 2);
+      }
+      __syncthreads();
+    }
+
+    // acc register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, feature l%32
+    const int k_first = max(1, s0 + 1 - P.has_base);
+    // opaque, so that the 16 * MB row addresses are not kept in registers through the groups' steps
+    int row0 = b0 + wm * MB * 32 + 4 * half;
+    asm volatile("" : "+v"(row0));
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      float xs[16];  // one memory round trip per row block
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        xs[r] = P.X[(long)min(row0 + mb * 32 + 8 * (r >> 2) + (r & 3), P.B - 1) * P.D_in + min(i, P.D_in - 1)];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int b = row0 + mb * 32 + 8 * (r >> 2) + (r & 3);
+        const long at = (long)b * P.D_in + i;
+        const float x = xs[r];
+        // T'_1 = 1, T'_{k+1} = 2 T_k + 2x T'_k - T'_{k-1}
+        float T = x, Tp = 1.0f, d = 1.0f, dp = 0.0f;
+        auto advance = [&]() {
+          const float Tn = __builtin_fmaf(2.0f * x, T, -Tp);
+          const float dn = __builtin_fmaf(2.0f * x, d, __builtin_fmaf(2.0f, T, -dp));
+          Tp = T;
+          T = Tn;
+          dp = d;
+          d = dn;
+        };
+        for (int k = 1; k < k_first; ++k) advance();
+        float dx = 0.0f, poly = 0.0f;
+#pragma unroll
+        for (int s = 0; s < SG; ++s) {
+          if (s == 0 && P.has_base && s0 == 0) {
+            dx = acc[mb][s][r] * silu_deriv_f32(x);
+          } else if (s0 + s < P.NS) {
+            poly = __builtin_fmaf(acc[mb][s][r], d, poly);
+            advance();
+          }
+        }
+        if (x >= -1.0f && x <= 1.0f) dx += poly;
+        if (b < P.B && i < P.D_in) out[at] = g == 0 ? dx : out[at] + dx;
+        // one value at a time: all of them side by side would spill the sums
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+}
+
+__global__ void k_sum_splits(const float* __restrict__ part, float* __restrict__ out, int splits, long n) {
+  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += (long)gridDim.x * blockDim.x) {
+    float s = 0.0f;
+    for (int k0 = 0; k0 < splits; k0 += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = k0 + u < splits ? part[(long)(k0 + u) * n + idx] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    out[idx] = s;
+  }
+}
+
+// K = 1 without the base branch: T_0 alone, dW[o, i] = dbias[o] and dX = 0.
+// One workgroup per 64 outputs, four row strides, summed through LDS.
+__global__ void __launch_bounds__(256) k_cheby_bwd_const(BwdArgs P) {
+  __shared__ float sums[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int o = blockIdx.x * 64 + lane;
+  float s = 0.0f;
+  if (o < P.D_out)
+    for (int b = w; b < P.B; b += 4) s += P.dY[(long)b * P.D_out + o];
+  sums[w][lane] = s;
+  __syncthreads();
+  const int o_end = min(P.D_out, (int)(blockIdx.x + 1) * 64);
+  for (int q = blockIdx.x * 64 + w; q < o_end; q += 4) {
+    const int l = q - blockIdx.x * 64;
+    const float d = (sums[0][l] + sums[1][l]) + (sums[2][l] + sums[3][l]);
+    if (lane == 0 && P.db != nullptr) P.db[q] = d;
+    for (int i = lane; i < P.D_in; i += 64) P.dW[(long)q * P.D_in + i] = d;
+  }
+}
+
+__global__ void k_fill_zero(float* __restrict__ p, long n) {
+  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += (long)gridDim.x * blockDim.x) p[idx] = 0.0f;
+}
+
+int reduce_blocks(long n) { return (int)std::min<long>((n + 255) / 256, 8192); }
+
+// Contraction splits of a grid of `tiles` workgroups (one per CU at a time, 256
+// CUs): the fewest that leave the CUs busy -- a further split has to fill the
+// last round of workgroups at least 10 % better -- with at least two steps
+// each, and no more than the workspace holds.
+int choose_splits(long tiles, int steps, long max_by_ws) {
+  auto fill = [&](long s) { return (double)(tiles * s) / (double)((tiles * s + 255) / 256 * 256); };
+  const long smax = std::min<long>({64, steps / 2, max_by_ws});
+  long best = 1;
+  for (long s = 2; s <= smax; ++s)
+    if (fill(s) > 1.1 * fill(best)) best = s;
+  return (int)best;
+}
+
+struct BwdPlan {
+  int SG, MB, groups, NS;
+  int splits_w, splits_x;
+  size_t ws_floats;
+};
+
+// Workspace cap of the split partial sums (floats).
+constexpr size_t kBwdWsFloats = size_t(64) << 20;
+
+BwdPlan plan_backward(int B, int D_in, int D_out, int K, int has_base, bool may_split) {
+  BwdPlan p{};
+  p.NS = K - 1 + has_base;
+  p.groups = std::max(1, (p.NS + kBwdMaxSG - 1) / kBwdMaxSG);
+  p.SG = std::max(1, (p.NS + p.groups - 1) / p.groups);
+  p.MB = p.SG <= 5 ? 2 : 1;
+  const int M = 4 * p.MB * 32;
+  const long f_tiles = (D_in + kBwdF - 1) / kBwdF;
+  const long per_w = (long)D_out * ((long)p.NS * D_in + 1), per_x = (long)B * D_in;
+  const long cap = may_split ? (long)kBwdWsFloats : 0;
+  p.splits_w = choose_splits(((D_out + M - 1) / M) * f_tiles * p.groups, (B + kBwdStep - 1) / kBwdStep, cap / per_w);
+  p.splits_x = choose_splits(((B + M - 1) / M) * f_tiles, (D_out + kBwdStep - 1) / kBwdStep, cap / per_x);
+  p.ws_floats = std::max(p.splits_w > 1 ? (size_t)(per_w * p.splits_w) : 0,
+                         p.splits_x > 1 ? (size_t)(per_x * p.splits_x) : 0);
+  return p;
+}
+
+template <int SG, int MB>
+hipError_t launch_bwd(BwdArgs A, const BwdPlan& p, float* ws, hipStream_t st) {
+  constexpr int M = 4 * MB * 32;
+  A.groups = p.groups;
+  A.f_tiles = (A.D_in + kBwdF - 1) / kBwdF;
+  // dW: outputs x (slot, feature), contraction over the batch
+  BwdArgs W = A;
+  W.m_tiles = (A.D_out + M - 1) / M;
+  W.steps = (A.B + kBwdStep - 1) / kBwdStep;
+  W.steps_per_split = (W.steps + p.splits_w - 1) / p.splits_w;
+  const int splits_w = (W.steps + W.steps_per_split - 1) / W.steps_per_split;
+  W.part = splits_w > 1 ? ws : nullptr;
+  W.dbp = splits_w > 1 ? ws + (size_t)splits_w * A.D_out * A.NS * A.D_in : nullptr;
+  hipLaunchKernelGGL((k_cheby_bwd_dw<SG, MB>), dim3(W.m_tiles * A.f_tiles * A.groups, splits_w), dim3(kBwdThreads), 0,
+                     st, W);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const dim3 gx((B + kBwdO - 1) / kBwdO, (D_in + kBwdF - 1) / kBwdF);
-  hipLaunchKernelGGL((k_cheby_bwd_dx<KPM>), gx, dim3(kBwdThreads), 0, st, dY, X, W, Wb, dX, B, D_in, D_out, K,
-                     has_base);
-  return hipGetLastError();
+  if (splits_w > 1) {
+    hipLaunchKernelGGL(k_cheby_bwd_dw_reduce, dim3(reduce_blocks((long)A.D_out * A.NS * A.D_in)), dim3(256), 0, st, W,
+                       splits_w);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  // dX: batch rows x (slot, feature), contraction over the outputs
+  BwdArgs X = A;
+  X.m_tiles = (A.B + M - 1) / M;
+  X.steps = (A.D_out + kBwdStep - 1) / kBwdStep;
+  X.steps_per_split = (X.steps + p.splits_x - 1) / p.splits_x;
+  const int splits_x = (X.steps + X.steps_per_split - 1) / X.steps_per_split;
+  X.part = splits_x > 1 ? ws : nullptr;
+  X.vec = A.D_out % 4 == 0 && ((uintptr_t)A.dY & 15) == 0;
+  hipLaunchKernelGGL((k_cheby_bwd_dx<SG, MB>), dim3(X.m_tiles * A.f_tiles, splits_x), dim3(kBwdThreads), 0, st, X);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (splits_x > 1) {
+    const long n = (long)A.B * A.D_in;
+    hipLaunchKernelGGL(k_sum_splits, dim3(reduce_blocks(n)), dim3(256), 0, st, ws, A.dX, splits_x, n);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 }  // namespace
 
-// Slots per feature padded to the instantiated register tile.
-hipError_t launch_cheby_backward(const float* dY, const float* X, const float* W, const float* Wb, float* dW,
-                                 float* dWb, float* db, float* dX, int B, int D_in, int D_out, int K, int has_base,
-                                 hipStream_t st) {
-  const int KP = K + has_base;
-  if (KP <= 4) return launch_bwd<4>(dY, X, W, Wb, dW, dWb, db, dX, B, D_in, D_out, K, has_base, st);
-  if (KP <= 8) return launch_bwd<8>(dY, X, W, Wb, dW, dWb, db, dX, B, D_in, D_out, K, has_base, st);
-  if (KP <= 12) return launch_bwd<12>(dY, X, W, Wb, dW, dWb, db, dX, B, D_in, D_out, K, has_base, st);
-  if (KP <= 16) return launch_bwd<16>(dY, X, W, Wb, dW, dWb, db, dX, B, D_in, D_out, K, has_base, st);
-  if (KP <= 24) return launch_bwd<24>(dY, X, W, Wb, dW, dWb, db, dX, B, D_in, D_out, K, has_base, st);
-  return launch_bwd<36>(dY, X, W, Wb, dW, dWb, db, dX, B, D_in, D_out, K, has_base, st);
+// ws: p.ws_floats floats when the plan splits, else unused.
+static hipError_t launch_cheby_backward(const float* dY, const float* X, const float* W, const float* Wb, float* dW,
+                                        float* dWb, float* db, float* dX, int B, int D_in, int D_out, int K,
+                                        int has_base, const BwdPlan& p, float* ws, hipStream_t st) {
+  BwdArgs A{};
+  A.dY = dY; A.X = X; A.W = W; A.Wb = Wb;
+  A.dW = dW; A.dWb = dWb; A.db = db; A.dX = dX;
+  A.B = B; A.D_in = D_in; A.D_out = D_out; A.K = K; A.has_base = has_base; A.NS = p.NS;
+  if (p.NS == 0) {
+    hipLaunchKernelGGL(k_cheby_bwd_const, dim3((D_out + 63) / 64), dim3(256), 0, st, A);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const long n = (long)B * D_in;
+    hipLaunchKernelGGL(k_fill_zero, dim3(reduce_blocks(n)), dim3(256), 0, st, dX, n);
+    return hipGetLastError();
+  }
+  switch (p.SG) {
+    case 1: return launch_bwd<1, 2>(A, p, ws, st);
+    case 2: return launch_bwd<2, 2>(A, p, ws, st);
+    case 3: return launch_bwd<3, 2>(A, p, ws, st);
+    case 4: return launch_bwd<4, 2>(A, p, ws, st);
+    case 5: return launch_bwd<5, 2>(A, p, ws, st);
+    case 6: return launch_bwd<6, 1>(A, p, ws, st);
+    case 7: return launch_bwd<7, 1>(A, p, ws, st);
+    case 8: return launch_bwd<8, 1>(A, p, ws, st);
+    case 9: return launch_bwd<9, 1>(A, p, ws, st);
+    default: return launch_bwd<10, 1>(A, p, ws, st);
+  }
 }
 
 }  // namespace kans
@@ -262,6 +594,31 @@ using namespace kans;
 
 namespace {
 
+// The split partial sums of a backward: one workspace of at most kBwdWsFloats
+// floats, shared by all calls (library lock held).  A call on another stream
+// than the last one's waits on the device until that one has read its sums.
+DevBuf g_ws;
+hipEvent_t g_ws_done = nullptr;
+hipStream_t g_ws_stream = nullptr;
+
+int acquire_ws(size_t floats, hipStream_t st, float** ws) {
+  *ws = nullptr;
+  if (floats == 0) return 0;
+  if (!g_ws_done) HIP_TRY(hipEventCreateWithFlags(&g_ws_done, hipEventDisableTiming));
+  else if (g_ws_stream != st) HIP_TRY(hipStreamWaitEvent(st, g_ws_done, 0));
+  int rc = g_ws.reserve(floats * sizeof(float));  // growing frees the old one, which waits for the device
+  if (rc) return rc;
+  *ws = (float*)g_ws.p;
+  return 0;
+}
+
+int release_ws(size_t floats, hipStream_t st) {
+  if (floats == 0) return 0;
+  HIP_TRY(hipEventRecord(g_ws_done, st));
+  g_ws_stream = st;
+  return 0;
+}
+
 int check_bwd(const void* dY, const void* X, const void* W, const void* Wb, const void* dW, const void* dWb,
               const void* dX, int B, int D_in, int D_out, int K, int has_base, int has_bias) {
   if (!dY || !X || !W || !dW || !dX) return kans_fail(KANS_ERR_ARG, "null dY, X, W, dW or dX");
@@ -269,6 +626,9 @@ int check_bwd(const void* dY, const void* X, const void* W, const void* Wb, cons
     return kans_fail(KANS_ERR_ARG, "bad dims B=%d D_in=%d D_out=%d K=%d (1 <= K <= %d)", B, D_in, D_out, K, kMaxK);
   if ((has_base != 0 && has_base != 1) || (has_bias != 0 && has_bias != 1))
     return kans_fail(KANS_ERR_ARG, "has_base / has_bias must be 0 or 1");
+  // the dX kernel's lane offsets are 32 bits: 36 bytes a reduction index of W, 1 KB an output of dY
+  if ((long)D_in * K > (1L << 26) || D_out > (1 << 21))
+    return kans_fail(KANS_ERR_UNSUPPORTED, "D_in * K = %ld above 2^26 or D_out = %d above 2^21", (long)D_in * K, D_out);
   if (has_base && (!Wb || !dWb)) return kans_fail(KANS_ERR_ARG, "has_base=1 but W_base or dW_base is null");
   return 0;
 }
@@ -294,8 +654,12 @@ int backward_host(const float* dY, const float* X, const float* W, const float* 
   HIP_TRY(hipMemcpyAsync(d_X, X, nX * 4, hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemcpyAsync(d_W, W, nW * 4, hipMemcpyHostToDevice, st));
   if (has_base) HIP_TRY(hipMemcpyAsync(d_Wb, Wb, nWb * 4, hipMemcpyHostToDevice, st));
+  const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, true);
+  float* ws;
+  if ((rc = acquire_ws(plan.ws_floats, st, &ws))) return rc;
   HIP_TRY(launch_cheby_backward(d_dY, d_X, d_W, has_base ? d_Wb : nullptr, d_dW, has_base ? d_dWb : nullptr,
-                                has_bias ? d_db : nullptr, d_dX, B, D_in, D_out, K, has_base, st));
+                                has_bias ? d_db : nullptr, d_dX, B, D_in, D_out, K, has_base, plan, ws, st));
+  if ((rc = release_ws(plan.ws_floats, st))) return rc;
   HIP_TRY(hipMemcpyAsync(dW, d_dW, nW * 4, hipMemcpyDeviceToHost, st));
   if (has_base) HIP_TRY(hipMemcpyAsync(dWb, d_dWb, nWb * 4, hipMemcpyDeviceToHost, st));
   if (has_bias) HIP_TRY(hipMemcpyAsync(db, d_db, nb * 4, hipMemcpyDeviceToHost, st));
@@ -316,9 +680,15 @@ int kans_cheby_backward(const float* dY, const float* X, const float* W, const f
   std::lock_guard<std::mutex> lk(kans_mutex());
   if ((rc = kans_ensure_init())) return rc;
   hipStream_t st = stream ? (hipStream_t)stream : kans_default_stream();
+  // a call recorded into a graph outlives this one: it gets no share of the common workspace
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, cap == hipStreamCaptureStatusNone);
+  float* ws;
+  if ((rc = acquire_ws(plan.ws_floats, st, &ws))) return rc;
   HIP_TRY(launch_cheby_backward(dY, X, W, has_base ? W_base : nullptr, dW, has_base ? dW_base : nullptr,
-                                has_bias ? dbias : nullptr, dX, B, D_in, D_out, K, has_base, st));
-  return 0;
+                                has_bias ? dbias : nullptr, dX, B, D_in, D_out, K, has_base, plan, ws, st));
+  return release_ws(plan.ws_floats, st);
 }
 
 int metal_kan_cheby_backward_fused(const float* dY, const float* X, const float* W_cheby, const float* W_base,

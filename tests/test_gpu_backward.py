@@ -186,3 +186,76 @@ def test_layer_backward_shapes_and_dtypes(gpu):
     ref = O.cheby_backward(dYh, xh.astype(np.float32), h.w_cheby.astype(np.float32),
                            h.w_base.astype(np.float32), True)
     assert O.rel_err(dXh, ref[3]) <= 1e-4 and O.rel_err(h.grad_w_cheby, ref[0]) <= 1e-4
+
+
+# Edges of the backward kernels' tiles: 32-row tiles in workgroups of 128 (NS = K - 1 + base > 5 slots) or 256
+# rows, 64 features, 16-deep steps; slot counts 1..10 and several groups of them; grids that split the
+# contraction and (the last two) grids that fill the chip without; odd widths (no 16-byte rows of dY).
+EDGES = [(1, 1, 1, 2, 0), (16, 64, 256, 3, 0), (17, 65, 257, 4, 1), (33, 63, 129, 6, 0), (128, 32, 128, 7, 0),
+         (129, 96, 127, 7, 1), (250, 31, 31, 8, 1), (64, 64, 64, 9, 1), (40, 33, 48, 11, 0), (40, 70, 50, 12, 1),
+         (48, 20, 36, 22, 1), (31, 40, 20, 32, 1), (40, 2048, 2050, 2, 0), (2050, 2048, 20, 2, 0)]
+
+
+@pytest.mark.parametrize("B,D_in,D_out,K,base", EDGES)
+def test_backward_tile_edges(gpu, B, D_in, D_out, K, base):
+    dY, X, W, Wb = case(B + K, B, D_in, D_out, K, bool(base), True)
+    got = run_host(gpu, gpu.metal_kan_cheby_backward_fused, dY, X, W, Wb, True)
+    # fp32 sums of at most 2050 terms: 2^-24 * sqrt(2050) = 3e-6 of the largest gradient
+    check(got, O.cheby_backward(dY, X, W, Wb, True), 1e-5)
+
+
+def test_backward_wide_range_and_infinities(gpu):
+    """Operands of 1e-30 .. 1e30 keep fp32 accuracy (their bf16 terms have fp32's exponent range), and an
+    infinite upstream gradient makes exactly the gradients it enters non-finite."""
+    B, D_in, D_out, K = 48, 40, 30, 5
+    dY, X, W, Wb = case(3, B, D_in, D_out, K, True, True)
+    scale = np.float32(10.0) ** np.linspace(-30, 30, B).astype(np.float32)
+    dY *= scale[:, None]
+    dX = run_host(gpu, gpu.metal_kan_cheby_backward_fused, dY, X, W, Wb, True)[3]
+    ref = O.cheby_backward(dY, X, W, Wb, True)[3]
+    for b in range(B):   # every row at its own scale
+        assert O.rel_err(dX[b], ref[b]) <= 1e-5, b
+    dY, X, W, Wb = case(4, B, D_in, D_out, K, True, True)
+    dY[7, 11] = np.inf
+    dW, dWb, db, dX = run_host(gpu, gpu.metal_kan_cheby_backward_fused, dY, X, W, Wb, True)
+    for g in (dW, dWb):
+        assert not np.isfinite(g[11]).any() and np.isfinite(np.delete(g, 11, 0)).all()
+    assert db[11] == np.inf and np.isfinite(np.delete(db, 11)).all()
+    assert not np.isfinite(dX[7][np.abs(X[7]) <= 1]).any() and np.isfinite(np.delete(dX, 7, 0)).all()
+
+
+def test_backward_streams_and_capture(gpu):
+    """Calls that share the partial-sum workspace from two streams, and a call recorded into a graph (which
+    gets no workspace), give the gradients of a call alone."""
+    torch = pytest.importorskip("torch")
+    from metal_kans import device
+    B, D_in, D_out, K = 512, 64, 96, 5
+    arrs = [case(20 + n, B, D_in, D_out, K, True, True) for n in range(2)]
+    dev = [[torch.from_numpy(a).cuda() for a in c] for c in arrs]
+    outs = [[torch.zeros(s, device="cuda") for s in ((D_out, D_in * K), (D_out, D_in), (D_out,), (B, D_in))]
+            for _ in range(2)]
+
+    def call(n, stream):
+        p = [t.data_ptr() for t in dev[n] + outs[n]]
+        device.check(gpu.kans_cheby_backward(*p, B, D_in, D_out, K, 1, 1, stream.cuda_stream), "backward")
+
+    refs = [O.cheby_backward(*c, True) for c in arrs]
+    s = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        call(0, s[0])
+        call(1, s[1])
+    torch.cuda.synchronize()
+    for n in range(2):
+        check([t.cpu().numpy() for t in outs[n]], refs[n], 1e-5)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s[0]):
+        call(0, s[0])
+    for _ in range(3):
+        for t in outs[0]:
+            t.zero_()
+        call(1, s[1])
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        check([t.cpu().numpy() for t in outs[0]], refs[0], 1e-5)
