@@ -14,7 +14,7 @@ struct DenseLaunch {
   int x_dtype, y_dtype;  // element types of X and Y: dtype, or DT_F32
   const void* X; long ldx;
   const void* Wt; int nob_pad;
-  const void* bias;
+  const float* bias;    // [D_out] constant term per output (bias, folded T_0 coefficients) or null
   void* Y; long ldy;
   float* part;          // split workspace (splits * B * D_out floats) or null
   int B, D_in, D_out, nfb;
@@ -22,6 +22,19 @@ struct DenseLaunch {
   int wm, nb, splits;   // tile config
   int ks = 1;           // wave groups per workgroup (4-wave block kernel, block_wave_groups_ok)
   int pair = 1;         // block kernels: two feature blocks per LDS stage when they fit (kan_fused_block)
+};
+
+// A layer's weights on the device into the fused kernels' layout (kans_dense.hip): W / Wb / bias of
+// src_dtype (the layer dtype, or DT_F32 for a converting upload; Wb / bias may be null) into Wt and, when
+// bias_out is set, the constant term per output.
+struct WeightUpload {
+  int src_dtype, dtype;
+  const void *W, *Wb, *bias;
+  void* Wt;
+  float* bias_out;
+  int D_in, D_out, K, has_base;
+  int fold;             // T_0 coefficients go into bias_out (BasisParams::k0)
+  int nfb, nob_pad;
 };
 
 // RBF parameters (centres, scaled centres, recurrence eligibility) of bp (bp.K set) from K centres and

@@ -42,7 +42,7 @@ constexpr int kMaxK = 32;
 
 // Basis parameters passed by value to the fused kernels.
 struct BasisParams {
-  int K;              // basis functions per feature (excluding the SiLU base slot)
+  int K;              // basis functions contracted per feature (excluding the SiLU base slot)
   int grid_size;      // B-spline: number of intervals G (K = G + 3)
   float grid_min;     // B-spline: left end of the grid
   float inv_h;        // B-spline: G / (max - min)
@@ -61,6 +61,11 @@ struct BasisParams {
   int rbf_rec;
   float rec_lo, rec_hi;  // clamp of t: [-kRbfRecPad, (K-1)*d + kRbfRecPad]
   float rec_2d, rec_c, rec_q;  // 2d, -d^2, exp2(-2d^2)
+  // Chebyshev: degree of the first basis function contracted.  1 when the
+  // layer's T_0 coefficients are folded into its bias (T_0 = 1 for every input,
+  // so they only add the constant sum_i W[o, i*K]): one slot less per feature
+  // in every product.
+  int k0;
 };
 
 // Recurrence limits: t is clamped to kRbfRecPad beyond the outer centres,
@@ -124,16 +129,19 @@ template <int BASIS, int NV> struct BasisGen;
 // registers r0, r1 hold consecutive T's; a step of parity P emits r_P and
 // advances it by two degrees (r_P <- 2t r_{1-P} - r_P), so consecutive steps
 // alternate registers without any register rotation.  ``begin(.., swap)``
-// places T_0 in r1 instead of r0 when basis 0 is emitted at an odd step.
+// places the first one (degree BasisParams::k0) in r1 instead of r0 when it is
+// emitted at an odd step.
 template <int NV> struct BasisGen<BASIS_CHEBY, NV> {
   float tw[NV], r0[NV], r1[NV];
-  __device__ __forceinline__ void begin(const float* x, const BasisParams&, bool swap = false) {
+  __device__ __forceinline__ void begin(const float* x, const BasisParams& bp, bool swap = false) {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       float t = __builtin_fminf(__builtin_fmaxf(x[v], -1.0f), 1.0f);
       tw[v] = t + t;
-      r0[v] = swap ? t : 1.0f;
-      r1[v] = swap ? 1.0f : t;
+      const float a = bp.k0 ? t : 1.0f;                                 // T_k0
+      const float b = bp.k0 ? __builtin_fmaf(tw[v], t, -1.0f) : t;      // T_{k0+1}
+      r0[v] = swap ? b : a;
+      r1[v] = swap ? a : b;
     }
   }
   template <int P>
@@ -167,20 +175,22 @@ template <int NV> struct BasisGen<BASIS_CHEBY, NV> {
 // advances its register and then emits the fresh value: step<P> does
 // r_P <- 2t r_{1-P} - r_P and returns r_P, so the emitted value is the result
 // of the step's own fma and no copy of the previous value has to stay alive.
-// Before the first step the registers hold T_{-2} = T_2 = 2t^2 - 1 and
-// T_{-1} = T_1 = t (T_{-k} = T_k), which yields T_0 = 2t*t - (2t^2 - 1) and
-// T_1 = 2t*T_0 - t; both are within an fp32 rounding of 1 and t, far below
-// the 16-bit rounding of the MFMA operands this generator feeds.
+// Before the first step the registers hold T_{k0-2} and T_{k0-1}: T_{-1} =
+// T_1 = t and T_0 = 1 for k0 = 1 (T_1 = 2t*1 - t is exact); T_{-2} = T_2 =
+// 2t^2 - 1 and T_{-1} for k0 = 0, whose T_0 = 2t*t - (2t^2 - 1) is within an
+// fp32 rounding of 1, far below the 16-bit rounding of the MFMA operands this
+// generator feeds.
 template <int NV> struct BasisGen<BASIS_CHEBY_POST, NV> {
   float tw[NV], r0[NV], r1[NV];
-  __device__ __forceinline__ void begin(const float* x, const BasisParams&, bool swap = false) {
+  __device__ __forceinline__ void begin(const float* x, const BasisParams& bp, bool swap = false) {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const float t = __builtin_fminf(__builtin_fmaxf(x[v], -1.0f), 1.0f);
       tw[v] = t + t;
-      const float tm2 = __builtin_fmaf(tw[v], t, -1.0f);
-      r0[v] = swap ? t : tm2;
-      r1[v] = swap ? tm2 : t;
+      const float a = bp.k0 ? t : __builtin_fmaf(tw[v], t, -1.0f);  // T_{k0-2}
+      const float b = bp.k0 ? 1.0f : t;                             // T_{k0-1}
+      r0[v] = swap ? b : a;
+      r1[v] = swap ? a : b;
     }
   }
   template <int P>

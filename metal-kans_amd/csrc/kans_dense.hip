@@ -50,7 +50,7 @@ template <typename T, typename TX, typename TY, int BASIS, int WM, int NB>
 __global__ void __launch_bounds__(kThreads, 2)
 kan_fused_dense(const TX* __restrict__ X, long ldx,
                 const uint4* __restrict__ Wt, int nob_pad,
-                const T* __restrict__ bias,
+                const float* __restrict__ bias,
                 TY* __restrict__ Y, long ldy,
                 float* __restrict__ Ypart,
                 int B, int D_in, int D_out, int m_tiles, int n_tiles,
@@ -278,7 +278,10 @@ kan_fused_dense(const TX* __restrict__ X, long ldx,
             if (rbase + dr < B) out[(long)dr * D_out] = acc[rb][nb][r];
           }
       } else {
-        const float bcol = bias != nullptr ? to_f32(bias[col]) : 0.0f;
+        // waited for here, once: left to the stores, each one's row test brought a wait for the
+        // load and with it for every store before (3 % of the 16384 x 1024 -> 1024 RBF kernel)
+        float bcol = bias != nullptr ? bias[col] : 0.0f;
+        asm volatile("" : "+v"(bcol));
         TY* out = Y + (long)rbase * ldy + col;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
@@ -369,7 +372,7 @@ template <typename T, typename TX, typename TY, int BASIS, int WM, int NB, int W
 __global__ void __launch_bounds__(WAVES * 64 * KS, block_min_wgs(WAVES, NB, KS))
 kan_fused_block(const TX* __restrict__ X, long ldx,
                 const uint4* __restrict__ Wt, int nob_pad,
-                const T* __restrict__ bias,
+                const float* __restrict__ bias,
                 TY* __restrict__ Y, long ldy,
                 float* __restrict__ Ypart,
                 int B, int D_in, int D_out, int m_tiles, int n_tiles,
@@ -770,7 +773,10 @@ kan_fused_block(const TX* __restrict__ X, long ldx,
             if (rbase + dr < B) out[(long)dr * D_out] = acc[rb][nb][r];
           }
       } else {
-        const float bcol = bias != nullptr ? to_f32(bias[col]) : 0.0f;
+        // waited for here, once: left to the stores, each one's row test brought a wait for the
+        // load and with it for every store before (3 % of the 16384 x 1024 -> 1024 RBF kernel)
+        float bcol = bias != nullptr ? bias[col] : 0.0f;
+        asm volatile("" : "+v"(bcol));
         TY* out = Y + (long)rbase * ldy + col;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
@@ -789,13 +795,13 @@ kan_fused_block(const TX* __restrict__ X, long ldx,
 }
 
 // Split reduction: y = sum_split part[split] + bias, converted to T.
-template <typename T, typename TY>
-__global__ void kan_split_finalize(const float* __restrict__ part, int splits, const T* __restrict__ bias,
+template <typename TY>
+__global__ void kan_split_finalize(const float* __restrict__ part, int splits, const float* __restrict__ bias,
                                    TY* __restrict__ Y, long ldy, int B, int D_out) {
   long n = (long)B * D_out;
   for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += (long)gridDim.x * blockDim.x) {
     int row = (int)(idx / D_out), col = (int)(idx - (long)row * D_out);
-    float s = bias ? to_f32(bias[col]) : 0.0f;
+    float s = bias ? bias[col] : 0.0f;
     // splits in order, loaded 8 at a time: one memory round trip per 8
     // splits instead of one per split
     for (int k0 = 0; k0 < splits; k0 += 8) {
@@ -813,8 +819,8 @@ __global__ void kan_split_finalize(const float* __restrict__ part, int splits, c
 // The same reduction for 4 consecutive columns per thread (D_out and ldy
 // multiples of 4, Y aligned to 4 elements): 16-byte partial loads and one
 // vector store, the same sum order per element.
-template <typename T, typename TY>
-__global__ void kan_split_finalize4(const float4* __restrict__ part, int splits, const T* __restrict__ bias,
+template <typename TY>
+__global__ void kan_split_finalize4(const float4* __restrict__ part, int splits, const float* __restrict__ bias,
                                     TY* __restrict__ Y, long ldy, int B, int D_out) {
   const long n4 = (long)B * D_out / 4;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (long)gridDim.x * blockDim.x) {
@@ -822,7 +828,7 @@ __global__ void kan_split_finalize4(const float4* __restrict__ part, int splits,
     const int row = (int)(idx / D_out), col = (int)(idx - (long)row * D_out);
     float s[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s[j] = bias ? to_f32(bias[col + j]) : 0.0f;
+    for (int j = 0; j < 4; ++j) s[j] = bias ? bias[col + j] : 0.0f;
     for (int k0 = 0; k0 < splits; k0 += 8) {
       float4 v[8];
 #pragma unroll
@@ -853,42 +859,69 @@ __global__ void kan_split_finalize4(const float4* __restrict__ part, int splits,
 // Repack raw weights W[D_out][D_in*K] (k fastest) and W_base[D_out][D_in], of
 // element type S, into the tiled layout W'[fb][s][ob][chunk][lane][e] of type T
 // (see kans_common.h), converting S -> T with round-to-nearest-even; zero
-// padding for o >= D_out and i >= D_in.
+// padding for o >= D_out and i >= D_in.  Slot s >= has_base holds coefficient
+// k = s - has_base + k0.
+//
+// One workgroup per (16 outputs, 16-feature block): its 16 row segments of 16 K
+// consecutive weights are read whole into LDS and written from there, a half
+// wave per slot (reading each slot straight from memory takes one value per
+// K-value stretch of a row and lane).  A training step repacks its weights on
+// every forward.
 template <typename S, typename T>
-__global__ void kan_repack_weights(const S* __restrict__ W, const S* __restrict__ Wb, uint4* __restrict__ Wt,
-                                   int D_in, int D_out, int K, int has_base, int nfb, int nob_pad) {
+__global__ void __launch_bounds__(256)
+kan_repack_weights(const S* __restrict__ W, const S* __restrict__ Wb, uint4* __restrict__ Wt,
+                   int D_in, int D_out, int K, int k0, int has_base, int nob_pad) {
   constexpr int CPL = Chunks<T>::CPL;
   constexpr int EPC = 16 / (int)sizeof(T);
-  const int KP = K + has_base;
-  const long total = (long)nfb * KP * nob_pad * CPL * 64;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
-    long r = idx;
-    const int lane = (int)(r % 64); r /= 64;
-    const int chunk = (int)(r % CPL); r /= CPL;
-    const int ob = (int)(r % nob_pad); r /= nob_pad;
-    const int s = (int)(r % KP); r /= KP;
-    const int fb = (int)r;
-    const int o = ob * 32 + (lane & 31);
-    const int ibase = fb * 16 + 8 * (lane >> 5) + chunk * EPC;
-    T vals[EPC];
+  extern __shared__ float seg[];  // [16][row]: 16 K coefficients, then 16 base weights
+  const int row = 16 * (K + has_base) + 1;  // odd: a column of rows spreads over the banks
+  const int ob = blockIdx.x >> 1, o_half = 16 * (blockIdx.x & 1), fb = blockIdx.y;
+  const int i0 = fb * 16, ni = min(16, D_in - i0);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int r = wave; r < 16; r += 4) {
+    const int o = ob * 32 + o_half + r;
+    for (int j = lane; j < 16 * K; j += 64)
+      seg[r * row + j] = o < D_out && j < ni * K ? to_f32(W[(long)o * D_in * K + (long)i0 * K + j]) : 0.0f;
+    if (has_base && lane < 16)
+      seg[r * row + 16 * K + lane] = o < D_out && lane < ni ? to_f32(Wb[(long)o * D_in + i0 + lane]) : 0.0f;
+  }
+  __syncthreads();
+  const int KP = K - k0 + has_base;
+  const int r = lane & 15, f0 = 8 * ((lane >> 4) & 1);
+  const float* src = seg + r * row;
+  const int dst_lane = o_half + r + 32 * ((lane >> 4) & 1);
+  for (int s = 2 * wave + (lane >> 5); s < KP; s += 8) {
+    const bool base = has_base && s == 0;
+    uint4* dst = Wt + (((long)fb * KP + s) * nob_pad + ob) * (64 * CPL) + dst_lane;
 #pragma unroll
-    for (int e = 0; e < EPC; ++e) {
-      const int i = ibase + e;
-      float w = 0.0f;
-      if (o < D_out && i < D_in) {
-        if (has_base && s == 0) w = to_f32(Wb[(long)o * D_in + i]);
-        else w = to_f32(W[((long)o * D_in + i) * K + (s - has_base)]);
+    for (int c = 0; c < CPL; ++c) {
+      T vals[EPC];
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) {
+        const int f = f0 + c * EPC + e;
+        vals[e] = from_f32<T>(src[base ? 16 * K + f : f * K + s - has_base + k0]);
       }
-      vals[e] = from_f32<T>(w);
+      uint4 u;
+      __builtin_memcpy(&u, vals, 16);
+      dst[c * 64] = u;
     }
-    Wt[idx] = *reinterpret_cast<uint4*>(vals);
   }
 }
 
+// The layer's constant term per output in fp32: bias[o] and, with fold, the T_0
+// coefficients sum_i W[o, i*K] (all rounded to the layer type T first, as the
+// products take them; summed in fp64).  One wave per output.
 template <typename S, typename T>
-__global__ void kan_convert(const S* __restrict__ src, T* __restrict__ dst, long n) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    dst[i] = from_f32<T>(to_f32(src[i]));
+__global__ void __launch_bounds__(256)
+kan_fold_bias(const S* __restrict__ W, const S* __restrict__ bias, float* __restrict__ out, int D_in, int D_out,
+              int K, int fold) {
+  const int o = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (o >= D_out) return;
+  double s = 0.0;
+  if (fold)
+    for (int i = lane; i < D_in; i += 64) s += (double)to_f32(from_f32<T>(to_f32(W[((long)o * D_in + i) * K])));
+  for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
+  if (lane == 0) out[o] = (float)(s + (bias ? (double)to_f32(from_f32<T>(to_f32(bias[o]))) : 0.0));
 }
 
 // ---------------------------------------------------------------------------
@@ -920,7 +953,7 @@ static hipError_t launch_dense_t(const DenseLaunch& L, hipStream_t st) {
       auto go = [&](auto KSC) {
         constexpr int KS = decltype(KSC)::value;
         hipLaunchKernelGGL((kan_fused_block<T, TX, TY, BB, WM, NB, 4, KS>), grid, dim3(256 * KS), 0, st,
-                           (const TX*)L.X, L.ldx, (const uint4*)L.Wt, L.nob_pad, (const T*)L.bias, (TY*)L.Y, L.ldy,
+                           (const TX*)L.X, L.ldx, (const uint4*)L.Wt, L.nob_pad, L.bias, (TY*)L.Y, L.ldy,
                            part, L.B, L.D_in, L.D_out, m_tiles, n_tiles, L.nfb, fbps, L.has_base, L.bp);
       };
       // wave groups (block_wave_groups_ok): 2 on (32,1) and (32,4), 4 on (32,1)
@@ -943,7 +976,7 @@ static hipError_t launch_dense_t(const DenseLaunch& L, hipStream_t st) {
         auto launch = [&](auto PC) {
           hipLaunchKernelGGL((kan_fused_block<T, TX, TY, BB, WM, NB, 8, 1, decltype(PC)::value>),
                              dim3(m_tiles8 * n_tiles, splits), dim3(512), 0, st, (const TX*)L.X, L.ldx,
-                             (const uint4*)L.Wt, L.nob_pad, (const T*)L.bias, (TY*)L.Y, L.ldy, part, L.B, L.D_in,
+                             (const uint4*)L.Wt, L.nob_pad, L.bias, (TY*)L.Y, L.ldy, part, L.B, L.D_in,
                              L.D_out, m_tiles8, n_tiles, L.nfb, fbps, L.has_base, L.bp);
         };
         // two feature blocks per LDS stage (Chebyshev, K + has_base <= 5)
@@ -970,7 +1003,7 @@ static hipError_t launch_dense_t(const DenseLaunch& L, hipStream_t st) {
     }
   } else {
     hipLaunchKernelGGL((kan_fused_dense<T, TX, TY, BASIS, WM, NB>), grid, dim3(kThreads), 0, st, (const TX*)L.X,
-                       L.ldx, (const uint4*)L.Wt, L.nob_pad, (const T*)L.bias, (TY*)L.Y, L.ldy, part, L.B, L.D_in,
+                       L.ldx, (const uint4*)L.Wt, L.nob_pad, L.bias, (TY*)L.Y, L.ldy, part, L.B, L.D_in,
                        L.D_out, m_tiles, n_tiles, L.nfb, fbps, L.has_base, L.bp);
   }
   hipError_t e = hipGetLastError();
@@ -979,12 +1012,12 @@ static hipError_t launch_dense_t(const DenseLaunch& L, hipStream_t st) {
     const long n = (long)L.B * L.D_out;
     if (L.D_out % 4 == 0 && L.ldy % 4 == 0 && ((uintptr_t)L.Y % (4 * sizeof(TY))) == 0) {
       const int blocks = (int)std::min<long>((n / 4 + 255) / 256, 4096);
-      hipLaunchKernelGGL((kan_split_finalize4<T, TY>), dim3(blocks), dim3(256), 0, st, (const float4*)part, splits,
-                         (const T*)L.bias, (TY*)L.Y, L.ldy, L.B, L.D_out);
+      hipLaunchKernelGGL((kan_split_finalize4<TY>), dim3(blocks), dim3(256), 0, st, (const float4*)part, splits,
+                         L.bias, (TY*)L.Y, L.ldy, L.B, L.D_out);
     } else {
       const int blocks = (int)std::min<long>((n + 255) / 256, 4096);
-      hipLaunchKernelGGL((kan_split_finalize<T, TY>), dim3(blocks), dim3(256), 0, st, part, splits,
-                         (const T*)L.bias, (TY*)L.Y, L.ldy, L.B, L.D_out);
+      hipLaunchKernelGGL((kan_split_finalize<TY>), dim3(blocks), dim3(256), 0, st, part, splits,
+                         L.bias, (TY*)L.Y, L.ldy, L.B, L.D_out);
     }
     e = hipGetLastError();
   }
@@ -1056,44 +1089,31 @@ hipError_t launch_dense(const DenseLaunch& L, hipStream_t st) {
 }
 
 template <typename S, typename T>
-static hipError_t repack_t(const void* W, const void* Wb, void* Wt, int D_in, int D_out, int K, int has_base,
-                           int nfb, int nob_pad, hipStream_t st) {
-  const int KP = K + has_base;
-  long total = (long)nfb * KP * nob_pad * Chunks<T>::CPL * 64;
-  int blocks = (int)std::min<long>((total + 255) / 256, 16384);
-  hipLaunchKernelGGL((kan_repack_weights<S, T>), dim3(blocks), dim3(256), 0, st, (const S*)W, (const S*)Wb,
-                     (uint4*)Wt, D_in, D_out, K, has_base, nfb, nob_pad);
+static hipError_t upload_t(const WeightUpload& U, hipStream_t st) {
+  const size_t lds = (size_t)16 * (16 * (U.K + U.has_base) + 1) * sizeof(float);
+  hipLaunchKernelGGL((kan_repack_weights<S, T>), dim3(2 * U.nob_pad, U.nfb), dim3(256), lds, st, (const S*)U.W,
+                     (const S*)U.Wb, (uint4*)U.Wt, U.D_in, U.D_out, U.K, U.fold, U.has_base, U.nob_pad);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || U.bias_out == nullptr) return e;
+  hipLaunchKernelGGL((kan_fold_bias<S, T>), dim3((U.D_out + 3) / 4), dim3(256), 0, st, (const S*)U.W,
+                     (const S*)U.bias, U.bias_out, U.D_in, U.D_out, U.K, U.fold);
   return hipGetLastError();
 }
 
-// src_dtype: element type of W / Wb (same as dtype, or DT_F32 for a converting upload).
-hipError_t launch_repack(int src_dtype, int dtype, const void* W, const void* Wb, void* Wt, int D_in, int D_out,
-                         int K, int has_base, int nfb, int nob_pad, hipStream_t st) {
-  if (src_dtype == dtype) {
-    switch (dtype) {
-      case DT_F16: return repack_t<_Float16, _Float16>(W, Wb, Wt, D_in, D_out, K, has_base, nfb, nob_pad, st);
-      case DT_BF16: return repack_t<__bf16, __bf16>(W, Wb, Wt, D_in, D_out, K, has_base, nfb, nob_pad, st);
-      default: return repack_t<float, float>(W, Wb, Wt, D_in, D_out, K, has_base, nfb, nob_pad, st);
+hipError_t launch_upload(const WeightUpload& U, hipStream_t st) {
+  if (U.src_dtype == U.dtype) {
+    switch (U.dtype) {
+      case DT_F16: return upload_t<_Float16, _Float16>(U, st);
+      case DT_BF16: return upload_t<__bf16, __bf16>(U, st);
+      default: return upload_t<float, float>(U, st);
     }
   }
-  if (src_dtype != DT_F32) return hipErrorInvalidValue;
-  switch (dtype) {
-    case DT_F16: return repack_t<float, _Float16>(W, Wb, Wt, D_in, D_out, K, has_base, nfb, nob_pad, st);
-    case DT_BF16: return repack_t<float, __bf16>(W, Wb, Wt, D_in, D_out, K, has_base, nfb, nob_pad, st);
+  if (U.src_dtype != DT_F32) return hipErrorInvalidValue;
+  switch (U.dtype) {
+    case DT_F16: return upload_t<float, _Float16>(U, st);
+    case DT_BF16: return upload_t<float, __bf16>(U, st);
     default: return hipErrorInvalidValue;
   }
-}
-
-hipError_t launch_convert(int src_dtype, int dtype, const void* src, void* dst, long n, hipStream_t st) {
-  int blocks = (int)std::min<long>((n + 255) / 256, 4096);
-  if (src_dtype != DT_F32 || dtype == DT_F32) return hipErrorInvalidValue;
-  if (dtype == DT_F16)
-    hipLaunchKernelGGL((kan_convert<float, _Float16>), dim3(blocks), dim3(256), 0, st, (const float*)src,
-                       (_Float16*)dst, n);
-  else
-    hipLaunchKernelGGL((kan_convert<float, __bf16>), dim3(blocks), dim3(256), 0, st, (const float*)src,
-                       (__bf16*)dst, n);
-  return hipGetLastError();
 }
 
 }  // namespace kans

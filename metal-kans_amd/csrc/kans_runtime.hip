@@ -40,9 +40,7 @@ hipError_t launch_dense(const DenseLaunch& L, hipStream_t st);
 bool dense_config_supported(int wm, int nb);
 bool block_wave_groups_ok(int wm, int nb, int ks);
 int block_waves(bool half, int basis, int wm, int nb, int KP);
-hipError_t launch_repack(int src_dtype, int dtype, const void* W, const void* Wb, void* Wt, int D_in, int D_out,
-                         int K, int has_base, int nfb, int nob_pad, hipStream_t st);
-hipError_t launch_convert(int src_dtype, int dtype, const void* src, void* dst, long n, hipStream_t st);
+hipError_t launch_upload(const WeightUpload& U, hipStream_t st);
 }  // namespace kans
 
 // ---------------------------------------------------------------------------
@@ -124,6 +122,7 @@ static size_t dtype_size(int dt) { return dt == DT_F32 ? 4 : 2; }
 struct kans_layer {
   int basis, dtype, D_in, D_out, K, has_base, has_bias;
   int D_in8, nfb, nob_pad;
+  int fold, slots;  // T_0 folded into the bias (BasisParams::k0); contracted slots per feature
   BasisParams bp{};
   DevBuf Wt, bias_d, part, x_d, y_d, raw_w, raw_wb;
   bool have_weights = false;
@@ -177,6 +176,18 @@ bool kans::kans_set_rbf_params(BasisParams& bp, const float* centers, float inv_
   return true;
 }
 
+// Sizes that follow from basis, D_in, D_out, K and has_base.
+static void layer_shape(kans_layer* L) {
+  L->D_in8 = round_up(L->D_in, 8);
+  L->nfb = (L->D_in + 15) / 16;
+  L->nob_pad = round_up((L->D_out + 31) / 32, kObPad);
+  // a T_0-only layer without a base branch keeps its one slot
+  L->fold = L->basis == BASIS_CHEBY && L->K + L->has_base > 1;
+  L->slots = L->K - L->fold + L->has_base;
+  L->bp.K = L->K - L->fold;
+  L->bp.k0 = L->fold;
+}
+
 static int validate_dims(int basis, int dtype, int D_in, int D_out, int K, int has_base, int has_bias) {
   if (basis < 0 || basis > 2) return kans_fail(KANS_ERR_ARG, "unknown basis %d", basis);
   if (dtype < 0 || dtype > 2) return kans_fail(KANS_ERR_ARG, "unknown dtype %d", dtype);
@@ -206,10 +217,7 @@ int kans_layer_create(int basis, int dtype, int D_in, int D_out, int K, int has_
   L->K = K;
   L->has_base = has_base;
   L->has_bias = has_bias;
-  L->D_in8 = round_up(D_in, 8);
-  L->nfb = (D_in + 15) / 16;
-  L->nob_pad = round_up((D_out + 31) / 32, kObPad);
-  L->bp.K = K;
+  layer_shape(L);
   *out = L;
   return 0;
 }
@@ -287,8 +295,7 @@ static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, con
   const size_t es = dtype_size(src_dtype);
   const size_t wbytes = (size_t)L->D_out * L->D_in * L->K * es;
   const size_t wbbytes = (size_t)L->D_out * L->D_in * es;
-  const int KP = L->K + L->has_base;
-  const size_t tbytes = (size_t)L->nfb * KP * L->nob_pad * 64 * 16 * (L->dtype == DT_F32 ? 2 : 1);
+  const size_t tbytes = (size_t)L->nfb * L->slots * L->nob_pad * 64 * 16 * (L->dtype == DT_F32 ? 2 : 1);
   int rc;
   void* old_wt = L->Wt.p;
   void* old_bias = L->bias_d.p;
@@ -311,17 +318,25 @@ static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, con
       wb_src = L->raw_wb.p;
     }
   }
-  HIP_TRY(launch_repack(src_dtype, L->dtype, w_src, L->has_base ? wb_src : nullptr, L->Wt.p, L->D_in, L->D_out,
-                        L->K, L->has_base, L->nfb, L->nob_pad, g_stream));
-  if (L->has_bias) {
-    const size_t bbytes = (size_t)L->D_out * dtype_size(L->dtype);
-    if ((rc = L->bias_d.reserve(bbytes))) return rc;
-    if (src_dtype == L->dtype) {
-      HIP_TRY(hipMemcpyAsync(L->bias_d.p, b_src, bbytes, hipMemcpyDeviceToDevice, g_stream));
-    } else {
-      HIP_TRY(launch_convert(src_dtype, L->dtype, b_src, L->bias_d.p, L->D_out, g_stream));
-    }
+  WeightUpload U{};
+  U.src_dtype = src_dtype;
+  U.dtype = L->dtype;
+  U.W = w_src;
+  U.Wb = L->has_base ? wb_src : nullptr;
+  U.bias = L->has_bias ? b_src : nullptr;
+  U.Wt = L->Wt.p;
+  U.D_in = L->D_in;
+  U.D_out = L->D_out;
+  U.K = L->K;
+  U.has_base = L->has_base;
+  U.fold = L->fold;
+  U.nfb = L->nfb;
+  U.nob_pad = L->nob_pad;
+  if (L->has_bias || L->fold) {
+    if ((rc = L->bias_d.reserve((size_t)L->D_out * sizeof(float)))) return rc;
+    U.bias_out = (float*)L->bias_d.p;
   }
+  HIP_TRY(launch_upload(U, g_stream));
   HIP_TRY(hipStreamSynchronize(g_stream));
   if (L->Wt.p != old_wt || L->bias_d.p != old_bias) ++L->gen;
   L->have_weights = true;
@@ -375,7 +390,7 @@ static void choose_tiling(const kans_layer* L, int B, int* wm, int* nb, int* spl
   const bool f32 = L->dtype == DT_F32;
   const int(*cand)[2] = (f32 && L->basis != BASIS_BSPLINE) ? pref_n4 : pref_n8;
   const int nob = (L->D_out + 31) / 32;
-  const int KP = L->K + L->has_base;
+  const int KP = L->slots;
   // workgroups of shape (ww, nn): the 8-wave block kernel's tile is 8 row blocks tall
   auto waves_of = [&](int ww, int nn) { return block_waves(!f32, L->basis, ww, nn, KP) == 8 ? 8 : 4; };
   auto wgs = [&](int ww, int nn) {
@@ -429,7 +444,7 @@ static void choose_tiling(const kans_layer* L, int B, int* wm, int* nb, int* spl
 // tile keeps one group unless the groups are forced too; a forced count that
 // the tile is not instantiated with falls back to 1.
 static int choose_wave_groups(const kans_layer* L, int B, int wm, int nb, int splits) {
-  if (block_waves(L->dtype != DT_F32, L->basis, wm, nb, L->K + L->has_base) != 4) return 1;
+  if (block_waves(L->dtype != DT_F32, L->basis, wm, nb, L->slots) != 4) return 1;
   if (L->forced_ks) return block_wave_groups_ok(wm, nb, L->forced_ks) ? L->forced_ks : 1;
   if (L->forced_wm) return 1;
   const long wgs = (long)((B + 4 * wm - 1) / (4 * wm)) * (((L->D_out + 31) / 32 + nb - 1) / nb) * splits;
@@ -484,7 +499,7 @@ static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, 
   D.ldx = ldx;
   D.Wt = L->Wt.p;
   D.nob_pad = L->nob_pad;
-  D.bias = L->has_bias ? L->bias_d.p : nullptr;
+  D.bias = L->has_bias || L->fold ? (const float*)L->bias_d.p : nullptr;
   D.Y = Y;
   D.ldy = ldy;
   D.B = B;
@@ -691,11 +706,11 @@ static int layer_kernel_name(const kans_layer* L, int B, bool io, int x_dtype, i
   choose_tiling(L, B, &wm, &nb, &splits);
   static const char* dt[] = {"float", "_Float16", "__bf16"};
   static const char* bs[] = {"BASIS_CHEBY", "BASIS_RBF", "BASIS_BSPLINE"};
-  const int waves = block_waves(L->dtype != DT_F32, L->basis, wm, nb, L->K + L->has_base);
+  const int waves = block_waves(L->dtype != DT_F32, L->basis, wm, nb, L->slots);
   const int ks = choose_wave_groups(L, B, wm, nb, splits);
   char groups[32] = "";
   if (ks > 1) snprintf(groups, sizeof groups, " x %d groups", ks);
-  const bool pairs = waves == 8 && L->basis == BASIS_CHEBY && L->block_pairs && 2 * (L->K + L->has_base) <= 10;
+  const bool pairs = waves == 8 && L->basis == BASIS_CHEBY && L->block_pairs && 2 * L->slots <= 10;
   char types[64];
   if (io)
     snprintf(types, sizeof types, "%s, %s, %s", dt[L->dtype], dt[x_dtype == DT_F32 ? DT_F32 : L->dtype],
@@ -891,10 +906,7 @@ static int sig_layer(int basis, int dtype, int D_in, int D_out, int K, int has_b
   L->K = K;
   L->has_base = has_base;
   L->has_bias = has_bias;
-  L->D_in8 = round_up(D_in, 8);
-  L->nfb = (D_in + 15) / 16;
-  L->nob_pad = round_up((D_out + 31) / 32, kObPad);
-  L->bp.K = K;
+  layer_shape(L.get());
   if (basis == BASIS_RBF) {
     for (int k = 0; k < K; ++k) L->bp.centers[k] = params[k];
     L->bp.have_centers = 1;
@@ -1341,10 +1353,7 @@ int metal_kan_chain_pipeline_cheby(const float* X, float* Y, int B, int num_laye
         L->K = degrees[l];
         L->has_base = key[5 * l + 3];
         L->has_bias = key[5 * l + 4];
-        L->D_in8 = round_up(L->D_in, 8);
-        L->nfb = (L->D_in + 15) / 16;
-        L->nob_pad = round_up((L->D_out + 31) / 32, kObPad);
-        L->bp.K = L->K;
+        layer_shape(L.get());
         ch->layers.push_back(L.get());
         ch->owned.push_back(std::move(L));
       }

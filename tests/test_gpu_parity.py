@@ -836,3 +836,26 @@ def test_gated_kan_dense_block_async(gpu):
         mk.set_async(False)
     for a, b in zip(outs, sync):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("K,base", [(1, True), (1, False), (2, False), (3, True), (32, True)])
+@pytest.mark.parametrize("d_in,d_out", [(1, 1), (15, 17), (17, 15), (40, 33), (129, 16)])
+def test_cheby_constant_coefficients(gpu, dtype, K, base, d_in, d_out):
+    """T_0 = 1: a Chebyshev layer's k = 0 coefficients reach the output through its constant term.  Layers
+    with only those coefficients (and a bias) give sum_i W[o, i*K] + bias[o] for every input, and with all
+    coefficients the oracle's output; sizes around the 16-output, 16-feature blocks of the re-tiling."""
+    import metal_kans as mk
+    L = make_layer(mk, "cheby", d_in, d_out, K, bias=True, base=base, seed=41)
+    x = np.random.default_rng(4).uniform(-1.2, 1.2, (37, d_in)).astype(np.float32)
+    assert O.rel_err(cast(L, dtype)(x), oracle_of(L, x)) <= TOL[dtype]
+    w = np.zeros_like(L.w_cheby)
+    w[:, ::K] = L.w_cheby[:, ::K]
+    L.w_cheby = w
+    if base:
+        L.w_base = np.zeros_like(L.w_base)
+    const = w.astype(np.float64).sum(1) + np.asarray(L.bias, np.float64)
+    y = np.asarray(L(x), np.float64)
+    # summed in more than fp32 and rounded once, to the output type (2^-24, 2^-11, 2^-8)
+    eps = {"float32": 2.0 ** -24, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[dtype]
+    assert np.all(np.abs(y - const) <= eps * np.abs(const) + 1e-7 * np.abs(w).sum(1))
