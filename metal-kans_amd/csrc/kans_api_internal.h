@@ -33,6 +33,7 @@ struct WeightUpload {
   void* Wt;
   float* bias_out;
   int D_in, D_out, K, has_base;
+  int sparse;           // layout of kan_fused_split_sparse (fp32 B-spline)
   int fold;             // T_0 coefficients go into bias_out (BasisParams::k0)
   int nfb, nob_pad;
 };

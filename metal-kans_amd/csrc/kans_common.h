@@ -92,6 +92,17 @@ constexpr float kRbfRecSpan = 6.0f;
 // so a lane's 16-byte chunk is exactly its MFMA B-operand for that slot, and one
 // (fb, s) step of an N-tile of NB output blocks is NB contiguous KB-sized tiles.
 // ---------------------------------------------------------------------------
+// fp32 B-spline layers with K >= 5 (kan_fused_split_sparse): of 8 consecutive
+// basis functions at most 4 consecutive ones are non-zero for an input, one of
+// each residue mod 4, so the groups {2P, 2P+4, 2P+1, 2P+5} (P = 0, 1) of a
+// block of 8 hold at most two: the 4:2 sparsity of the sparse MFMA.  After the
+// base slot their W' holds kSparseSteps steps per block of 8 functions (K
+// padded to a multiple of 8), each of two slots' size:
+//   step (m, P, fh), element j = 0..15 of lane l (column l%32, hb = l/32):
+//     function 8m + 2P + 4(j%2) + (j/2)%2,  feature 8(j/8) + 4fh + 2hb + (j/4)%2
+constexpr int kSparseSteps = 4;
+__host__ __device__ inline int sparse_blocks(int K) { return (K + 7) / 8; }
+
 constexpr int kObPad = 8;  // output blocks padded to a multiple of 8 (max NB)
 
 __host__ __device__ inline int round_up(int a, int b) { return (a + b - 1) / b * b; }

@@ -18,8 +18,8 @@
 //     them straight into the MFMA A-fragment;
 //   * the B-fragments come from LDS, filled from the pre-tiled weights (one
 //     (fb, s) step of an N-tile is NB contiguous KB);
-//   * fp16 / bf16 use v_mfma_f32_32x32x16_{f16,bf16}; fp32 uses
-//     v_mfma_f32_32x32x2_f32 eight times per step.  Accumulation is fp32.
+//   * v_mfma_f32_32x32x16_{f16,bf16}, fp32 accumulation (fp32 layers:
+//     kan_fused_split, kans_dense_split.hip);
 //   * an optional split over feature blocks writes fp32 partials that a finalize
 //     kernel reduces (used when the output tile count alone cannot fill the GPU);
 //     the 4-wave block kernel can also split a tile's feature blocks over KS
@@ -30,10 +30,11 @@
 //                    B-spline with K+base <= 9 on the 256 x 256 tile (8 waves):
 //                    one barrier per feature block, global->LDS DMA of the next
 //                    block's weights, basis generation interleaved with the MFMAs;
-//   kan_fused_dense  everything else (fp32, other tiles, larger K): one
-//                    barrier per slot, register-staged weights.
+//   kan_fused_dense  the other 16-bit tiles and larger K: one barrier per slot,
+//                    register-staged weights.
 #include "kans_common.h"
 #include "kans_api_internal.h"
+#include "kans_split.h"
 #include "kans_tile.h"
 #include <algorithm>
 #include <type_traits>
@@ -58,10 +59,10 @@ kan_fused_dense(const TX* __restrict__ X, long ldx,
   constexpr int RB = WM / 32;           // 32-row blocks per wave
   constexpr int NV = RB * 8;            // inputs held per lane
   constexpr int CPL = Chunks<T>::CPL;   // uint4 per lane per 32-col block
+  static_assert(sizeof(T) == 2, "fp32 layers: kan_fused_split");
   constexpr int CPX = Chunks<TX>::CPL;  // uint4 per lane per row block of inputs
   constexpr int SU = NB * 64 * CPL;     // uint4 per pipeline stage
   constexpr int LPT = (SU + kThreads - 1) / kThreads;
-  constexpr bool kHalf = sizeof(T) == 2;
 
   __shared__ uint4 lds[kStages][SU];
 
@@ -172,41 +173,18 @@ kan_fused_dense(const TX* __restrict__ X, long ldx,
     const bool pf = t + 2 < nsteps;
     if (pf) gload(t + 2);
     const uint4* st = lds[t % kStages];
-    if constexpr (kHalf) {
-      typedef typename Mfma<T>::frag frag;
-      frag a[RB];
+    typedef typename Mfma<T>::frag frag;
+    frag a[RB];
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) a[rb][j] = from_f32<T>(v[rb * 8 + j]);
+      for (int j = 0; j < 8; ++j) a[rb][j] = from_f32<T>(v[rb * 8 + j]);
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        uint4 u = st[nb * 64 + lane];
-        frag b = *reinterpret_cast<frag*>(&u);
+    for (int nb = 0; nb < NB; ++nb) {
+      uint4 u = st[nb * 64 + lane];
+      frag b = *reinterpret_cast<frag*>(&u);
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) acc[rb][nb] = Mfma<T>::mma(a[rb], b, acc[rb][nb]);
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        float bv[NB][4];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          uint4 u = st[(nb * 2 + c) * 64 + lane];
-          bv[nb][0] = __uint_as_float(u.x);
-          bv[nb][1] = __uint_as_float(u.y);
-          bv[nb][2] = __uint_as_float(u.z);
-          bv[nb][3] = __uint_as_float(u.w);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-              acc[rb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[rb * 8 + c * 4 + e], bv[nb][e], acc[rb][nb],
-                                                                  0, 0, 0);
-      }
+      for (int rb = 0; rb < RB; ++rb) acc[rb][nb] = Mfma<T>::mma(a[rb], b, acc[rb][nb]);
     }
     if (pf) lstore(t + 2);
     ++t;
@@ -858,8 +836,8 @@ __global__ void kan_split_finalize4(const float4* __restrict__ part, int splits,
 
 // Repack raw weights W[D_out][D_in*K] (k fastest) and W_base[D_out][D_in], of
 // element type S, into the tiled layout W'[fb][s][ob][chunk][lane][e] of type T
-// (see kans_common.h), converting S -> T with round-to-nearest-even; zero
-// padding for o >= D_out and i >= D_in.  Slot s >= has_base holds coefficient
+// (see kans_common.h), converting S -> T with round-to-nearest-even (T = float:
+// splitting into three bf16 terms); zero padding for o >= D_out and i >= D_in.  Slot s >= has_base holds coefficient
 // k = s - has_base + k0.
 //
 // One workgroup per (16 outputs, 16-feature block): its 16 row segments of 16 K
@@ -870,9 +848,8 @@ __global__ void kan_split_finalize4(const float4* __restrict__ part, int splits,
 template <typename S, typename T>
 __global__ void __launch_bounds__(256)
 kan_repack_weights(const S* __restrict__ W, const S* __restrict__ Wb, uint4* __restrict__ Wt,
-                   int D_in, int D_out, int K, int k0, int has_base, int nob_pad) {
-  constexpr int CPL = Chunks<T>::CPL;
-  constexpr int EPC = 16 / (int)sizeof(T);
+                   int D_in, int D_out, int K, int k0, int has_base, int nob_pad, int sparse) {
+  constexpr int CPL = sizeof(T) == 4 ? 3 : 1;  // 16-byte chunks per lane: the three bf16 terms of fp32 weights
   extern __shared__ float seg[];  // [16][row]: 16 K coefficients, then 16 base weights
   const int row = 16 * (K + has_base) + 1;  // odd: a column of rows spreads over the banks
   const int ob = blockIdx.x >> 1, o_half = 16 * (blockIdx.x & 1), fb = blockIdx.y;
@@ -886,6 +863,41 @@ kan_repack_weights(const S* __restrict__ W, const S* __restrict__ Wb, uint4* __r
       seg[r * row + 16 * K + lane] = o < D_out && lane < ni ? to_f32(Wb[(long)o * D_in + i0 + lane]) : 0.0f;
   }
   __syncthreads();
+  if constexpr (sizeof(T) == 4) {
+    if (sparse) {
+      // units of one slot's size: the base slot, then two per step (kans_common.h, kSparseSteps)
+      const int steps = kSparseSteps * sparse_blocks(K), units = has_base + 2 * steps;
+      const int r = lane & 15, hb = (lane >> 4) & 1, dst_lane = o_half + r + 32 * hb;
+      const float* src = seg + r * row;
+      for (int u = 2 * wave + (lane >> 5); u < has_base + steps; u += 8) {
+        float v[16];
+        if (u < has_base) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = src[16 * K + 8 * hb + j];
+          const Split8 t = split8(v);
+          uint4* dst = Wt + ((long)fb * units * nob_pad + ob) * 192 + dst_lane;
+#pragma unroll
+          for (int c = 0; c < 3; ++c) dst[c * 64] = t.t[c];
+        } else {
+          const int st = u - has_base, m = st >> 2, P = (st >> 1) & 1, fh = st & 1;
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const int k = 8 * m + 2 * P + 4 * (j & 1) + ((j >> 1) & 1);
+            const int f = 8 * (j >> 3) + 4 * fh + 2 * hb + ((j >> 2) & 1);
+            v[j] = k < K ? src[f * K + k] : 0.0f;
+          }
+          const Split8 t0 = split8(v), t1 = split8(v + 8);
+          uint4* dst = Wt + (((long)fb * units + has_base + 2 * st) * nob_pad + 2 * ob) * 192 + dst_lane;
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            dst[2 * c * 64] = t0.t[c];
+            dst[(2 * c + 1) * 64] = t1.t[c];
+          }
+        }
+      }
+      return;
+    }
+  }
   const int KP = K - k0 + has_base;
   const int r = lane & 15, f0 = 8 * ((lane >> 4) & 1);
   const float* src = seg + r * row;
@@ -893,17 +905,20 @@ kan_repack_weights(const S* __restrict__ W, const S* __restrict__ Wb, uint4* __r
   for (int s = 2 * wave + (lane >> 5); s < KP; s += 8) {
     const bool base = has_base && s == 0;
     uint4* dst = Wt + (((long)fb * KP + s) * nob_pad + ob) * (64 * CPL) + dst_lane;
+    float v[8];
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-      T vals[EPC];
+    for (int e = 0; e < 8; ++e) v[e] = src[base ? 16 * K + f0 + e : (f0 + e) * K + s - has_base + k0];
+    if constexpr (sizeof(T) == 4) {
+      const Split8 t = split8(v);
 #pragma unroll
-      for (int e = 0; e < EPC; ++e) {
-        const int f = f0 + c * EPC + e;
-        vals[e] = from_f32<T>(src[base ? 16 * K + f : f * K + s - has_base + k0]);
-      }
+      for (int c = 0; c < CPL; ++c) dst[c * 64] = t.t[c];
+    } else {
+      T vals[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vals[e] = from_f32<T>(v[e]);
       uint4 u;
       __builtin_memcpy(&u, vals, 16);
-      dst[c * 64] = u;
+      *dst = u;
     }
   }
 }
@@ -930,6 +945,23 @@ kan_fold_bias(const S* __restrict__ W, const S* __restrict__ bias, float* __rest
 
 
 int block_waves(bool half, int basis, int wm, int nb, int KP);
+hipError_t launch_split(const DenseLaunch& L, int splits, int fbps, float* part, hipStream_t st);
+
+// y = sum of the splits' partials + the constant term.
+template <typename TY>
+static hipError_t finalize_splits(const DenseLaunch& L, const float* part, int splits, hipStream_t st) {
+  const long n = (long)L.B * L.D_out;
+  if (L.D_out % 4 == 0 && L.ldy % 4 == 0 && ((uintptr_t)L.Y % (4 * sizeof(TY))) == 0) {
+    const int blocks = (int)std::min<long>((n / 4 + 255) / 256, 4096);
+    hipLaunchKernelGGL((kan_split_finalize4<TY>), dim3(blocks), dim3(256), 0, st, (const float4*)part, splits,
+                       L.bias, (TY*)L.Y, L.ldy, L.B, L.D_out);
+  } else {
+    const int blocks = (int)std::min<long>((n + 255) / 256, 4096);
+    hipLaunchKernelGGL((kan_split_finalize<TY>), dim3(blocks), dim3(256), 0, st, part, splits, L.bias, (TY*)L.Y,
+                       L.ldy, L.B, L.D_out);
+  }
+  return hipGetLastError();
+}
 
 template <typename T, typename TX, typename TY, int BASIS, int WM, int NB>
 static hipError_t launch_dense_t(const DenseLaunch& L, hipStream_t st) {
@@ -943,10 +975,10 @@ static hipError_t launch_dense_t(const DenseLaunch& L, hipStream_t st) {
   // Kernel choice for 16-bit layers whose feature block fits one LDS stage:
   //   Chebyshev, tiles up to NB = 4        -> block kernel, 4 waves;
   //   RBF / B-spline, tile (32,8)          -> block kernel, 8 waves (256 x 256);
-  // everything else (fp32, other tiles, larger K) -> the per-slot kernel.
-  const int waves = block_waves(sizeof(T) == 2, BASIS, WM, NB, L.bp.K + L.has_base);
-  constexpr bool kBlock4 = sizeof(T) == 2 && BASIS == BASIS_CHEBY && NB <= 4;
-  constexpr bool kBlock8 = sizeof(T) == 2 && WM == 32 && NB == 8;
+  // everything else (other tiles, larger K) -> the per-slot kernel.
+  const int waves = block_waves(true, BASIS, WM, NB, L.bp.K + L.has_base);
+  constexpr bool kBlock4 = BASIS == BASIS_CHEBY && NB <= 4;
+  constexpr bool kBlock8 = WM == 32 && NB == 8;
   if (waves == 4) {
     if constexpr (kBlock4) {
       constexpr int BB = BASIS == BASIS_CHEBY ? BASIS_CHEBY_POST : BASIS;
@@ -1008,20 +1040,7 @@ static hipError_t launch_dense_t(const DenseLaunch& L, hipStream_t st) {
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (splits > 1) {
-    const long n = (long)L.B * L.D_out;
-    if (L.D_out % 4 == 0 && L.ldy % 4 == 0 && ((uintptr_t)L.Y % (4 * sizeof(TY))) == 0) {
-      const int blocks = (int)std::min<long>((n / 4 + 255) / 256, 4096);
-      hipLaunchKernelGGL((kan_split_finalize4<TY>), dim3(blocks), dim3(256), 0, st, (const float4*)part, splits,
-                         L.bias, (TY*)L.Y, L.ldy, L.B, L.D_out);
-    } else {
-      const int blocks = (int)std::min<long>((n + 255) / 256, 4096);
-      hipLaunchKernelGGL((kan_split_finalize<TY>), dim3(blocks), dim3(256), 0, st, part, splits,
-                         L.bias, (TY*)L.Y, L.ldy, L.B, L.D_out);
-    }
-    e = hipGetLastError();
-  }
-  return e;
+  return splits > 1 ? finalize_splits<TY>(L, part, splits, st) : e;
 }
 
 // Workgroup waves of the block kernel for this configuration, 0 when the
@@ -1069,22 +1088,26 @@ static hipError_t launch_dense_io(const DenseLaunch& L, hipStream_t st) {
 // x_dtype / y_dtype: the layer dtype or DT_F32 (fp32 activations around a 16-bit layer).
 template <typename T>
 static hipError_t launch_dense_type(const DenseLaunch& L, hipStream_t st) {
-  const bool xf = L.x_dtype == DT_F32 && L.dtype != DT_F32;
-  const bool yf = L.y_dtype == DT_F32 && L.dtype != DT_F32;
+  const bool xf = L.x_dtype == DT_F32, yf = L.y_dtype == DT_F32;
   if (!xf && !yf) return launch_dense_io<T, T, T>(L, st);
-  if constexpr (sizeof(T) == 2) {
-    if (xf && yf) return launch_dense_io<T, float, float>(L, st);
-    if (xf) return launch_dense_io<T, float, T>(L, st);
-    return launch_dense_io<T, T, float>(L, st);
-  }
-  return hipErrorInvalidValue;
+  if (xf && yf) return launch_dense_io<T, float, float>(L, st);
+  if (xf) return launch_dense_io<T, float, T>(L, st);
+  return launch_dense_io<T, T, float>(L, st);
+}
+
+static hipError_t launch_dense_f32(const DenseLaunch& L, hipStream_t st) {
+  const int fbps = (L.nfb + L.splits - 1) / L.splits;
+  const int splits = (L.nfb + fbps - 1) / fbps;
+  float* part = splits > 1 ? L.part : nullptr;
+  hipError_t e = launch_split(L, splits, fbps, part, st);
+  return e == hipSuccess && splits > 1 ? finalize_splits<float>(L, part, splits, st) : e;
 }
 
 hipError_t launch_dense(const DenseLaunch& L, hipStream_t st) {
   switch (L.dtype) {
     case DT_F16: return launch_dense_type<_Float16>(L, st);
     case DT_BF16: return launch_dense_type<__bf16>(L, st);
-    default: return launch_dense_type<float>(L, st);
+    default: return launch_dense_f32(L, st);
   }
 }
 
@@ -1092,7 +1115,7 @@ template <typename S, typename T>
 static hipError_t upload_t(const WeightUpload& U, hipStream_t st) {
   const size_t lds = (size_t)16 * (16 * (U.K + U.has_base) + 1) * sizeof(float);
   hipLaunchKernelGGL((kan_repack_weights<S, T>), dim3(2 * U.nob_pad, U.nfb), dim3(256), lds, st, (const S*)U.W,
-                     (const S*)U.Wb, (uint4*)U.Wt, U.D_in, U.D_out, U.K, U.fold, U.has_base, U.nob_pad);
+                     (const S*)U.Wb, (uint4*)U.Wt, U.D_in, U.D_out, U.K, U.fold, U.has_base, U.nob_pad, U.sparse);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || U.bias_out == nullptr) return e;
   hipLaunchKernelGGL((kan_fold_bias<S, T>), dim3((U.D_out + 3) / 4), dim3(256), 0, st, (const S*)U.W,

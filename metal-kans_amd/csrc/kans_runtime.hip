@@ -40,6 +40,8 @@ hipError_t launch_dense(const DenseLaunch& L, hipStream_t st);
 bool dense_config_supported(int wm, int nb);
 bool block_wave_groups_ok(int wm, int nb, int ks);
 int block_waves(bool half, int basis, int wm, int nb, int KP);
+int split_waves(int wm, int nb);
+bool split_sparse(int basis, int K);
 hipError_t launch_upload(const WeightUpload& U, hipStream_t st);
 }  // namespace kans
 
@@ -122,7 +124,8 @@ static size_t dtype_size(int dt) { return dt == DT_F32 ? 4 : 2; }
 struct kans_layer {
   int basis, dtype, D_in, D_out, K, has_base, has_bias;
   int D_in8, nfb, nob_pad;
-  int fold, slots;  // T_0 folded into the bias (BasisParams::k0); contracted slots per feature
+  // T_0 folded into the bias (BasisParams::k0); fp32 B-spline in the sparse layout; slots of W' per feature
+  int fold, sparse, slots;
   BasisParams bp{};
   DevBuf Wt, bias_d, part, x_d, y_d, raw_w, raw_wb;
   bool have_weights = false;
@@ -183,7 +186,8 @@ static void layer_shape(kans_layer* L) {
   L->nob_pad = round_up((L->D_out + 31) / 32, kObPad);
   // a T_0-only layer without a base branch keeps its one slot
   L->fold = L->basis == BASIS_CHEBY && L->K + L->has_base > 1;
-  L->slots = L->K - L->fold + L->has_base;
+  L->sparse = L->dtype == DT_F32 && split_sparse(L->basis, L->K);
+  L->slots = L->sparse ? 8 * sparse_blocks(L->K) + L->has_base : L->K - L->fold + L->has_base;
   L->bp.K = L->K - L->fold;
   L->bp.k0 = L->fold;
 }
@@ -295,7 +299,7 @@ static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, con
   const size_t es = dtype_size(src_dtype);
   const size_t wbytes = (size_t)L->D_out * L->D_in * L->K * es;
   const size_t wbbytes = (size_t)L->D_out * L->D_in * es;
-  const size_t tbytes = (size_t)L->nfb * L->slots * L->nob_pad * 64 * 16 * (L->dtype == DT_F32 ? 2 : 1);
+  const size_t tbytes = (size_t)L->nfb * L->slots * L->nob_pad * 64 * 16 * (L->dtype == DT_F32 ? 3 : 1);
   int rc;
   void* old_wt = L->Wt.p;
   void* old_bias = L->bias_d.p;
@@ -329,6 +333,7 @@ static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, con
   U.D_out = L->D_out;
   U.K = L->K;
   U.has_base = L->has_base;
+  U.sparse = L->sparse;
   U.fold = L->fold;
   U.nfb = L->nfb;
   U.nob_pad = L->nob_pad;
@@ -385,16 +390,19 @@ int kans_layer_load_weights_device(kans_layer* L, const void* W, const void* W_b
 //    ways on the per-slot kernel.
 static void choose_tiling(const kans_layer* L, int B, int* wm, int* nb, int* splits) {
   static const int pref_n8[4][2] = {{32, 8}, {64, 4}, {32, 4}, {32, 1}};
-  static const int pref_n4[4][2] = {{32, 4}, {64, 4}, {32, 8}, {32, 1}};
   static const int pref_small[4][2] = {{32, 4}, {32, 8}, {64, 4}, {32, 1}};
   const bool f32 = L->dtype == DT_F32;
-  const int(*cand)[2] = (f32 && L->basis != BASIS_BSPLINE) ? pref_n4 : pref_n8;
+  const int(*cand)[2] = pref_n8;
   const int nob = (L->D_out + 31) / 32;
   const int KP = L->slots;
   // workgroups of shape (ww, nn): the 8-wave block kernel's tile is 8 row blocks tall
-  auto waves_of = [&](int ww, int nn) { return block_waves(!f32, L->basis, ww, nn, KP) == 8 ? 8 : 4; };
+  // (fp32: 32 rows per wave, 8 or 4 waves)
+  auto waves_of = [&](int ww, int nn) {
+    if (f32) return split_waves(ww, nn);
+    return block_waves(true, L->basis, ww, nn, KP) == 8 ? 8 : 4;
+  };
   auto wgs = [&](int ww, int nn) {
-    const int rows = waves_of(ww, nn) * ww;
+    const int rows = waves_of(ww, nn) * (f32 ? 32 : ww);
     return ((B + rows - 1) / rows) * ((nob + nn - 1) / nn);
   };
   auto slots = [&](int ww, int nn) { return waves_of(ww, nn) == 8 ? 256 : 512; };
@@ -725,6 +733,9 @@ static int layer_kernel_name(const kans_layer* L, int B, bool io, int x_dtype, i
                      ? (L->has_base ? "BASIS_BSPLINE_TAB" : "BASIS_BSPLINE_TAB0")
                      : bs[L->basis],
                  wm, nb, waves, groups);
+  else if (L->dtype == DT_F32)
+    n = snprintf(name, len, "kans::kan_fused_split%s<%s, %s, %d, %d, %d waves>", L->sparse ? "_sparse" : "", types,
+                 bs[L->basis], wm, nb, split_waves(wm, nb));
   else
     n = snprintf(name, len, "kans::kan_fused_dense<%s, %s, %d, %d>", types, bs[L->basis], wm, nb);
   if (n >= 0 && splits > 1)

@@ -27,31 +27,30 @@ __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
   return u;
 }
 
-// What is left of v after its bf16 rounding hf.  An infinite or NaN hf leaves
-// nothing: the product then is what h alone gives (inf - inf would turn an
-// infinity into NaN).
-__device__ __forceinline__ float bf16_rest(float v, float hf) {
-  const float r = v - hf;
-  return __builtin_fabsf(hf) < __builtin_inff() ? r : 0.0f;
-}
-
-// The three bf16 terms of 8 fp32 values, each packed as one MFMA operand.
+// The three bf16 terms of 8 fp32 values, each packed as one MFMA operand.  An
+// infinite or NaN value (and a finite one that rounds to infinity in bf16,
+// above 3.3895e38) goes into the l term alone: of the six products it then
+// enters one, l_a h_b, where h = inf, m = l = 0 would meet zeros and terms of
+// the other sign in three more and turn an infinite sum into NaN.
 struct Split8 {
   uint4 t[3];
 };
 
 __device__ __forceinline__ Split8 split8(const float* v) {
+  constexpr float kFiniteMax = 0x1.fep+127f;  // largest bf16
   unsigned d[3][4];
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     const float a = v[2 * p], b = v[2 * p + 1];
-    const unsigned h = bf16_pair(a, b);
-    const float ra = bf16_rest(a, __uint_as_float(h << 16));
-    const float rb = bf16_rest(b, __uint_as_float(h & 0xffff0000u));
+    const bool fa = __builtin_fabsf(a) <= kFiniteMax, fb = __builtin_fabsf(b) <= kFiniteMax;
+    const float ca = fa ? a : 0.0f, cb = fb ? b : 0.0f;
+    const unsigned h = bf16_pair(ca, cb);
+    const float ra = ca - __uint_as_float(h << 16), rb = cb - __uint_as_float(h & 0xffff0000u);
     const unsigned m = bf16_pair(ra, rb);
+    const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
     d[0][p] = h;
     d[1][p] = m;
-    d[2][p] = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+    d[2][p] = bf16_pair(fa ? sa : a, fb ? sb : b);
   }
   Split8 s;
 #pragma unroll
@@ -68,6 +67,35 @@ __device__ __forceinline__ floatx16 mma_split(const bf16x8 (&a)[3], const bf16x8
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+  return acc;
+}
+
+// The same with the five small products in an accumulator of their own, 2^-8 of
+// the sum: the sum itself is then rounded once per product tile, not six times.
+__device__ __forceinline__ void mma_split2(const bf16x8 (&a)[3], const bf16x8 (&b)[3], floatx16& acc, floatx16& small) {
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], small, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+}
+
+// The same with a 4:2 sparse left operand of 32 contraction indices (two
+// non-zeros in each group of four, their places in the low 16 bits of idx):
+// v_smfmac_f32_32x32x32_bf16 takes the time of the 16-deep dense MFMA.
+// Lane l of A (row l%32, h = l/32) holds the non-zeros of groups g = 0..3 at
+// elements 2g, 2g+1, whose places (0..3 in their group) are bits 4g..4g+1 and
+// 4g+2..4g+3 of idx; group g of half h meets elements 8h + 4(g%2) .. +3 of B's
+// lane half g/2 (B: column l%32, contraction indices 16(l/32) .. +15).
+typedef __bf16 bf16x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ floatx16 smfma_split(const bf16x8 (&a)[3], const bf16x16 (&b)[3], int idx, floatx16 acc) {
+  acc = __builtin_amdgcn_smfmac_f32_32x32x32_bf16(a[2], b[0], acc, idx, 0, 0);
+  acc = __builtin_amdgcn_smfmac_f32_32x32x32_bf16(a[1], b[1], acc, idx, 0, 0);
+  acc = __builtin_amdgcn_smfmac_f32_32x32x32_bf16(a[0], b[2], acc, idx, 0, 0);
+  acc = __builtin_amdgcn_smfmac_f32_32x32x32_bf16(a[1], b[0], acc, idx, 0, 0);
+  acc = __builtin_amdgcn_smfmac_f32_32x32x32_bf16(a[0], b[1], acc, idx, 0, 0);
+  acc = __builtin_amdgcn_smfmac_f32_32x32x32_bf16(a[0], b[0], acc, idx, 0, 0);
   return acc;
 }
 

@@ -859,3 +859,53 @@ def test_cheby_constant_coefficients(gpu, dtype, K, base, d_in, d_out):
     # summed in more than fp32 and rounded once, to the output type (2^-24, 2^-11, 2^-8)
     eps = {"float32": 2.0 ** -24, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[dtype]
     assert np.all(np.abs(y - const) <= eps * np.abs(const) + 1e-7 * np.abs(w).sum(1))
+
+
+@pytest.mark.parametrize("wm,nb", [(64, 4), (32, 8), (32, 4), (32, 1)])
+@pytest.mark.parametrize("kind,K", [("bspline", 4), ("bspline", 5), ("bspline", 8), ("bspline", 9), ("bspline", 13),
+                                    ("bspline", 17), ("cheby", 9), ("rbf", 7)])
+def test_f32_split_kernels_edges(gpu, wm, nb, kind, K):
+    """fp32 layers on the bf16 matrix cores (three terms per operand): B-splines of K = 4 take dense steps,
+    K >= 5 sparse ones in one, two or three blocks of 8 functions (K at and around their ends); inputs on every
+    knot, on the ends of the grid and outside it; ragged sizes, one and several feature blocks, feature splits."""
+    import metal_kans as mk
+    for d_in, base, splits in ((7, True, 1), (41, False, 2), (90, True, 1)):
+        L = make_layer(mk, kind, d_in, 75, K, bias=True, base=base, seed=K + d_in)
+        rng = np.random.default_rng(K)
+        x = rng.uniform(-1.3, 1.3, (70, d_in)).astype(np.float32)
+        if kind == "bspline":
+            knots = np.linspace(-1, 1, K - 2).astype(np.float32)
+            x[::7, :] = rng.choice(knots, x[::7, :].shape)
+            x[3], x[4] = 1e4, -1e4
+        L.set_tiling(wm, nb, splits)
+        # fp32 operands taken exactly, at most 90 * 18 products per sum: 2^-24 * sqrt(1620) = 2.4e-6, and the
+        # fp32 basis values (up to ~1e-6 for K = 9 Chebyshev, 2e-6 at positions next to a knot)
+        assert O.rel_err(L(x), oracle_of(L, x)) <= 1e-5, (d_in, base, splits)
+
+
+def test_f32_long_contraction(gpu):
+    """738 steps on the 256-column tile: more than one run of sums (kRun)."""
+    import metal_kans as mk
+    L = make_layer(mk, "cheby", 1300, 40, 9, bias=True, base=True, seed=5)
+    x = np.random.default_rng(8).uniform(-1, 1, (300, 1300)).astype(np.float32)
+    y_ref = oracle_of(L, x)
+    for splits in (1, 2):
+        L.set_tiling(32, 8, splits)
+        assert O.rel_err(L(x), y_ref) <= 1e-5
+
+
+@pytest.mark.parametrize("kind,K", [("cheby", 5), ("rbf", 8), ("bspline", 8)])
+def test_f32_infinite_and_nan_inputs(gpu, kind, K):
+    """An infinite input reaches the output through the SiLU branch as in one fp32 sum: +inf times the sign of
+    its weight; NaN and -inf (SiLU(-inf) = -inf * 0) make their row NaN, every other row stays finite."""
+    import metal_kans as mk
+    L = make_layer(mk, kind, 40, 30, K, bias=True, base=True, seed=6)
+    x = np.random.default_rng(9).uniform(-1, 1, (20, 40)).astype(np.float32)
+    ref = np.asarray(L(x))
+    bad = x.copy()
+    bad[3, 7], bad[5, 8], bad[6, 9] = np.inf, np.nan, -np.inf
+    y = np.asarray(L(bad))
+    rows = [r for r in range(20) if r not in (3, 5, 6)]
+    assert np.array_equal(y[rows], ref[rows])
+    assert np.array_equal(y[3], np.sign(L.w_base[:, 7]) * np.inf)
+    assert np.isnan(y[5]).all() and np.isnan(y[6]).all()
