@@ -82,6 +82,10 @@ __host__ __device__ constexpr int qp_period(int K, int GS) {
     }
   return 1;
 }
+// Chebyshev layers keep their T_0 coefficients out of the contraction (T_0 = 1:
+// they add sum_i W[o, i*K] to every row, part of the constant term per output);
+// a K = 1 layer without the base branch keeps its one slot.
+__host__ __device__ constexpr int qp_fold(bool cheby, int K, int has_base) { return cheby && K + has_base > 1 ? 1 : 0; }
 __host__ __device__ constexpr int qp_chunk_bytes(int qt) { return qt == 0 ? 4 : qt == 2 ? 8 : 2; }  // Q_INT4/TERN/INT8
 __host__ __device__ constexpr int qp_group(int qt) { return qt == 1 ? 32 : 64; }
 __host__ __device__ constexpr int qp_param_floats(int qt) { return qt == 1 ? 1 : 2; }
@@ -103,7 +107,7 @@ struct QPMat {
   long ldp;                 // parameter row stride (nob_pad * 32 outputs)
   int nob_pad;              // 32-column blocks, padded to a multiple of 8
   int D_out;
-  const void* bias;         // [D_out] (bias_dt) or null
+  const void* bias;         // [D_out] (bias_dt), with the folded T_0 coefficients (qp_fold), or null
 };
 
 // One fused prefill launch: y = forward(x) of matrix m[0] (grp = 8: all eight
@@ -154,6 +158,12 @@ hipError_t qp_run_tern_b1(const QPLaunch& L, const QPGrid& G, hipStream_t st);
 hipError_t qp_tile_affine(int bits, const unsigned char* qw, long rowbytes, const float* scales, const float* biases,
                           int gpr, int D_out, int D_in, int Kseg, int nfb, int nob_pad, int G_alloc, void* codes,
                           float* params, hipStream_t st);
+// out[o] = bias[o] + sum_i W[o, i*K] of the dequantized weights, summed in fp64 (bias may be null).
+hipError_t q_fold_affine(int bits, const unsigned char* qw, long rowbytes, const float* scales, const float* biases,
+                         int gpr, int D_out, int D_in, int K, const void* bias, int bias_dt, float* out,
+                         hipStream_t st);
+hipError_t q_fold_tern(const unsigned* wp, int wpr, const float* scales, int gpr, int D_out, int D_in, int K,
+                       const void* bias, int bias_dt, float* out, hipStream_t st);
 hipError_t qp_tile_tern(const unsigned* wp, int wpr, const float* scales, int gpr, int D_out, int D_in, int Kseg,
                         int nfb, int nob_pad, int G_alloc, void* codes, float* params, hipStream_t st);
 

@@ -132,6 +132,61 @@ __global__ void k_qp_tile_tern(const unsigned* __restrict__ wp, int wpr, int D_o
   }
 }
 
+// The constant term of a Chebyshev layer: one wave per output, w(i) = W[o, i*K].
+template <typename F>
+__device__ __forceinline__ void fold_row(int D_out, int D_in, const void* bias, int bias_dt, float* out, F&& w) {
+  const int o = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (o >= D_out) return;
+  double s = 0.0;
+  for (int i = lane; i < D_in; i += 64) s += (double)w(o, i);
+  for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
+  if (lane == 0) out[o] = (float)(s + (bias ? (double)load_any_f(bias, o, bias_dt) : 0.0));
+}
+
+template <int BITS>
+__global__ void __launch_bounds__(256)
+k_q_fold_affine(const unsigned char* __restrict__ qw, long rowbytes, const float* __restrict__ scales,
+                const float* __restrict__ biases, int gpr, int D_out, int D_in, int K, const void* bias, int bias_dt,
+                float* __restrict__ out) {
+  fold_row(D_out, D_in, bias, bias_dt, out, [&](int o, int i) {
+    const long j = (long)i * K, g = (long)o * gpr + j / 64;
+    const unsigned b = qw[(long)o * rowbytes + (BITS == 8 ? j : j >> 1)];
+    const float q = (float)(BITS == 8 ? b : (j & 1) ? b >> 4 : b & 15u);
+    return __fadd_rn(__fmul_rn(q, scales[g]), biases[g]);  // quantization.py:136-148
+  });
+}
+
+__global__ void __launch_bounds__(256)
+k_q_fold_tern(const unsigned* __restrict__ wp, int wpr, const float* __restrict__ scales, int gpr, int D_out, int D_in,
+              int K, const void* bias, int bias_dt, float* __restrict__ out) {
+  fold_row(D_out, D_in, bias, bias_dt, out, [&](int o, int i) {
+    const long j = (long)i * K;
+    const unsigned c = (wp[(long)o * wpr + (j >> 4)] >> (2 * (j & 15))) & 3u;
+    const float s = scales[(long)o * gpr + j / 32];
+    return c == 0 ? -s : c == 2 ? s : 0.0f;
+  });
+}
+
+hipError_t q_fold_affine(int bits, const unsigned char* qw, long rowbytes, const float* scales, const float* biases,
+                         int gpr, int D_out, int D_in, int K, const void* bias, int bias_dt, float* out,
+                         hipStream_t st) {
+  const dim3 grid((D_out + 3) / 4);
+  if (bits == 8)
+    hipLaunchKernelGGL(k_q_fold_affine<8>, grid, dim3(256), 0, st, qw, rowbytes, scales, biases, gpr, D_out, D_in, K,
+                       bias, bias_dt, out);
+  else
+    hipLaunchKernelGGL(k_q_fold_affine<4>, grid, dim3(256), 0, st, qw, rowbytes, scales, biases, gpr, D_out, D_in, K,
+                       bias, bias_dt, out);
+  return hipGetLastError();
+}
+
+hipError_t q_fold_tern(const unsigned* wp, int wpr, const float* scales, int gpr, int D_out, int D_in, int K,
+                       const void* bias, int bias_dt, float* out, hipStream_t st) {
+  hipLaunchKernelGGL(k_q_fold_tern, dim3((D_out + 3) / 4), dim3(256), 0, st, wp, wpr, scales, gpr, D_out, D_in, K, bias,
+                     bias_dt, out);
+  return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launch.
 // ---------------------------------------------------------------------------

@@ -283,7 +283,10 @@ struct QPArgs {
 // ---------------------------------------------------------------------------
 template <int QT, int KQ, int HB, int BASIS = BASIS_CHEBY_POST, bool PAIR = false>
 __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
-  constexpr int KP = KQ + HB;
+  // Chebyshev: the T_0 coefficients are in the constant term (QPMat::bias), so the
+  // contraction starts at k = F: K + base = 5 slots become 4
+  constexpr int F = qp_fold(BASIS == BASIS_CHEBY_POST, KQ, HB);
+  constexpr int KP = KQ - F + HB;
   constexpr int NV = 8;
   constexpr int SLOT = kQNB * 64;  // uint4 per slot of the N-tile
   constexpr int CB = qp_chunk_bytes(QT);
@@ -293,7 +296,7 @@ __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
   constexpr int NCB = QT == Q_TERN ? (KQ == 1 ? 1 : (KQ + 1) / 2) : (KQ * CB) / 4;
   constexpr int NCW = QT == Q_INT8 ? 2 : 1;  // base code dwords
   typedef half8 frag;
-  static_assert(KQ >= 1 && KQ <= kQPMaxK && KP <= 10, "K + base slots of fp16 B-tiles in two LDS stages");
+  static_assert(KQ >= 1 && KQ <= kQPMaxK && KP >= 1 && KP <= 10, "K + base slots of fp16 B-tiles in two LDS stages");
   // quantization groups a half-block's codes meet, and the phases of the
   // feature block index that place them differently (qp_ngroups, qp_period)
   constexpr int NGRP = qp_ngroups(KQ, GS);
@@ -389,7 +392,9 @@ __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
     }
   };
   auto load_all = [&](int fbq, auto PHC, QRegs& r) __attribute__((always_inline)) {
-    static_for<0, NG>([&](auto G) __attribute__((always_inline)) { load_cb(fbq, decltype(G)::value, r); });
+    // (a word group that holds only k = 0 is not read)
+    constexpr int G0 = F && (QT != Q_TERN || KQ == 1) ? 1 : 0;
+    static_for<G0, NG>([&](auto G) __attribute__((always_inline)) { load_cb(fbq, decltype(G)::value, r); });
     if constexpr (HB) load_cw(fbq, r);
     load_params(fbq, PHC, r);
   };
@@ -399,7 +404,7 @@ __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
     if constexpr (HB && SC == 0) {
       load_cw(fbq, r);
     } else {
-      constexpr int k = SC - HB;
+      constexpr int k = SC - HB + F;
       if constexpr (QT != Q_TERN || KQ == 1) load_cb(fbq, k, r);
       else if constexpr ((k & 1) || k == KQ - 1) load_cb(fbq, k / 2, r);  // every slot of the word decoded
     }
@@ -416,7 +421,7 @@ __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
       else if constexpr (QT == Q_INT8) return dq_int8<1, GS, 0, 0>(r.cw[0], r.cw[1], pw, m0, dk);
       else return dq_tern<1, GS, 0, 0, 0>(tern_spread(r.cw[0]), pw, m0, dk);
     } else {
-      constexpr int k = SC - HB;
+      constexpr int k = SC - HB + F;
       if constexpr (QT == Q_INT4) return dq_int4<KQ, GS, ph, k>(r.cb[k], pb, m0, dk);
       else if constexpr (QT == Q_INT8) return dq_int8<KQ, GS, ph, k>(r.cb[2 * k], r.cb[2 * k + 1], pb, m0, dk);
       else if constexpr (KQ == 1) return dq_tern<KQ, GS, ph, k, 0>(tern_spread(r.cb[0]), pb, m0, dk);
@@ -594,7 +599,11 @@ __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
     load_params(fb + AH + 1, PhNN{}, R);
     bread(bf, cur, 0);
     if constexpr (kTab) gen.begin(xf, bp, bs_sel);
-    else gen.begin(xf, bp, HB != 0);
+    else if constexpr (BASIS == BASIS_CHEBY_POST) {
+      BasisParams first;  // the only field this generator reads
+      first.k0 = F;
+      gen.begin(xf, first, HB != 0);
+    } else gen.begin(xf, bp, HB != 0);
     {
       float v[NV];
       if constexpr (HB) {
@@ -724,8 +733,10 @@ __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
     for (int nb = 0; nb < 4; ++nb) {
       const int c = (n_tile * 4 + nb) * 32 + (lane & 31);
       if (c < A.m[0].D_out) {
-        const float bg = A.m[0].bias ? load_any_f(A.m[0].bias, c, A.bias_dt) : 0.0f;
-        const float bu = A.m[1].bias ? load_any_f(A.m[1].bias, c, A.bias_dt) : 0.0f;
+        // loaded and waited for once, before the row tests (see kan_fused_block)
+        float bg = A.m[0].bias ? load_any_f(A.m[0].bias, c, A.bias_dt) : 0.0f;
+        float bu = A.m[1].bias ? load_any_f(A.m[1].bias, c, A.bias_dt) : 0.0f;
+        asm volatile("" : "+v"(bg), "+v"(bu));
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int dr = 8 * (r >> 2) + (r & 3);
@@ -744,7 +755,8 @@ __global__ void __launch_bounds__(kQThreads, 1) kan_qfused_block(QPArgs A) {
   for (int nb = 0; nb < kQNB; ++nb) {
     const int c = (n_tile * 8 + nb) * 32 + (lane & 31);
     if (c < A.m[0].D_out) {
-      const float bc = A.m[0].bias ? load_any_f(A.m[0].bias, c, A.bias_dt) : 0.0f;
+      float bc = A.m[0].bias ? load_any_f(A.m[0].bias, c, A.bias_dt) : 0.0f;
+      asm volatile("" : "+v"(bc));
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int dr = 8 * (r >> 2) + (r & 3);

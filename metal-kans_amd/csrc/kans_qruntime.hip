@@ -32,6 +32,7 @@ struct kans_qlayer {
   int nrb_pad;               // 16-row blocks, padded to a multiple of nw
   bool decode = false;       // decode records built (INT4 / ternary)
   DevBuf R, bias;            // re-tiled records (codes + group parameters), bias (bias_dtype)
+  DevBuf cbias;              // fp32 bias + sum_i W[o, i*K]: the Chebyshev constant term (qp_fold)
   int bias_dtype = DT_F32;
   // decode workspace: activation basis, its group sums, split-K partials
   DevBuf Phi, S, part;
@@ -191,7 +192,11 @@ void prefill_geometry(kans_qlayer* L) {
   L->p_nob_pad = round_up((L->D_out + 31) / 32, 8);
 }
 
-QPMat qp_mat(const kans_qlayer* L) {
+// Whether the prefill of a layer with this basis takes its constant term from cbias.
+bool prefill_fold(const kans_qlayer* L, int basis) { return qp_fold(basis == BASIS_CHEBY, L->K, L->has_base); }
+int prefill_bias_dtype(const kans_qlayer* L, int basis) { return prefill_fold(L, basis) ? DT_F32 : L->bias_dtype; }
+
+QPMat qp_mat(const kans_qlayer* L, int basis) {
   QPMat m;
   m.cb = (const unsigned char*)L->PCb.p;
   m.cw = (const unsigned char*)L->PCw.p;
@@ -200,7 +205,7 @@ QPMat qp_mat(const kans_qlayer* L) {
   m.ldp = (long)L->p_nob_pad * 32;
   m.nob_pad = L->p_nob_pad;
   m.D_out = L->D_out;
-  m.bias = L->has_bias ? L->bias.p : nullptr;
+  m.bias = prefill_fold(L, basis) ? L->cbias.p : L->has_bias ? L->bias.p : nullptr;
   return m;
 }
 
@@ -370,10 +375,10 @@ int prefill_layer_locked(kans_qlayer* L, const void* X, int x_dtype, long ldx, v
   P.X = X;
   P.ldx = ldx;
   P.x_dtype = x_dtype;
-  P.m[0] = qp_mat(L);
+  P.m[0] = qp_mat(L, L->basis);
   P.m[1] = P.m[0];
   P.grp = 8;
-  P.bias_dtype = L->bias_dtype;
+  P.bias_dtype = prefill_bias_dtype(L, L->basis);
   P.Y = Y;
   P.ldy = ldy;
   P.y_dtype = y_dtype;
@@ -437,10 +442,11 @@ int plan_gated_prefill(kans_gated* G, const void* X, int x_dtype, long ldx, void
   P1.X = X;
   P1.ldx = ldx;
   P1.x_dtype = x_dtype;
-  P1.m[0] = qp_mat(g);
-  P1.m[1] = qp_mat(u);
+  P1.m[0] = qp_mat(g, BASIS_CHEBY);
+  P1.m[1] = qp_mat(u, BASIS_CHEBY);
   P1.grp = 4;
-  P1.bias_dtype = g->has_bias ? g->bias_dtype : u->bias_dtype;
+  // (gate and up have one K and one base flag, so both terms are folded or neither)
+  P1.bias_dtype = prefill_fold(g, BASIS_CHEBY) ? DT_F32 : g->has_bias ? g->bias_dtype : u->bias_dtype;
   P1.ldy = ldh;
   P1.y_dtype = hdt;
   P1.B = B;
@@ -454,10 +460,10 @@ int plan_gated_prefill(kans_gated* G, const void* X, int x_dtype, long ldx, void
   P2.has_base = d->has_base;
   P2.ldx = ldh;
   P2.x_dtype = hdt;
-  P2.m[0] = qp_mat(d);
+  P2.m[0] = qp_mat(d, BASIS_CHEBY);
   P2.m[1] = P2.m[0];
   P2.grp = 8;
-  P2.bias_dtype = d->bias_dtype;
+  P2.bias_dtype = prefill_bias_dtype(d, BASIS_CHEBY);
   P2.Y = Y;
   P2.ldy = ldy;
   P2.y_dtype = y_dtype;
@@ -710,12 +716,18 @@ int create_affine(int bits, int D_in, int D_out, int K, int has_base, int has_bi
     if (L->prefill &&
         (r = build_ptiles(L, seg, tq.p, rowbytes, (const float*)ts.p, (const float*)tb.p, (int)gpr, st)))
       return r;
+    if (seg == 0) {
+      if ((r = L->cbias.reserve((size_t)D_out * sizeof(float)))) return r;
+      HIP_TRY(q_fold_affine(bits, (const unsigned char*)tq.p, rowbytes, (const float*)ts.p, (const float*)tb.p,
+                            (int)gpr, D_out, D_in, K, has_bias ? L->bias.p : nullptr, bias_dtype,
+                            (float*)L->cbias.p, st));
+    }
     HIP_TRY(hipStreamSynchronize(st));  // the temporaries die here
     return 0;
   };
+  if ((rc = upload_bias(L, bias, bias_dtype))) return fail(rc);
   if ((rc = segment(0, qweight, scales, biases))) return fail(rc);
   if (has_base && (rc = segment(1, qweight_base, scales_base, biases_base))) return fail(rc);
-  if ((rc = upload_bias(L, bias, bias_dtype))) return fail(rc);
   HIP_TRY(hipStreamSynchronize(st));
   *out = L;
   return 0;
@@ -889,12 +901,17 @@ int kans_qlayer_create_ternary(int D_in, int D_out, int K, int has_base, int has
                               seg ? L->Cw : L->Cb, seg ? L->Cb : 0, L->C_tot, L->R.p, st);
     if (e != hipSuccess) return kans_fail(KANS_ERR_HIP, "ternary re-tiling failed: %s", hipGetErrorString(e));
     if (L->prefill && (r = build_ptiles(L, seg, tw.p, wpr, (const float*)ts.p, nullptr, gpr, st))) return r;
+    if (seg == 0) {
+      if ((r = L->cbias.reserve((size_t)D_out * sizeof(float)))) return r;
+      HIP_TRY(q_fold_tern((const unsigned*)tw.p, wpr, (const float*)ts.p, gpr, D_out, D_in, K,
+                          has_bias ? L->bias.p : nullptr, bias_dtype, (float*)L->cbias.p, st));
+    }
     HIP_TRY(hipStreamSynchronize(st));  // the temporaries die here
     return 0;
   };
+  if ((rc = upload_bias(L, bias, bias_dtype))) return fail(rc);
   if ((rc = segment(0, w_packed, scales))) return fail(rc);
   if (has_base && (rc = segment(1, w_packed_base, scales_base))) return fail(rc);
-  if ((rc = upload_bias(L, bias, bias_dtype))) return fail(rc);
   HIP_TRY(hipStreamSynchronize(st));
   *out = L;
   return 0;
