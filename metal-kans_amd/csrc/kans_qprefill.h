@@ -135,7 +135,7 @@ extern int g_qp_block_pairs;
 // Split-K workspace floats a launch needs (0 when unsplit).
 long qp_part_floats(const QPLaunch& L);
 // Feature splits the launcher picks for B rows (so the grid fills the GPU).
-int qp_choose_splits(int B, int D_in, int n_cols, int grp);
+int qp_choose_splits(int B, int D_in, int n_cols, int grp, int slots);
 hipError_t qp_launch(const QPLaunch& L, hipStream_t st);
 
 // Grid of one fused launch: m_tiles x n_tiles output tiles by nsp feature

@@ -22,9 +22,20 @@ __global__ void k_qp_finalize(const float* __restrict__ part, int splits, int B,
     const long sstride = (long)B * ncols;
     float g = bias0 ? load_any_f(bias0, c, bias_dt) : 0.0f;
     float u = (epi == QP_EPI_SWIGLU && bias1) ? load_any_f(bias1, c, bias_dt) : 0.0f;
-    for (int k = 0; k < splits; ++k) {
-      g += p[k * sstride];
-      if (epi == QP_EPI_SWIGLU) u += p[k * sstride + 128];
+    // splits in order, loaded 4 at a time
+    for (int k0 = 0; k0 < splits; k0 += 4) {
+      float a[4], b[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bool ok = k0 + q < splits;
+        a[q] = ok ? p[(k0 + q) * sstride] : 0.0f;
+        b[q] = ok && epi == QP_EPI_SWIGLU ? p[(k0 + q) * sstride + 128] : 0.0f;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        g += a[q];
+        u += b[q];
+      }
     }
     if (epi == QP_EPI_SWIGLU) {
       g = round16v(g, round16);
@@ -219,14 +230,37 @@ hipError_t qp_tile_tern(const unsigned* wp, int wpr, const float* scales, int gp
   return hipGetLastError();
 }
 
-int qp_choose_splits(int B, int D_in, int n_cols, int grp) {
-  const int m_tiles = (B + 255) / 256;
-  const int n_tiles = (n_cols + 32 * grp - 1) / (32 * grp);
-  const int tiles = m_tiles * n_tiles;
+// Feature splits of one launch: the estimate of its time is the rounds of
+// workgroups (one per CU, 256 CUs) times a workgroup's feature blocks at
+// kSlotUs per slot and kRoundUs to start and drain, plus for a split launch the
+// partial sums written and read once and the reduce kernel.  A grid between one
+// and two workgroups per CU (172 at 512 rows of a 11008-wide gate|up pair)
+// leaves a third of the chip idle in its last round unless it is split into
+// several short rounds; a split that only spills into one more round costs
+// more than it gives.
+// GatedKAN 4096 / 11008, INT4, us per block at 33 / 256 / 512 / 1024 / 2048 rows:
+// one workgroup per CU as the only aim 412 / 498 / 773 / 1440 / 2370, this
+// estimate 315 / 377 / 674 / 1233 / 2346 (ternary 1024 / 2816: 55 / 68 / 100 /
+// 154 / 231 and 50 / 64 / 83 / 126 / 200).
+int qp_choose_splits(int B, int D_in, int n_cols, int grp, int slots) {
+  constexpr double kSlotUs = 0.5, kRoundUs = 5.0, kReduceUs = 4.0, kBytesPerUs = 6.0e6;
+  const long m_tiles = (B + 255) / 256;
+  const long n_tiles = (n_cols + 32 * grp - 1) / (32 * grp);
+  const long tiles = m_tiles * n_tiles;
   const int nfb = (D_in + 15) / 16;
-  if (tiles >= 256) return 1;
-  // towards one workgroup per CU, at least 8 feature blocks per split
-  return std::max(1, std::min((256 + tiles - 1) / tiles, nfb / 8));
+  double best = 0.0;
+  int bs = 1;
+  // at least 8 feature blocks per split
+  for (int s = 1; s <= std::max(1, std::min(nfb / 8, 32)); ++s) {
+    const long rounds = (tiles * s + 255) / 256, fbps = (nfb + s - 1) / s;
+    double t = (double)rounds * (fbps * slots * kSlotUs + kRoundUs);
+    if (s > 1) t += kReduceUs + 8.0 * s * B * n_tiles * 256 / kBytesPerUs;
+    if (s == 1 || t < 0.97 * best) {
+      best = t;
+      bs = s;
+    }
+  }
+  return bs;
 }
 
 long qp_part_floats(const QPLaunch& L) {

@@ -384,7 +384,7 @@ int prefill_layer_locked(kans_qlayer* L, const void* X, int x_dtype, long ldx, v
   P.y_dtype = y_dtype;
   P.B = B;
   P.D_in = L->D_in;
-  P.splits = qp_choose_splits(B, L->D_in, L->D_out, 8);
+  P.splits = qp_choose_splits(B, L->D_in, L->D_out, 8, L->K + L->has_base - prefill_fold(L, L->basis));
   P.epi = QP_EPI_PLAIN;
   const long pf = qp_part_floats(P);
   if (pf > 0) {
@@ -451,7 +451,7 @@ int plan_gated_prefill(kans_gated* G, const void* X, int x_dtype, long ldx, void
   P1.y_dtype = hdt;
   P1.B = B;
   P1.D_in = g->D_in;
-  P1.splits = qp_choose_splits(B, g->D_in, h, 4);
+  P1.splits = qp_choose_splits(B, g->D_in, h, 4, g->K + g->has_base - prefill_fold(g, BASIS_CHEBY));
   P1.epi = QP_EPI_SWIGLU;
   P1.round16 = round16;
   P2 = QPLaunch{};
@@ -469,7 +469,7 @@ int plan_gated_prefill(kans_gated* G, const void* X, int x_dtype, long ldx, void
   P2.y_dtype = y_dtype;
   P2.B = B;
   P2.D_in = h;
-  P2.splits = qp_choose_splits(B, h, d->D_out, 8);
+  P2.splits = qp_choose_splits(B, h, d->D_out, 8, d->K + d->has_base - prefill_fold(d, BASIS_CHEBY));
   P2.epi = QP_EPI_PLAIN;
   GP.hidden_bytes = (size_t)B * ldh * dt_bytes(hdt);
   GP.part_bytes = (size_t)std::max(qp_part_floats(P1), qp_part_floats(P2)) * sizeof(float);
@@ -1093,6 +1093,11 @@ int kans_gated_forward_noalloc(kans_gated* G, const void* X, int x_dtype, long l
   if (B > kMaxDecodeB || !g->decode) {
     GatedPrefill GP;
     if ((rc = plan_gated_prefill(G, X, x_dtype, ldx, Y, y_dtype, ldy, B, round16, GP))) return rc;
+    // fewer splits where the chosen ones do not fit the scratch
+    for (QPLaunch* P : {&GP.P1, &GP.P2})
+      while (P->splits > 1 && GP.hidden_bytes + qp_part_floats(*P) * sizeof(float) + 1024 > kScratchBytes - kScratchCnt)
+        --P->splits;
+    GP.part_bytes = (size_t)std::max(qp_part_floats(GP.P1), qp_part_floats(GP.P2)) * sizeof(float);
     void* hidden = sc.take<char>(GP.hidden_bytes);
     float* part = GP.part_bytes ? sc.take<float>(GP.part_bytes) : nullptr;
     if (sc.need > kScratchBytes) return too_big(sc.need);
