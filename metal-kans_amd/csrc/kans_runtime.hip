@@ -121,6 +121,11 @@ static size_t dtype_size(int dt) { return dt == DT_F32 ? 4 : 2; }
 // ---------------------------------------------------------------------------
 // Layer
 // ---------------------------------------------------------------------------
+// Tile (wm rows per wave, nb 32-column blocks), feature splits and wave groups of a forward.
+struct TileCfg {
+  int wm, nb, splits, ks;
+};
+
 struct kans_layer {
   int basis, dtype, D_in, D_out, K, has_base, has_bias;
   int D_in8, nfb, nob_pad;
@@ -133,6 +138,9 @@ struct kans_layer {
   int forced_ks = 0;  // wave groups per workgroup override (0 = heuristic)
   int block_pairs = 1;  // block kernels: two feature blocks per LDS stage when they fit
   unsigned gen = 0;  // bumped whenever a buffer captured by a graph may have moved
+  TileCfg cfg{};     // tile_cfg_locked: the configuration of a forward of cfg_B rows
+  int cfg_B = -1;
+  unsigned tile_gen = 0, cfg_gen = 0;  // tile_gen: bumped whenever a tiling override changes
 };
 
 // Scaled-centre table of the RBF basis: phi_k = exp2(-(s*x - s*c_k)^2) with
@@ -269,6 +277,7 @@ int kans_layer_set_tiling(kans_layer* L, int wm, int nb, int splits) {
   L->forced_wm = wm;
   L->forced_nb = nb;
   L->forced_splits = splits;
+  ++L->tile_gen;
   ++L->gen;
   return 0;
 }
@@ -278,6 +287,7 @@ int kans_layer_set_wave_groups(kans_layer* L, int groups) {
   if (groups != 0 && groups != 1 && groups != 2 && groups != 4)
     return kans_fail(KANS_ERR_ARG, "wave groups must be 0 (automatic), 1, 2 or 4");
   L->forced_ks = groups;
+  ++L->tile_gen;
   ++L->gen;
   return 0;
 }
@@ -374,102 +384,148 @@ int kans_layer_load_weights_device(kans_layer* L, const void* W, const void* W_b
 
 }  // extern "C"
 
-// Tile configuration.  Preference orders come from MI355X timings at
-// 16384 x 1024 -> 1024 (16-bit) and 8192 x 1024 -> {1024, 4096} (fp32):
-//   16-bit, every basis (32,8) -- the 8-wave block kernel: 8 basis values per
-//                                lane feed 8 MFMAs;
-//   fp32 Chebyshev / RBF (32,4); fp32 B-spline (32,8).
-// 1. The first shape in that order whose tiles alone fill every CU's resident
-//    workgroup slots (256 for the 8-wave block kernel, 512 otherwise).
-// 2. Else the first of (32,4), (32,8), (64,4), (32,1) that fills half of them
-//    with a feature split of at most nfb / 8 (>= 8 feature blocks per split):
-//    measured on the config-2 chain's layers (4096 x 784 -> 256 best at
-//    (32,4) x 4 splits, 4096 x 256 -> 256 at (32,1) unsplit).
-// 3. Else the shape with the most tiles, split towards 512 workgroups, at most
-//    nfb / 2 ways on the block kernel (4096 x 256 -> 10: (32,1) x 8) and nfb
-//    ways on the per-slot kernel.
-static void choose_tiling(const kans_layer* L, int B, int* wm, int* nb, int* splits) {
-  static const int pref_n8[4][2] = {{32, 8}, {64, 4}, {32, 4}, {32, 1}};
-  static const int pref_small[4][2] = {{32, 4}, {32, 8}, {64, 4}, {32, 1}};
-  const bool f32 = L->dtype == DT_F32;
-  const int(*cand)[2] = pref_n8;
-  const int nob = (L->D_out + 31) / 32;
-  const int KP = L->slots;
-  // workgroups of shape (ww, nn): the 8-wave block kernel's tile is 8 row blocks tall
-  // (fp32: 32 rows per wave, 8 or 4 waves)
-  auto waves_of = [&](int ww, int nn) {
-    if (f32) return split_waves(ww, nn);
-    return block_waves(true, L->basis, ww, nn, KP) == 8 ? 8 : 4;
-  };
-  auto wgs = [&](int ww, int nn) {
-    const int rows = waves_of(ww, nn) * (f32 ? 32 : ww);
-    return ((B + rows - 1) / rows) * ((nob + nn - 1) / nn);
-  };
-  auto slots = [&](int ww, int nn) { return waves_of(ww, nn) == 8 ? 256 : 512; };
-  auto mostly_padding = [&](int nn) {
-    const int padded = ((nob + nn - 1) / nn) * nn;
-    return nn > 1 && 2 * nob < padded;  // over half of the N-tile would be padding
-  };
-  int bw = 0, bn = 0, s = 1;
-  for (int i = 0; i < 4 && !bw; ++i) {
-    const int* c = cand[i];
-    if (!mostly_padding(c[1]) && wgs(c[0], c[1]) >= slots(c[0], c[1])) { bw = c[0]; bn = c[1]; }
-  }
-  const int smax = std::max(1, L->nfb / 8);
-  for (int i = 0; i < 4 && !bw; ++i) {
-    const int* c = pref_small[i];
-    if (mostly_padding(c[1])) continue;
-    const int t = wgs(c[0], c[1]), need = slots(c[0], c[1]) / 2;
-    const int sc = std::min(smax, (need + t - 1) / t);
-    if ((long)t * sc >= need) { bw = c[0]; bn = c[1]; s = sc; }
-  }
-  if (!bw) {
-    bw = 32; bn = 1;
-    int bt = wgs(32, 1);  // (32, 1) always fits
-    for (int i = 0; i < 4; ++i) {
-      const int* c = cand[i];
-      if (mostly_padding(c[1])) continue;
-      if (wgs(c[0], c[1]) > bt) { bw = c[0]; bn = c[1]; bt = wgs(c[0], c[1]); }
-    }
-    // at most one feature block per split on the per-slot kernel (one barrier per
-    // slot: a shorter chain pays; 256 x 64 -> 64 fp32: 4 splits 9.0 us, 2 splits
-    // 12.8 us), two on the block kernel
-    const bool per_slot = block_waves(!f32, L->basis, bw, bn, KP) == 0;
-    s = std::max(1, std::min((512 + bt - 1) / bt, std::max(1, per_slot ? L->nfb : L->nfb / 2)));
-  }
-  if (L->forced_wm && L->forced_nb) { bw = L->forced_wm; bn = L->forced_nb; }
-  if (L->forced_splits) s = L->forced_splits;
-  *wm = bw;
-  *nb = bn;
-  *splits = s;
+// Tile, feature splits and wave groups of one forward: those with the least
+// estimated time.  A configuration's estimate is, with n workgroups on the
+// fullest of the 256 CUs, F feature blocks per workgroup (per wave group) and
+// S slots per block,
+//   n = 1:  F S alone + F block + wg                   one workgroup on a CU
+//   n > 1:  n (F S shared + F block + wg)              (rate with neighbours)
+//   + launch + (splits > 1: split_us + split_mb * MB of partial sums)
+// in us.  The coefficients are non-negative least-squares fits (relative error
+// 5 to 14 %) to 11 500 timings: three bases, K = 4 to 9, fp16 and fp32, rows
+// 256 to 8192, widths 10 to 2048, 1 to 16 splits.  Choosing by them came within
+// 2 % of the fastest configuration on average (18 % at most); the earlier rule
+// (a preference order, first shape whose tiles fill the chip) took 1.47 times
+// the fastest on average and up to 5.5 times: it preferred 32-column tiles
+// without a split, which generate every basis value anew for each 32 columns,
+// to larger tiles with one.  4096 x 1024 -> 1024, K = 8 + base, fp16, us: RBF
+// 273 -> 94, B-spline 413 -> 95; fp32 738 -> 374 and 655 -> 262.
+struct TileCost {
+  int wm, nb, ks;
+  float alone, shared, wg, block, split_us, split_mb, launch;
+};
+
+// 16-bit Chebyshev (block kernels)
+static const TileCost kCostCheby16[] = {
+    {32, 8, 1, 0.286f, 0.285f, 0.0f, 0.581f, 2.88f, 0.194f, 3.42f},
+    {64, 4, 1, 0.179f, 0.105f, 0.0f, 0.66f, 2.0f, 0.187f, 4.76f},
+    {32, 4, 1, 0.117f, 0.0723f, 0.0f, 0.353f, 2.17f, 0.172f, 3.85f},
+    {32, 4, 2, 0.181f, 0.178f, 0.0f, 0.642f, 1.74f, 0.249f, 4.52f},
+    {32, 1, 1, 0.0823f, 0.0321f, 0.0f, 0.257f, 2.35f, 0.106f, 3.98f},
+    {32, 1, 2, 0.102f, 0.0609f, 0.0f, 0.5f, 2.59f, 0.118f, 3.79f},
+    {32, 1, 4, 0.13f, 0.123f, 0.747f, 1.11f, 2.22f, 0.151f, 3.48f}};
+// 16-bit RBF, and the per-slot kernel of any basis whose slots exceed the block
+// kernels' (its (32, 8) tile has 128 rows: about the (64, 4) one's work)
+static const TileCost kCostRbf16[] = {
+    {32, 8, 1, 0.352f, 0.36f, 0.0f, 0.0f, 3.25f, 0.197f, 2.8f},
+    {64, 4, 1, 0.462f, 0.268f, 0.0f, 0.0f, 1.97f, 0.195f, 4.89f},
+    {32, 4, 1, 0.35f, 0.164f, 0.0f, 0.0f, 2.94f, 0.163f, 3.39f},
+    {32, 1, 1, 0.244f, 0.0964f, 0.0f, 0.0f, 1.8f, 0.0901f, 5.2f}};
+static const TileCost kCostBspline16[] = {
+    {32, 8, 1, 0.369f, 0.369f, 0.0f, 0.0f, 3.22f, 0.193f, 3.49f},
+    {64, 4, 1, 0.741f, 0.465f, 0.0f, 0.0f, 2.71f, 0.17f, 4.65f},
+    {32, 4, 1, 0.423f, 0.205f, 0.0f, 0.0f, 2.74f, 0.154f, 3.96f},
+    {32, 1, 1, 0.335f, 0.156f, 0.0f, 0.0f, 1.59f, 0.0826f, 5.57f}};
+// fp32 (kan_fused_split, B-spline K >= 5 kan_fused_split_sparse)
+static const TileCost kCostCheby32[] = {
+    {32, 8, 1, 1.91f, 1.93f, 1.42f, 0.53f, 5.05f, 0.284f, 2.59f},
+    {64, 4, 1, 1.0f, 1.04f, 0.0f, 0.292f, 2.7f, 0.242f, 4.34f},
+    {32, 4, 1, 0.775f, 0.555f, 0.0f, 0.265f, 2.75f, 0.191f, 4.38f},
+    {32, 1, 1, 0.363f, 0.238f, 0.0f, 0.196f, 2.39f, 0.171f, 4.27f}};
+static const TileCost kCostRbf32[] = {
+    {32, 8, 1, 1.96f, 2.0f, 2.42f, 0.0f, 6.81f, 0.294f, 0.0f},
+    {64, 4, 1, 1.09f, 1.11f, 0.0f, 0.0f, 3.66f, 0.248f, 3.26f},
+    {32, 4, 1, 0.873f, 0.618f, 0.0f, 0.0f, 3.5f, 0.189f, 3.58f},
+    {32, 1, 1, 0.443f, 0.285f, 0.0f, 0.0f, 2.35f, 0.162f, 4.46f}};
+static const TileCost kCostSparse32[] = {
+    {32, 8, 1, 1.32f, 1.34f, 2.99f, 0.0f, 4.02f, 0.247f, 0.0f},
+    {64, 4, 1, 0.838f, 0.827f, 0.0f, 0.0f, 3.27f, 0.233f, 3.33f},
+    {32, 4, 1, 0.709f, 0.482f, 0.0f, 0.0f, 3.01f, 0.182f, 3.82f},
+    {32, 1, 1, 0.357f, 0.252f, 0.0f, 0.0f, 2.51f, 0.147f, 4.01f}};
+
+// Rows of a workgroup's tile.
+static int tile_rows(const kans_layer* L, int wm, int nb) {
+  if (L->dtype == DT_F32) return 32 * split_waves(wm, nb);
+  return (block_waves(true, L->basis, wm, nb, L->slots) == 8 ? 8 : 4) * wm;
 }
 
-// Wave groups per workgroup (KS) of the 4-wave block kernel for a forward of
-// batch B on tile (wm, nb) x splits.  A layer that leaves at most one such
-// workgroup per CU gets 4 groups on (32,1) or 2 on (32,4), when each group
-// still has at least 4 feature blocks: one workgroup per CU then holds 4·KS
-// waves instead of 4, each with a KS times shorter chain of blocks.  A forced
-// tile keeps one group unless the groups are forced too; a forced count that
-// the tile is not instantiated with falls back to 1.
-static int choose_wave_groups(const kans_layer* L, int B, int wm, int nb, int splits) {
-  if (block_waves(L->dtype != DT_F32, L->basis, wm, nb, L->slots) != 4) return 1;
-  if (L->forced_ks) return block_wave_groups_ok(wm, nb, L->forced_ks) ? L->forced_ks : 1;
-  if (L->forced_wm) return 1;
-  const long wgs = (long)((B + 4 * wm - 1) / (4 * wm)) * (((L->D_out + 31) / 32 + nb - 1) / nb) * splits;
-  const int fbps = (L->nfb + splits - 1) / splits;
-  if (wgs > 256) return 1;
-  if (block_wave_groups_ok(wm, nb, 4) && fbps >= 16) return 4;
-  if (block_wave_groups_ok(wm, nb, 2) && fbps >= 8) return 2;
-  return 1;
+static bool tile_groups_ok(const kans_layer* L, int wm, int nb, int ks) {
+  return ks == 1 || (L->dtype != DT_F32 && block_waves(true, L->basis, wm, nb, L->slots) == 4 &&
+                     block_wave_groups_ok(wm, nb, ks));
+}
+
+// Partial sums of a split forward are kept below this.
+constexpr double kMaxPartMB = 256.0;
+
+static TileCfg choose_tiling(const kans_layer* L, int B) {
+  const TileCost* table;
+  int rows = 4;
+  if (L->dtype == DT_F32) {
+    table = L->sparse ? kCostSparse32 : L->basis == BASIS_CHEBY ? kCostCheby32 : kCostRbf32;
+  } else if (L->basis == BASIS_CHEBY && block_waves(true, L->basis, 32, 4, L->slots) == 4) {
+    table = kCostCheby16;
+    rows = (int)(sizeof(kCostCheby16) / sizeof(kCostCheby16[0]));
+  } else {
+    table = L->basis == BASIS_BSPLINE ? kCostBspline16 : kCostRbf16;
+  }
+  const bool per_slot8 = L->dtype != DT_F32 && block_waves(true, L->basis, 32, 8, L->slots) == 0;
+  const int nob = (L->D_out + 31) / 32;
+  TileCfg best{32, 1, 1, 1};
+  double best_t = 0.0;
+  bool any = false;
+  for (int i = 0; i < rows; ++i) {
+    const TileCost& c = per_slot8 && i == 0 ? table[1] : table[i];  // coefficients
+    const int wm = table[i].wm, nb = table[i].nb, ks = table[i].ks;
+    if (L->forced_wm && (wm != L->forced_wm || nb != L->forced_nb || ks != 1)) continue;
+    const int tr = tile_rows(L, wm, nb);
+    const long tiles = (long)((B + tr - 1) / tr) * ((nob + nb - 1) / nb);
+    int last = 0;  // splits that come to the same feature blocks each are looked at once
+    for (int s = 1; s <= std::min(L->nfb, 32); ++s) {
+      const int fbps = L->forced_splits ? (L->nfb + L->forced_splits - 1) / L->forced_splits : (L->nfb + s - 1) / s;
+      if (fbps == last || (ks > 1 && fbps < 2 * ks)) continue;
+      last = fbps;
+      const int splits = (L->nfb + fbps - 1) / fbps;
+      const double mb = splits > 1 ? 8e-6 * splits * B * L->D_out : 0.0;
+      if (splits > 1 && mb > 2.0 * kMaxPartMB && !L->forced_splits) break;
+      const double n = (double)((tiles * splits + 255) / 256), F = (fbps + ks - 1) / ks;
+      double t = n * (F * L->slots * (n > 1 ? c.shared : c.alone) + F * c.block + c.wg) + c.launch;
+      if (splits > 1) t += c.split_us + mb * c.split_mb;
+      if (!any || t < best_t) {
+        any = true;
+        best_t = t;
+        best = TileCfg{wm, nb, L->forced_splits ? L->forced_splits : splits, ks};
+      }
+    }
+  }
+  if (L->forced_wm) {
+    best.wm = L->forced_wm;
+    best.nb = L->forced_nb;
+    best.ks = 1;
+    // a forced tile keeps one split unless the splits are forced too
+    best.splits = L->forced_splits ? L->forced_splits : best.splits;
+  }
+  // a forced group count that the tile is not instantiated with falls back to 1
+  if (L->forced_ks) best.ks = tile_groups_ok(L, best.wm, best.nb, L->forced_ks) ? L->forced_ks : 1;
+  return best;
+}
+
+// The configuration of a forward of batch B, kept for the last batch size (library lock held; gen changes
+// with every setting it depends on).
+static const TileCfg& tile_cfg_locked(kans_layer* L, int B) {
+  if (L->cfg_B != B || L->cfg_gen != L->tile_gen) {
+    L->cfg = choose_tiling(L, B);
+    L->cfg_B = B;
+    L->cfg_gen = L->tile_gen;
+  }
+  return L->cfg;
 }
 
 // Reserve the split workspace a forward of batch B needs (no launch).
 static int layer_reserve_locked(kans_layer* L, int B) {
-  int wm, nb, splits;
-  choose_tiling(L, B, &wm, &nb, &splits);
-  if (splits > 1) {
+  const TileCfg& cfg = tile_cfg_locked(L, B);
+  if (cfg.splits > 1) {
     void* old = L->part.p;
-    int rc = L->part.reserve((size_t)splits * B * L->D_out * sizeof(float));
+    int rc = L->part.reserve((size_t)cfg.splits * B * L->D_out * sizeof(float));
     if (rc) return rc;
     if (old != L->part.p) ++L->gen;
   }
@@ -480,9 +536,10 @@ static int layer_reserve_locked(kans_layer* L, int B) {
 // ran before (the chain relies on this while capturing a graph).
 // cfg_B > 0: use the tile configuration a forward of cfg_B rows would use (the
 // chunked host forward launches row chunks of a batch with the whole batch's
-// configuration, so every row gets the same result as in one launch).
+// configuration, so every row gets the same result as in one launch; row0, the
+// chunk's first row, gives each chunk its own part of the split workspace).
 static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, long ldy, int B, hipStream_t st,
-                               int x_dtype = -1, int y_dtype = -1, int cfg_B = 0) {
+                               int x_dtype = -1, int y_dtype = -1, int cfg_B = 0, long row0 = 0) {
   if (x_dtype < 0) x_dtype = L->dtype;
   if (y_dtype < 0) y_dtype = L->dtype;
   if ((x_dtype != L->dtype && x_dtype != DT_F32) || (y_dtype != L->dtype && y_dtype != DT_F32))
@@ -516,13 +573,16 @@ static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, 
   D.nfb = L->nfb;
   D.bp = L->bp;
   if (cfg_B <= 0) cfg_B = B;
-  choose_tiling(L, cfg_B, &D.wm, &D.nb, &D.splits);
-  D.ks = choose_wave_groups(L, cfg_B, D.wm, D.nb, D.splits);
+  const TileCfg& cfg = tile_cfg_locked(L, cfg_B);
+  D.wm = cfg.wm;
+  D.nb = cfg.nb;
+  D.splits = cfg.splits;
+  D.ks = cfg.ks;
   D.pair = L->block_pairs;
   if (D.splits > 1) {
-    if (L->part.cap < (size_t)D.splits * B * L->D_out * sizeof(float))
+    if (L->part.cap < (size_t)D.splits * (row0 + B) * L->D_out * sizeof(float))
       return kans_fail(KANS_ERR_STATE, "split workspace not reserved");
-    D.part = (float*)L->part.p;
+    D.part = (float*)L->part.p + (size_t)D.splits * row0 * L->D_out;
   }
   HIP_TRY(launch_dense(D, st));
   return 0;
@@ -540,9 +600,9 @@ static int layer_forward_locked(kans_layer* L, const void* X, long ldx, void* Y,
 // the PCIe transfers in both directions and the kernels of different chunks
 // overlap; the host copies of chunk c + 1 run while the device works on
 // chunk c.  Every chunk is launched with the tile configuration of the whole
-// batch, which leaves each row's result exactly what one launch gives; only
-// configurations without a feature split are chunked (no workspace is shared
-// by chunk kernels that may run at the same time).  Chunks are whole 256-row
+// batch, which leaves each row's result exactly what one launch gives, and
+// chunk kernels, which may run at the same time, have their own rows of the
+// split workspace.  Chunks are whole 256-row
 // tiles.  Measured on one MI355X, FastKAN fp16 16384 x 1024 -> 1024 from and
 // into host arrays: 2.06 -> 1.54 ms per call (the C entry point, output array
 // reused), 2.87 -> 1.92 ms through FastKAN.__call__ (a fresh output array).
@@ -592,7 +652,7 @@ static int layer_forward_host_chunked(kans_layer* L, const void* X, void* Y, int
     if (hipEventRecord(e_in, g_copy_in) != hipSuccess || hipStreamWaitEvent(cs, e_in, 0) != hipSuccess)
       return fail(kans_fail(KANS_ERR_HIP, "chunked host forward: input event"));
     if ((rc = layer_launch_locked(L, xd + r0 * pitch_in, ldx, yd + r0 * row_out, L->D_out, rows, cs, x_dtype,
-                                  L->dtype, B)))
+                                  L->dtype, B, r0)))
       return fail(rc);
     if (hipEventRecord(e_k, cs) != hipSuccess || hipStreamWaitEvent(g_copy_out, e_k, 0) != hipSuccess)
       return fail(kans_fail(KANS_ERR_HIP, "chunked host forward: kernel event"));
@@ -642,11 +702,7 @@ static int layer_forward_host_locked(kans_layer* L, const void* X, void* Y, int 
   }
   if ((rc = pinned_reserve(g_pin_in, xbytes))) return rc;
   if ((rc = pinned_reserve(g_pin_out, ybytes))) return rc;
-  if (xbytes + ybytes >= kChunkedBytes && B >= 2 * 256) {
-    int wm, nb, splits;
-    choose_tiling(L, B, &wm, &nb, &splits);
-    if (splits == 1) return layer_forward_host_chunked(L, X, Y, B, x_dtype);
-  }
+  if (xbytes + ybytes >= kChunkedBytes && B >= 2 * 256) return layer_forward_host_chunked(L, X, Y, B, x_dtype);
   if ((rc = stage_in(L->x_d.p, X, row_in, pitch_in, B, g_pin_in.p, g_stream))) return rc;
   if ((rc = layer_launch_locked(L, L->x_d.p, ldx, L->y_d.p, L->D_out, B, g_stream, x_dtype, L->dtype))) {
     (void)hipStreamSynchronize(g_stream);  // the input DMAs read g_pin_in; finish them before it is reused
@@ -701,7 +757,10 @@ int kans_layer_forward_host_ex(kans_layer* L, const void* X, int x_dtype, void* 
 
 int kans_layer_describe(const kans_layer* L, int B, int* wm, int* nb, int* splits) {
   if (!L || !wm || !nb || !splits) return kans_fail(KANS_ERR_ARG, "null argument");
-  choose_tiling(L, B, wm, nb, splits);
+  const TileCfg cfg = choose_tiling(L, B);
+  *wm = cfg.wm;
+  *nb = cfg.nb;
+  *splits = cfg.splits;
   return 0;
 }
 
@@ -710,12 +769,11 @@ int kans_layer_describe(const kans_layer* L, int B, int* wm, int* nb, int* split
 // types of X and Y as well, in template order ("kans::kan_fused_block<_Float16, _Float16, _Float16,
 // BASIS_RBF_REC, 32, 8, 8 waves>"), as launch_dense routes x_dtype / y_dtype.
 static int layer_kernel_name(const kans_layer* L, int B, bool io, int x_dtype, int y_dtype, char* name, int len) {
-  int wm, nb, splits;
-  choose_tiling(L, B, &wm, &nb, &splits);
+  const TileCfg cfg = choose_tiling(L, B);
+  const int wm = cfg.wm, nb = cfg.nb, splits = cfg.splits, ks = cfg.ks;
   static const char* dt[] = {"float", "_Float16", "__bf16"};
   static const char* bs[] = {"BASIS_CHEBY", "BASIS_RBF", "BASIS_BSPLINE"};
   const int waves = block_waves(L->dtype != DT_F32, L->basis, wm, nb, L->slots);
-  const int ks = choose_wave_groups(L, B, wm, nb, splits);
   char groups[32] = "";
   if (ks > 1) snprintf(groups, sizeof groups, " x %d groups", ks);
   const bool pairs = waves == 8 && L->basis == BASIS_CHEBY && L->block_pairs && 2 * L->slots <= 10;

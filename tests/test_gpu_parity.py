@@ -909,3 +909,28 @@ def test_f32_infinite_and_nan_inputs(gpu, kind, K):
     assert np.array_equal(y[rows], ref[rows])
     assert np.array_equal(y[3], np.sign(L.w_base[:, 7]) * np.inf)
     assert np.isnan(y[5]).all() and np.isnan(y[6]).all()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("kind,K", [("cheby", 4), ("cheby", 9), ("cheby", 14), ("rbf", 8), ("rbf", 11), ("bspline", 8),
+                                    ("bspline", 6)])
+@pytest.mark.parametrize("B,d_in,d_out", [(1, 3, 5), (257, 33, 65), (700, 300, 500), (1300, 130, 33), (300, 777, 260)])
+def test_automatic_configuration(gpu, dtype, kind, K, B, d_in, d_out):
+    """The tile, splits and wave groups that a forward chooses by itself, from one row to several tiles, against
+    the oracle on sampled rows and against an unsplit (32, 4) forward; a rerun is bit-identical."""
+    import metal_kans as mk
+    L = make_layer(mk, kind, d_in, d_out, K, bias=True, base=True, seed=B)
+    x = np.random.default_rng(K).uniform(-1.2, 1.2, (B, d_in)).astype(np.float32)
+    rows = np.unique(np.linspace(0, B - 1, 24).astype(int))
+    y_ref = oracle_of(L, x[rows])
+    cast(L, dtype)
+    y = np.asarray(L(x))
+    assert O.rel_err(y[rows], y_ref) <= TOL[dtype]
+    assert np.array_equal(np.asarray(L(x)), y)
+    wm, nb, sp = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    h = L._engine().handle
+    assert gpu.kans_layer_describe(h, B, ctypes.byref(wm), ctypes.byref(nb), ctypes.byref(sp)) == 0
+    assert (wm.value, nb.value) in ((64, 4), (32, 8), (32, 4), (32, 1)) and 1 <= sp.value <= (d_in + 15) // 16
+    L.set_tiling(32, 4, 1)
+    # the same products in another order: fp32 rounding, then the output type's
+    assert O.rel_err(y, np.asarray(L(x), np.float64)) <= {"float32": 4e-6, "float16": 2e-3}[dtype]
