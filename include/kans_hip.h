@@ -41,6 +41,10 @@ extern "C" {
 #define KANS_DT_F16 1
 #define KANS_DT_BF16 2
 
+/* `stream` arguments: a hipStream_t, NULL for the library's own stream (kans_stream()), or this for HIP's
+ * default stream, whose own handle is null */
+#define KANS_STREAM_LEGACY ((void*)1)
+
 const char* kans_last_error(void);
 
 /* ======================================================================= *
@@ -200,6 +204,11 @@ int kans_layer_kernel_ex(const kans_layer* layer, int B, int x_dtype, int y_dtyp
 /* weights in the layer dtype: W [D_out][D_in*K] (k fastest), W_base [D_out][D_in], bias [D_out] */
 int kans_layer_load_weights(kans_layer* layer, const void* W, const void* W_base, const void* bias);
 int kans_layer_load_weights_device(kans_layer* layer, const void* W, const void* W_base, const void* bias);
+/* as kans_layer_load_weights_device, enqueued on `stream` (NULL = kans_stream()) and not waited for: forwards
+ * on this stream run behind it, forwards on other streams wait for it on the device; the arrays stay as they
+ * are until the stream has passed the call (a training step re-tiles its weights before every forward) */
+int kans_layer_load_weights_stream(kans_layer* layer, const void* W, const void* W_base, const void* bias,
+                                   void* stream);
 /* host fp32 weights converted on the device to the layer dtype (round to nearest even) */
 int kans_layer_load_weights_f32(kans_layer* layer, const float* W, const float* W_base, const float* bias);
 /* device pointers; X [B][ldx] with ldx >= round_up(D_in, 8), ldx % 8 == 0, X 16-byte aligned and

@@ -74,6 +74,15 @@ int kans_fail(int code, const char* fmt, ...);
 // called by the library's initialisation with `device` current.
 int kans_noalloc_setup(int device);
 hipStream_t kans_default_stream();
+// The stream of an entry point's `stream` argument: NULL is the library's own, KANS_STREAM_LEGACY the HIP
+// default stream (whose handle is itself null; the runtime's own pseudo-handle for it must not reach event
+// calls: waiting for an event recorded through it crashed).
+inline hipStream_t kans_caller_stream(void* stream) {
+  if (!stream) return kans_default_stream();
+  return stream == KANS_STREAM_LEGACY ? (hipStream_t) nullptr : (hipStream_t)stream;
+}
+// Whether st is under graph capture (the default stream never is).
+hipError_t kans_capturing(hipStream_t st, bool* capturing);
 // fp32 Chebyshev forward (no base branch) of host X on device-resident fp32 weights (kans_runtime.hip);
 // call with the library lock held.
 int kans_ref_cheby_forward_devw_locked(const float* X, const float* W_dev, const float* bias_dev, float* Y, int B,

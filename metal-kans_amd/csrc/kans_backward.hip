@@ -679,11 +679,11 @@ int kans_cheby_backward(const float* dY, const float* X, const float* W, const f
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(kans_mutex());
   if ((rc = kans_ensure_init())) return rc;
-  hipStream_t st = stream ? (hipStream_t)stream : kans_default_stream();
+  hipStream_t st = kans_caller_stream(stream);
   // a call recorded into a graph outlives this one: it gets no share of the common workspace
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(st, &cap));
-  const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, cap == hipStreamCaptureStatusNone);
+  bool capturing = false;
+  HIP_TRY(kans_capturing(st, &capturing));
+  const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, !capturing);
   float* ws;
   if ((rc = acquire_ws(plan.ws_floats, st, &ws))) return rc;
   HIP_TRY(launch_cheby_backward(dY, X, W, has_base ? W_base : nullptr, dW, has_base ? dW_base : nullptr,

@@ -962,7 +962,7 @@ int kans_qlayer_forward(kans_qlayer* L, const void* X, int x_dtype, long ldx, vo
   std::lock_guard<std::mutex> lk(kans_mutex());
   int rc = kans_ensure_init();
   if (rc) return rc;
-  hipStream_t st = stream ? (hipStream_t)stream : kans_default_stream();
+  hipStream_t st = kans_caller_stream(stream);
   return qlayer_forward_locked(L, X, x_dtype, ldx, Y, y_dtype, ldy, B, st);
 }
 
@@ -1047,7 +1047,7 @@ int kans_gated_forward(kans_gated* G, const void* X, int x_dtype, long ldx, void
   std::lock_guard<std::mutex> lk(kans_mutex());
   int rc = kans_ensure_init();
   if (rc) return rc;
-  hipStream_t st = stream ? (hipStream_t)stream : kans_default_stream();
+  hipStream_t st = kans_caller_stream(stream);
   return gated_forward_locked(G, X, x_dtype, ldx, Y, y_dtype, ldy, B, round16, st);
 }
 
@@ -1079,7 +1079,7 @@ int kans_gated_forward_noalloc(kans_gated* G, const void* X, int x_dtype, long l
   HIP_TRY(hipGetDevice(&dev));
   auto it = g_scratch.find(dev);
   if (it == g_scratch.end()) return kans_fail(KANS_ERR_STATE, "no scratch set up on device %d", dev);
-  hipStream_t st = stream ? (hipStream_t)stream : kans_default_stream();
+  hipStream_t st = kans_caller_stream(stream);
   kans_qlayer *g = G->gate, *d = G->down;
   if ((rc = check_y(Y, y_dtype, ldy, d->D_out))) return rc;
   if (B < 0) return kans_fail(KANS_ERR_ARG, "B=%d < 0", B);

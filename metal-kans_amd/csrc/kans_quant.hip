@@ -316,7 +316,7 @@ int kans_dequantize_affine_device(const void* q, const float* scales, const floa
   int rc = kans_init();
   if (rc) return rc;
   return dequant_affine_device(q, scales, biases, out, num_groups, group_size, bits,
-                               stream ? (hipStream_t)stream : kans_default_stream());
+                               kans_caller_stream(stream));
 }
 
 int kans_dequantize_ternary_device(const uint32_t* packed, const float* scales, float* out, int D_out, int K_dim,
@@ -326,7 +326,7 @@ int kans_dequantize_ternary_device(const uint32_t* packed, const float* scales, 
   int rc = kans_init();
   if (rc) return rc;
   return dequant_ternary_device(packed, scales, out, D_out, K_dim, group_size,
-                                stream ? (hipStream_t)stream : kans_default_stream());
+                                kans_caller_stream(stream));
 }
 
 // Device copy of `bytes` (multiple of 16, 16-byte aligned pointers) with a plain kernel.
@@ -337,7 +337,7 @@ int kans_copy_device(void* dst, const void* src, size_t bytes, void* stream) {
   if (rc) return rc;
   const long n = (long)(bytes / 16);
   hipLaunchKernelGGL(k_copy_u4, dim3(std::min<long>((n + 255) / 256, 8192)), dim3(256), 0,
-                     stream ? (hipStream_t)stream : kans_default_stream(), (const uint4*)src, (uint4*)dst, n);
+                     kans_caller_stream(stream), (const uint4*)src, (uint4*)dst, n);
   HIP_TRY(hipGetLastError());
   return 0;
 }

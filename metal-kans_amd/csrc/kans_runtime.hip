@@ -106,6 +106,13 @@ static int ensure_init() {
 
 hipStream_t kans_default_stream() { return g_stream; }
 
+hipError_t kans_capturing(hipStream_t st, bool* capturing) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const hipError_t e = st ? hipStreamIsCapturing(st, &cap) : hipSuccess;
+  *capturing = cap != hipStreamCaptureStatusNone;
+  return e;
+}
+
 std::mutex& kans_mutex() { return g_mu; }
 int kans_ensure_init() { return ensure_init(); }
 int kans_pinned_stage(int which, size_t bytes, void** p) {
@@ -134,6 +141,17 @@ struct kans_layer {
   BasisParams bp{};
   DevBuf Wt, bias_d, part, x_d, y_d, raw_w, raw_wb;
   bool have_weights = false;
+  // weights re-tiled on a caller's stream (kans_layer_load_weights_stream) without waiting for them: work on
+  // another stream waits for w_done first
+  bool w_pending = false;
+  hipStream_t w_stream = nullptr;
+  hipEvent_t w_done = nullptr;
+  // streams the forwards since the last re-tiling ran on: none, one (use_stream), or several
+  bool used = false, used_many = false;
+  hipStream_t use_stream = nullptr;
+  ~kans_layer() {
+    if (w_done) (void)hipEventDestroy(w_done);
+  }
   int forced_wm = 0, forced_nb = 0, forced_splits = 0;  // tuning overrides (0 = heuristic)
   int forced_ks = 0;  // wave groups per workgroup override (0 = heuristic)
   int block_pairs = 1;  // block kernels: two feature blocks per LDS stage when they fit
@@ -305,7 +323,7 @@ int kans_layer_set_block_pairs(kans_layer* L, int on) {
 // W_base: [D_out][D_in] (ignored unless has_base); bias: [D_out] (ignored
 // unless has_bias).  Re-tiles W/W_base into the fused kernel's layout.
 static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, const void* bias, bool device_src,
-                               int src_dtype) {
+                               int src_dtype, hipStream_t st, bool wait) {
   const size_t es = dtype_size(src_dtype);
   const size_t wbytes = (size_t)L->D_out * L->D_in * L->K * es;
   const size_t wbbytes = (size_t)L->D_out * L->D_in * es;
@@ -351,10 +369,14 @@ static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, con
     if ((rc = L->bias_d.reserve((size_t)L->D_out * sizeof(float)))) return rc;
     U.bias_out = (float*)L->bias_d.p;
   }
-  HIP_TRY(launch_upload(U, g_stream));
-  HIP_TRY(hipStreamSynchronize(g_stream));
+  HIP_TRY(launch_upload(U, st));
+  if (wait) {
+    HIP_TRY(hipStreamSynchronize(st));
+    L->w_pending = false;
+  }
   if (L->Wt.p != old_wt || L->bias_d.p != old_bias) ++L->gen;
   L->have_weights = true;
+  L->used = L->used_many = false;
   return 0;
 }
 
@@ -363,7 +385,7 @@ int kans_layer_load_weights(kans_layer* L, const void* W, const void* W_base, co
   if (L->has_base && !W_base) return kans_fail(KANS_ERR_ARG, "has_base=1 but W_base is null");
   if (L->has_bias && !bias) return kans_fail(KANS_ERR_ARG, "has_bias=1 but bias is null");
   std::lock_guard<std::mutex> lk(g_mu);
-  return layer_upload_locked(L, W, W_base, bias, false, L->dtype);
+  return layer_upload_locked(L, W, W_base, bias, false, L->dtype, g_stream, true);
 }
 
 int kans_layer_load_weights_f32(kans_layer* L, const float* W, const float* W_base, const float* bias) {
@@ -371,7 +393,7 @@ int kans_layer_load_weights_f32(kans_layer* L, const float* W, const float* W_ba
   if (L->has_base && !W_base) return kans_fail(KANS_ERR_ARG, "has_base=1 but W_base is null");
   if (L->has_bias && !bias) return kans_fail(KANS_ERR_ARG, "has_bias=1 but bias is null");
   std::lock_guard<std::mutex> lk(g_mu);
-  return layer_upload_locked(L, W, W_base, bias, false, DT_F32);
+  return layer_upload_locked(L, W, W_base, bias, false, DT_F32, g_stream, true);
 }
 
 int kans_layer_load_weights_device(kans_layer* L, const void* W, const void* W_base, const void* bias) {
@@ -379,7 +401,26 @@ int kans_layer_load_weights_device(kans_layer* L, const void* W, const void* W_b
   if (L->has_base && !W_base) return kans_fail(KANS_ERR_ARG, "has_base=1 but W_base is null");
   if (L->has_bias && !bias) return kans_fail(KANS_ERR_ARG, "has_bias=1 but bias is null");
   std::lock_guard<std::mutex> lk(g_mu);
-  return layer_upload_locked(L, W, W_base, bias, true, L->dtype);
+  return layer_upload_locked(L, W, W_base, bias, true, L->dtype, g_stream, true);
+}
+
+int kans_layer_load_weights_stream(kans_layer* L, const void* W, const void* W_base, const void* bias, void* stream) {
+  if (!L || !W) return kans_fail(KANS_ERR_ARG, "null layer or W");
+  if (L->has_base && !W_base) return kans_fail(KANS_ERR_ARG, "has_base=1 but W_base is null");
+  if (L->has_bias && !bias) return kans_fail(KANS_ERR_ARG, "has_bias=1 but bias is null");
+  std::lock_guard<std::mutex> lk(g_mu);
+  hipStream_t st = kans_caller_stream(stream);
+  int rc;
+  // the last re-tiling, and every forward that may still read the tiles, must be done or ahead on this stream
+  if (L->used_many || (L->used && L->use_stream != st) || (L->w_pending && L->w_stream != st))
+    HIP_TRY(hipDeviceSynchronize());
+  if (!L->w_done) HIP_TRY(hipEventCreateWithFlags(&L->w_done, hipEventDisableTiming));
+  L->w_pending = false;
+  if ((rc = layer_upload_locked(L, W, W_base, bias, true, L->dtype, st, false))) return rc;
+  HIP_TRY(hipEventRecord(L->w_done, st));
+  L->w_pending = true;
+  L->w_stream = st;
+  return 0;
 }
 
 }  // extern "C"
@@ -532,6 +573,28 @@ static int layer_reserve_locked(kans_layer* L, int B) {
   return 0;
 }
 
+// Before a kernel on stream st reads the layer's weights: behind a re-tiling still on another stream.  A
+// stream under graph capture cannot wait for an event from outside, so the host waits for it.
+static int layer_use_weights(kans_layer* L, hipStream_t st) {
+  if (L->used && L->use_stream != st) L->used_many = true;
+  L->used = true;
+  L->use_stream = st;
+  if (!L->w_pending || L->w_stream == st) return 0;
+  bool capturing = false;
+  HIP_TRY(kans_capturing(st, &capturing));
+  if (!capturing) {
+    HIP_TRY(hipStreamWaitEvent(st, L->w_done, 0));
+    return 0;
+  }
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  const hipError_t e = hipEventSynchronize(L->w_done);
+  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  HIP_TRY(e);
+  L->w_pending = false;
+  return 0;
+}
+
 // Enqueue one fused forward; allocates nothing when layer_reserve_locked(L, B)
 // ran before (the chain relies on this while capturing a graph).
 // cfg_B > 0: use the tile configuration a forward of cfg_B rows would use (the
@@ -554,6 +617,8 @@ static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, 
     return kans_fail(KANS_ERR_ARG, "fp32 X must be 32-byte aligned");
   if (ldy < L->D_out) return kans_fail(KANS_ERR_ARG, "ldy=%ld < D_out=%d", ldy, L->D_out);
   if (((uintptr_t)X & 15) != 0) return kans_fail(KANS_ERR_ARG, "X must be 16-byte aligned");
+  int rc = layer_use_weights(L, st);
+  if (rc) return rc;
   DenseLaunch D{};
   D.dtype = L->dtype;
   D.x_dtype = x_dtype;
@@ -727,7 +792,7 @@ extern "C" {
 int kans_layer_forward(kans_layer* L, const void* X, long ldx, void* Y, long ldy, int B, void* stream) {
   if (!L || !X || !Y) return kans_fail(KANS_ERR_ARG, "null argument");
   std::lock_guard<std::mutex> lk(g_mu);
-  return layer_forward_locked(L, X, ldx, Y, ldy, B, stream ? (hipStream_t)stream : g_stream);
+  return layer_forward_locked(L, X, ldx, Y, ldy, B, kans_caller_stream(stream));
 }
 
 int kans_layer_forward_ex(kans_layer* L, const void* X, int x_dtype, long ldx, void* Y, int y_dtype, long ldy, int B,
@@ -736,7 +801,7 @@ int kans_layer_forward_ex(kans_layer* L, const void* X, int x_dtype, long ldx, v
   std::lock_guard<std::mutex> lk(g_mu);
   int rc = layer_reserve_locked(L, B);
   if (rc) return rc;
-  return layer_launch_locked(L, X, ldx, Y, ldy, B, stream ? (hipStream_t)stream : g_stream, x_dtype, y_dtype);
+  return layer_launch_locked(L, X, ldx, Y, ldy, B, kans_caller_stream(stream), x_dtype, y_dtype);
 }
 
 int kans_layer_forward_host(kans_layer* L, const void* X, void* Y, int B) {
@@ -1004,7 +1069,7 @@ static int ref_forward(int basis, int dtype, const void* X, const void* W, const
   std::lock_guard<std::mutex> lk(g_mu);
   kans_layer* L;
   if ((rc = sig_layer(basis, dtype, D_in, D_out, K, has_base, has_bias, params, &L))) return rc;
-  if ((rc = layer_upload_locked(L, W, Wb, bias, false, dtype))) return rc;
+  if ((rc = layer_upload_locked(L, W, Wb, bias, false, dtype, g_stream, true))) return rc;
   return layer_forward_host_locked(L, X, Y, B);
 }
 
@@ -1020,7 +1085,7 @@ int kans_ref_cheby_forward_devw_locked(const float* X, const float* W_dev, const
   if (rc) return rc;
   kans_layer* L;
   if ((rc = sig_layer(BASIS_CHEBY, DT_F32, D_in, D_out, K, 0, has_bias, {}, &L))) return rc;
-  if ((rc = layer_upload_locked(L, W_dev, nullptr, bias_dev, true, DT_F32))) return rc;
+  if ((rc = layer_upload_locked(L, W_dev, nullptr, bias_dev, true, DT_F32, g_stream, true))) return rc;
   return layer_forward_host_locked(L, X, Y, B);
 }
 
@@ -1357,7 +1422,7 @@ int kans_chain_forward(kans_chain* C, const void* X, long ldx, void* Y, long ldy
   int rc = chain_reserve(C, B);
   if (rc) return rc;
   C->in_dtype = C->dtype;
-  return chain_launch(C, X, ldx, Y, ldy, B, stream ? (hipStream_t)stream : g_stream);
+  return chain_launch(C, X, ldx, Y, ldy, B, kans_caller_stream(stream));
 }
 
 // Time `iters` replays of the chain graph; include_copies = 1 also replays the
@@ -1441,7 +1506,7 @@ int metal_kan_chain_pipeline_cheby(const float* X, float* Y, int B, int num_laye
     for (int l = 0; l < num_layers; ++l) {
       kans_layer* L = C->layers[l];
       rc = layer_upload_locked(L, W_chebys[l], L->has_base ? W_bases[l] : nullptr, L->has_bias ? biases[l] : nullptr,
-                               false, DT_F32);
+                               false, DT_F32, g_stream, true);
       if (rc) return rc;
     }
   }
@@ -1644,7 +1709,7 @@ int kans_gated_dense_forward(kans_gated_dense* D, const void* X, int x_dtype, lo
   std::lock_guard<std::mutex> lk(g_mu);
   int rc = dgated_reserve(D, B);
   if (rc) return rc;
-  return dgated_launch(D, X, x_dtype, ldx, Y, ldy, B, stream ? (hipStream_t)stream : g_stream);
+  return dgated_launch(D, X, x_dtype, ldx, Y, ldy, B, kans_caller_stream(stream));
 }
 
 // Host arrays [B][d] (x_dtype: the block dtype, or fp32 for a 16-bit block) -> [B][d] (block dtype):

@@ -176,16 +176,16 @@ class LayerEngine:
             self.params = params
 
     def prepare_device(self, dt: int, W_ptr: int, W_base_ptr: Optional[int], bias_ptr: Optional[int],
-                       params: tuple, key: tuple) -> None:
+                       params: tuple, key: tuple, stream=None) -> None:
         """Make the device copy current from device arrays in dtype ``dt`` (e.g. torch tensors); ``key``
-        identifies their contents (pointers and version counters): equal keys skip the re-tiling.  The
-        caller has finished writing the arrays (the upload runs on the library's stream)."""
+        identifies their contents (pointers and version counters): equal keys skip the re-tiling, which is
+        enqueued on ``stream`` behind whatever wrote the arrays there."""
         lib = self._ensure_handle(dt)
         self._set_params(lib, params)
         if self.snaps is None and self.dev_key == key:
             return
-        device.check(lib.kans_layer_load_weights_device(self.handle, W_ptr, W_base_ptr, bias_ptr),
-                     "kans_layer_load_weights_device")
+        device.check(lib.kans_layer_load_weights_stream(self.handle, W_ptr, W_base_ptr, bias_ptr, stream),
+                     "kans_layer_load_weights_stream")
         self.snaps = None
         self.dev_key = key
 

@@ -80,6 +80,7 @@ SIGNATURES = {
     "metal_kan_cheby_backward": (c_int, [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int]),
     "kans_layer_load_weights": (c_int, [P, P, P, P]),
     "kans_layer_load_weights_device": (c_int, [P, P, P, P]),
+    "kans_layer_load_weights_stream": (c_int, [P, P, P, P, P]),
     "kans_layer_load_weights_f32": (c_int, [P, P, P, P]),
     "kans_layer_forward": (c_int, [P, P, c_long, P, c_long, c_int, P]),
     "kans_layer_forward_ex": (c_int, [P, P, c_int, c_long, P, c_int, c_long, c_int, P]),

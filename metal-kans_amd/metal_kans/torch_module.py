@@ -53,6 +53,15 @@ def _aligned_rows(x: torch.Tensor, d_in: int, align: int) -> tuple:
     return xp, ldx
 
 
+# KANS_STREAM_LEGACY: torch's default stream has the handle 0, which the library takes for its own stream
+_LEGACY_STREAM = 1
+
+
+def _stream_of(dev: torch.device) -> ctypes.c_void_p:
+    """Handle of torch's current stream on ``dev``."""
+    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream or _LEGACY_STREAM)
+
+
 class _KANFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, base_weight, bias, module):
@@ -159,11 +168,10 @@ class TorchMetalKANLinear(nn.Module):
                    bias.contiguous() if bias is not None else None]
         key = tuple((p.data_ptr(), p._version) if p is not None else None for p in params)
         eng = self.metal_layer._engine()
-        if eng.dt != dt or eng.dev_key != key or eng.snaps is not None:
-            torch.cuda.current_stream(x.device).synchronize()   # parameter writes done before the re-tiling
+        stream = _stream_of(x.device)
         eng.prepare_device(dt, params[0].data_ptr(), params[1].data_ptr() if params[1] is not None else None,
                            params[2].data_ptr() if params[2] is not None else None,
-                           self.metal_layer._basis_params(), key)
+                           self.metal_layer._basis_params(), key, stream)
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
         if x2.shape[0] == 0:
@@ -171,7 +179,6 @@ class TorchMetalKANLinear(nn.Module):
         xdt = dt if x.dtype == pdt else DT_F32
         xa, ldx = _aligned_rows(x2, self.in_features, 32)
         y = torch.empty((x2.shape[0], self.out_features), dtype=x.dtype, device=x.device)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
         lib = device.get_metal_bridge()
         device.check(lib.kans_layer_forward_ex(eng.handle, ctypes.c_void_p(xa.data_ptr()), xdt, ldx,
                                                ctypes.c_void_p(y.data_ptr()), xdt, self.out_features,
@@ -190,7 +197,7 @@ class TorchMetalKANLinear(nn.Module):
         db = torch.empty((self.out_features,), dtype=torch.float32, device=dev) if bias is not None else None
         dX = torch.empty((B, self.in_features), dtype=torch.float32, device=dev)
         ptr = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        stream = _stream_of(dev)
         device.check(device.get_metal_bridge().kans_cheby_backward(
             ptr(dy), ptr(xs), ptr(W), ptr(Wb), ptr(dW), ptr(dWb), ptr(db), ptr(dX), B, self.in_features,
             self.out_features, self._K, int(Wb is not None), int(db is not None), stream), "kans_cheby_backward")

@@ -141,3 +141,51 @@ def test_device_half_module(cuda):
     y32 = m(x)   # fp32 input to the half module: read unrounded, fp32 output
     assert y32.dtype == torch.float32
     assert O.rel_err(y32.detach().cpu().numpy(), ref) <= 2e-2
+
+
+def test_retiling_and_results_follow_the_streams(cuda):
+    """Weights changed on one stream, forwards and backward on the default stream, on the same stream and on
+    another one: every result is the one of the weights at that point of its stream (the re-tiling is not
+    waited for on the host).  The layer is large enough that a kernel that did not wait would read old tiles."""
+    import metal_kans as mk
+    np.random.seed(0)
+    m = mk.TorchMetalKANLinear(512, 768, degree=6).to(cuda)
+    x = torch.rand(2048, 512, device=cuda) * 2 - 1
+    g = torch.randn(2048, 768, device=cuda)
+    scales = (1.0, 2.0, 0.5, 4.0)
+    with torch.no_grad():
+        base = [p.clone() for p in m.parameters()]
+        torch.cuda.synchronize()
+        refs = []
+        for s in scales:
+            for p, b in zip(m.parameters(), base):
+                p.copy_(b * s)
+            torch.cuda.synchronize()
+            y = m(x)
+            torch.cuda.synchronize()
+            refs.append(y.clone())
+    torch.cuda.synchronize()
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    for stream in (torch.cuda.default_stream(cuda), side):
+        with torch.no_grad(), torch.cuda.stream(stream):
+            outs = []
+            for s in scales * 3:
+                for p, b in zip(m.parameters(), base):
+                    p.copy_(b * s)
+                outs.append(m(x).clone())          # read on the stream right behind
+                other.wait_stream(stream)
+                with torch.cuda.stream(other):     # the re-tiling is still on `stream`
+                    outs.append(m(x).clone())
+                stream.wait_stream(other)
+        torch.cuda.synchronize()
+        for n, y in enumerate(outs):
+            assert torch.equal(y, refs[n // 2 % len(scales)]), n
+        with torch.cuda.stream(stream):
+            xr = x.clone().requires_grad_(True)
+            m.zero_grad(set_to_none=True)
+            m(xr).backward(g)
+            got = [t.grad * 1.0 for t in (xr, *m.parameters())]
+        torch.cuda.synchronize()
+        if stream is side:
+            assert all(torch.equal(a, b) for a, b in zip(got, first))
+        first = got
