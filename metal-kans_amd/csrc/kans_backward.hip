@@ -1,4 +1,4 @@
-// Fused Chebyshev KAN layer backward for gfx950 (fp32), without materialising
+// Fused Chebyshev KAN layer backward for gfx950, without materialising
 // the basis tensor Phi.
 //
 // Reference: metal_kan_cheby_backward_fused (metal_kan_bridge.mm:4532-4632),
@@ -51,6 +51,14 @@
 // Grids that leave CUs idle split the contraction (choose_splits) into partial
 // sums that a second kernel adds in order: 64 workgroups of dW at that shape
 // become 256, and the sums cost 27 us.
+//
+// 16-bit arrays are read as they are and every gradient is rounded once, from
+// its fp32 sum: a dX product is one MFMA, a bf16 dW product four (BwdTerms).
+// The steps are too short there for the matrix pipe to be the bound; the loads'
+// latency and, in dW, the 43 MB of partial sums are.  2000 x 300 -> 500, K = 6,
+// bf16: dW 36 us (41 us with the loads converted as they arrive), its sum 13 us,
+// dX 28 us; through fp32 copies of the arrays and back the training step took
+// 245 us, now 203 us.
 #include "kans_common.h"
 #include "kans_api_internal.h"
 #include "kans_split.h"
@@ -65,9 +73,11 @@ constexpr int kBwdF = 64;      // features per workgroup
 constexpr int kBwdStep = 16;   // contraction indices per step (one MFMA)
 constexpr int kBwdMaxSG = 10;  // slots per workgroup
 
+// T: element type of the layer's arrays (dY, X, W and the gradients).
+template <typename T>
 struct BwdArgs {
-  const float *dY, *X, *W, *Wb;
-  float *dW, *dWb, *db, *dX;
+  const T *dY, *X, *W, *Wb;
+  T *dW, *dWb, *db, *dX;
   float* part;   // split partial sums (null: one split, results written directly)
   float* dbp;    // split partial sums of dbias
   int B, D_in, D_out, K, has_base, NS;
@@ -76,39 +86,82 @@ struct BwdArgs {
   int vec;       // dX: rows of dY readable with 16-byte loads
 };
 
+// Terms of an operand in LDS.  fp32: the three of kans_split.h.  16-bit layers:
+//   dX: dY and W are MFMA operands as they are, one product, exact;
+//   dW: dY in bf16 is one bf16 term (a second one holds its infinities and
+//       NaNs, which must not meet the zeros among the slot values' lower
+//       terms); in fp16 it is split like fp32.  The slot values keep three terms.
+template <typename T> struct BwdTerms { static constexpr int dw_a = 3, dx = 1; };
+template <> struct BwdTerms<float> { static constexpr int dw_a = 3, dx = 3; };
+template <> struct BwdTerms<__bf16> { static constexpr int dw_a = 2, dx = 1; };
+template <typename T> struct BwdFrag { typedef typename Mfma<T>::frag frag; };
+template <> struct BwdFrag<float> { typedef bf16x8 frag; };
+
 __device__ __forceinline__ float silu_deriv_f32(float x) {
   const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * kLog2e));
   return s * (1.0f + x * (1.0f - s));
 }
 
-// One operand tile (32 x 16) of a stage: three terms of 64 lanes x 16 bytes.
-__device__ __forceinline__ void put_tile(uint4* stage, int tile, int lane, const float* v) {
+// An operand tile (32 x 16) of a stage: N terms of 64 lanes x 16 bytes, from
+// its term `at` on.
+__device__ __forceinline__ void put_tile(uint4* stage, int at, int lane, const float* v) {
   const Split8 s = split8(v);
 #pragma unroll
-  for (int q = 0; q < 3; ++q) stage[(tile * 3 + q) * 64 + lane] = s.t[q];
+  for (int q = 0; q < 3; ++q) stage[(at + q) * 64 + lane] = s.t[q];
+}
+// bf16 values: the finite ones, and the others
+__device__ __forceinline__ void put_tile_bf16(uint4* stage, int at, int lane, const float* v) {
+  unsigned d[2][4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const float a = v[2 * p], b = v[2 * p + 1];
+    const bool fa = __builtin_fabsf(a) < __builtin_inff(), fb = __builtin_fabsf(b) < __builtin_inff();
+    d[0][p] = bf16_pair(fa ? a : 0.0f, fb ? b : 0.0f);
+    d[1][p] = bf16_pair(fa ? 0.0f : a, fb ? 0.0f : b);
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) stage[(at + q) * 64 + lane] = make_uint4(d[q][0], d[q][1], d[q][2], d[q][3]);
 }
 
-__device__ __forceinline__ void get_tile(const uint4* stage, int tile, int lane, bf16x8 (&f)[3]) {
+template <int N, typename Frag>
+__device__ __forceinline__ void get_tile(const uint4* stage, int at, int lane, Frag (&f)[N]) {
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const uint4 u = stage[(tile * 3 + q) * 64 + lane];
-    f[q] = *reinterpret_cast<const bf16x8*>(&u);
+  for (int q = 0; q < N; ++q) {
+    const uint4 u = stage[(at + q) * 64 + lane];
+    __builtin_memcpy(&f[q], &u, 16);
   }
 }
 
-// One step of the wave's MB x SG tiles from a stage (A tiles first, then the
-// 2 x SG B tiles).
-template <int SG, int MB>
+// acc += a b for operands of TA and TB terms (see BwdTerms)
+template <typename T, int TA, int TB, typename Frag>
+__device__ __forceinline__ floatx16 mma_terms(const Frag (&a)[TA], const Frag (&b)[TB], floatx16 acc) {
+  if constexpr (TA == 3 && TB == 3) {
+    return mma_split(a, b, acc);
+  } else if constexpr (TA == 2 && TB == 3) {
+    acc = Mfma<__bf16>::mma(a[1], b[0], acc);
+    acc = Mfma<__bf16>::mma(a[0], b[2], acc);
+    acc = Mfma<__bf16>::mma(a[0], b[1], acc);
+    return Mfma<__bf16>::mma(a[0], b[0], acc);
+  } else {
+    static_assert(TA == 1 && TB == 1, "terms");
+    return Mfma<T>::mma(a[0], b[0], acc);
+  }
+}
+
+// One step of the wave's MB x SG tiles from a stage (4 MB tiles of A, then the
+// 2 x SG of B).
+template <typename T, int SG, int MB, int TA, int TB, typename Frag>
 __device__ __forceinline__ void multiply(const uint4* stage, int wm, int wf, int lane, floatx16 (&acc)[MB][SG]) {
-  bf16x8 a[MB][3], b[2][3];
+  Frag a[MB][TA], b[2][TB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) get_tile(stage, wm * MB + mb, lane, a[mb]);
-  get_tile(stage, 4 * MB + wf * SG, lane, b[0]);
+  for (int mb = 0; mb < MB; ++mb) get_tile(stage, (wm * MB + mb) * TA, lane, a[mb]);
+  const int b0 = 4 * MB * TA + wf * SG * TB;
+  get_tile(stage, b0, lane, b[0]);
 #pragma unroll
   for (int s = 0; s < SG; ++s) {
-    if (s + 1 < SG) get_tile(stage, 4 * MB + wf * SG + s + 1, lane, b[(s + 1) & 1]);
+    if (s + 1 < SG) get_tile(stage, b0 + (s + 1) * TB, lane, b[(s + 1) & 1]);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[mb][s] = mma_split(a[mb], b[s & 1], acc[mb][s]);
+    for (int mb = 0; mb < MB; ++mb) acc[mb][s] = mma_terms<T>(a[mb], b[s & 1], acc[mb][s]);
   }
 }
 
@@ -122,10 +175,10 @@ __device__ __forceinline__ void clear(floatx16 (&acc)[MB][SG]) {
       for (int r = 0; r < 16; ++r) acc[mb][s][r] = 0.0f;
 }
 
-template <int SG, int MB>
-__global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
-  constexpr int NA = 4 * MB;
-  __shared__ uint4 stage[2][(NA + 2 * SG) * 3 * 64];
+template <typename T, int SG, int MB>
+__global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs<T> P) {
+  constexpr int NA = 4 * MB, TA = BwdTerms<T>::dw_a;
+  __shared__ uint4 stage[2][(NA * TA + 2 * SG * 3) * 64];
   __shared__ float dbs[NA * 32];
   const int lane = threadIdx.x & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -148,23 +201,24 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
   // lanes past D_out / D_in repeat the last one: their sums are not stored
   const int ocol = min(o0 + a_tile * 32 + (lane & 31), P.D_out - 1);
   const int icol = min(i0 + wf * 32 + (lane & 31), P.D_in - 1);
-  float ra[8], rx[8];
+  // as loaded: a conversion here would wait for the loads before the products that hide them
+  T la[8], lx[8];
   auto load = [&](int t) {
     const int b0 = (t0 + t) * kBwdStep + 8 * half;
-    const float* pa = P.dY + (long)b0 * P.D_out + ocol;
-    const float* px = P.X + (long)b0 * P.D_in + icol;
+    const T* pa = P.dY + (long)b0 * P.D_out + ocol;
+    const T* px = P.X + (long)b0 * P.D_in + icol;
     if ((t0 + t + 1) * kBwdStep <= P.B) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        if (do_a) ra[j] = pa[(long)j * P.D_out];
-        rx[j] = px[(long)j * P.D_in];
+        if (do_a) la[j] = pa[(long)j * P.D_out];
+        lx[j] = px[(long)j * P.D_in];
       }
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const bool ok = b0 + j < P.B;
-        if (do_a) ra[j] = ok ? pa[(long)j * P.D_out] : 0.0f;
-        rx[j] = ok ? px[(long)j * P.D_in] : 0.0f;
+        if (do_a) la[j] = ok ? pa[(long)j * P.D_out] : from_f32<T>(0.0f);
+        lx[j] = ok ? px[(long)j * P.D_in] : from_f32<T>(0.0f);
       }
     }
   };
@@ -172,8 +226,15 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
   const bool base0 = P.has_base != 0 && s0 == 0;
   const int k_first = s0 + 1 - P.has_base;  // T index of the group's first slot (g > 0)
   auto produce = [&](uint4* st) {
+    float rx[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) rx[j] = to_f32(lx[j]);
     if (do_a) {
-      put_tile(st, a_tile, lane, ra);
+      float ra[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ra[j] = to_f32(la[j]);
+      if constexpr (TA == 2) put_tile_bf16(st, a_tile * TA, lane, ra);
+      else put_tile(st, a_tile * TA, lane, ra);
       bsum += ((ra[0] + ra[1]) + (ra[2] + ra[3])) + ((ra[4] + ra[5]) + (ra[6] + ra[7]));
     }
     float tw[8], c[8], p[8];  // 2t, T_k, T_{k-1}
@@ -201,10 +262,10 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
           float v[8];
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[j] = silu_f32(rx[j]);
-          put_tile(st, NA + wf * SG + s, lane, v);
+          put_tile(st, NA * TA + (wf * SG + s) * 3, lane, v);
         }
       } else {
-        if (mine) put_tile(st, NA + wf * SG + s, lane, c);
+        if (mine) put_tile(st, NA * TA + (wf * SG + s) * 3, lane, c);
         if (s + 1 < SG) advance();
       }
     }
@@ -224,7 +285,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
       produce(nxt);
       if (t + 2 < nk) load(t + 2);
     }
-    multiply<SG, MB>(cur, wm, wf, lane, acc);
+    multiply<T, SG, MB, TA, 3, bf16x8>(cur, wm, wf, lane, acc);
     if (wf != 0 && more) {
       produce(nxt);
       if (t + 2 < nk) load(t + 2);
@@ -238,7 +299,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
   const int tid = threadIdx.x;
   if (f_tile == 0 && g == 0 && tid < NA * 32 && o0 + tid < P.D_out) {
     if (P.part != nullptr) P.dbp[(long)split * P.D_out + o0 + tid] = dbs[tid];
-    else if (P.db != nullptr) P.db[o0 + tid] = dbs[tid];
+    else if (P.db != nullptr) P.db[o0 + tid] = from_f32<T>(dbs[tid]);
   }
   // acc register r of lane l holds output 8*(r/4) + 4*(l/32) + r%4, feature l%32
   const int i = i0 + wf * 32 + (lane & 31);
@@ -256,12 +317,12 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
         for (int s = 0; s < SG; ++s)
           if (s0 + s < P.NS) out[(long)s * P.D_in] = acc[mb][s][r];
       } else {
-        float* out = P.dW + (long)o * Kd + (long)i * P.K;
-        if (g == 0) out[0] = dbs[ol];
+        T* out = P.dW + (long)o * Kd + (long)i * P.K;
+        if (g == 0) out[0] = from_f32<T>(dbs[ol]);
 #pragma unroll
         for (int s = 0; s < SG; ++s) {
-          if (s == 0 && base0) P.dWb[(long)o * P.D_in + i] = acc[mb][s][r];
-          else if (s0 + s < P.NS) out[s0 + s + 1 - P.has_base] = acc[mb][s][r];
+          if (s == 0 && base0) P.dWb[(long)o * P.D_in + i] = from_f32<T>(acc[mb][s][r]);
+          else if (s0 + s < P.NS) out[s0 + s + 1 - P.has_base] = from_f32<T>(acc[mb][s][r]);
         }
       }
     }
@@ -270,7 +331,8 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs P) {
 // Sum of the splits' partial sums, in split order, into dW / dW_base / dbias.
 // One thread per (output, slot, feature); slot 0's threads also write the
 // k = 0 coefficient, which is dbias.
-__global__ void k_cheby_bwd_dw_reduce(BwdArgs P, int splits) {
+template <typename T>
+__global__ void k_cheby_bwd_dw_reduce(BwdArgs<T> P, int splits) {
   const long n = (long)P.D_out * P.NS * P.D_in;
   for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += (long)gridDim.x * blockDim.x) {
     const long row = idx / P.D_in;
@@ -283,23 +345,23 @@ __global__ void k_cheby_bwd_dw_reduce(BwdArgs P, int splits) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) s += v[u];
     }
-    float* out = P.dW + ((long)o * P.D_in + i) * P.K;
+    T* out = P.dW + ((long)o * P.D_in + i) * P.K;
     if (sl == 0) {
       float d = 0.0f;
       for (int k = 0; k < splits; ++k) d += P.dbp[(long)k * P.D_out + o];
-      out[0] = d;
-      if (i == 0 && P.db != nullptr) P.db[o] = d;
+      out[0] = from_f32<T>(d);
+      if (i == 0 && P.db != nullptr) P.db[o] = from_f32<T>(d);
     }
-    if (sl == 0 && P.has_base) P.dWb[(long)o * P.D_in + i] = s;
-    else out[sl + 1 - P.has_base] = s;
+    if (sl == 0 && P.has_base) P.dWb[(long)o * P.D_in + i] = from_f32<T>(s);
+    else out[sl + 1 - P.has_base] = from_f32<T>(s);
   }
 }
 
-template <int SG, int MB>
-__global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
-  constexpr int NA = 4 * MB, NT = NA + 2 * SG;
+template <typename T, int SG, int MB>
+__global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
+  constexpr int NA = 4 * MB, NT = NA + 2 * SG, TT = BwdTerms<T>::dx;
   constexpr int R = (NT + 7) / 8;  // operand tiles a wave loads and splits per step
-  __shared__ uint4 stage[2][NT * 3 * 64];
+  __shared__ uint4 stage[2][NT * TT * 64];
   const int lane = threadIdx.x & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave & 3, wf = wave >> 2;
@@ -311,7 +373,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
   const int t0 = split * P.steps_per_split;
   const int nk = min(P.steps - t0, P.steps_per_split);
   const long Kd = (long)P.D_in * P.K;
-  float* const out = P.part != nullptr ? P.part + (long)split * P.B * P.D_in : P.dX;
+  float* const part = P.part != nullptr ? P.part + (long)split * P.B * P.D_in : nullptr;
   const int i = i0 + wf * 32 + (lane & 31);
 
   for (int g = 0; g < P.groups; ++g) {
@@ -319,17 +381,17 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
     // operand tile r * 8 + wave: A (dY rows, contiguous outputs) below NA, else
     // slot weights; lanes past B / D_in and slots past NS repeat the last one
     // (src: the wave's first address, lane_off: this lane's bytes from it)
-    const float* src[R];
+    const T* src[R];
     unsigned lane_off[R];
     long stride[R];
-    float raw[R][8];
+    T raw[R][8];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int id = r * 8 + wave;
       const long o = (long)t0 * kBwdStep;
       if (id < NA) {
         src[r] = P.dY + (long)b0 * P.D_out + o;
-        lane_off[r] = 4u * ((unsigned)(min(b0 + id * 32 + (lane & 31), P.B - 1) - b0) * P.D_out + 8 * half);
+        lane_off[r] = (unsigned)sizeof(T) * ((unsigned)(min(b0 + id * 32 + (lane & 31), P.B - 1) - b0) * P.D_out + 8 * half);
         stride[r] = 1;
       } else {
         const int q = min(id, NT - 1) - NA, f = q / SG;
@@ -338,7 +400,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
         const bool base = P.has_base != 0 && sl == 0;
         stride[r] = base ? P.D_in : Kd;
         src[r] = (base ? P.Wb : P.W + k) + o * stride[r];
-        lane_off[r] = 4u * (8u * half * (unsigned)stride[r] + (unsigned)ic * (base ? 1 : P.K));
+        lane_off[r] = (unsigned)sizeof(T) * (8u * half * (unsigned)stride[r] + (unsigned)ic * (base ? 1 : P.K));
       }
     }
     auto load = [&](int t) {
@@ -348,25 +410,36 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
       for (int r = 0; r < R; ++r) {
         const int id = r * 8 + wave;
         if (id >= NT) continue;
-        const float* p = src[r] + (long)t * kBwdStep * stride[r];
-        auto at = [&](int j) { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(p + j * stride[r]) + lane_off[r]); };
+        const T* p = src[r] + (long)t * kBwdStep * stride[r];
+        auto at = [&](int j) { return reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + j * stride[r]) + lane_off[r]); };
         if (full && id < NA && P.vec) {
-          const float4 u = *reinterpret_cast<const float4*>(at(0)), w = *reinterpret_cast<const float4*>(at(4));
-          raw[r][0] = u.x; raw[r][1] = u.y; raw[r][2] = u.z; raw[r][3] = u.w;
-          raw[r][4] = w.x; raw[r][5] = w.y; raw[r][6] = w.z; raw[r][7] = w.w;
+          constexpr int EPL = 16 / (int)sizeof(T);  // elements of a 16-byte load
+#pragma unroll
+          for (int q = 0; q < 8 / EPL; ++q) {
+            const uint4 u = *reinterpret_cast<const uint4*>(at(q * EPL));
+            __builtin_memcpy(&raw[r][q * EPL], &u, 16);
+          }
         } else if (full) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) raw[r][j] = *at(j);
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) raw[r][j] = j < left ? *at(j) : 0.0f;
+          for (int j = 0; j < 8; ++j) raw[r][j] = j < left ? *at(j) : from_f32<T>(0.0f);
         }
       }
     };
     auto produce = [&](uint4* st) {
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        if (r * 8 + wave < NT) put_tile(st, r * 8 + wave, lane, raw[r]);
+        if (r * 8 + wave < NT) {
+          if constexpr (TT == 3) {
+            put_tile(st, (r * 8 + wave) * TT, lane, raw[r]);
+          } else {
+            uint4 u;
+            __builtin_memcpy(&u, raw[r], 16);
+            st[(r * 8 + wave) * 64 + lane] = u;
+          }
+        }
     };
 
     floatx16 acc[MB][SG];
@@ -383,7 +456,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
         produce(nxt);
         if (t + 2 < nk) load(t + 2);
       }
-      multiply<SG, MB>(cur, wm, wf, lane, acc);
+      multiply<T, SG, MB, TT, TT, typename BwdFrag<T>::frag>(cur, wm, wf, lane, acc);
       if (wf != 0 && more) {
         produce(nxt);
         if (t + 2 < nk) load(t + 2);
@@ -401,19 +474,19 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
       float xs[16];  // one memory round trip per row block
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        xs[r] = P.X[(long)min(row0 + mb * 32 + 8 * (r >> 2) + (r & 3), P.B - 1) * P.D_in + min(i, P.D_in - 1)];
+        xs[r] = to_f32(P.X[(long)min(row0 + mb * 32 + 8 * (r >> 2) + (r & 3), P.B - 1) * P.D_in + min(i, P.D_in - 1)]);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int b = row0 + mb * 32 + 8 * (r >> 2) + (r & 3);
         const long at = (long)b * P.D_in + i;
         const float x = xs[r];
         // T'_1 = 1, T'_{k+1} = 2 T_k + 2x T'_k - T'_{k-1}
-        float T = x, Tp = 1.0f, d = 1.0f, dp = 0.0f;
+        float t = x, tp = 1.0f, d = 1.0f, dp = 0.0f;
         auto advance = [&]() {
-          const float Tn = __builtin_fmaf(2.0f * x, T, -Tp);
-          const float dn = __builtin_fmaf(2.0f * x, d, __builtin_fmaf(2.0f, T, -dp));
-          Tp = T;
-          T = Tn;
+          const float tn = __builtin_fmaf(2.0f * x, t, -tp);
+          const float dn = __builtin_fmaf(2.0f * x, d, __builtin_fmaf(2.0f, t, -dp));
+          tp = t;
+          t = tn;
           dp = d;
           d = dn;
         };
@@ -429,7 +502,12 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
           }
         }
         if (x >= -1.0f && x <= 1.0f) dx += poly;
-        if (b < P.B && i < P.D_in) out[at] = g == 0 ? dx : out[at] + dx;
+        if (b < P.B && i < P.D_in) {
+          // several slot groups (fp32 only): each adds to the one before
+          if (part != nullptr) part[at] = g == 0 ? dx : part[at] + dx;
+          else if constexpr (sizeof(T) == 4) P.dX[at] = g == 0 ? dx : P.dX[at] + dx;
+          else P.dX[at] = from_f32<T>(dx);
+        }
         // one value at a time: all of them side by side would spill the sums
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -437,7 +515,8 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs P) {
   }
 }
 
-__global__ void k_sum_splits(const float* __restrict__ part, float* __restrict__ out, int splits, long n) {
+template <typename T>
+__global__ void k_sum_splits(const float* __restrict__ part, T* __restrict__ out, int splits, long n) {
   for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += (long)gridDim.x * blockDim.x) {
     float s = 0.0f;
     for (int k0 = 0; k0 < splits; k0 += 8) {
@@ -447,13 +526,13 @@ __global__ void k_sum_splits(const float* __restrict__ part, float* __restrict__
 #pragma unroll
       for (int u = 0; u < 8; ++u) s += v[u];
     }
-    out[idx] = s;
+    out[idx] = from_f32<T>(s);
   }
 }
 
 // K = 1 without the base branch: T_0 alone, dW[o, i] = dbias[o] and dX = 0.
 // One workgroup per 64 outputs, four row strides, summed through LDS.
-__global__ void __launch_bounds__(256) k_cheby_bwd_const(BwdArgs P) {
+__global__ void __launch_bounds__(256) k_cheby_bwd_const(BwdArgs<float> P) {
   __shared__ float sums[4][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int o = blockIdx.x * 64 + lane;
@@ -516,76 +595,85 @@ BwdPlan plan_backward(int B, int D_in, int D_out, int K, int has_base, bool may_
   return p;
 }
 
-template <int SG, int MB>
-hipError_t launch_bwd(BwdArgs A, const BwdPlan& p, float* ws, hipStream_t st) {
+template <typename T, int SG, int MB>
+hipError_t launch_bwd(BwdArgs<T> A, const BwdPlan& p, float* ws, hipStream_t st) {
   constexpr int M = 4 * MB * 32;
   A.groups = p.groups;
   A.f_tiles = (A.D_in + kBwdF - 1) / kBwdF;
   // dW: outputs x (slot, feature), contraction over the batch
-  BwdArgs W = A;
+  BwdArgs<T> W = A;
   W.m_tiles = (A.D_out + M - 1) / M;
   W.steps = (A.B + kBwdStep - 1) / kBwdStep;
   W.steps_per_split = (W.steps + p.splits_w - 1) / p.splits_w;
   const int splits_w = (W.steps + W.steps_per_split - 1) / W.steps_per_split;
   W.part = splits_w > 1 ? ws : nullptr;
   W.dbp = splits_w > 1 ? ws + (size_t)splits_w * A.D_out * A.NS * A.D_in : nullptr;
-  hipLaunchKernelGGL((k_cheby_bwd_dw<SG, MB>), dim3(W.m_tiles * A.f_tiles * A.groups, splits_w), dim3(kBwdThreads), 0,
+  hipLaunchKernelGGL((k_cheby_bwd_dw<T, SG, MB>), dim3(W.m_tiles * A.f_tiles * A.groups, splits_w), dim3(kBwdThreads), 0,
                      st, W);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (splits_w > 1) {
-    hipLaunchKernelGGL(k_cheby_bwd_dw_reduce, dim3(reduce_blocks((long)A.D_out * A.NS * A.D_in)), dim3(256), 0, st, W,
+    hipLaunchKernelGGL((k_cheby_bwd_dw_reduce<T>), dim3(reduce_blocks((long)A.D_out * A.NS * A.D_in)), dim3(256), 0, st, W,
                        splits_w);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   // dX: batch rows x (slot, feature), contraction over the outputs
-  BwdArgs X = A;
+  BwdArgs<T> X = A;
   X.m_tiles = (A.B + M - 1) / M;
   X.steps = (A.D_out + kBwdStep - 1) / kBwdStep;
   X.steps_per_split = (X.steps + p.splits_x - 1) / p.splits_x;
   const int splits_x = (X.steps + X.steps_per_split - 1) / X.steps_per_split;
   X.part = splits_x > 1 ? ws : nullptr;
-  X.vec = A.D_out % 4 == 0 && ((uintptr_t)A.dY & 15) == 0;
-  hipLaunchKernelGGL((k_cheby_bwd_dx<SG, MB>), dim3(X.m_tiles * A.f_tiles, splits_x), dim3(kBwdThreads), 0, st, X);
+  X.vec = A.D_out % (16 / (int)sizeof(T)) == 0 && ((uintptr_t)A.dY & 15) == 0;
+  hipLaunchKernelGGL((k_cheby_bwd_dx<T, SG, MB>), dim3(X.m_tiles * A.f_tiles, splits_x), dim3(kBwdThreads), 0, st, X);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (splits_x > 1) {
     const long n = (long)A.B * A.D_in;
-    hipLaunchKernelGGL(k_sum_splits, dim3(reduce_blocks(n)), dim3(256), 0, st, ws, A.dX, splits_x, n);
+    hipLaunchKernelGGL((k_sum_splits<T>), dim3(reduce_blocks(n)), dim3(256), 0, st, ws, A.dX, splits_x, n);
     e = hipGetLastError();
   }
   return e;
 }
 
+
+template <typename T>
+hipError_t launch_slots(const BwdArgs<T>& A, const BwdPlan& p, float* ws, hipStream_t st) {
+  switch (p.SG) {
+    case 1: return launch_bwd<T, 1, 2>(A, p, ws, st);
+    case 2: return launch_bwd<T, 2, 2>(A, p, ws, st);
+    case 3: return launch_bwd<T, 3, 2>(A, p, ws, st);
+    case 4: return launch_bwd<T, 4, 2>(A, p, ws, st);
+    case 5: return launch_bwd<T, 5, 2>(A, p, ws, st);
+    case 6: return launch_bwd<T, 6, 1>(A, p, ws, st);
+    case 7: return launch_bwd<T, 7, 1>(A, p, ws, st);
+    case 8: return launch_bwd<T, 8, 1>(A, p, ws, st);
+    case 9: return launch_bwd<T, 9, 1>(A, p, ws, st);
+    default: return launch_bwd<T, 10, 1>(A, p, ws, st);
+  }
+}
+
 }  // namespace
 
 // ws: p.ws_floats floats when the plan splits, else unused.
-static hipError_t launch_cheby_backward(const float* dY, const float* X, const float* W, const float* Wb, float* dW,
-                                        float* dWb, float* db, float* dX, int B, int D_in, int D_out, int K,
+template <typename T>
+static hipError_t launch_cheby_backward(const void* dY, const void* X, const void* W, const void* Wb, void* dW,
+                                        void* dWb, void* db, void* dX, int B, int D_in, int D_out, int K,
                                         int has_base, const BwdPlan& p, float* ws, hipStream_t st) {
-  BwdArgs A{};
-  A.dY = dY; A.X = X; A.W = W; A.Wb = Wb;
-  A.dW = dW; A.dWb = dWb; A.db = db; A.dX = dX;
+  BwdArgs<T> A{};
+  A.dY = (const T*)dY; A.X = (const T*)X; A.W = (const T*)W; A.Wb = (const T*)Wb;
+  A.dW = (T*)dW; A.dWb = (T*)dWb; A.db = (T*)db; A.dX = (T*)dX;
   A.B = B; A.D_in = D_in; A.D_out = D_out; A.K = K; A.has_base = has_base; A.NS = p.NS;
-  if (p.NS == 0) {
-    hipLaunchKernelGGL(k_cheby_bwd_const, dim3((D_out + 63) / 64), dim3(256), 0, st, A);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const long n = (long)B * D_in;
-    hipLaunchKernelGGL(k_fill_zero, dim3(reduce_blocks(n)), dim3(256), 0, st, dX, n);
-    return hipGetLastError();
+  if constexpr (sizeof(T) == 4) {
+    if (p.NS == 0) {
+      hipLaunchKernelGGL(k_cheby_bwd_const, dim3((D_out + 63) / 64), dim3(256), 0, st, A);
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      const long n = (long)B * D_in;
+      hipLaunchKernelGGL(k_fill_zero, dim3(reduce_blocks(n)), dim3(256), 0, st, (float*)dX, n);
+      return hipGetLastError();
+    }
   }
-  switch (p.SG) {
-    case 1: return launch_bwd<1, 2>(A, p, ws, st);
-    case 2: return launch_bwd<2, 2>(A, p, ws, st);
-    case 3: return launch_bwd<3, 2>(A, p, ws, st);
-    case 4: return launch_bwd<4, 2>(A, p, ws, st);
-    case 5: return launch_bwd<5, 2>(A, p, ws, st);
-    case 6: return launch_bwd<6, 1>(A, p, ws, st);
-    case 7: return launch_bwd<7, 1>(A, p, ws, st);
-    case 8: return launch_bwd<8, 1>(A, p, ws, st);
-    case 9: return launch_bwd<9, 1>(A, p, ws, st);
-    default: return launch_bwd<10, 1>(A, p, ws, st);
-  }
+  return launch_slots<T>(A, p, ws, st);
 }
 
 }  // namespace kans
@@ -657,7 +745,7 @@ int backward_host(const float* dY, const float* X, const float* W, const float* 
   const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, true);
   float* ws;
   if ((rc = acquire_ws(plan.ws_floats, st, &ws))) return rc;
-  HIP_TRY(launch_cheby_backward(d_dY, d_X, d_W, has_base ? d_Wb : nullptr, d_dW, has_base ? d_dWb : nullptr,
+  HIP_TRY(launch_cheby_backward<float>(d_dY, d_X, d_W, has_base ? d_Wb : nullptr, d_dW, has_base ? d_dWb : nullptr,
                                 has_bias ? d_db : nullptr, d_dX, B, D_in, D_out, K, has_base, plan, ws, st));
   if ((rc = release_ws(plan.ws_floats, st))) return rc;
   HIP_TRY(hipMemcpyAsync(dW, d_dW, nW * 4, hipMemcpyDeviceToHost, st));
@@ -672,11 +760,16 @@ int backward_host(const float* dY, const float* X, const float* W, const float* 
 
 extern "C" {
 
-int kans_cheby_backward(const float* dY, const float* X, const float* W, const float* W_base, float* dW,
-                        float* dW_base, float* dbias, float* dX, int B, int D_in, int D_out, int K, int has_base,
-                        int has_bias, void* stream) {
+int kans_cheby_backward_ex(int dtype, const void* dY, const void* X, const void* W, const void* W_base, void* dW,
+                           void* dW_base, void* dbias, void* dX, int B, int D_in, int D_out, int K, int has_base,
+                           int has_bias, void* stream) {
   int rc = check_bwd(dY, X, W, W_base, dW, dW_base, dX, B, D_in, D_out, K, has_base, has_bias);
   if (rc) return rc;
+  if (dtype != DT_F32 && dtype != DT_F16 && dtype != DT_BF16) return kans_fail(KANS_ERR_ARG, "unknown dtype %d", dtype);
+  // partial gradients of several slot groups are added up in the output, which has to hold fp32
+  if (dtype != DT_F32 && (K - 1 + has_base < 1 || K - 1 + has_base > kBwdMaxSG))
+    return kans_fail(KANS_ERR_UNSUPPORTED, "16-bit backward takes 1 to %d slots (K - 1 + has_base = %d)", kBwdMaxSG,
+                     K - 1 + has_base);
   std::lock_guard<std::mutex> lk(kans_mutex());
   if ((rc = kans_ensure_init())) return rc;
   hipStream_t st = kans_caller_stream(stream);
@@ -686,9 +779,19 @@ int kans_cheby_backward(const float* dY, const float* X, const float* W, const f
   const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, !capturing);
   float* ws;
   if ((rc = acquire_ws(plan.ws_floats, st, &ws))) return rc;
-  HIP_TRY(launch_cheby_backward(dY, X, W, has_base ? W_base : nullptr, dW, has_base ? dW_base : nullptr,
-                                has_bias ? dbias : nullptr, dX, B, D_in, D_out, K, has_base, plan, ws, st));
+  auto* go = dtype == DT_F16 ? launch_cheby_backward<_Float16>
+             : dtype == DT_BF16 ? launch_cheby_backward<__bf16>
+                                : launch_cheby_backward<float>;
+  HIP_TRY(go(dY, X, W, has_base ? W_base : nullptr, dW, has_base ? dW_base : nullptr, has_bias ? dbias : nullptr, dX, B,
+             D_in, D_out, K, has_base, plan, ws, st));
   return release_ws(plan.ws_floats, st);
+}
+
+int kans_cheby_backward(const float* dY, const float* X, const float* W, const float* W_base, float* dW,
+                        float* dW_base, float* dbias, float* dX, int B, int D_in, int D_out, int K, int has_base,
+                        int has_bias, void* stream) {
+  return kans_cheby_backward_ex(DT_F32, dY, X, W, W_base, dW, dW_base, dbias, dX, B, D_in, D_out, K, has_base, has_bias,
+                                stream);
 }
 
 int metal_kan_cheby_backward_fused(const float* dY, const float* X, const float* W_cheby, const float* W_base,

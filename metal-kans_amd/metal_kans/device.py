@@ -76,6 +76,7 @@ SIGNATURES = {
     "kans_layer_kernel": (c_int, [P, c_int, ctypes.c_char_p, c_int]),
     "kans_layer_kernel_ex": (c_int, [P, c_int, c_int, c_int, ctypes.c_char_p, c_int]),
     "kans_cheby_backward": (c_int, [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P]),
+    "kans_cheby_backward_ex": (c_int, [c_int, P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P]),
     "metal_kan_cheby_backward_fused": (c_int, [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int]),
     "metal_kan_cheby_backward": (c_int, [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int]),
     "kans_layer_load_weights": (c_int, [P, P, P, P]),

@@ -187,20 +187,26 @@ class TorchMetalKANLinear(nn.Module):
 
     def _backward_device(self, grad_out, x, weight, base_weight, bias):
         B = grad_out.numel() // self.out_features
-        f32 = lambda t: None if t is None else t.detach().float().contiguous()  # noqa: E731
-        dy = f32(grad_out).reshape(B, self.out_features)
-        xs = f32(x).reshape(B, self.in_features)
-        W, Wb = f32(weight), f32(base_weight)
+        # 16-bit arrays as they are where the kernels take them (all of one dtype, 1 to 10 slots), else in fp32
+        dt = weight.dtype
+        slots = self._K - 1 + int(base_weight is not None)
+        given = [t for t in (x, grad_out, base_weight, bias) if t is not None]
+        if dt not in _DT or any(t.dtype != dt for t in given) or not 1 <= slots <= 10:
+            dt = torch.float32
+        as_dt = lambda t: None if t is None else t.detach().to(dt).contiguous()  # noqa: E731
+        dy = as_dt(grad_out).reshape(B, self.out_features)
+        xs = as_dt(x).reshape(B, self.in_features)
+        W, Wb = as_dt(weight), as_dt(base_weight)
         dev = x.device
         dW = torch.empty_like(W)
         dWb = torch.empty_like(Wb) if Wb is not None else None
-        db = torch.empty((self.out_features,), dtype=torch.float32, device=dev) if bias is not None else None
-        dX = torch.empty((B, self.in_features), dtype=torch.float32, device=dev)
+        db = torch.empty((self.out_features,), dtype=dt, device=dev) if bias is not None else None
+        dX = torch.empty((B, self.in_features), dtype=dt, device=dev)
         ptr = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
         stream = _stream_of(dev)
-        device.check(device.get_metal_bridge().kans_cheby_backward(
-            ptr(dy), ptr(xs), ptr(W), ptr(Wb), ptr(dW), ptr(dWb), ptr(db), ptr(dX), B, self.in_features,
-            self.out_features, self._K, int(Wb is not None), int(db is not None), stream), "kans_cheby_backward")
+        device.check(device.get_metal_bridge().kans_cheby_backward_ex(
+            _DT[dt], ptr(dy), ptr(xs), ptr(W), ptr(Wb), ptr(dW), ptr(dWb), ptr(db), ptr(dX), B, self.in_features,
+            self.out_features, self._K, int(Wb is not None), int(db is not None), stream), "kans_cheby_backward_ex")
         cast = lambda g, p: None if g is None else g.to(p.dtype)  # noqa: E731
         return (dX.reshape(x.shape).to(x.dtype), cast(dW, weight), cast(dWb, base_weight), cast(db, bias))
 

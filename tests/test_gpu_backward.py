@@ -262,3 +262,53 @@ def test_backward_streams_and_capture(gpu):
         graph.replay()
         torch.cuda.synchronize()
         check([t.cpu().numpy() for t in outs[0]], refs[0], 1e-5)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("B,D_in,D_out,K,base", [e for e in EDGES if e[3] - 1 + e[4] <= 10] + [(40, 33, 48, 10, 1)])
+def test_backward_16bit_arrays(gpu, dtype, B, D_in, D_out, K, base):
+    """kans_cheby_backward_ex on 16-bit arrays: the gradients of those values, each rounded once."""
+    torch = pytest.importorskip("torch")
+    dt = getattr(torch, dtype)
+    dev = [None if a is None else torch.from_numpy(a).cuda().to(dt) for a in case(B + K, B, D_in, D_out, K, bool(base), True)]
+    outs = [torch.empty(s, device="cuda", dtype=dt) if s else None
+            for s in ((D_out, D_in * K), (D_out, D_in) if base else None, (D_out,), (B, D_in))]
+    torch.cuda.synchronize()
+    assert gpu.kans_cheby_backward_ex({"float16": 1, "bfloat16": 2}[dtype],
+                                      *(t.data_ptr() if t is not None else None for t in dev + outs),
+                                      B, D_in, D_out, K, base, 1, None) == 0, gpu.kans_last_error()
+    assert gpu.kans_synchronize() == 0
+    ref = O.cheby_backward(*(None if t is None else t.float().cpu().numpy() for t in dev), True)
+    # half a unit in the last place of a 16-bit result, beside the fp32 sums' 1e-5 of the largest gradient
+    half_ulp = 2.0 ** (-11 if dtype == "float16" else -8)
+    for got, r, name in zip(outs, ref, ("dW", "dW_base", "dbias", "dX")):
+        if got is None:
+            continue
+        g = got.double().cpu().numpy()
+        bound = half_ulp * np.abs(r) + 1e-5 * np.abs(r).max() + 2.0 ** -24
+        assert (np.abs(g - r) <= bound).all(), f"{name}: {np.max(np.abs(g - r) / bound):.3f} of the bound"
+
+
+def test_backward_16bit_infinities_and_limits(gpu):
+    """An infinite 16-bit upstream gradient makes exactly the gradients it enters non-finite; slot counts that
+    the 16-bit kernels don't take and unknown types are refused."""
+    torch = pytest.importorskip("torch")
+    B, D_in, D_out, K = 48, 40, 30, 5
+    for code, dt in ((1, torch.float16), (2, torch.bfloat16)):
+        dev = [torch.from_numpy(a).cuda().to(dt) for a in case(4, B, D_in, D_out, K, True, True)]
+        dev[0][7, 11] = float("inf")
+        outs = [torch.empty(s, device="cuda", dtype=dt) for s in ((D_out, D_in * K), (D_out, D_in), (D_out,), (B, D_in))]
+        ptrs = [t.data_ptr() for t in dev + outs]
+        torch.cuda.synchronize()
+        assert gpu.kans_cheby_backward_ex(code, *ptrs, B, D_in, D_out, K, 1, 1, None) == 0
+        assert gpu.kans_synchronize() == 0
+        dW, dWb, db, dX = (t.float().cpu().numpy() for t in outs)
+        x = dev[1][7].float().cpu().numpy()
+        assert np.isfinite(np.delete(dW, 11, 0)).all() and np.isfinite(np.delete(dWb, 11, 0)).all()
+        np.testing.assert_array_equal(dWb[11], np.sign(x) * np.inf)
+        np.testing.assert_array_equal(dW[11].reshape(D_in, K)[:, 1], np.sign(x) * np.inf)
+        assert db[11] == np.inf and np.isfinite(np.delete(db, 11)).all()
+        assert not np.isfinite(dX[7][np.abs(x) <= 1]).any() and np.isfinite(np.delete(dX, 7, 0)).all()
+        assert gpu.kans_cheby_backward_ex(code, *ptrs, B, D_in, D_out, 11, 1, 1, None) < 0
+        assert gpu.kans_cheby_backward_ex(code, *ptrs, B, D_in, D_out, 1, 0, 1, None) < 0
+    assert gpu.kans_cheby_backward_ex(7, *ptrs, B, D_in, D_out, K, 1, 1, None) < 0
