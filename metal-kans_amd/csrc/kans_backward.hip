@@ -390,8 +390,9 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
       const int id = r * 8 + wave;
       const long o = (long)t0 * kBwdStep;
       if (id < NA) {
-        src[r] = P.dY + (long)b0 * P.D_out + o;
-        lane_off[r] = (unsigned)sizeof(T) * ((unsigned)(min(b0 + id * 32 + (lane & 31), P.B - 1) - b0) * P.D_out + 8 * half);
+        const int row = min(b0 + id * 32, P.B - 1);
+        src[r] = P.dY + (long)row * P.D_out + o;
+        lane_off[r] = (unsigned)sizeof(T) * ((unsigned)min(lane & 31, P.B - 1 - row) * P.D_out + 8 * half);
         stride[r] = 1;
       } else {
         const int q = min(id, NT - 1) - NA, f = q / SG;
@@ -683,27 +684,33 @@ using namespace kans;
 namespace {
 
 // The split partial sums of a backward: one workspace of at most kBwdWsFloats
-// floats, shared by all calls (library lock held).  A call on another stream
-// than the last one's waits on the device until that one has read its sums.
+// floats, shared by all calls (library lock held).  A call waits on the device
+// until the last one has read its sums (no wait by stream handle: the handle of
+// a destroyed stream can come back for another).
 DevBuf g_ws;
 hipEvent_t g_ws_done = nullptr;
-hipStream_t g_ws_stream = nullptr;
 
-int acquire_ws(size_t floats, hipStream_t st, float** ws) {
+// The plan of one backward and its workspace; where the device has no memory
+// for the partial sums, the plan without splits.
+int acquire_ws(int B, int D_in, int D_out, int K, int has_base, bool may_split, hipStream_t st, BwdPlan* plan,
+               float** ws) {
   *ws = nullptr;
-  if (floats == 0) return 0;
+  *plan = plan_backward(B, D_in, D_out, K, has_base, may_split);
+  if (plan->ws_floats == 0) return 0;
   if (!g_ws_done) HIP_TRY(hipEventCreateWithFlags(&g_ws_done, hipEventDisableTiming));
-  else if (g_ws_stream != st) HIP_TRY(hipStreamWaitEvent(st, g_ws_done, 0));
-  int rc = g_ws.reserve(floats * sizeof(float));  // growing frees the old one, which waits for the device
-  if (rc) return rc;
+  else HIP_TRY(hipStreamWaitEvent(st, g_ws_done, 0));
+  // growing frees the old one, which waits for the device
+  if (g_ws.reserve(plan->ws_floats * sizeof(float))) {
+    (void)hipGetLastError();  // the launches report the errors that they find
+    *plan = plan_backward(B, D_in, D_out, K, has_base, false);
+    return 0;
+  }
   *ws = (float*)g_ws.p;
   return 0;
 }
 
-int release_ws(size_t floats, hipStream_t st) {
-  if (floats == 0) return 0;
-  HIP_TRY(hipEventRecord(g_ws_done, st));
-  g_ws_stream = st;
+int release_ws(const BwdPlan& plan, hipStream_t st) {
+  if (plan.ws_floats != 0) HIP_TRY(hipEventRecord(g_ws_done, st));
   return 0;
 }
 
@@ -714,9 +721,9 @@ int check_bwd(const void* dY, const void* X, const void* W, const void* Wb, cons
     return kans_fail(KANS_ERR_ARG, "bad dims B=%d D_in=%d D_out=%d K=%d (1 <= K <= %d)", B, D_in, D_out, K, kMaxK);
   if ((has_base != 0 && has_base != 1) || (has_bias != 0 && has_bias != 1))
     return kans_fail(KANS_ERR_ARG, "has_base / has_bias must be 0 or 1");
-  // the dX kernel's lane offsets are 32 bits: 36 bytes a reduction index of W, 1 KB an output of dY
-  if ((long)D_in * K > (1L << 26) || D_out > (1 << 21))
-    return kans_fail(KANS_ERR_UNSUPPORTED, "D_in * K = %ld above 2^26 or D_out = %d above 2^21", (long)D_in * K, D_out);
+  // the dX kernel's lane offsets are 32 bits: 36 bytes a reduction index of W, 124 bytes an output of dY
+  if ((long)D_in * K > (1L << 26) || D_out > (1 << 25))
+    return kans_fail(KANS_ERR_UNSUPPORTED, "D_in * K = %ld above 2^26 or D_out = %d above 2^25", (long)D_in * K, D_out);
   if (has_base && (!Wb || !dWb)) return kans_fail(KANS_ERR_ARG, "has_base=1 but W_base or dW_base is null");
   return 0;
 }
@@ -742,12 +749,12 @@ int backward_host(const float* dY, const float* X, const float* W, const float* 
   HIP_TRY(hipMemcpyAsync(d_X, X, nX * 4, hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemcpyAsync(d_W, W, nW * 4, hipMemcpyHostToDevice, st));
   if (has_base) HIP_TRY(hipMemcpyAsync(d_Wb, Wb, nWb * 4, hipMemcpyHostToDevice, st));
-  const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, true);
+  BwdPlan plan;
   float* ws;
-  if ((rc = acquire_ws(plan.ws_floats, st, &ws))) return rc;
+  if ((rc = acquire_ws(B, D_in, D_out, K, has_base, true, st, &plan, &ws))) return rc;
   HIP_TRY(launch_cheby_backward<float>(d_dY, d_X, d_W, has_base ? d_Wb : nullptr, d_dW, has_base ? d_dWb : nullptr,
                                 has_bias ? d_db : nullptr, d_dX, B, D_in, D_out, K, has_base, plan, ws, st));
-  if ((rc = release_ws(plan.ws_floats, st))) return rc;
+  if ((rc = release_ws(plan, st))) return rc;
   HIP_TRY(hipMemcpyAsync(dW, d_dW, nW * 4, hipMemcpyDeviceToHost, st));
   if (has_base) HIP_TRY(hipMemcpyAsync(dWb, d_dWb, nWb * 4, hipMemcpyDeviceToHost, st));
   if (has_bias) HIP_TRY(hipMemcpyAsync(db, d_db, nb * 4, hipMemcpyDeviceToHost, st));
@@ -776,15 +783,15 @@ int kans_cheby_backward_ex(int dtype, const void* dY, const void* X, const void*
   // a call recorded into a graph outlives this one: it gets no share of the common workspace
   bool capturing = false;
   HIP_TRY(kans_capturing(st, &capturing));
-  const BwdPlan plan = plan_backward(B, D_in, D_out, K, has_base, !capturing);
+  BwdPlan plan;
   float* ws;
-  if ((rc = acquire_ws(plan.ws_floats, st, &ws))) return rc;
+  if ((rc = acquire_ws(B, D_in, D_out, K, has_base, !capturing, st, &plan, &ws))) return rc;
   auto* go = dtype == DT_F16 ? launch_cheby_backward<_Float16>
              : dtype == DT_BF16 ? launch_cheby_backward<__bf16>
                                 : launch_cheby_backward<float>;
   HIP_TRY(go(dY, X, W, has_base ? W_base : nullptr, dW, has_base ? dW_base : nullptr, has_bias ? dbias : nullptr, dX, B,
              D_in, D_out, K, has_base, plan, ws, st));
-  return release_ws(plan.ws_floats, st);
+  return release_ws(plan, st);
 }
 
 int kans_cheby_backward(const float* dY, const float* X, const float* W, const float* W_base, float* dW,

@@ -264,6 +264,22 @@ def test_backward_streams_and_capture(gpu):
         check([t.cpu().numpy() for t in outs[0]], refs[0], 1e-5)
 
 
+def test_backward_wide_output(gpu):
+    """More outputs than 32-bit offsets over the 256 rows of a dX tile reach (2^32 / 1024), two row blocks."""
+    B, D_in, D_out, K = 33, 1, (1 << 22) + 3, 2
+    dY, X, W, Wb = case(9, B, D_in, D_out, K, False, True)
+    got = run_host(gpu, gpu.metal_kan_cheby_backward_fused, dY, X, W, Wb, True)
+    # T_0 = 1, T_1 = x; dX = dY W[:, 1] where |x| <= 1
+    t = np.clip(X[:, 0].astype(np.float64), -1, 1)
+    db = dY.sum(0, dtype=np.float64)
+    dW = np.stack([db, t @ dY], 1)
+    dX = (dY.astype(np.float64) @ W[:, 1].astype(np.float64))[:, None] * (np.abs(X) <= 1)
+    check(got[:3], (dW, None, db), 1e-5)
+    # dX adds 64 partial sums of 4096 steps, six products each: as many roundings of half a unit (2^-24), which add
+    # like a random walk, four deviations
+    assert O.rel_err(got[3], dX) <= 4 * np.sqrt(6 * 4096) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("B,D_in,D_out,K,base", [e for e in EDGES if e[3] - 1 + e[4] <= 10] + [(40, 33, 48, 10, 1)])
 def test_backward_16bit_arrays(gpu, dtype, B, D_in, D_out, K, base):
