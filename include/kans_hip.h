@@ -206,7 +206,8 @@ int kans_layer_load_weights(kans_layer* layer, const void* W, const void* W_base
 int kans_layer_load_weights_device(kans_layer* layer, const void* W, const void* W_base, const void* bias);
 /* as kans_layer_load_weights_device, enqueued on `stream` (NULL = kans_stream()) and not waited for: forwards
  * on this stream run behind it, forwards on other streams wait for it on the device; the arrays stay as they
- * are until the stream has passed the call (a training step re-tiles its weights before every forward) */
+ * are until the stream has passed the call (a training step re-tiles its weights before every forward).
+ * Refused (KANS_ERR_UNSUPPORTED) on a stream under graph capture. */
 int kans_layer_load_weights_stream(kans_layer* layer, const void* W, const void* W_base, const void* bias,
                                    void* stream);
 /* host fp32 weights converted on the device to the layer dtype (round to nearest even) */

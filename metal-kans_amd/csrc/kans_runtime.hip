@@ -411,6 +411,10 @@ int kans_layer_load_weights_stream(kans_layer* L, const void* W, const void* W_b
   std::lock_guard<std::mutex> lk(g_mu);
   hipStream_t st = kans_caller_stream(stream);
   int rc;
+  // recorded into a graph, the tiles would not be there for the forwards outside it
+  bool capturing = false;
+  HIP_TRY(kans_capturing(st, &capturing));
+  if (capturing) return kans_fail(KANS_ERR_UNSUPPORTED, "weights cannot be loaded on a stream under graph capture");
   // the last re-tiling, and every forward that may still read the tiles, must be done or ahead on this stream
   if (L->used_many || (L->used && L->use_stream != st) || (L->w_pending && L->w_stream != st))
     HIP_TRY(hipDeviceSynchronize());
@@ -573,19 +577,21 @@ static int layer_reserve_locked(kans_layer* L, int B) {
   return 0;
 }
 
-// Before a kernel on stream st reads the layer's weights: behind a re-tiling still on another stream.  A
-// stream under graph capture cannot wait for an event from outside, so the host waits for it.
+// Before a kernel on stream st reads the layer's weights: behind a re-tiling that may still run.  A
+// stream under graph capture cannot wait for an event from outside, so the host waits for it; on the stream
+// that now captures, the re-tiling ran ahead of the capture (and its event cannot be asked for).
 static int layer_use_weights(kans_layer* L, hipStream_t st) {
   if (L->used && L->use_stream != st) L->used_many = true;
   L->used = true;
   L->use_stream = st;
-  if (!L->w_pending || L->w_stream == st) return 0;
+  if (!L->w_pending) return 0;
   bool capturing = false;
   HIP_TRY(kans_capturing(st, &capturing));
   if (!capturing) {
     HIP_TRY(hipStreamWaitEvent(st, L->w_done, 0));
     return 0;
   }
+  if (L->w_stream == st) return 0;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
   const hipError_t e = hipEventSynchronize(L->w_done);

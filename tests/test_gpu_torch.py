@@ -189,3 +189,33 @@ def test_retiling_and_results_follow_the_streams(cuda):
         if stream is side:
             assert all(torch.equal(a, b) for a, b in zip(got, first))
         first = got
+
+
+def test_weights_loaded_under_capture_are_refused(cuda):
+    """Changed weights re-tiled inside a graph capture would leave forwards outside the graph without tiles: the
+    call is refused, and the module gives the new weights' results afterwards.  A forward of unchanged weights is
+    recorded, and replays follow its input."""
+    import metal_kans as mk
+    np.random.seed(1)
+    m = mk.TorchMetalKANLinear(40, 48, degree=4).to(cuda)
+    side = torch.cuda.Stream()
+    with torch.no_grad(), torch.cuda.stream(side):
+        x = torch.rand(64, 40, device=cuda) * 2 - 1
+        refs = [m(x).clone()]
+        for p in m.parameters():
+            p.mul_(2.0)
+        side.synchronize()
+        with pytest.raises(Exception):
+            with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=side):
+                m(x)
+        refs.append(m(x).clone())
+        assert O.rel_err(refs[1].cpu().numpy(), 2.0 * refs[0].cpu().numpy()) <= 1e-6   # powers of two scale exactly
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            y = m(x)
+        for n in range(3):
+            x.copy_(torch.rand(64, 40, device=cuda) * 2 - 1)
+            graph.replay()
+            want = m(x)
+            side.synchronize()
+            assert torch.equal(y, want), n
