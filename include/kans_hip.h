@@ -175,6 +175,9 @@ typedef struct kans_layer kans_layer;
 
 int kans_init(void);
 void* kans_stream(void); /* the library's HIP stream (hipStream_t) */
+/* the caller keeps `stream` until the process ends: work on other streams is then ordered behind it on the
+ * device, where the library otherwise waits on the host (weights loaded behind forwards on another stream) */
+int kans_stream_keep(void* stream);
 int kans_synchronize(void);
 
 int kans_layer_create(int basis, int dtype, int D_in, int D_out, int K, int has_base, int has_bias,

@@ -18,12 +18,14 @@
 //     returns 0 or a negative code; kans_last_error() describes the failure.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <cmath>
 #include <string>
 #include <tuple>
@@ -113,6 +115,21 @@ hipError_t kans_capturing(hipStream_t st, bool* capturing) {
   return e;
 }
 
+// Streams that exist until the process ends: HIP's default stream, the library's own and those that the
+// caller has named (kans_stream_keep).
+static std::set<hipStream_t> g_kept;
+static bool stream_kept(hipStream_t st) {
+  return st == nullptr || st == g_stream || st == g_compute2 || g_kept.count(st) != 0;
+}
+
+// Allows this thread the calls that a capture running in another one forbids by default (waiting for the
+// device or an event, allocations); none of them concerns a capturing stream.
+struct CaptureRelaxed {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 std::mutex& kans_mutex() { return g_mu; }
 int kans_ensure_init() { return ensure_init(); }
 int kans_pinned_stage(int which, size_t bytes, void** p) {
@@ -133,6 +150,11 @@ struct TileCfg {
   int wm, nb, splits, ks;
 };
 
+// Streams are told apart by their handles.  A destroyed stream's handle can come back for another one, but
+// hipStreamDestroy returns when the stream's work is done, so equal handles still mean ordered work
+// (test_destroyed_stream_is_drained).  hipStreamPerThread is a stream of each thread and equals nothing.
+constexpr size_t kMaxReaders = 64;
+
 struct kans_layer {
   int basis, dtype, D_in, D_out, K, has_base, has_bias;
   int D_in8, nfb, nob_pad;
@@ -141,16 +163,16 @@ struct kans_layer {
   BasisParams bp{};
   DevBuf Wt, bias_d, part, x_d, y_d, raw_w, raw_wb;
   bool have_weights = false;
-  // weights re-tiled on a caller's stream (kans_layer_load_weights_stream) without waiting for them: work on
-  // another stream waits for w_done first
-  bool w_pending = false;
+  // Order between the tiles' writer and their readers (layer_use_weights, layer_claim_weights).
+  bool w_pending = false;           // re-tiled on w_stream (kans_layer_load_weights_stream), not known to be done
   hipStream_t w_stream = nullptr;
-  hipEvent_t w_done = nullptr;
-  // streams the forwards since the last re-tiling ran on: none, one (use_stream), or several
-  bool used = false, used_many = false;
-  hipStream_t use_stream = nullptr;
+  hipEvent_t w_done = nullptr;      // recorded behind the re-tiling
+  std::vector<hipStream_t> readers; // streams of the forwards since the last re-tiling, each ordered behind it
+  bool unnamed_reader = false;      // a forward that readers does not hold
+  hipEvent_t r_done = nullptr;
   ~kans_layer() {
     if (w_done) (void)hipEventDestroy(w_done);
+    if (r_done) (void)hipEventDestroy(r_done);
   }
   int forced_wm = 0, forced_nb = 0, forced_splits = 0;  // tuning overrides (0 = heuristic)
   int forced_ks = 0;  // wave groups per workgroup override (0 = heuristic)
@@ -318,6 +340,32 @@ int kans_layer_set_block_pairs(kans_layer* L, int on) {
   return 0;
 }
 
+// Before the tiles are written on stream st (not under capture): behind the last
+// re-tiling and behind every forward that may still read them.  A reader's event
+// is recorded now, not behind each forward, where it costs 3.5 us of GPU time (a
+// small forward takes 27); that needs a stream that still exists.  One that the
+// caller may have destroyed, or that is being captured, is waited for on the host
+// with the device.
+static int layer_claim_weights(kans_layer* L, hipStream_t st) {
+  CaptureRelaxed relaxed;
+  if (L->w_pending && L->w_stream != st) HIP_TRY(hipStreamWaitEvent(st, L->w_done, 0));
+  bool sync = L->unnamed_reader;
+  for (hipStream_t r : L->readers) {
+    if (r == st) continue;
+    bool capturing = true;
+    if (stream_kept(r)) HIP_TRY(kans_capturing(r, &capturing));
+    if (capturing) {
+      sync = true;
+      continue;
+    }
+    if (!L->r_done) HIP_TRY(hipEventCreateWithFlags(&L->r_done, hipEventDisableTiming));
+    HIP_TRY(hipEventRecord(L->r_done, r));
+    HIP_TRY(hipStreamWaitEvent(st, L->r_done, 0));
+  }
+  if (sync) HIP_TRY(hipDeviceSynchronize());
+  return 0;
+}
+
 // Upload weights (host or device memory) whose element type is src_dtype (the
 // layer dtype, or fp32 for a converting upload).  W: [D_out][D_in*K];
 // W_base: [D_out][D_in] (ignored unless has_base); bias: [D_out] (ignored
@@ -376,7 +424,8 @@ static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, con
   }
   if (L->Wt.p != old_wt || L->bias_d.p != old_bias) ++L->gen;
   L->have_weights = true;
-  L->used = L->used_many = false;
+  L->readers.clear();
+  L->unnamed_reader = false;
   return 0;
 }
 
@@ -415,12 +464,11 @@ int kans_layer_load_weights_stream(kans_layer* L, const void* W, const void* W_b
   bool capturing = false;
   HIP_TRY(kans_capturing(st, &capturing));
   if (capturing) return kans_fail(KANS_ERR_UNSUPPORTED, "weights cannot be loaded on a stream under graph capture");
-  // the last re-tiling, and every forward that may still read the tiles, must be done or ahead on this stream
-  if (L->used_many || (L->used && L->use_stream != st) || (L->w_pending && L->w_stream != st))
-    HIP_TRY(hipDeviceSynchronize());
+  if ((rc = layer_claim_weights(L, st))) return rc;
   if (!L->w_done) HIP_TRY(hipEventCreateWithFlags(&L->w_done, hipEventDisableTiming));
   L->w_pending = false;
-  if ((rc = layer_upload_locked(L, W, W_base, bias, true, L->dtype, st, false))) return rc;
+  if ((rc = layer_upload_locked(L, W, W_base, bias, true, L->dtype, st, st == hipStreamPerThread))) return rc;
+  if (st == hipStreamPerThread) return 0;  // one handle for a stream of each thread: waited for above
   HIP_TRY(hipEventRecord(L->w_done, st));
   L->w_pending = true;
   L->w_stream = st;
@@ -577,27 +625,32 @@ static int layer_reserve_locked(kans_layer* L, int B) {
   return 0;
 }
 
-// Before a kernel on stream st reads the layer's weights: behind a re-tiling that may still run.  A
-// stream under graph capture cannot wait for an event from outside, so the host waits for it; on the stream
-// that now captures, the re-tiling ran ahead of the capture (and its event cannot be asked for).
+// Before a kernel on stream st reads the layer's tiles: behind a re-tiling that
+// may still run.  Each stream waits once per re-tiling; after that the forward
+// makes no call here but the capture query (0.05 us).  A stream under capture
+// cannot wait for an event from outside, so the host waits for it, and the graph's
+// replays are the caller's to order.  Captured on the stream that loaded the
+// weights, the graph is to be launched behind that stream's work, as any graph is:
+// the event cannot be asked for while its stream is captured.
 static int layer_use_weights(kans_layer* L, hipStream_t st) {
-  if (L->used && L->use_stream != st) L->used_many = true;
-  L->used = true;
-  L->use_stream = st;
-  if (!L->w_pending) return 0;
+  const bool known = std::find(L->readers.begin(), L->readers.end(), st) != L->readers.end();
+  if (known && !L->w_pending) return 0;
   bool capturing = false;
   HIP_TRY(kans_capturing(st, &capturing));
-  if (!capturing) {
-    HIP_TRY(hipStreamWaitEvent(st, L->w_done, 0));
+  const bool behind = L->w_pending && (st == hipStreamPerThread || L->w_stream != st);
+  if (capturing || st == hipStreamPerThread) {
+    if (behind) {
+      CaptureRelaxed relaxed;
+      HIP_TRY(hipEventSynchronize(L->w_done));
+      L->w_pending = false;
+    }
+    if (!capturing) L->unnamed_reader = true;
     return 0;
   }
-  if (L->w_stream == st) return 0;
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-  const hipError_t e = hipEventSynchronize(L->w_done);
-  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-  HIP_TRY(e);
-  L->w_pending = false;
+  if (known) return 0;
+  if (behind) HIP_TRY(hipStreamWaitEvent(st, L->w_done, 0));
+  if (L->readers.size() < kMaxReaders) L->readers.push_back(st);
+  else L->unnamed_reader = true;
   return 0;
 }
 
@@ -894,6 +947,14 @@ int kans_init(void) {
 }
 
 void* kans_stream(void) { return (void*)g_stream; }
+
+int kans_stream_keep(void* stream) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  hipStream_t st = kans_caller_stream(stream);
+  if (st == hipStreamPerThread) return kans_fail(KANS_ERR_ARG, "hipStreamPerThread names a stream of each thread");
+  if (st) g_kept.insert(st);
+  return 0;
+}
 
 int kans_dev_malloc(void** p, size_t bytes) {
   if (!p) return kans_fail(KANS_ERR_ARG, "null argument");

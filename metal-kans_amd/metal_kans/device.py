@@ -64,6 +64,7 @@ SIGNATURES = {
     # device-resident layer API
     "kans_init": (c_int, []),
     "kans_stream": (c_void_p, []),
+    "kans_stream_keep": (c_int, [P]),
     "kans_synchronize": (c_int, []),
     "kans_layer_create": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, ctypes.POINTER(c_void_p)]),
     "kans_layer_destroy": (c_int, [P]),

@@ -57,9 +57,18 @@ def _aligned_rows(x: torch.Tensor, d_in: int, align: int) -> tuple:
 _LEGACY_STREAM = 1
 
 
+# streams the library may name later: torch's own, which live until the process ends
+_kept = {0}
+
+
 def _stream_of(dev: torch.device) -> ctypes.c_void_p:
     """Handle of torch's current stream on ``dev``."""
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream or _LEGACY_STREAM)
+    s = torch.cuda.current_stream(dev)
+    h = s.cuda_stream
+    if h not in _kept and s.stream_id != h:  # (an external stream has its handle for id)
+        device.check(device.get_metal_bridge().kans_stream_keep(h), "kans_stream_keep")
+        _kept.add(h)
+    return ctypes.c_void_p(h or _LEGACY_STREAM)
 
 
 class _KANFunction(torch.autograd.Function):

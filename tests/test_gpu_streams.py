@@ -1,0 +1,91 @@
+"""Order between streams: weights re-tiled, forwards, graph replays and split workspaces (run on an MI355X).
+
+Races are provoked by holding one stream up with a long kernel (``torch.cuda._sleep``) while the others go on,
+and every result is compared with the same call made alone.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+HOLD = 200_000_000  # cycles of a held stream: 0.1 to 2 s
+
+
+@pytest.fixture(scope="module")
+def cuda(gpu):
+    if not torch.cuda.is_available():
+        pytest.skip("torch sees no GPU")
+    return torch.device("cuda:0")
+
+
+def module(d_in, d_out, **kw):
+    import metal_kans as mk
+    np.random.seed(0)
+    return mk.TorchMetalKANLinear(d_in, d_out, **kw).to("cuda")
+
+
+def scale(m, s):
+    with torch.no_grad():
+        for p in m.parameters():
+            p.mul_(s)
+
+
+def alone(m, x):
+    torch.cuda.synchronize()
+    y = m(x).clone()
+    torch.cuda.synchronize()
+    return y
+
+
+def hip_runtime():
+    """The HIP runtime that this process uses."""
+    with open("/proc/self/maps") as f:
+        paths = {line.split()[-1] for line in f if "libamdhip64" in line}
+    assert len(paths) == 1, paths
+    return ctypes.CDLL(paths.pop())
+
+
+def test_destroyed_stream_is_drained(cuda):
+    """A stream's handle is taken for the stream: hipStreamDestroy returns when the stream's work is done, so a
+    handle that comes back for another stream finds nothing of the old one still running."""
+    hip = hip_runtime()
+    h = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(h), 1) == 0
+    done = torch.cuda.Event()
+    with torch.cuda.stream(torch.cuda.ExternalStream(h.value)):
+        torch.cuda._sleep(HOLD)
+        done.record()
+    assert not done.query()
+    assert hip.hipStreamDestroy(h) == 0
+    assert done.query()
+
+
+def test_retiling_behind_another_streams_forward_keeps_the_host_free(cuda):
+    """Weights changed and re-tiled on one stream while a forward of the old ones still waits on another: the
+    forward reads the old tiles, and the call that re-tiles does not wait for it on the host."""
+    m = module(512, 768, degree=6)
+    x = torch.rand(512, 512, device=cuda) * 2 - 1
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.no_grad():
+        old = alone(m, x)
+        scale(m, 2.0)
+        new = alone(m, x)
+        scale(m, 0.5)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            m(x)
+        with torch.cuda.stream(b):
+            torch.cuda._sleep(HOLD)
+            yb = m(x)
+            held = torch.cuda.Event()
+            held.record()
+        with torch.cuda.stream(a):
+            scale(m, 2.0)
+            ya = m(x)
+        assert not held.query()
+    torch.cuda.synchronize()
+    assert torch.equal(yb, old) and torch.equal(ya, new)
