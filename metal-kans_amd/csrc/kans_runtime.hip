@@ -376,7 +376,8 @@ static int layer_upload_locked(kans_layer* L, const void* W, const void* Wb, con
   const size_t wbytes = (size_t)L->D_out * L->D_in * L->K * es;
   const size_t wbbytes = (size_t)L->D_out * L->D_in * es;
   const size_t tbytes = (size_t)L->nfb * L->slots * L->nob_pad * 64 * 16 * (L->dtype == DT_F32 ? 3 : 1);
-  int rc;
+  int rc = layer_claim_weights(L, st);
+  if (rc) return rc;
   void* old_wt = L->Wt.p;
   void* old_bias = L->bias_d.p;
   if ((rc = L->Wt.reserve(tbytes))) return rc;
@@ -464,9 +465,7 @@ int kans_layer_load_weights_stream(kans_layer* L, const void* W, const void* W_b
   bool capturing = false;
   HIP_TRY(kans_capturing(st, &capturing));
   if (capturing) return kans_fail(KANS_ERR_UNSUPPORTED, "weights cannot be loaded on a stream under graph capture");
-  if ((rc = layer_claim_weights(L, st))) return rc;
   if (!L->w_done) HIP_TRY(hipEventCreateWithFlags(&L->w_done, hipEventDisableTiming));
-  L->w_pending = false;
   if ((rc = layer_upload_locked(L, W, W_base, bias, true, L->dtype, st, st == hipStreamPerThread))) return rc;
   if (st == hipStreamPerThread) return 0;  // one handle for a stream of each thread: waited for above
   HIP_TRY(hipEventRecord(L->w_done, st));

@@ -89,3 +89,26 @@ def test_retiling_behind_another_streams_forward_keeps_the_host_free(cuda):
         assert not held.query()
     torch.cuda.synchronize()
     assert torch.equal(yb, old) and torch.equal(ya, new)
+
+
+def test_host_load_behind_a_queued_retiling(cuda):
+    """Weights re-tiled on a held stream, then other weights loaded from host arrays: the later load stays."""
+    m = module(96, 80, degree=5)
+    layer = m.metal_layer
+    xh = (np.random.default_rng(0).random((64, 96)) * 2 - 1).astype(np.float32)
+    x = torch.from_numpy(xh).to(cuda)
+    want = layer(xh)                         # the layer's own arrays
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        scale(m, 2.0)                        # the module's parameters
+        doubled = alone(m, x)
+        scale(m, 1.0)                        # (a new version of the same values)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(HOLD)
+            y = m(x)                         # its re-tiling waits on the held stream
+    first = layer(xh)
+    torch.cuda.synchronize()
+    assert torch.equal(y, doubled)
+    np.testing.assert_array_equal(first, want)
+    np.testing.assert_array_equal(layer(xh), want)   # nothing loaded again
