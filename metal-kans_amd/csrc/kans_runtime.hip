@@ -1397,6 +1397,17 @@ static int chain_graph_ready(kans_chain* C, int B, bool copies) {
   return chain_capture(C, B, copies);
 }
 
+// Replay the chain's graph on g_stream, behind loads of its layers' weights on other streams (a load moves
+// nothing that the graph holds, so the graph stays as it is).
+static int chain_replay(kans_chain* C) {
+  for (kans_layer* L : C->layers) {
+    int rc = layer_use_weights(L, g_stream);
+    if (rc) return rc;
+  }
+  HIP_TRY(hipGraphLaunch(C->exec, g_stream));
+  return 0;
+}
+
 extern "C" {
 
 int kans_chain_create(kans_layer** layers, int n, kans_chain** out) {
@@ -1463,16 +1474,16 @@ int kans_chain_forward_host_ex(kans_chain* C, const void* X, int x_dtype, void* 
     g_pending.push_back({pin_out, nullptr, 0});
     const size_t out_idx = g_pending.size() - 1;
     if ((rc = stage_in(C->x_d.p, X, row_in, pitch_in, B, pin_in, g_stream))) return rc;
-    HIP_TRY(hipGraphLaunch(C->exec, g_stream));
+    if ((rc = chain_replay(C))) return rc;
     HIP_TRY(hipMemcpyAsync(pin_out, C->y_d.p, out_bytes, hipMemcpyDeviceToHost, g_stream));
     g_pending[out_idx].dst = Y;
     g_pending[out_idx].bytes = out_bytes;
     return 0;
   }
   if ((rc = stage_in(C->x_d.p, X, row_in, pitch_in, B, C->pin_in.p, g_stream))) return rc;
-  if (hipGraphLaunch(C->exec, g_stream) != hipSuccess) {
+  if ((rc = chain_replay(C))) {
     (void)hipStreamSynchronize(g_stream);  // the input DMAs read pin_in; finish them before it is reused
-    return kans_fail(KANS_ERR_HIP, "hipGraphLaunch failed");
+    return rc;
   }
   return stage_out(Y, C->y_d.p, out_bytes, C->pin_out.p, g_stream);
 }
@@ -1498,12 +1509,14 @@ int kans_chain_time(kans_chain* C, int B, int warmup, int iters, int include_cop
   std::lock_guard<std::mutex> lk(g_mu);  // replays the graph of the last host call's input dtype
   int rc = chain_graph_ready(C, B, include_copies != 0);
   if (rc) return rc;
-  for (int i = 0; i < warmup; ++i) HIP_TRY(hipGraphLaunch(C->exec, g_stream));
+  for (int i = 0; i < warmup; ++i)
+    if ((rc = chain_replay(C))) return rc;
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   HIP_TRY(hipEventRecord(e0, g_stream));
-  for (int i = 0; i < iters; ++i) HIP_TRY(hipGraphLaunch(C->exec, g_stream));
+  for (int i = 0; i < iters; ++i)
+    if ((rc = chain_replay(C))) return rc;
   HIP_TRY(hipEventRecord(e1, g_stream));
   HIP_TRY(hipEventSynchronize(e1));
   float t = 0;
@@ -1730,6 +1743,16 @@ static int dgated_graph_ready(kans_gated_dense* D, int B, bool copies) {
   return dgated_capture(D, B, copies);
 }
 
+// As chain_replay.
+static int dgated_replay(kans_gated_dense* D) {
+  for (kans_layer* L : {D->gate, D->up, D->down}) {
+    int rc = layer_use_weights(L, g_stream);
+    if (rc) return rc;
+  }
+  HIP_TRY(hipGraphLaunch(D->exec, g_stream));
+  return 0;
+}
+
 extern "C" {
 
 int kans_gated_dense_create(kans_layer* gate, kans_layer* up, kans_layer* down, kans_gated_dense** out) {
@@ -1805,16 +1828,16 @@ int kans_gated_dense_forward_host(kans_gated_dense* D, const void* X, int x_dtyp
     g_pending.push_back({pin_out, nullptr, 0});
     const size_t out_idx = g_pending.size() - 1;
     if ((rc = stage_in(D->x_d.p, X, row_in, pitch_in, B, pin_in, g_stream))) return rc;
-    HIP_TRY(hipGraphLaunch(D->exec, g_stream));
+    if ((rc = dgated_replay(D))) return rc;
     HIP_TRY(hipMemcpyAsync(pin_out, D->y_d.p, out_bytes, hipMemcpyDeviceToHost, g_stream));
     g_pending[out_idx].dst = Y;
     g_pending[out_idx].bytes = out_bytes;
     return 0;
   }
   if ((rc = stage_in(D->x_d.p, X, row_in, pitch_in, B, D->pin_in.p, g_stream))) return rc;
-  if (hipGraphLaunch(D->exec, g_stream) != hipSuccess) {
+  if ((rc = dgated_replay(D))) {
     (void)hipStreamSynchronize(g_stream);  // the input DMAs read pin_in; finish them before it is reused
-    return kans_fail(KANS_ERR_HIP, "hipGraphLaunch failed");
+    return rc;
   }
   return stage_out(Y, D->y_d.p, out_bytes, D->pin_out.p, g_stream);
 }
@@ -1826,12 +1849,14 @@ int kans_gated_dense_time(kans_gated_dense* D, int B, int warmup, int iters, int
   std::lock_guard<std::mutex> lk(g_mu);
   int rc = dgated_graph_ready(D, B, include_copies != 0);
   if (rc) return rc;
-  for (int i = 0; i < warmup; ++i) HIP_TRY(hipGraphLaunch(D->exec, g_stream));
+  for (int i = 0; i < warmup; ++i)
+    if ((rc = dgated_replay(D))) return rc;
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   HIP_TRY(hipEventRecord(e0, g_stream));
-  for (int i = 0; i < iters; ++i) HIP_TRY(hipGraphLaunch(D->exec, g_stream));
+  for (int i = 0; i < iters; ++i)
+    if ((rc = dgated_replay(D))) return rc;
   HIP_TRY(hipEventRecord(e1, g_stream));
   HIP_TRY(hipEventSynchronize(e1));
   float t = 0;

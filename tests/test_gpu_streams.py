@@ -112,3 +112,57 @@ def test_host_load_behind_a_queued_retiling(cuda):
     assert torch.equal(y, doubled)
     np.testing.assert_array_equal(first, want)
     np.testing.assert_array_equal(layer(xh), want)   # nothing loaded again
+
+
+def load_on(lib, m, stream, s):
+    """The module's weights times s into its layer, on `stream`; returns the arrays, which the load reads."""
+    import metal_kans as mk
+    ws = [(p.detach() * s).contiguous() for p in (m.weight, m.base_weight, m.bias_param)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(HOLD)
+    mk.device.check(lib.kans_layer_load_weights_stream(m.metal_layer._engine().handle, *[w.data_ptr() for w in ws],
+                                                       stream.cuda_stream), "kans_layer_load_weights_stream")
+    return ws
+
+
+@pytest.mark.parametrize("kind", ["chain", "gated"])
+def test_graph_replays_follow_a_load_on_another_stream(gpu, cuda, kind):
+    """A chain's and a dense gated block's graph, built before, replayed while a load of new weights is still
+    queued on a held stream: the result is the new weights'."""
+    import metal_kans as mk
+    lib = gpu
+    dims = ((24, 40), (40, 16)) if kind == "chain" else ((24, 40), (24, 40), (40, 24))
+    ms = [module(a, b, degree=4) for a, b in dims]
+    with torch.no_grad():
+        for m in ms:
+            m(torch.zeros(1, m.in_features, device=cuda))   # the handles
+    torch.cuda.synchronize()
+    handles = [m.metal_layer._engine().handle for m in ms]
+    obj = ctypes.c_void_p()
+    if kind == "chain":
+        arr = (ctypes.c_void_p * 2)(*[h.value for h in handles])
+        mk.device.check(lib.kans_chain_create(arr, 2, ctypes.byref(obj)), "kans_chain_create")
+        call = lambda x, y: lib.kans_chain_forward_host(obj, x.ctypes.data, y.ctypes.data, len(x))  # noqa: E731
+    else:
+        mk.device.check(lib.kans_gated_dense_create(*handles, ctypes.byref(obj)), "kans_gated_dense_create")
+        call = lambda x, y: lib.kans_gated_dense_forward_host(obj, x.ctypes.data, 0, y.ctypes.data, len(x))  # noqa: E731
+    x = (np.random.default_rng(1).random((32, 24)) * 2 - 1).astype(np.float32)
+
+    def forward():
+        y = np.empty((32, dims[-1][1]), np.float32)
+        mk.device.check(call(x, y), kind)
+        return y
+    try:
+        old = forward()
+        side = torch.cuda.Stream()
+        keep = load_on(lib, ms[0], side, 0.5)
+        new = forward()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(forward(), new)
+        assert not np.array_equal(old, new)
+        keep += load_on(lib, ms[0], side, 1.0)
+        np.testing.assert_array_equal(forward(), old)
+    finally:
+        torch.cuda.synchronize()
+        (lib.kans_chain_destroy if kind == "chain" else lib.kans_gated_dense_destroy)(obj)
