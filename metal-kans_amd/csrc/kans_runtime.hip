@@ -549,7 +549,9 @@ static bool tile_groups_ok(const kans_layer* L, int wm, int nb, int ks) {
 // Partial sums of a split forward are kept below this.
 constexpr double kMaxPartMB = 256.0;
 
-static TileCfg choose_tiling(const kans_layer* L, int B) {
+// unsplit: one split whatever is forced.
+static TileCfg choose_tiling(const kans_layer* L, int B, bool unsplit = false) {
+  const int forced_splits = unsplit ? 1 : L->forced_splits;
   const TileCost* table;
   int rows = 4;
   if (L->dtype == DT_F32) {
@@ -573,19 +575,19 @@ static TileCfg choose_tiling(const kans_layer* L, int B) {
     const long tiles = (long)((B + tr - 1) / tr) * ((nob + nb - 1) / nb);
     int last = 0;  // splits that come to the same feature blocks each are looked at once
     for (int s = 1; s <= std::min(L->nfb, 32); ++s) {
-      const int fbps = L->forced_splits ? (L->nfb + L->forced_splits - 1) / L->forced_splits : (L->nfb + s - 1) / s;
+      const int fbps = forced_splits ? (L->nfb + forced_splits - 1) / forced_splits : (L->nfb + s - 1) / s;
       if (fbps == last || (ks > 1 && fbps < 2 * ks)) continue;
       last = fbps;
       const int splits = (L->nfb + fbps - 1) / fbps;
       const double mb = splits > 1 ? 8e-6 * splits * B * L->D_out : 0.0;
-      if (splits > 1 && mb > 2.0 * kMaxPartMB && !L->forced_splits) break;
+      if (splits > 1 && mb > 2.0 * kMaxPartMB && !forced_splits) break;
       const double n = (double)((tiles * splits + 255) / 256), F = (fbps + ks - 1) / ks;
       double t = n * (F * L->slots * (n > 1 ? c.shared : c.alone) + F * c.block + c.wg) + c.launch;
       if (splits > 1) t += c.split_us + mb * c.split_mb;
       if (!any || t < best_t) {
         any = true;
         best_t = t;
-        best = TileCfg{wm, nb, L->forced_splits ? L->forced_splits : splits, ks};
+        best = TileCfg{wm, nb, forced_splits ? forced_splits : splits, ks};
       }
     }
   }
@@ -593,16 +595,16 @@ static TileCfg choose_tiling(const kans_layer* L, int B) {
     best.wm = L->forced_wm;
     best.nb = L->forced_nb;
     best.ks = 1;
-    // a forced tile keeps one split unless the splits are forced too
-    best.splits = L->forced_splits ? L->forced_splits : best.splits;
+    // (the splits estimated for that tile, unless they are forced too)
+    if (forced_splits) best.splits = forced_splits;
   }
   // a forced group count that the tile is not instantiated with falls back to 1
   if (L->forced_ks) best.ks = tile_groups_ok(L, best.wm, best.nb, L->forced_ks) ? L->forced_ks : 1;
   return best;
 }
 
-// The configuration of a forward of batch B, kept for the last batch size (library lock held; gen changes
-// with every setting it depends on).
+// The configuration of a forward of batch B, kept for the last batch size (library lock held; tile_gen
+// changes with every setting it depends on).
 static const TileCfg& tile_cfg_locked(kans_layer* L, int B) {
   if (L->cfg_B != B || L->cfg_gen != L->tile_gen) {
     L->cfg = choose_tiling(L, B);
@@ -612,14 +614,18 @@ static const TileCfg& tile_cfg_locked(kans_layer* L, int B) {
   return L->cfg;
 }
 
-// Reserve the split workspace a forward of batch B needs (no launch).
+// Reserve the split workspace a forward of batch B needs (no launch).  Where the device has no memory for it
+// the forwards of this batch size run unsplit.
 static int layer_reserve_locked(kans_layer* L, int B) {
   const TileCfg& cfg = tile_cfg_locked(L, B);
   if (cfg.splits > 1) {
     void* old = L->part.p;
-    int rc = L->part.reserve((size_t)cfg.splits * B * L->D_out * sizeof(float));
-    if (rc) return rc;
+    const int rc = L->part.reserve((size_t)cfg.splits * B * L->D_out * sizeof(float));
     if (old != L->part.p) ++L->gen;
+    if (rc) {
+      (void)hipGetLastError();  // the launches report the errors that they find
+      L->cfg = choose_tiling(L, B, true);
+    }
   }
   return 0;
 }

@@ -166,3 +166,18 @@ def test_graph_replays_follow_a_load_on_another_stream(gpu, cuda, kind):
     finally:
         torch.cuda.synchronize()
         (lib.kans_chain_destroy if kind == "chain" else lib.kans_gated_dense_destroy)(obj)
+
+
+def test_forward_without_memory_for_its_splits(cuda):
+    """Partial sums larger than the device (550 GB): the forward runs unsplit, with the unsplit forward's bits."""
+    m = module(4096, 2048, degree=2, bias=False, use_base=False).half()
+    eng = m.metal_layer._engine()
+    x = torch.rand(262144, 4096, device=cuda, dtype=torch.float16) * 2 - 1
+    with torch.no_grad():
+        eng.set_tiling(0, 0, 1)
+        want = m(x)
+        eng.set_tiling(0, 0, 256)
+        assert torch.equal(m(x), want)
+        eng.set_tiling(0, 0, 0)
+        small = m(x[:64])
+    assert torch.isfinite(small).all()
