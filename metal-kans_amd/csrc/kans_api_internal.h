@@ -83,6 +83,26 @@ inline hipStream_t kans_caller_stream(void* stream) {
 }
 // Whether st is under graph capture (the default stream never is).
 hipError_t kans_capturing(hipStream_t st, bool* capturing);
+// Workspace for the partial sums of a split kernel on stream st, `bytes` large: one per stream, which all
+// calls on the stream share, since their kernels run one after the other (library lock held; st not under
+// capture by a caller).  Null where there is none -- no memory for it, or hipStreamPerThread, one handle
+// for several streams: the caller then runs unsplit.  It grows with the calls and stays until the next
+// larger request, until kMaxWorkspaces other streams have asked since, or until the library's last object
+// is destroyed (WorkspaceUser).
+float* kans_stream_workspace(hipStream_t st, size_t bytes);
+struct WorkspaceUser {
+  WorkspaceUser();
+  ~WorkspaceUser();
+  WorkspaceUser(const WorkspaceUser&) = delete;
+  WorkspaceUser& operator=(const WorkspaceUser&) = delete;
+};
+// Allows this thread the calls that a capture running in another one forbids by default (waiting for the
+// device or an event, allocations); none of them concerns a capturing stream.
+struct CaptureRelaxed {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
 // fp32 Chebyshev forward (no base branch) of host X on device-resident fp32 weights (kans_runtime.hip);
 // call with the library lock held.
 int kans_ref_cheby_forward_devw_locked(const float* X, const float* W_dev, const float* bias_dev, float* Y, int B,

@@ -122,13 +122,58 @@ static bool stream_kept(hipStream_t st) {
   return st == nullptr || st == g_stream || st == g_compute2 || g_kept.count(st) != 0;
 }
 
-// Allows this thread the calls that a capture running in another one forbids by default (waiting for the
-// device or an event, allocations); none of them concerns a capturing stream.
-struct CaptureRelaxed {
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-  ~CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+// Split workspaces (kans_stream_workspace), of at most kMaxWorkspaces streams.  Dropping one frees it, which
+// waits for the device.
+struct StreamWorkspace {
+  explicit StreamWorkspace(hipStream_t s) : st(s) {}
+  hipStream_t st;
+  unsigned long asked = 0;  // g_ws_clock of the last request
+  DevBuf buf;
+  size_t refused = SIZE_MAX;  // bytes that could not be had; not tried again before g_ws_clock = retry
+  unsigned long retry = 0;
 };
+constexpr size_t kMaxWorkspaces = 8;
+static auto& g_ws = *new std::vector<std::unique_ptr<StreamWorkspace>>();  // (never destroyed: used by static objects)
+static unsigned long g_ws_clock = 0;
+static unsigned g_ws_gen = 0;  // bumped when g_stream's moves: captured graphs hold it
+static long g_ws_users = 0;
+
+float* kans_stream_workspace(hipStream_t st, size_t bytes) {
+  if (st == hipStreamPerThread) return nullptr;
+  CaptureRelaxed relaxed;
+  auto at = std::find_if(g_ws.begin(), g_ws.end(), [&](const auto& w) { return w->st == st; });
+  if (at == g_ws.end()) {
+    if (g_ws.size() >= kMaxWorkspaces)
+      g_ws.erase(std::min_element(g_ws.begin(), g_ws.end(), [](const auto& a, const auto& b) {
+        return (a->st == g_stream) != (b->st == g_stream) ? b->st == g_stream : a->asked < b->asked;
+      }));
+    g_ws.emplace_back(new StreamWorkspace(st));
+    at = g_ws.end() - 1;
+  }
+  StreamWorkspace& w = **at;
+  w.asked = ++g_ws_clock;
+  if (bytes <= w.buf.cap) return (float*)w.buf.p;
+  if (bytes >= w.refused && g_ws_clock < w.retry) return nullptr;
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();  // the launches report the errors that they find
+    w.refused = bytes;
+    w.retry = g_ws_clock + 256;
+    return nullptr;
+  }
+  if (w.buf.p) (void)hipFree(w.buf.p);  // waits for the device: nothing uses it any more
+  w.buf.p = p;
+  w.buf.cap = bytes;
+  w.refused = SIZE_MAX;
+  if (st == g_stream) ++g_ws_gen;
+  return (float*)p;
+}
+WorkspaceUser::WorkspaceUser() { ++g_ws_users; }
+WorkspaceUser::~WorkspaceUser() {
+  if (--g_ws_users > 0) return;
+  g_ws.clear();
+  ++g_ws_gen;
+}
 
 std::mutex& kans_mutex() { return g_mu; }
 int kans_ensure_init() { return ensure_init(); }
@@ -161,7 +206,8 @@ struct kans_layer {
   // T_0 folded into the bias (BasisParams::k0); fp32 B-spline in the sparse layout; slots of W' per feature
   int fold, sparse, slots;
   BasisParams bp{};
-  DevBuf Wt, bias_d, part, x_d, y_d, raw_w, raw_wb;
+  DevBuf Wt, bias_d, x_d, y_d, raw_w, raw_wb;
+  WorkspaceUser ws_user;
   bool have_weights = false;
   // Order between the tiles' writer and their readers (layer_use_weights, layer_claim_weights).
   bool w_pending = false;           // re-tiled on w_stream (kans_layer_load_weights_stream), not known to be done
@@ -614,20 +660,21 @@ static const TileCfg& tile_cfg_locked(kans_layer* L, int B) {
   return L->cfg;
 }
 
-// Reserve the split workspace a forward of batch B needs (no launch).  Where the device has no memory for it
-// the forwards of this batch size run unsplit.
-static int layer_reserve_locked(kans_layer* L, int B) {
-  const TileCfg& cfg = tile_cfg_locked(L, B);
-  if (cfg.splits > 1) {
-    void* old = L->part.p;
-    const int rc = L->part.reserve((size_t)cfg.splits * B * L->D_out * sizeof(float));
-    if (old != L->part.p) ++L->gen;
-    if (rc) {
-      (void)hipGetLastError();  // the launches report the errors that they find
-      L->cfg = choose_tiling(L, B, true);
-    }
+// How one forward runs: its configuration and, where that is split, its workspace.
+struct FwdPlan {
+  TileCfg cfg;
+  float* part = nullptr;  // [splits][B][D_out]
+};
+
+// The plan of a forward of B rows on stream st.  Without a workspace it is unsplit.
+static FwdPlan layer_plan_locked(kans_layer* L, int B, hipStream_t st) {
+  FwdPlan p;
+  p.cfg = tile_cfg_locked(L, B);
+  if (p.cfg.splits > 1) {
+    p.part = kans_stream_workspace(st, (size_t)p.cfg.splits * B * L->D_out * sizeof(float));
+    if (!p.part) p.cfg = choose_tiling(L, B, true);
   }
-  return 0;
+  return p;
 }
 
 // Before a kernel on stream st reads the layer's tiles: behind a re-tiling that
@@ -659,14 +706,14 @@ static int layer_use_weights(kans_layer* L, hipStream_t st) {
   return 0;
 }
 
-// Enqueue one fused forward; allocates nothing when layer_reserve_locked(L, B)
+// Enqueue one fused forward; allocates nothing when layer_plan_locked(L, B, st)
 // ran before (the chain relies on this while capturing a graph).
-// cfg_B > 0: use the tile configuration a forward of cfg_B rows would use (the
-// chunked host forward launches row chunks of a batch with the whole batch's
-// configuration, so every row gets the same result as in one launch; row0, the
-// chunk's first row, gives each chunk its own part of the split workspace).
+// whole: the plan of the batch that these are rows row0.. of (the chunked host
+// forward launches row chunks with the whole batch's configuration, so every row
+// gets the same result as in one launch, and each in its own part of the split
+// workspace).
 static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, long ldy, int B, hipStream_t st,
-                               int x_dtype = -1, int y_dtype = -1, int cfg_B = 0, long row0 = 0) {
+                               int x_dtype = -1, int y_dtype = -1, const FwdPlan* whole = nullptr, long row0 = 0) {
   if (x_dtype < 0) x_dtype = L->dtype;
   if (y_dtype < 0) y_dtype = L->dtype;
   if ((x_dtype != L->dtype && x_dtype != DT_F32) || (y_dtype != L->dtype && y_dtype != DT_F32))
@@ -681,8 +728,10 @@ static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, 
     return kans_fail(KANS_ERR_ARG, "fp32 X must be 32-byte aligned");
   if (ldy < L->D_out) return kans_fail(KANS_ERR_ARG, "ldy=%ld < D_out=%d", ldy, L->D_out);
   if (((uintptr_t)X & 15) != 0) return kans_fail(KANS_ERR_ARG, "X must be 16-byte aligned");
-  int rc = layer_use_weights(L, st);
-  if (rc) return rc;
+  if (!whole) {  // (the chunked forward has done this for both of its streams)
+    int rc = layer_use_weights(L, st);
+    if (rc) return rc;
+  }
   DenseLaunch D{};
   D.dtype = L->dtype;
   D.x_dtype = x_dtype;
@@ -701,26 +750,15 @@ static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, 
   D.D_out = L->D_out;
   D.nfb = L->nfb;
   D.bp = L->bp;
-  if (cfg_B <= 0) cfg_B = B;
-  const TileCfg& cfg = tile_cfg_locked(L, cfg_B);
-  D.wm = cfg.wm;
-  D.nb = cfg.nb;
-  D.splits = cfg.splits;
-  D.ks = cfg.ks;
+  const FwdPlan plan = whole ? *whole : layer_plan_locked(L, B, st);
+  D.wm = plan.cfg.wm;
+  D.nb = plan.cfg.nb;
+  D.splits = plan.cfg.splits;
+  D.ks = plan.cfg.ks;
   D.pair = L->block_pairs;
-  if (D.splits > 1) {
-    if (L->part.cap < (size_t)D.splits * (row0 + B) * L->D_out * sizeof(float))
-      return kans_fail(KANS_ERR_STATE, "split workspace not reserved");
-    D.part = (float*)L->part.p + (size_t)D.splits * row0 * L->D_out;
-  }
+  if (plan.part) D.part = plan.part + (size_t)D.splits * row0 * L->D_out;
   HIP_TRY(launch_dense(D, st));
   return 0;
-}
-
-static int layer_forward_locked(kans_layer* L, const void* X, long ldx, void* Y, long ldy, int B, hipStream_t st) {
-  int rc = layer_reserve_locked(L, B);
-  if (rc) return rc;
-  return layer_launch_locked(L, X, ldx, Y, ldy, B, st);
 }
 
 // Large synchronous host forwards as a pipeline of row chunks: chunk c's input
@@ -730,8 +768,9 @@ static int layer_forward_locked(kans_layer* L, const void* X, long ldx, void* Y,
 // overlap; the host copies of chunk c + 1 run while the device works on
 // chunk c.  Every chunk is launched with the tile configuration of the whole
 // batch, which leaves each row's result exactly what one launch gives, and
-// chunk kernels, which may run at the same time, have their own rows of the
-// split workspace.  Chunks are whole 256-row
+// chunk kernels, which may run at the same time, have their own rows of
+// g_stream's split workspace (nothing else on g_stream runs until the call
+// has drained both).  Chunks are whole 256-row
 // tiles.  Measured on one MI355X, FastKAN fp16 16384 x 1024 -> 1024 from and
 // into host arrays: 2.06 -> 1.54 ms per call (the C entry point, output array
 // reused), 2.87 -> 1.92 ms through FastKAN.__call__ (a fresh output array).
@@ -751,6 +790,8 @@ static int layer_forward_host_chunked(kans_layer* L, const void* X, void* Y, int
     HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     g_chunk_events.push_back(e);
   }
+  const FwdPlan plan = layer_plan_locked(L, B, g_stream);
+  if ((rc = layer_use_weights(L, g_stream))) return rc;
   // the side streams start after everything already on g_stream (a weight upload and its re-tiling
   // kernel, say); the call returns only after every chunk's output copy, so nothing outlives it
   hipEvent_t e0 = g_chunk_events[2 * n];
@@ -781,7 +822,7 @@ static int layer_forward_host_chunked(kans_layer* L, const void* X, void* Y, int
     if (hipEventRecord(e_in, g_copy_in) != hipSuccess || hipStreamWaitEvent(cs, e_in, 0) != hipSuccess)
       return fail(kans_fail(KANS_ERR_HIP, "chunked host forward: input event"));
     if ((rc = layer_launch_locked(L, xd + r0 * pitch_in, ldx, yd + r0 * row_out, L->D_out, rows, cs, x_dtype,
-                                  L->dtype, B, r0)))
+                                  L->dtype, &plan, r0)))
       return fail(rc);
     if (hipEventRecord(e_k, cs) != hipSuccess || hipStreamWaitEvent(g_copy_out, e_k, 0) != hipSuccess)
       return fail(kans_fail(KANS_ERR_HIP, "chunked host forward: kernel event"));
@@ -806,7 +847,6 @@ static int layer_forward_host_locked(kans_layer* L, const void* X, void* Y, int 
   int rc;
   if ((rc = L->x_d.reserve(xbytes))) return rc;
   if ((rc = L->y_d.reserve(ybytes))) return rc;
-  if ((rc = layer_reserve_locked(L, B))) return rc;
   // rows padded with zeros to a multiple of 8 features
   const size_t row_in = (size_t)L->D_in * xes, pitch_in = (size_t)ldx * xes;
   if (g_async) {  // per-call pinned buffers; the result lands in Y at metal_kan_sync
@@ -856,15 +896,13 @@ extern "C" {
 int kans_layer_forward(kans_layer* L, const void* X, long ldx, void* Y, long ldy, int B, void* stream) {
   if (!L || !X || !Y) return kans_fail(KANS_ERR_ARG, "null argument");
   std::lock_guard<std::mutex> lk(g_mu);
-  return layer_forward_locked(L, X, ldx, Y, ldy, B, kans_caller_stream(stream));
+  return layer_launch_locked(L, X, ldx, Y, ldy, B, kans_caller_stream(stream));
 }
 
 int kans_layer_forward_ex(kans_layer* L, const void* X, int x_dtype, long ldx, void* Y, int y_dtype, long ldy, int B,
                           void* stream) {
   if (!L || !X || !Y) return kans_fail(KANS_ERR_ARG, "null argument");
   std::lock_guard<std::mutex> lk(g_mu);
-  int rc = layer_reserve_locked(L, B);
-  if (rc) return rc;
   return layer_launch_locked(L, X, ldx, Y, ldy, B, kans_caller_stream(stream), x_dtype, y_dtype);
 }
 
@@ -1011,13 +1049,13 @@ int kans_layer_time_forward(kans_layer* L, const void* X, long ldx, void* Y, lon
   std::lock_guard<std::mutex> lk(g_mu);
   int rc;
   for (int i = 0; i < warmup; ++i)
-    if ((rc = layer_forward_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
+    if ((rc = layer_launch_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   HIP_TRY(hipEventRecord(e0, g_stream));
   for (int i = 0; i < iters; ++i)
-    if ((rc = layer_forward_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
+    if ((rc = layer_launch_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
   HIP_TRY(hipEventRecord(e1, g_stream));
   HIP_TRY(hipEventSynchronize(e1));
   float t = 0;
@@ -1042,7 +1080,7 @@ int kans_layer_time_window(kans_layer* L, const void* X, long ldx, void* Y, long
   const auto s0 = std::chrono::steady_clock::now();
   do {
     for (int i = 0; i < 16; ++i)
-      if ((rc = layer_forward_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
+      if ((rc = layer_launch_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
     HIP_TRY(hipStreamSynchronize(g_stream));
   } while (std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - s0).count() < settle_ms);
   hipEvent_t e0, e1;
@@ -1052,7 +1090,7 @@ int kans_layer_time_window(kans_layer* L, const void* X, long ldx, void* Y, long
   const auto t0 = std::chrono::steady_clock::now();
   HIP_TRY(hipEventRecord(e0, g_stream));
   for (int i = 0; i < iters; ++i)
-    if ((rc = layer_forward_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
+    if ((rc = layer_launch_locked(L, X, ldx, Y, ldy, B, g_stream))) return rc;
   HIP_TRY(hipEventRecord(e1, g_stream));
   HIP_TRY(hipStreamSynchronize(g_stream));
   const auto t1 = std::chrono::steady_clock::now();
@@ -1311,7 +1349,7 @@ struct kans_chain {
 };
 
 static unsigned chain_gen(const kans_chain* C) {
-  unsigned g = 0;
+  unsigned g = g_ws_gen;
   for (auto* L : C->layers) g = g * 31u + L->gen;
   return g;
 }
@@ -1341,8 +1379,6 @@ static int chain_reserve(kans_chain* C, int B) {
     for (int i = 0; i < 4; ++i)
       if (olds[i] != news[i]) C->graph_B = -1;
   }
-  for (auto* L : C->layers)
-    if ((rc = layer_reserve_locked(L, B))) return rc;
   return 0;
 }
 
@@ -1397,6 +1433,7 @@ static int chain_capture(kans_chain* C, int B, bool copies) {
 static int chain_graph_ready(kans_chain* C, int B, bool copies) {
   int rc = chain_reserve(C, B);
   if (rc) return rc;
+  for (auto* L : C->layers) (void)layer_plan_locked(L, B, g_stream);  // the workspace, before the capture
   if (C->exec && C->graph_B == B && C->graph_in == C->in_dtype && C->graph_gen == chain_gen(C) &&
       C->graph_copies == copies)
     return 0;
@@ -1669,7 +1706,7 @@ struct kans_gated_dense {
 };
 
 static unsigned dgated_gen(const kans_gated_dense* D) {
-  return (D->gate->gen * 31u + D->up->gen) * 31u + D->down->gen;
+  return ((g_ws_gen * 31u + D->gate->gen) * 31u + D->up->gen) * 31u + D->down->gen;
 }
 
 static int dgated_reserve(kans_gated_dense* D, int B) {
@@ -1696,8 +1733,6 @@ static int dgated_reserve(kans_gated_dense* D, int B) {
     for (int i = 0; i < 5; ++i)
       if (olds[i] != news[i]) D->graph_B = -1;
   }
-  for (kans_layer* L : {D->gate, D->up, D->down})
-    if ((rc = layer_reserve_locked(L, B))) return rc;
   return 0;
 }
 
@@ -1743,6 +1778,7 @@ static int dgated_capture(kans_gated_dense* D, int B, bool copies) {
 static int dgated_graph_ready(kans_gated_dense* D, int B, bool copies) {
   int rc = dgated_reserve(D, B);
   if (rc) return rc;
+  for (kans_layer* L : {D->gate, D->up, D->down}) (void)layer_plan_locked(L, B, g_stream);
   if (D->exec && D->graph_B == B && D->graph_in == D->in_dtype && D->graph_gen == dgated_gen(D) &&
       D->graph_copies == copies)
     return 0;

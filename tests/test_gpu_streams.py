@@ -181,3 +181,30 @@ def test_forward_without_memory_for_its_splits(cuda):
         eng.set_tiling(0, 0, 0)
         small = m(x[:64])
     assert torch.isfinite(small).all()
+
+
+def splits_of(lib, m, B):
+    wm, nb, splits = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    assert lib.kans_layer_describe(m.metal_layer._engine().handle, B, ctypes.byref(wm), ctypes.byref(nb),
+                                   ctypes.byref(splits)) == 0
+    return splits.value
+
+
+@pytest.mark.parametrize("basis,dtype", [("rbf", torch.float16), ("cheby", torch.float32)])
+def test_split_forwards_of_one_layer_on_several_streams(gpu, cuda, basis, dtype):
+    """Unordered forwards of a layer whose features are split, on more streams than workspaces are kept for:
+    each has partial sums of its own."""
+    m = module(1024, 1024, basis=basis, degree=8).to(dtype)
+    B, streams = 2048, [torch.cuda.Stream() for _ in range(12)]
+    with torch.no_grad():
+        xs = [(torch.rand(B, 1024, device=cuda) * 2 - 1).to(dtype) for _ in streams]
+        want = [alone(m, x) for x in xs]
+        assert splits_of(gpu, m, B) > 1
+        for pair in (streams[:2], streams):
+            outs = []
+            for _ in range(8 if len(pair) == 2 else 1):
+                for s, x in zip(pair, xs):
+                    with torch.cuda.stream(s):
+                        outs.append(m(x))
+            torch.cuda.synchronize()
+            assert all(torch.equal(y, want[n % len(pair)]) for n, y in enumerate(outs))
