@@ -140,9 +140,9 @@ static long g_ws_users = 0;
 
 float* kans_stream_workspace(hipStream_t st, size_t bytes) {
   if (st == hipStreamPerThread) return nullptr;
-  CaptureRelaxed relaxed;
   auto at = std::find_if(g_ws.begin(), g_ws.end(), [&](const auto& w) { return w->st == st; });
   if (at == g_ws.end()) {
+    CaptureRelaxed relaxed;
     if (g_ws.size() >= kMaxWorkspaces)
       g_ws.erase(std::min_element(g_ws.begin(), g_ws.end(), [](const auto& a, const auto& b) {
         return (a->st == g_stream) != (b->st == g_stream) ? b->st == g_stream : a->asked < b->asked;
@@ -154,6 +154,7 @@ float* kans_stream_workspace(hipStream_t st, size_t bytes) {
   w.asked = ++g_ws_clock;
   if (bytes <= w.buf.cap) return (float*)w.buf.p;
   if (bytes >= w.refused && g_ws_clock < w.retry) return nullptr;
+  CaptureRelaxed relaxed;
   void* p = nullptr;
   if (hipMalloc(&p, bytes) != hipSuccess) {
     (void)hipGetLastError();  // the launches report the errors that they find
@@ -208,6 +209,9 @@ struct kans_layer {
   BasisParams bp{};
   DevBuf Wt, bias_d, x_d, y_d, raw_w, raw_wb;
   WorkspaceUser ws_user;
+  // workspaces of forwards that callers have captured, one each: their graphs hold them (layer_capture_part)
+  std::vector<std::unique_ptr<DevBuf>> captured;
+  size_t captured_bytes = 0;
   bool have_weights = false;
   // Order between the tiles' writer and their readers (layer_use_weights, layer_claim_weights).
   bool w_pending = false;           // re-tiled on w_stream (kans_layer_load_weights_stream), not known to be done
@@ -666,15 +670,33 @@ struct FwdPlan {
   float* part = nullptr;  // [splits][B][D_out]
 };
 
-// The plan of a forward of B rows on stream st.  Without a workspace it is unsplit.
-static FwdPlan layer_plan_locked(kans_layer* L, int B, hipStream_t st) {
-  FwdPlan p;
-  p.cfg = tile_cfg_locked(L, B);
-  if (p.cfg.splits > 1) {
-    p.part = kans_stream_workspace(st, (size_t)p.cfg.splits * B * L->D_out * sizeof(float));
-    if (!p.part) p.cfg = choose_tiling(L, B, true);
+// Workspace of a forward that a caller captures.  The graph keeps the pointer and may be replayed beside any
+// other work, so it is the graph's own, until the layer is destroyed (as the tiles are, which the graph holds
+// too).  Null once the layer's captured forwards hold kMaxPartMB.
+static float* layer_capture_part(kans_layer* L, size_t bytes) {
+  if (L->captured_bytes + bytes > (size_t)(kMaxPartMB * 1e6)) return nullptr;
+  CaptureRelaxed relaxed;
+  auto buf = std::make_unique<DevBuf>();
+  if (buf->reserve(bytes)) {
+    (void)hipGetLastError();
+    return nullptr;
   }
-  return p;
+  L->captured_bytes += bytes;
+  L->captured.push_back(std::move(buf));
+  return (float*)L->captured.back()->p;
+}
+
+// The plan of a forward of B rows on stream st.  Without a workspace it is unsplit.
+static int layer_plan_locked(kans_layer* L, int B, hipStream_t st, FwdPlan* p) {
+  p->cfg = tile_cfg_locked(L, B);
+  p->part = nullptr;
+  if (p->cfg.splits <= 1) return 0;
+  const size_t bytes = (size_t)p->cfg.splits * B * L->D_out * sizeof(float);
+  bool capturing = false;
+  HIP_TRY(kans_capturing(st, &capturing));
+  p->part = capturing ? layer_capture_part(L, bytes) : kans_stream_workspace(st, bytes);
+  if (!p->part) p->cfg = choose_tiling(L, B, true);
+  return 0;
 }
 
 // Before a kernel on stream st reads the layer's tiles: behind a re-tiling that
@@ -706,14 +728,14 @@ static int layer_use_weights(kans_layer* L, hipStream_t st) {
   return 0;
 }
 
-// Enqueue one fused forward; allocates nothing when layer_plan_locked(L, B, st)
-// ran before (the chain relies on this while capturing a graph).
-// whole: the plan of the batch that these are rows row0.. of (the chunked host
-// forward launches row chunks with the whole batch's configuration, so every row
-// gets the same result as in one launch, and each in its own part of the split
-// workspace).
+// Enqueue one fused forward.
+// given: the plan to run by, from a caller that has ordered st behind the layer's
+// weights (the library's own graphs, which order every replay; the chunked host
+// forward, which launches rows row0.. with the whole batch's plan, so that every
+// row gets the same result as in one launch, and each in its own part of the
+// split workspace).
 static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, long ldy, int B, hipStream_t st,
-                               int x_dtype = -1, int y_dtype = -1, const FwdPlan* whole = nullptr, long row0 = 0) {
+                               int x_dtype = -1, int y_dtype = -1, const FwdPlan* given = nullptr, long row0 = 0) {
   if (x_dtype < 0) x_dtype = L->dtype;
   if (y_dtype < 0) y_dtype = L->dtype;
   if ((x_dtype != L->dtype && x_dtype != DT_F32) || (y_dtype != L->dtype && y_dtype != DT_F32))
@@ -728,9 +750,12 @@ static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, 
     return kans_fail(KANS_ERR_ARG, "fp32 X must be 32-byte aligned");
   if (ldy < L->D_out) return kans_fail(KANS_ERR_ARG, "ldy=%ld < D_out=%d", ldy, L->D_out);
   if (((uintptr_t)X & 15) != 0) return kans_fail(KANS_ERR_ARG, "X must be 16-byte aligned");
-  if (!whole) {  // (the chunked forward has done this for both of its streams)
+  FwdPlan plan;
+  if (given) {
+    plan = *given;
+  } else {
     int rc = layer_use_weights(L, st);
-    if (rc) return rc;
+    if (rc || (rc = layer_plan_locked(L, B, st, &plan))) return rc;
   }
   DenseLaunch D{};
   D.dtype = L->dtype;
@@ -750,7 +775,6 @@ static int layer_launch_locked(kans_layer* L, const void* X, long ldx, void* Y, 
   D.D_out = L->D_out;
   D.nfb = L->nfb;
   D.bp = L->bp;
-  const FwdPlan plan = whole ? *whole : layer_plan_locked(L, B, st);
   D.wm = plan.cfg.wm;
   D.nb = plan.cfg.nb;
   D.splits = plan.cfg.splits;
@@ -790,8 +814,8 @@ static int layer_forward_host_chunked(kans_layer* L, const void* X, void* Y, int
     HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     g_chunk_events.push_back(e);
   }
-  const FwdPlan plan = layer_plan_locked(L, B, g_stream);
-  if ((rc = layer_use_weights(L, g_stream))) return rc;
+  FwdPlan plan;
+  if ((rc = layer_use_weights(L, g_stream)) || (rc = layer_plan_locked(L, B, g_stream, &plan))) return rc;
   // the side streams start after everything already on g_stream (a weight upload and its re-tiling
   // kernel, say); the call returns only after every chunk's output copy, so nothing outlives it
   hipEvent_t e0 = g_chunk_events[2 * n];
@@ -1382,8 +1406,21 @@ static int chain_reserve(kans_chain* C, int B) {
   return 0;
 }
 
-// Enqueue all layers: X (ldx) -> ... -> Y (ldy) through the ping-pong buffers.
-static int chain_launch(kans_chain* C, const void* X, long ldx, void* Y, long ldy, int B, hipStream_t st) {
+// The plans of `n` layers that run on g_stream in one graph: every workspace request first, since each may
+// move the workspace.
+static int graph_plans(kans_layer* const* layers, size_t n, int B, std::vector<FwdPlan>* plans) {
+  plans->resize(n);
+  for (int pass = 0; pass < 2; ++pass)
+    for (size_t l = 0; l < n; ++l) {
+      int rc = layer_plan_locked(layers[l], B, g_stream, &(*plans)[l]);
+      if (rc) return rc;
+    }
+  return 0;
+}
+
+// Enqueue all layers: X (ldx) -> ... -> Y (ldy) through the ping-pong buffers (plans: for a graph).
+static int chain_launch(kans_chain* C, const void* X, long ldx, void* Y, long ldy, int B, hipStream_t st,
+                        const std::vector<FwdPlan>* plans = nullptr) {
   const void* src = X;
   long lds = ldx;
   const size_t n = C->layers.size();
@@ -1392,7 +1429,7 @@ static int chain_launch(kans_chain* C, const void* X, long ldx, void* Y, long ld
     long ldd = (l + 1 == n) ? ldy : C->ld_mid;
     const int xdt = (l == 0) ? C->in_dtype : C->mid_dtype;
     const int ydt = (l + 1 == n) ? C->dtype : C->mid_dtype;
-    int rc = layer_launch_locked(C->layers[l], src, lds, dst, ldd, B, st, xdt, ydt);
+    int rc = layer_launch_locked(C->layers[l], src, lds, dst, ldd, B, st, xdt, ydt, plans ? &(*plans)[l] : nullptr);
     if (rc) return rc;
     src = dst;
     lds = ldd;
@@ -1400,7 +1437,7 @@ static int chain_launch(kans_chain* C, const void* X, long ldx, void* Y, long ld
   return 0;
 }
 
-static int chain_capture(kans_chain* C, int B, bool copies) {
+static int chain_capture(kans_chain* C, int B, bool copies, const std::vector<FwdPlan>& plans) {
   if (C->exec) { (void)hipGraphExecDestroy(C->exec); C->exec = nullptr; }
   if (C->graph) { (void)hipGraphDestroy(C->graph); C->graph = nullptr; }
   const size_t es = dtype_size(C->dtype);
@@ -1411,7 +1448,7 @@ static int chain_capture(kans_chain* C, int B, bool copies) {
     hipError_t e = hipMemcpyAsync(C->x_d.p, C->pin_in.p, (size_t)B * C->ld_in * ies, hipMemcpyHostToDevice, g_stream);
     if (e != hipSuccess) rc = kans_fail(KANS_ERR_HIP, "capture H2D: %s", hipGetErrorString(e));
   }
-  if (!rc) rc = chain_launch(C, C->x_d.p, C->ld_in, C->y_d.p, C->ld_out, B, g_stream);
+  if (!rc) rc = chain_launch(C, C->x_d.p, C->ld_in, C->y_d.p, C->ld_out, B, g_stream, &plans);
   if (!rc && copies) {
     hipError_t e = hipMemcpyAsync(C->pin_out.p, C->y_d.p, (size_t)B * C->ld_out * es, hipMemcpyDeviceToHost,
                                   g_stream);
@@ -1433,11 +1470,12 @@ static int chain_capture(kans_chain* C, int B, bool copies) {
 static int chain_graph_ready(kans_chain* C, int B, bool copies) {
   int rc = chain_reserve(C, B);
   if (rc) return rc;
-  for (auto* L : C->layers) (void)layer_plan_locked(L, B, g_stream);  // the workspace, before the capture
+  std::vector<FwdPlan> plans;
+  if ((rc = graph_plans(C->layers.data(), C->layers.size(), B, &plans))) return rc;
   if (C->exec && C->graph_B == B && C->graph_in == C->in_dtype && C->graph_gen == chain_gen(C) &&
       C->graph_copies == copies)
     return 0;
-  return chain_capture(C, B, copies);
+  return chain_capture(C, B, copies, plans);
 }
 
 // Replay the chain's graph on g_stream, behind loads of its layers' weights on other streams (a load moves
@@ -1738,15 +1776,16 @@ static int dgated_reserve(kans_gated_dense* D, int B) {
 
 // Enqueue gate, up, SwiGLU and down: X (x_dtype, ldx) -> Y (block dtype, ldy).
 static int dgated_launch(kans_gated_dense* D, const void* X, int x_dtype, long ldx, void* Y, long ldy, int B,
-                         hipStream_t st) {
+                         hipStream_t st, const std::vector<FwdPlan>* plans = nullptr) {
+  auto plan = [&](int l) { return plans ? &(*plans)[l] : nullptr; };
   int rc;
-  if ((rc = layer_launch_locked(D->gate, X, ldx, D->g_d.p, D->ld_h, B, st, x_dtype, D->dtype))) return rc;
-  if ((rc = layer_launch_locked(D->up, X, ldx, D->u_d.p, D->ld_h, B, st, x_dtype, D->dtype))) return rc;
+  if ((rc = layer_launch_locked(D->gate, X, ldx, D->g_d.p, D->ld_h, B, st, x_dtype, D->dtype, plan(0)))) return rc;
+  if ((rc = layer_launch_locked(D->up, X, ldx, D->u_d.p, D->ld_h, B, st, x_dtype, D->dtype, plan(1)))) return rc;
   HIP_TRY(launch_gated_swiglu(D->dtype, D->g_d.p, D->u_d.p, D->h_d.p, D->ld_h, B, D->h, st));
-  return layer_launch_locked(D->down, D->h_d.p, D->ld_h, Y, ldy, B, st, D->dtype, D->dtype);
+  return layer_launch_locked(D->down, D->h_d.p, D->ld_h, Y, ldy, B, st, D->dtype, D->dtype, plan(2));
 }
 
-static int dgated_capture(kans_gated_dense* D, int B, bool copies) {
+static int dgated_capture(kans_gated_dense* D, int B, bool copies, const std::vector<FwdPlan>& plans) {
   if (D->exec) { (void)hipGraphExecDestroy(D->exec); D->exec = nullptr; }
   if (D->graph) { (void)hipGraphDestroy(D->graph); D->graph = nullptr; }
   const size_t es = dtype_size(D->dtype), ies = dtype_size(D->in_dtype);
@@ -1756,7 +1795,7 @@ static int dgated_capture(kans_gated_dense* D, int B, bool copies) {
     hipError_t e = hipMemcpyAsync(D->x_d.p, D->pin_in.p, (size_t)B * D->ld_in * ies, hipMemcpyHostToDevice, g_stream);
     if (e != hipSuccess) rc = kans_fail(KANS_ERR_HIP, "capture H2D: %s", hipGetErrorString(e));
   }
-  if (!rc) rc = dgated_launch(D, D->x_d.p, D->in_dtype, D->ld_in, D->y_d.p, D->ld_out, B, g_stream);
+  if (!rc) rc = dgated_launch(D, D->x_d.p, D->in_dtype, D->ld_in, D->y_d.p, D->ld_out, B, g_stream, &plans);
   if (!rc && copies) {
     hipError_t e = hipMemcpyAsync(D->pin_out.p, D->y_d.p, (size_t)B * D->ld_out * es, hipMemcpyDeviceToHost,
                                   g_stream);
@@ -1778,11 +1817,13 @@ static int dgated_capture(kans_gated_dense* D, int B, bool copies) {
 static int dgated_graph_ready(kans_gated_dense* D, int B, bool copies) {
   int rc = dgated_reserve(D, B);
   if (rc) return rc;
-  for (kans_layer* L : {D->gate, D->up, D->down}) (void)layer_plan_locked(L, B, g_stream);
+  kans_layer* const layers[] = {D->gate, D->up, D->down};
+  std::vector<FwdPlan> plans;
+  if ((rc = graph_plans(layers, 3, B, &plans))) return rc;
   if (D->exec && D->graph_B == B && D->graph_in == D->in_dtype && D->graph_gen == dgated_gen(D) &&
       D->graph_copies == copies)
     return 0;
-  return dgated_capture(D, B, copies);
+  return dgated_capture(D, B, copies, plans);
 }
 
 // As chain_replay.

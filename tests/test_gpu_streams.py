@@ -208,3 +208,55 @@ def test_split_forwards_of_one_layer_on_several_streams(gpu, cuda, basis, dtype)
                         outs.append(m(x))
             torch.cuda.synchronize()
             assert all(torch.equal(y, want[n % len(pair)]) for n, y in enumerate(outs))
+
+
+def test_captured_split_forward_keeps_its_workspace(gpu, cuda):
+    """A forward with split features in a graph: its replays give the eager bits after larger eager forwards (whose
+    workspace has grown since) and beside others; the graphs captured once the layer's captured workspaces are
+    used up (256 MB) run unsplit."""
+    m = module(1024, 1024, basis="rbf", degree=4).half()
+    B = 2048
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def inputs(n):
+        return (torch.rand(n, 1024, device=cuda) * 2 - 1).half()
+    with torch.no_grad(), torch.cuda.stream(side):
+        x = inputs(B)
+        m(x)
+        assert splits_of(gpu, m, B) > 1
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            y = m(x)
+        big = inputs(3 * B)
+        with torch.cuda.stream(other):
+            m(big)
+        m(big)
+        for n in range(4):
+            x.copy_(inputs(B))
+            side.synchronize()
+            graph.replay()
+            with torch.cuda.stream(other):
+                beside = m(big)
+            side.synchronize()
+            got = y.clone()
+            assert torch.equal(got, m(x)), n
+            torch.cuda.synchronize()
+            assert torch.equal(beside, m(big)), n
+        part = splits_of(gpu, m, B) * B * 1024 * 4
+        graphs = []
+        for _ in range(256_000_000 // part + 2):
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=side):
+                yg = m(x)
+            graphs.append((g, yg))
+        want = m(x)
+        for g, _ in graphs:
+            g.replay()
+        side.synchronize()
+        assert torch.equal(graphs[0][1], want)
+        # The same products summed in another order: 1024 * 5 / 16 = 320 matrix steps, each of which rounds a sum of
+        # at most S = sum |w| (basis values and SiLU(x) are at most 1 here) to fp32, on either side; then one unit in
+        # the last place of fp16.
+        S = sum(p.double().abs().reshape(1024, -1).sum(1) for p in m.parameters())
+        err = (graphs[-1][1].double() - want.double()).abs()
+        assert (err <= 2 * 320 * 2.0 ** -24 * S + 2.0 ** -10 * want.double().abs()).all()
