@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include "kans_common.h"
 #include "../../include/kans_hip.h"
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -70,6 +71,33 @@ int stage_out_drain(StagedOut& out);
 }  // namespace kans
 
 int kans_fail(int code, const char* fmt, ...);
+#define HIP_TRY(expr)                                                                       \
+  do {                                                                                      \
+    hipError_t _e = (expr);                                                                 \
+    if (_e != hipSuccess)                                                                   \
+      return kans_fail(KANS_ERR_HIP, "%s failed: %s (%s:%d)", #expr, hipGetErrorString(_e), \
+                       __FILE__, __LINE__);                                                 \
+  } while (0)
+
+// Grow-only device buffer.
+struct DevBuf {
+  void* p = nullptr;
+  size_t cap = 0;
+  DevBuf() = default;
+  DevBuf(const DevBuf&) = delete;
+  DevBuf& operator=(const DevBuf&) = delete;
+  ~DevBuf() { if (p) (void)hipFree(p); }
+  int reserve(size_t bytes) {
+    if (bytes <= cap) return 0;
+    if (p) HIP_TRY(hipFree(p));
+    p = nullptr;
+    cap = 0;
+    HIP_TRY(hipMalloc(&p, bytes));
+    cap = bytes;
+    return 0;
+  }
+};
+
 // Per-device set-up of kans_gated_forward_noalloc's scratch (kans_qruntime.hip);
 // called by the library's initialisation with `device` current.
 int kans_noalloc_setup(int device);
@@ -103,6 +131,18 @@ struct CaptureRelaxed {
   CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
   ~CaptureRelaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
+// Workspaces of calls that callers have captured on an object's behalf.  A graph keeps the pointer and may be
+// replayed beside any other work, so each call has its own, until the object is destroyed (as its weights are,
+// which the graph holds too).  Null once they hold kMaxCapturedBytes, or without memory.
+struct CapturedWorkspaces {
+  std::vector<std::unique_ptr<DevBuf>> bufs;
+  size_t bytes = 0;
+  float* take(size_t n);
+};
+constexpr size_t kMaxCapturedBytes = size_t(256) << 20;
+// The workspace of a split call on st: the stream's, or one of its own under a caller's capture.
+// *part is null where there is none.
+int kans_split_workspace(CapturedWorkspaces& captured, hipStream_t st, size_t bytes, float** part);
 // fp32 Chebyshev forward (no base branch) of host X on device-resident fp32 weights (kans_runtime.hip);
 // call with the library lock held.
 int kans_ref_cheby_forward_devw_locked(const float* X, const float* W_dev, const float* bias_dev, float* Y, int B,
@@ -115,33 +155,6 @@ int kans_ref_cheby_forward_devw_locked(const float* X, const float* W_dev, const
 std::mutex& kans_mutex();
 int kans_ensure_init();
 int kans_pinned_stage(int which, size_t bytes, void** p);
-
-#define HIP_TRY(expr)                                                                       \
-  do {                                                                                      \
-    hipError_t _e = (expr);                                                                 \
-    if (_e != hipSuccess)                                                                   \
-      return kans_fail(KANS_ERR_HIP, "%s failed: %s (%s:%d)", #expr, hipGetErrorString(_e), \
-                       __FILE__, __LINE__);                                                 \
-  } while (0)
-
-// Grow-only device buffer.
-struct DevBuf {
-  void* p = nullptr;
-  size_t cap = 0;
-  DevBuf() = default;
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-  ~DevBuf() { if (p) (void)hipFree(p); }
-  int reserve(size_t bytes) {
-    if (bytes <= cap) return 0;
-    if (p) HIP_TRY(hipFree(p));
-    p = nullptr;
-    cap = 0;
-    HIP_TRY(hipMalloc(&p, bytes));
-    cap = bytes;
-    return 0;
-  }
-};
 
 // Grow-only pinned host buffer.
 struct Pinned {

@@ -250,8 +250,10 @@ int qp_choose_splits(int B, int D_in, int n_cols, int grp, int slots) {
   const int nfb = (D_in + 15) / 16;
   double best = 0.0;
   int bs = 1;
-  // at least 8 feature blocks per split
+  // at least 8 feature blocks per split, and partial sums of at most kMaxPartBytes
+  constexpr double kMaxPartBytes = 512e6;
   for (int s = 1; s <= std::max(1, std::min(nfb / 8, 32)); ++s) {
+    if (s > 1 && 4.0 * s * B * n_tiles * 256 > kMaxPartBytes) break;
     const long rounds = (tiles * s + 255) / 256, fbps = (nfb + s - 1) / s;
     double t = (double)rounds * (fbps * slots * kSlotUs + kRoundUs);
     if (s > 1) t += kReduceUs + 8.0 * s * B * n_tiles * 256 / kBytesPerUs;

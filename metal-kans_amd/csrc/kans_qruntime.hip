@@ -42,14 +42,16 @@ struct kans_qlayer {
   bool prefill = false;
   int p_nfb = 0, p_nob_pad = 0;
   DevBuf PCb, PCw, PPb, PPw;
-  DevBuf p_part;             // prefill split workspace
+  WorkspaceUser ws_user;     // prefill splits: kans_split_workspace
+  CapturedWorkspaces captured;
   DevBuf hx, hy;             // staging of the host-pointer forward (grow-only)
 };
 
 struct kans_gated {
   kans_qlayer *gate, *up, *down;
   DevBuf hidden;  // SwiGLU(gate, up): [B][h] fp32 (decode, separate kernels) or [B][ld_h] (prefill)
-  DevBuf p_part;  // prefill split workspace
+  WorkspaceUser ws_user;  // prefill splits: kans_split_workspace
+  CapturedWorkspaces captured;
   DevBuf hx, hy;  // staging of the host-pointer forward (grow-only)
 };
 
@@ -387,10 +389,8 @@ int prefill_layer_locked(kans_qlayer* L, const void* X, int x_dtype, long ldx, v
   P.splits = qp_choose_splits(B, L->D_in, L->D_out, 8, L->K + L->has_base - prefill_fold(L, L->basis));
   P.epi = QP_EPI_PLAIN;
   const long pf = qp_part_floats(P);
-  if (pf > 0) {
-    if ((rc = L->p_part.reserve((size_t)pf * sizeof(float)))) return rc;
-    P.part = (float*)L->p_part.p;
-  }
+  if (pf > 0 && (rc = kans_split_workspace(L->captured, st, (size_t)pf * sizeof(float), &P.part))) return rc;
+  if (!P.part) P.splits = 1;
   HIP_TRY(qp_launch(P, st));
   return 0;
 }
@@ -487,13 +487,18 @@ int run_gated_prefill(GatedPrefill& GP, void* hidden, float* part, hipStream_t s
 }
 
 int prefill_gated_locked(kans_gated* G, const void* X, int x_dtype, long ldx, void* Y, int y_dtype, long ldy, int B,
-                         int round16, hipStream_t st) {
+                         int round16, hipStream_t st, bool own_graph) {
   GatedPrefill GP;
   int rc = plan_gated_prefill(G, X, x_dtype, ldx, Y, y_dtype, ldy, B, round16, GP);
   if (rc) return rc;
   if ((rc = G->hidden.reserve(GP.hidden_bytes))) return rc;
-  if (GP.part_bytes && (rc = G->p_part.reserve(GP.part_bytes))) return rc;
-  return run_gated_prefill(GP, G->hidden.p, GP.part_bytes ? (float*)G->p_part.p : nullptr, st);
+  float* part = nullptr;
+  if (GP.part_bytes) {
+    if (own_graph) part = kans_stream_workspace(st, GP.part_bytes);
+    else if ((rc = kans_split_workspace(G->captured, st, GP.part_bytes, &part))) return rc;
+    if (!part) GP.P1.splits = GP.P2.splits = 1;
+  }
+  return run_gated_prefill(GP, G->hidden.p, part, st);
 }
 
 // Decode GEMV split-K of the gated block's two GEMVs for batch B.
@@ -564,15 +569,17 @@ int gated_decode(kans_gated* G, const void* X, int x_dtype, long ldx, void* Y, i
   return gemv_reduce_locked(d, B, ks2, Y, y_dtype, ldy, nt, ws.phi2, ws.s2, ws.part2, st);
 }
 
+// own_graph: captured by the library, which has run the call on st before and replays the graph there before
+// anything else asks for st's workspace.
 int gated_forward_locked(kans_gated* G, const void* X, int x_dtype, long ldx, void* Y, int y_dtype, long ldy, int B,
-                         int round16, hipStream_t st) {
+                         int round16, hipStream_t st, bool own_graph = false) {
   kans_qlayer *g = G->gate, *u = G->up, *d = G->down;
   int rc = check_y(Y, y_dtype, ldy, d->D_out);
   if (rc) return rc;
   if (B < 0) return kans_fail(KANS_ERR_ARG, "B=%d < 0", B);
   if (B == 0) return 0;
   if (B > kMaxDecodeB || !g->decode)
-    return prefill_gated_locked(G, X, x_dtype, ldx, Y, y_dtype, ldy, B, round16, st);
+    return prefill_gated_locked(G, X, x_dtype, ldx, Y, y_dtype, ldy, B, round16, st, own_graph);
   if ((rc = check_x(X, x_dtype, ldx, g->D_in, B))) return rc;
   int ks1, ks2;
   gated_ksplits(G, B, &ks1, &ks2);
@@ -752,16 +759,15 @@ int time_blocks_locked(kans_gated* const* Gs, int n, const void* X, int x_dtype,
       if (g) (void)hipGraphDestroy(g);
   };
   int rc = 0;
-  for (int b = 0; b < n && !rc; ++b) {
-    // one eager call sizes every workspace before any capture
-    if ((rc = gated_forward_locked(Gs[b], X, x_dtype, d, Y, y_dtype, d, B, 1, st))) break;
-    if (!use_graph) continue;
+  // one eager call each sizes every workspace before any capture
+  for (int b = 0; b < n && !rc; ++b) rc = gated_forward_locked(Gs[b], X, x_dtype, d, Y, y_dtype, d, B, 1, st);
+  for (int b = 0; b < n && !rc && use_graph; ++b) {
     hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
       rc = kans_fail(KANS_ERR_HIP, "hipStreamBeginCapture: %s", hipGetErrorString(e));
       break;
     }
-    rc = gated_forward_locked(Gs[b], X, x_dtype, d, Y, y_dtype, d, B, 1, st);
+    rc = gated_forward_locked(Gs[b], X, x_dtype, d, Y, y_dtype, d, B, 1, st, true);
     e = hipStreamEndCapture(st, &graphs[b]);
     if (!rc && e != hipSuccess) rc = kans_fail(KANS_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
     if (!rc && (e = hipGraphInstantiate(&execs[b], graphs[b], nullptr, nullptr, 0)) != hipSuccess)
@@ -804,21 +810,21 @@ static int time_step_locked(kans_gated* const* Gs, int n, void* X, int dtype, vo
   for (int b = 0; b < n; ++b)
     if (Gs[b]->gate->D_in != d || Gs[b]->down->D_out != d)
       return kans_fail(KANS_ERR_ARG, "a decode step chains blocks of one width d -> d");
-  auto step = [&]() -> int {
+  auto step = [&](bool own_graph) -> int {
     for (int b = 0; b < n; ++b) {
       const void* in = (b & 1) ? Y : X;
       void* out = (b & 1) ? X : Y;
-      int rc = gated_forward_locked(Gs[b], in, dtype, d, out, dtype, d, B, 1, st);
+      int rc = gated_forward_locked(Gs[b], in, dtype, d, out, dtype, d, B, 1, st, own_graph);
       if (rc) return rc;
     }
     return 0;
   };
-  int rc = step();  // sizes every workspace before the capture
+  int rc = step(false);  // sizes every workspace before the capture
   if (rc) return rc;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  rc = step();
+  rc = step(true);
   hipError_t e = hipStreamEndCapture(st, &graph);
   if (!rc && e != hipSuccess) rc = kans_fail(KANS_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
   if (!rc && (e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0)) != hipSuccess)

@@ -169,6 +169,27 @@ float* kans_stream_workspace(hipStream_t st, size_t bytes) {
   if (st == g_stream) ++g_ws_gen;
   return (float*)p;
 }
+
+float* CapturedWorkspaces::take(size_t n) {
+  if (bytes + n > kMaxCapturedBytes) return nullptr;
+  CaptureRelaxed relaxed;
+  auto buf = std::make_unique<DevBuf>();
+  if (buf->reserve(n)) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  bytes += n;
+  bufs.push_back(std::move(buf));
+  return (float*)bufs.back()->p;
+}
+
+int kans_split_workspace(CapturedWorkspaces& captured, hipStream_t st, size_t bytes, float** part) {
+  bool capturing = false;
+  HIP_TRY(kans_capturing(st, &capturing));
+  *part = capturing ? captured.take(bytes) : kans_stream_workspace(st, bytes);
+  return 0;
+}
+
 WorkspaceUser::WorkspaceUser() { ++g_ws_users; }
 WorkspaceUser::~WorkspaceUser() {
   if (--g_ws_users > 0) return;
@@ -209,9 +230,7 @@ struct kans_layer {
   BasisParams bp{};
   DevBuf Wt, bias_d, x_d, y_d, raw_w, raw_wb;
   WorkspaceUser ws_user;
-  // workspaces of forwards that callers have captured, one each: their graphs hold them (layer_capture_part)
-  std::vector<std::unique_ptr<DevBuf>> captured;
-  size_t captured_bytes = 0;
+  CapturedWorkspaces captured;
   bool have_weights = false;
   // Order between the tiles' writer and their readers (layer_use_weights, layer_claim_weights).
   bool w_pending = false;           // re-tiled on w_stream (kans_layer_load_weights_stream), not known to be done
@@ -670,31 +689,13 @@ struct FwdPlan {
   float* part = nullptr;  // [splits][B][D_out]
 };
 
-// Workspace of a forward that a caller captures.  The graph keeps the pointer and may be replayed beside any
-// other work, so it is the graph's own, until the layer is destroyed (as the tiles are, which the graph holds
-// too).  Null once the layer's captured forwards hold kMaxPartMB.
-static float* layer_capture_part(kans_layer* L, size_t bytes) {
-  if (L->captured_bytes + bytes > (size_t)(kMaxPartMB * 1e6)) return nullptr;
-  CaptureRelaxed relaxed;
-  auto buf = std::make_unique<DevBuf>();
-  if (buf->reserve(bytes)) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  L->captured_bytes += bytes;
-  L->captured.push_back(std::move(buf));
-  return (float*)L->captured.back()->p;
-}
-
 // The plan of a forward of B rows on stream st.  Without a workspace it is unsplit.
 static int layer_plan_locked(kans_layer* L, int B, hipStream_t st, FwdPlan* p) {
   p->cfg = tile_cfg_locked(L, B);
   p->part = nullptr;
   if (p->cfg.splits <= 1) return 0;
-  const size_t bytes = (size_t)p->cfg.splits * B * L->D_out * sizeof(float);
-  bool capturing = false;
-  HIP_TRY(kans_capturing(st, &capturing));
-  p->part = capturing ? layer_capture_part(L, bytes) : kans_stream_workspace(st, bytes);
+  int rc = kans_split_workspace(L->captured, st, (size_t)p->cfg.splits * B * L->D_out * sizeof(float), &p->part);
+  if (rc) return rc;
   if (!p->part) p->cfg = choose_tiling(L, B, true);
   return 0;
 }

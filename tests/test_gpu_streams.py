@@ -260,3 +260,50 @@ def test_captured_split_forward_keeps_its_workspace(gpu, cuda):
         S = sum(p.double().abs().reshape(1024, -1).sum(1) for p in m.parameters())
         err = (graphs[-1][1].double() - want.double()).abs()
         assert (err <= 2 * 320 * 2.0 ** -24 * S + 2.0 ** -10 * want.double().abs()).all()
+
+
+@pytest.mark.parametrize("fmt", ["int4", "ternary"])
+def test_split_quantized_prefill_on_several_streams_and_captured(gpu, cuda, fmt):
+    """A quantized layer's prefill with split features: unordered on two streams, and captured before the
+    workspace of the eager calls grows."""
+    from test_gpu_qprefill import make_qlayer
+    import metal_kans as mk
+    h, _ = make_qlayer(gpu, fmt, 1024, 520, 4, True, True, 3)
+    B = 300
+
+    def forward(x, stream):
+        with torch.cuda.stream(stream):
+            y = torch.empty((x.shape[0], 520), device=cuda)
+        mk.device.check(gpu.kans_qlayer_forward(h, x.data_ptr(), 0, 1024, y.data_ptr(), 0, 520, x.shape[0],
+                                                stream.cuda_stream), "kans_qlayer_forward")
+        return y
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    try:
+        xs = [torch.rand(B, 1024, device=cuda) * 2 - 1 for _ in range(2)]
+        torch.cuda.synchronize()
+        want = []
+        for x in xs:
+            want.append(forward(x, a))
+            a.synchronize()
+        outs = [forward(x, s) for _ in range(8) for x, s in zip(xs, (a, b))]
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, want[n % 2]) for n, y in enumerate(outs))
+        graph = torch.cuda.CUDAGraph()
+        x = xs[0].clone()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=a):
+            y = forward(x, a)
+        big = torch.rand(8 * B, 1024, device=cuda)
+        torch.cuda.synchronize()
+        forward(big, a)
+        for n in range(4):
+            x.copy_(xs[n % 2])
+            torch.cuda.synchronize()
+            forward(big, b)
+            with torch.cuda.stream(a):
+                graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want[n % 2]), n
+    finally:
+        torch.cuda.synchronize()
+        gpu.kans_qlayer_destroy(h)
