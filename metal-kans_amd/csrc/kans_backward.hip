@@ -683,35 +683,14 @@ using namespace kans;
 
 namespace {
 
-// The split partial sums of a backward: one workspace of at most kBwdWsFloats
-// floats, shared by all calls (library lock held).  A call waits on the device
-// until the last one has read its sums (no wait by stream handle: the handle of
-// a destroyed stream can come back for another).
-DevBuf g_ws;
-hipEvent_t g_ws_done = nullptr;
-
-// The plan of one backward and its workspace; where the device has no memory
-// for the partial sums, the plan without splits.
-int acquire_ws(int B, int D_in, int D_out, int K, int has_base, bool may_split, hipStream_t st, BwdPlan* plan,
-               float** ws) {
+// The plan of one backward and the stream's workspace for its partial sums; without one the plan without splits.
+void acquire_ws(int B, int D_in, int D_out, int K, int has_base, bool may_split, hipStream_t st, BwdPlan* plan,
+                float** ws) {
   *ws = nullptr;
   *plan = plan_backward(B, D_in, D_out, K, has_base, may_split);
-  if (plan->ws_floats == 0) return 0;
-  if (!g_ws_done) HIP_TRY(hipEventCreateWithFlags(&g_ws_done, hipEventDisableTiming));
-  else HIP_TRY(hipStreamWaitEvent(st, g_ws_done, 0));
-  // growing frees the old one, which waits for the device
-  if (g_ws.reserve(plan->ws_floats * sizeof(float))) {
-    (void)hipGetLastError();  // the launches report the errors that they find
-    *plan = plan_backward(B, D_in, D_out, K, has_base, false);
-    return 0;
-  }
-  *ws = (float*)g_ws.p;
-  return 0;
-}
-
-int release_ws(const BwdPlan& plan, hipStream_t st) {
-  if (plan.ws_floats != 0) HIP_TRY(hipEventRecord(g_ws_done, st));
-  return 0;
+  if (plan->ws_floats == 0) return;
+  *ws = kans_stream_workspace(st, plan->ws_floats * sizeof(float));
+  if (!*ws) *plan = plan_backward(B, D_in, D_out, K, has_base, false);
 }
 
 int check_bwd(const void* dY, const void* X, const void* W, const void* Wb, const void* dW, const void* dWb,
@@ -751,10 +730,9 @@ int backward_host(const float* dY, const float* X, const float* W, const float* 
   if (has_base) HIP_TRY(hipMemcpyAsync(d_Wb, Wb, nWb * 4, hipMemcpyHostToDevice, st));
   BwdPlan plan;
   float* ws;
-  if ((rc = acquire_ws(B, D_in, D_out, K, has_base, true, st, &plan, &ws))) return rc;
+  acquire_ws(B, D_in, D_out, K, has_base, true, st, &plan, &ws);
   HIP_TRY(launch_cheby_backward<float>(d_dY, d_X, d_W, has_base ? d_Wb : nullptr, d_dW, has_base ? d_dWb : nullptr,
                                 has_bias ? d_db : nullptr, d_dX, B, D_in, D_out, K, has_base, plan, ws, st));
-  if ((rc = release_ws(plan, st))) return rc;
   HIP_TRY(hipMemcpyAsync(dW, d_dW, nW * 4, hipMemcpyDeviceToHost, st));
   if (has_base) HIP_TRY(hipMemcpyAsync(dWb, d_dWb, nWb * 4, hipMemcpyDeviceToHost, st));
   if (has_bias) HIP_TRY(hipMemcpyAsync(db, d_db, nb * 4, hipMemcpyDeviceToHost, st));
@@ -780,18 +758,18 @@ int kans_cheby_backward_ex(int dtype, const void* dY, const void* X, const void*
   std::lock_guard<std::mutex> lk(kans_mutex());
   if ((rc = kans_ensure_init())) return rc;
   hipStream_t st = kans_caller_stream(stream);
-  // a call recorded into a graph outlives this one: it gets no share of the common workspace
+  // a call recorded into a graph outlives this one: it gets no share of the stream's workspace
   bool capturing = false;
   HIP_TRY(kans_capturing(st, &capturing));
   BwdPlan plan;
   float* ws;
-  if ((rc = acquire_ws(B, D_in, D_out, K, has_base, !capturing, st, &plan, &ws))) return rc;
+  acquire_ws(B, D_in, D_out, K, has_base, !capturing, st, &plan, &ws);
   auto* go = dtype == DT_F16 ? launch_cheby_backward<_Float16>
              : dtype == DT_BF16 ? launch_cheby_backward<__bf16>
                                 : launch_cheby_backward<float>;
   HIP_TRY(go(dY, X, W, has_base ? W_base : nullptr, dW, has_base ? dW_base : nullptr, has_bias ? dbias : nullptr, dX, B,
              D_in, D_out, K, has_base, plan, ws, st));
-  return release_ws(plan, st);
+  return 0;
 }
 
 int kans_cheby_backward(const float* dY, const float* X, const float* W, const float* W_base, float* dW,

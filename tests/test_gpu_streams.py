@@ -307,3 +307,41 @@ def test_split_quantized_prefill_on_several_streams_and_captured(gpu, cuda, fmt)
     finally:
         torch.cuda.synchronize()
         gpu.kans_qlayer_destroy(h)
+
+
+def test_per_thread_stream(gpu, cuda):
+    """hipStreamPerThread, one handle for a stream of each thread: no workspace is kept for it (split forwards and
+    backwards run unsplit) and weights loaded on it are waited for."""
+    import metal_kans as mk
+    per_thread = ctypes.c_void_p(2)
+    m = module(512, 512, degree=5)
+    x, g = torch.rand(256, 512, device=cuda) * 2 - 1, torch.randn(256, 512, device=cuda)
+    with torch.no_grad():
+        y1 = alone(m, x)
+        scale(m, 2.0)
+        want = alone(m, x)
+        torch.cuda.synchronize()
+    assert splits_of(gpu, m, 256) > 1
+    h = m.metal_layer._engine().handle
+    xr = x.clone().requires_grad_(True)
+    m(xr).backward(g)
+    grads = [t.grad for t in (*m.parameters(), xr)]
+    ws = [p.detach() for p in (m.weight, m.base_weight, m.bias_param)]
+    y, outs = torch.empty_like(want), [torch.empty_like(t) for t in grads]
+    torch.cuda.synchronize()
+    hip = hip_runtime()
+    for s in (0.5, 1.0):
+        half = [(w * s).contiguous() for w in ws]
+        torch.cuda.synchronize()
+        mk.device.check(gpu.kans_layer_load_weights_stream(h, *[w.data_ptr() for w in half], per_thread), "load")
+        mk.device.check(gpu.kans_layer_forward_ex(h, x.data_ptr(), 0, 512, y.data_ptr(), 0, 512, 256, per_thread), "forward")
+        assert hip.hipStreamSynchronize(per_thread) == 0
+        ref = y1 if s == 0.5 else want
+        # other order of 512 * 5 fp32 sums
+        assert (y - ref).abs().max() <= 1e-5 * ref.abs().max()
+    mk.device.check(gpu.kans_cheby_backward(g.data_ptr(), x.data_ptr(), ws[0].data_ptr(), ws[1].data_ptr(),
+                                            *[t.data_ptr() for t in outs], 256, 512, 512, 5, 1, 1, per_thread), "backward")
+    assert hip.hipStreamSynchronize(per_thread) == 0
+    for a, b in zip(outs, grads):
+        assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+    assert gpu.kans_stream_keep(per_thread) < 0
