@@ -848,11 +848,11 @@ __global__ void kan_split_finalize4(const float4* __restrict__ part, int splits,
 template <typename S, typename T>
 __global__ void __launch_bounds__(256)
 kan_repack_weights(const S* __restrict__ W, const S* __restrict__ Wb, uint4* __restrict__ Wt,
-                   int D_in, int D_out, int K, int k0, int has_base, int nob_pad, int sparse) {
+                   int D_in, int D_out, int K, int k0, int has_base, int nob_pad, int sparse, int x0) {
   constexpr int CPL = sizeof(T) == 4 ? 3 : 1;  // 16-byte chunks per lane: the three bf16 terms of fp32 weights
   extern __shared__ float seg[];  // [16][row]: 16 K coefficients, then 16 base weights
   const int row = 16 * (K + has_base) + 1;  // odd: a column of rows spreads over the banks
-  const int ob = blockIdx.x >> 1, o_half = 16 * (blockIdx.x & 1), fb = blockIdx.y;
+  const int ox = x0 + blockIdx.x, ob = ox >> 1, o_half = 16 * (ox & 1), fb = blockIdx.y;
   const int i0 = fb * 16, ni = min(16, D_in - i0);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int r = wave; r < 16; r += 4) {
@@ -930,13 +930,14 @@ template <typename S, typename T>
 __global__ void __launch_bounds__(256)
 kan_fold_bias(const S* __restrict__ W, const S* __restrict__ bias, float* __restrict__ out, int D_in, int D_out,
               int K, int fold) {
-  const int o = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (o >= D_out) return;
-  double s = 0.0;
-  if (fold)
-    for (int i = lane; i < D_in; i += 64) s += (double)to_f32(from_f32<T>(to_f32(W[((long)o * D_in + i) * K])));
-  for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
-  if (lane == 0) out[o] = (float)(s + (bias ? (double)to_f32(from_f32<T>(to_f32(bias[o]))) : 0.0));
+  const int lane = threadIdx.x & 63;
+  for (long o = blockIdx.x * 4 + (threadIdx.x >> 6); o < D_out; o += (long)gridDim.x * 4) {
+    double s = 0.0;
+    if (fold)
+      for (int i = lane; i < D_in; i += 64) s += (double)to_f32(from_f32<T>(to_f32(W[(o * D_in + i) * K])));
+    for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
+    if (lane == 0) out[o] = (float)(s + (bias ? (double)to_f32(from_f32<T>(to_f32(bias[o]))) : 0.0));
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1114,11 +1115,17 @@ hipError_t launch_dense(const DenseLaunch& L, hipStream_t st) {
 template <typename S, typename T>
 static hipError_t upload_t(const WeightUpload& U, hipStream_t st) {
   const size_t lds = (size_t)16 * (16 * (U.K + U.has_base) + 1) * sizeof(float);
-  hipLaunchKernelGGL((kan_repack_weights<S, T>), dim3(2 * U.nob_pad, U.nfb), dim3(256), lds, st, (const S*)U.W,
-                     (const S*)U.Wb, (uint4*)U.Wt, U.D_in, U.D_out, U.K, U.fold, U.has_base, U.nob_pad, U.sparse);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || U.bias_out == nullptr) return e;
-  hipLaunchKernelGGL((kan_fold_bias<S, T>), dim3((U.D_out + 3) / 4), dim3(256), 0, st, (const S*)U.W,
+  // a grid holds fewer than 2^32 threads along x
+  constexpr int kMaxX = 1 << 22;
+  for (int x = 0; x < 2 * U.nob_pad; x += kMaxX) {
+    hipLaunchKernelGGL((kan_repack_weights<S, T>), dim3(std::min(kMaxX, 2 * U.nob_pad - x), U.nfb), dim3(256), lds, st,
+                       (const S*)U.W, (const S*)U.Wb, (uint4*)U.Wt, U.D_in, U.D_out, U.K, U.fold, U.has_base, U.nob_pad,
+                       U.sparse, x);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (U.bias_out == nullptr) return hipSuccess;
+  hipLaunchKernelGGL((kan_fold_bias<S, T>), dim3(std::min(U.D_out / 4 + 1, 1 << 22)), dim3(256), 0, st, (const S*)U.W,
                      (const S*)U.bias, U.bias_out, U.D_in, U.D_out, U.K, U.fold);
   return hipGetLastError();
 }

@@ -146,12 +146,13 @@ __global__ void k_qp_tile_tern(const unsigned* __restrict__ wp, int wpr, int D_o
 // The constant term of a Chebyshev layer: one wave per output, w(i) = W[o, i*K].
 template <typename F>
 __device__ __forceinline__ void fold_row(int D_out, int D_in, const void* bias, int bias_dt, float* out, F&& w) {
-  const int o = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (o >= D_out) return;
-  double s = 0.0;
-  for (int i = lane; i < D_in; i += 64) s += (double)w(o, i);
-  for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
-  if (lane == 0) out[o] = (float)(s + (bias ? (double)load_any_f(bias, o, bias_dt) : 0.0));
+  const int lane = threadIdx.x & 63;
+  for (long o = blockIdx.x * 4 + (threadIdx.x >> 6); o < D_out; o += (long)gridDim.x * 4) {
+    double s = 0.0;
+    for (int i = lane; i < D_in; i += 64) s += (double)w((int)o, i);
+    for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
+    if (lane == 0) out[o] = (float)(s + (bias ? (double)load_any_f(bias, o, bias_dt) : 0.0));
+  }
 }
 
 template <int BITS>
@@ -178,10 +179,12 @@ k_q_fold_tern(const unsigned* __restrict__ wp, int wpr, const float* __restrict_
   });
 }
 
+static int fold_blocks(int D_out) { return std::min(D_out / 4 + 1, 1 << 22); }
+
 hipError_t q_fold_affine(int bits, const unsigned char* qw, long rowbytes, const float* scales, const float* biases,
                          int gpr, int D_out, int D_in, int K, const void* bias, int bias_dt, float* out,
                          hipStream_t st) {
-  const dim3 grid((D_out + 3) / 4);
+  const dim3 grid(fold_blocks(D_out));
   if (bits == 8)
     hipLaunchKernelGGL(k_q_fold_affine<8>, grid, dim3(256), 0, st, qw, rowbytes, scales, biases, gpr, D_out, D_in, K,
                        bias, bias_dt, out);
@@ -193,7 +196,7 @@ hipError_t q_fold_affine(int bits, const unsigned char* qw, long rowbytes, const
 
 hipError_t q_fold_tern(const unsigned* wp, int wpr, const float* scales, int gpr, int D_out, int D_in, int K,
                        const void* bias, int bias_dt, float* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_q_fold_tern, dim3((D_out + 3) / 4), dim3(256), 0, st, wp, wpr, scales, gpr, D_out, D_in, K, bias,
+  hipLaunchKernelGGL(k_q_fold_tern, dim3(fold_blocks(D_out)), dim3(256), 0, st, wp, wpr, scales, gpr, D_out, D_in, K, bias,
                      bias_dt, out);
   return hipGetLastError();
 }

@@ -934,3 +934,14 @@ def test_automatic_configuration(gpu, dtype, kind, K, B, d_in, d_out):
     L.set_tiling(32, 4, 1)
     # the same products in another order: fp32 rounding, then the output type's
     assert O.rel_err(y, np.asarray(L(x), np.float64)) <= {"float32": 4e-6, "float16": 2e-3}[dtype]
+
+
+def test_outputs_beyond_a_grid_of_threads(gpu):
+    """2^26 + 5 outputs: the constant term takes a wave each, more than the 2^32 threads of a grid."""
+    import metal_kans as mk
+    L = cast(mk.ChebyKAN(1, (1 << 26) + 5, degree=2, bias=False, use_base=False), "float16")
+    x = np.array([[-0.75], [0.5]], np.float32)
+    y = np.asarray(L(x))
+    W = L.w_cheby.astype(np.float32)
+    for b in range(2):   # T_0 = 1, T_1 = x exactly; only the result, below 2, is rounded to fp16
+        assert np.abs(y[b] - (W[:, 0] + x[b, 0] * W[:, 1])).max() <= 2.0 ** -11
