@@ -104,19 +104,18 @@ __device__ __forceinline__ float silu_deriv_f32(float x) {
 
 // An operand tile (32 x 16) of a stage: N terms of 64 lanes x 16 bytes, from
 // its term `at` on.
-__device__ __forceinline__ void put_tile(uint4* stage, int at, int lane, const float* v) {
-  const Split8 s = split8(v);
+__device__ __forceinline__ void put_tile(uint4* stage, int at, int lane, const Split8& s) {
 #pragma unroll
   for (int q = 0; q < 3; ++q) stage[(at + q) * 64 + lane] = s.t[q];
 }
-// bf16 values: the finite ones, and the others
+// bf16 values: the finite ones (+-1 in the others' place, as split8's h), and the others
 __device__ __forceinline__ void put_tile_bf16(uint4* stage, int at, int lane, const float* v) {
   unsigned d[2][4];
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     const float a = v[2 * p], b = v[2 * p + 1];
     const bool fa = __builtin_fabsf(a) < __builtin_inff(), fb = __builtin_fabsf(b) < __builtin_inff();
-    d[0][p] = bf16_pair(fa ? a : 0.0f, fb ? b : 0.0f);
+    d[0][p] = bf16_pair(fa ? a : __builtin_copysignf(1.0f, a), fb ? b : __builtin_copysignf(1.0f, b));
     d[1][p] = bf16_pair(fa ? 0.0f : a, fb ? 0.0f : b);
   }
 #pragma unroll
@@ -234,7 +233,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs<T> P) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) ra[j] = to_f32(la[j]);
       if constexpr (TA == 2) put_tile_bf16(st, a_tile * TA, lane, ra);
-      else put_tile(st, a_tile * TA, lane, ra);
+      else put_tile(st, a_tile * TA, lane, split8(ra));
       bsum += ((ra[0] + ra[1]) + (ra[2] + ra[3])) + ((ra[4] + ra[5]) + (ra[6] + ra[7]));
     }
     float tw[8], c[8], p[8];  // 2t, T_k, T_{k-1}
@@ -262,10 +261,10 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs<T> P) {
           float v[8];
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[j] = silu_f32(rx[j]);
-          put_tile(st, NA * TA + (wf * SG + s) * 3, lane, v);
+          put_tile(st, NA * TA + (wf * SG + s) * 3, lane, split8(v));
         }
       } else {
-        if (mine) put_tile(st, NA * TA + (wf * SG + s) * 3, lane, c);
+        if (mine) put_tile(st, NA * TA + (wf * SG + s) * 3, lane, split8_bounded(c));
         if (s + 1 < SG) advance();
       }
     }
@@ -434,7 +433,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
       for (int r = 0; r < R; ++r)
         if (r * 8 + wave < NT) {
           if constexpr (TT == 3) {
-            put_tile(st, (r * 8 + wave) * TT, lane, raw[r]);
+            put_tile(st, (r * 8 + wave) * TT, lane, split8(raw[r]));
           } else {
             uint4 u;
             __builtin_memcpy(&u, raw[r], 16);

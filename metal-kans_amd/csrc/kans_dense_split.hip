@@ -126,16 +126,18 @@ kan_fused_split(const float* __restrict__ X, long ldx, const uint4* __restrict__
     if (fb + 1 < fb_end) xload(fb + 1);
     gen.begin(xf, bp);
   };
-  auto values = [&](int s, float* v) {
+  // A operand of slot s
+  auto frags = [&](int s, bf16x8 (&a)[3]) {
+    float v[8];
+    Split8 t;
     if (has_base && s == 0) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = silu_f32(xf[j]);
+      t = split8(v);
     } else {
       gen.next(s - has_base, bp, rbf_tab, v);
+      t = split8_bounded(v);
     }
-  };
-  auto frags = [&](const float* v, bf16x8 (&a)[3]) {
-    const Split8 t = split8(v);
 #pragma unroll
     for (int q = 0; q < 3; ++q) a[q] = *reinterpret_cast<const bf16x8*>(&t.t[q]);
   };
@@ -164,10 +166,8 @@ kan_fused_split(const float* __restrict__ X, long ldx, const uint4* __restrict__
   int fb = fb_begin, s = 0;
   bf16x8 a[3];
   {
-    float v[8];
     begin_block(fb);
-    values(0, v);
-    frags(v, a);
+    frags(0, a);
   }
   auto chunk = [&](int c, const uint4* cur, uint4* nxt) {
     if ((c + 1) * CS < nsteps) dma(c + 1, nxt);
@@ -178,10 +178,8 @@ kan_fused_split(const float* __restrict__ X, long ldx, const uint4* __restrict__
         s = 0;
         if (++fb < fb_end) begin_block(fb);
       }
-      float v[8];
-      values(s, v);
       bf16x8 an[3];
-      frags(v, an);
+      frags(s, an);
       const uint4* st = cur + q * STEP + lane;
       bf16x8 b[2][3];
       auto bread = [&](int nb) {
@@ -324,8 +322,7 @@ kan_fused_split_sparse(const float* __restrict__ X, long ldx, const uint4* __res
     }
     if (fb + 1 < fb_end) xload(fb + 1);
   };
-  auto frags = [&](const float* v, bf16x8 (&a)[3]) {
-    const Split8 t = split8(v);
+  auto frags = [&](const Split8& t, bf16x8 (&a)[3]) {
 #pragma unroll
     for (int q = 0; q < 3; ++q) a[q] = *reinterpret_cast<const bf16x8*>(&t.t[q]);
   };
@@ -365,7 +362,7 @@ kan_fused_split_sparse(const float* __restrict__ X, long ldx, const uint4* __res
       v[2 * g + 1] = (unsigned)k1 < 8u ? v1 : 0.0f;
       idx |= (((k0 >> 2) & 1) | (k1 & 4) | 8) << (4 * g);
     }
-    frags(v, a);
+    frags(split8_bounded(v), a);
   };
 
   floatx16 acc[NB];
@@ -387,7 +384,7 @@ kan_fused_split_sparse(const float* __restrict__ X, long ldx, const uint4* __res
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = silu_f32(xf[j]);
         bf16x8 a[3];
-        frags(v, a);
+        frags(split8(v), a);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
           bf16x8 b[3];

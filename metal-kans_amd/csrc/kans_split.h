@@ -1,8 +1,11 @@
 // fp32 products on the bf16 matrix cores (gfx950).
 //
 // An fp32 value is the sum of three bf16 values h + m + l (8 + 8 + 8 significant
-// bits, each the rounding of what the ones before it left): exact while l stays
-// a normal number, i.e. for |v| >= 2^-110.  A product of two such values is
+// bits, each the rounding of what the ones before it left), as in published
+// work on products in emulated precision (Henry, Tang and Heinecke, "Leveraging
+// the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", 2019).  Exact for |v| >= 2^-110; smaller values keep all bits
+// down to 2^-133, the smallest bf16 number (error at most 2^-134 a value).  A product of two such values is
 // taken as the six MFMAs
 //   l_a h_b, m_a m_b, h_a l_b, m_a h_b, h_a m_b, h_a h_b
 // whose bf16 x bf16 products are exact in fp32; what is left out (m l, l m,
@@ -27,31 +30,65 @@ __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
   return u;
 }
 
-// The three bf16 terms of 8 fp32 values, each packed as one MFMA operand.  An
-// infinite or NaN value (and a finite one that rounds to infinity in bf16,
-// above 3.3895e38) goes into the l term alone: of the six products it then
-// enters one, l_a h_b, where h = inf, m = l = 0 would meet zeros and terms of
-// the other sign in three more and turn an infinite sum into NaN.
+// The three bf16 terms of 8 fp32 values, each packed as one MFMA operand.
 struct Split8 {
   uint4 t[3];
 };
 
-__device__ __forceinline__ Split8 split8(const float* v) {
-  constexpr float kFiniteMax = 0x1.fep+127f;  // largest bf16
+// Finite values of at most the largest bf16 one (0x1.fep127), and basis values
+// (|v| <= 1 or NaN: a NaN makes all three terms NaN).
+__device__ __forceinline__ Split8 split8_bounded(const float* v) {
   unsigned d[3][4];
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     const float a = v[2 * p], b = v[2 * p + 1];
-    const bool fa = __builtin_fabsf(a) <= kFiniteMax, fb = __builtin_fabsf(b) <= kFiniteMax;
-    const float ca = fa ? a : 0.0f, cb = fb ? b : 0.0f;
-    const unsigned h = bf16_pair(ca, cb);
-    const float ra = ca - __uint_as_float(h << 16), rb = cb - __uint_as_float(h & 0xffff0000u);
+    const unsigned h = bf16_pair(a, b);
+    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
     const unsigned m = bf16_pair(ra, rb);
-    const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
     d[0][p] = h;
     d[1][p] = m;
-    d[2][p] = bf16_pair(fa ? sa : a, fb ? sb : b);
+    d[2][p] = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
   }
+  Split8 s;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) s.t[q] = make_uint4(d[q][0], d[q][1], d[q][2], d[q][3]);
+  return s;
+}
+
+// Any fp32 values.  Above the largest bf16 value the h term of a finite one is cut
+// off there instead of rounding to infinity; m and l still hold what is left.  An
+// infinite or NaN value goes into the l term, with h = +-1 and m = 0: of the six
+// products l_a h_b and h_a l_b give the infinite result or the NaN, with the right
+// sign also where both values are infinite, and the others stay finite (an infinite
+// h would meet terms of the other sign and the zeros of m and l, which turns an
+// infinite sum into NaN).  A wave takes this path only if one of its values needs
+// it (for all of them it would cost 1.3 % of a training step).
+__device__ __forceinline__ Split8 split8(const float* v) {
+  constexpr float kMaxBf16 = 0x1.fep+127f;
+  float sum = 0.0f;  // of the magnitudes: infinite or NaN if one of them is
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) sum += __builtin_fabsf(v[j]) + __builtin_fabsf(v[j + 1]);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= kMaxBf16)) == 0, 1)) return split8_bounded(v);
+  float c[8], l[8];
+  unsigned d[3][4];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) c[j] = __builtin_fabsf(v[j]) < __builtin_inff() ? v[j] : __builtin_copysignf(1.0f, v[j]);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const float a = c[2 * p], b = c[2 * p + 1];
+    const unsigned h = bf16_pair(__builtin_amdgcn_fmed3f(a, -kMaxBf16, kMaxBf16), __builtin_amdgcn_fmed3f(b, -kMaxBf16, kMaxBf16));
+    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+    const unsigned m = bf16_pair(ra, rb);
+    d[0][p] = h;
+    d[1][p] = m;
+    l[2 * p] = ra - __uint_as_float(m << 16);
+    l[2 * p + 1] = rb - __uint_as_float(m & 0xffff0000u);
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    if (!(__builtin_fabsf(v[j]) < __builtin_inff())) l[j] = v[j];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) d[2][p] = bf16_pair(l[2 * p], l[2 * p + 1]);
   Split8 s;
 #pragma unroll
   for (int q = 0; q < 3; ++q) s.t[q] = make_uint4(d[q][0], d[q][1], d[q][2], d[q][3]);

@@ -328,3 +328,28 @@ def test_backward_16bit_infinities_and_limits(gpu):
         assert gpu.kans_cheby_backward_ex(code, *ptrs, B, D_in, D_out, 11, 1, 1, None) < 0
         assert gpu.kans_cheby_backward_ex(code, *ptrs, B, D_in, D_out, 1, 0, 1, None) < 0
     assert gpu.kans_cheby_backward_ex(7, *ptrs, B, D_in, D_out, K, 1, 1, None) < 0
+
+
+def test_backward_largest_values_and_products_of_infinities(gpu):
+    """Gradients of the largest finite size stay finite, and an infinite gradient times an infinite weight or
+    activation is an infinity of the right sign."""
+    B, D_in, D_out, K = 40, 36, 34, 5
+    dY, X, W, Wb = case(5, B, D_in, D_out, K, True, True, -0.9, 0.9)
+    big = np.float32(np.finfo(np.float32).max)
+    W *= np.float32(0.01)
+    Wb *= np.float32(0.01)
+    dY[:] = 0
+    dY[np.arange(34), np.arange(34)] = big * np.where(np.arange(34) % 2, 1, -1).astype(np.float32)
+    got = run_host(gpu, gpu.metal_kan_cheby_backward_fused, dY, X, W, Wb, True)
+    ref = O.cheby_backward(dY, X, W, Wb, True)
+    for g, r in zip(got, ref):   # one product in each sum, of fp32 factors (T'_k and SiLU' of a few roundings)
+        assert np.isfinite(g).all()
+        assert (np.abs(g - r) <= 2.0 ** -20 * np.abs(r) + 2.0 ** -22 * np.abs(r).max()).all()
+    dY, X, W, Wb = case(6, B, D_in, D_out, K, True, True, -0.9, 0.9)
+    dY[7, 11], X[7, 2], Wb[11, 4] = -np.inf, np.inf, np.inf
+    dW, dWb, db, dX = run_host(gpu, gpu.metal_kan_cheby_backward_fused, dY, X, W, Wb, True)
+    assert dWb[11, 2] == -np.inf              # -inf * SiLU(inf)
+    assert dX[7, 4] == -np.inf or np.isnan(dX[7, 4])
+    keep = np.delete(np.arange(D_out), 11)
+    assert np.isfinite(dWb[np.ix_(keep, np.delete(np.arange(D_in), 2))]).all()
+    np.testing.assert_array_equal(dWb[keep, 2], np.sign(dY[7, keep]) * np.inf)

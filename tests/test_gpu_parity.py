@@ -945,3 +945,48 @@ def test_outputs_beyond_a_grid_of_threads(gpu):
     W = L.w_cheby.astype(np.float32)
     for b in range(2):   # T_0 = 1, T_1 = x exactly; only the result, below 2, is rounded to fp16
         assert np.abs(y[b] - (W[:, 0] + x[b, 0] * W[:, 1])).max() <= 2.0 ** -11
+
+
+@pytest.mark.parametrize("kind,K", [("cheby", 4), ("rbf", 5), ("bspline", 4), ("bspline", 8)])
+def test_fp32_range_of_the_operands(gpu, kind, K):
+    """fp32 layers multiply three bf16 terms of each operand: the largest finite weights stay finite, infinities
+    keep their sign (one infinite factor or two), and weights below 2^-110 are off by at most 2^-134 each."""
+    import metal_kans as mk
+    d_in, d_out = 24, 40
+    rng = np.random.default_rng(11)
+    x = rng.uniform(-0.9, 0.9, (33, d_in)).astype(np.float32)
+    L = make_layer(mk, kind, d_in, d_out, K, bias=False)
+    W0, Wb0 = getattr(L, L._weight_attr).copy(), L.w_base.copy()
+    # one weight of the largest finite value in each output, the others below a thousandth of it
+    big = np.float32(np.finfo(np.float32).max)
+    W = (W0 / np.abs(W0).max() * np.float32(1e34)).astype(np.float32)
+    k = 1 + np.arange(d_out) % (K - 1)                     # (T_0 takes no part in the products)
+    W[np.arange(d_out), (np.arange(d_out) % d_in) * K + k] = big * rng.choice([-1, 1], d_out).astype(np.float32)
+    setattr(L, L._weight_attr, W)
+    ref = oracle_of(L, x)
+    y = np.asarray(L(x))
+    inside = np.abs(ref) < 3.3e38
+    assert np.isfinite(y[inside]).all()
+    # the large weight times a basis value that is computed in fp32 (values up to 1, a few roundings: 2^-21), beside
+    # which the others' rounding is nothing
+    assert (np.abs(y - ref)[inside] <= 2.0 ** -21 * float(big)).all()
+    # weights below 2^-110
+    for scale in (1e-34, 1e-36, 1e-38):
+        setattr(L, L._weight_attr, (W0 * scale).astype(np.float32))
+        L.w_base = (Wb0 * scale).astype(np.float32)
+        y = np.asarray(L(x), np.float64)
+        # (basis values and SiLU are below 1; T_0's coefficients are summed apart)
+        assert np.abs(y - oracle_of(L, x)).max() <= d_in * (K + 1) * 2.0 ** -134 + 1e-6 * np.abs(y).max()
+    # an infinite weight, and an infinite input times an infinite weight
+    setattr(L, L._weight_attr, W0)
+    L.w_base = Wb0.copy()
+    x[5, 3] = np.inf
+    if L.has_base:
+        L.w_base[7, 3], L.w_base[8, 3], L.w_base[9, 3] = np.inf, -np.inf, np.nan
+        y = np.asarray(L(x))
+        assert y[5, 7] == np.inf and y[5, 8] == -np.inf and np.isnan(y[:, 9]).all()
+        others = np.delete(np.arange(d_out), [7, 8, 9])
+        np.testing.assert_array_equal(y[5, others], np.sign(L.w_base[others, 3]) * np.inf)
+        rows = np.delete(np.arange(33), 5)
+        np.testing.assert_array_equal(y[rows, 7], np.sign(x[rows, 3]) * np.inf)
+        assert np.isfinite(y[np.ix_(rows, others)]).all()
