@@ -273,7 +273,7 @@ int kans_cheby_backward(const float* dY, const float* X, const float* W, const f
                         int has_bias, void* stream);
 
 /* as kans_cheby_backward for arrays of `dtype` (all of them: operands and gradients; 16-bit for
- * 1 <= K - 1 + has_base <= 10, else KANS_ERR_UNSUPPORTED).  16-bit values enter the products as they are, the
+ * 1 <= K - 1 + has_base <= 10, D_in * K <= 2^26 and D_out <= 2^25, else KANS_ERR_UNSUPPORTED).  16-bit values enter the products as they are, the
  * sums are fp32 and each gradient is rounded once. */
 int kans_cheby_backward_ex(int dtype, const void* dY, const void* X, const void* W, const void* W_base, void* dW,
                            void* dW_base, void* dbias, void* dX, int B, int D_in, int D_out, int K, int has_base,

@@ -64,6 +64,7 @@
 #include "kans_split.h"
 #include "kans_tile.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace kans {
 namespace {
@@ -81,7 +82,8 @@ struct BwdArgs {
   float* part;   // split partial sums (null: one split, results written directly)
   float* dbp;    // split partial sums of dbias
   int B, D_in, D_out, K, has_base, NS;
-  int m_tiles, f_tiles, groups;
+  int m_tiles, f_tiles, groups;  // of this launch, whose first feature tile is f0
+  int f0;
   int steps, steps_per_split;
   int vec;       // dX: rows of dY readable with 16-byte loads
 };
@@ -188,6 +190,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dw(BwdArgs<T> P) {
   const int g = lin / tiles;
   int m_tile, f_tile;
   tile_of(lin - g * tiles, P.m_tiles, P.f_tiles, m_tile, f_tile);
+  f_tile += P.f0;
   const int o0 = m_tile * (NA * 32), i0 = f_tile * kBwdF, s0 = g * SG;
   const int split = blockIdx.y;
   const int t0 = split * P.steps_per_split;
@@ -356,8 +359,10 @@ __global__ void k_cheby_bwd_dw_reduce(BwdArgs<T> P, int splits) {
   }
 }
 
-template <typename T, int SG, int MB>
+// kWide: lane offsets in 64 bits, for rows of W or dY that 32 bits do not reach over (wide_rows).
+template <typename T, int SG, int MB, bool kWide>
 __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
+  typedef typename std::conditional<kWide, size_t, unsigned>::type offset;
   constexpr int NA = 4 * MB, NT = NA + 2 * SG, TT = BwdTerms<T>::dx;
   constexpr int R = (NT + 7) / 8;  // operand tiles a wave loads and splits per step
   __shared__ uint4 stage[2][NT * TT * 64];
@@ -367,6 +372,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
 
   int m_tile, f_tile;
   tile_of(xcd_remap(blockIdx.x, P.m_tiles * P.f_tiles), P.m_tiles, P.f_tiles, m_tile, f_tile);
+  f_tile += P.f0;
   const int b0 = m_tile * (NA * 32), i0 = f_tile * kBwdF;
   const int split = blockIdx.y;
   const int t0 = split * P.steps_per_split;
@@ -381,7 +387,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
     // slot weights; lanes past B / D_in and slots past NS repeat the last one
     // (src: the wave's first address, lane_off: this lane's bytes from it)
     const T* src[R];
-    unsigned lane_off[R];
+    offset lane_off[R];
     long stride[R];
     T raw[R][8];
 #pragma unroll
@@ -391,7 +397,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
       if (id < NA) {
         const int row = min(b0 + id * 32, P.B - 1);
         src[r] = P.dY + (long)row * P.D_out + o;
-        lane_off[r] = (unsigned)sizeof(T) * ((unsigned)min(lane & 31, P.B - 1 - row) * P.D_out + 8 * half);
+        lane_off[r] = (offset)sizeof(T) * ((offset)min(lane & 31, P.B - 1 - row) * P.D_out + 8 * half);
         stride[r] = 1;
       } else {
         const int q = min(id, NT - 1) - NA, f = q / SG;
@@ -400,7 +406,7 @@ __global__ void __launch_bounds__(kBwdThreads) k_cheby_bwd_dx(BwdArgs<T> P) {
         const bool base = P.has_base != 0 && sl == 0;
         stride[r] = base ? P.D_in : Kd;
         src[r] = (base ? P.Wb : P.W + k) + o * stride[r];
-        lane_off[r] = (unsigned)sizeof(T) * (8u * half * (unsigned)stride[r] + (unsigned)ic * (base ? 1 : P.K));
+        lane_off[r] = (offset)sizeof(T) * ((offset)(8 * half) * (offset)stride[r] + (offset)ic * (base ? 1 : P.K));
       }
     }
     auto load = [&](int t) {
@@ -569,11 +575,19 @@ int choose_splits(long tiles, int steps, long max_by_ws) {
   return (int)best;
 }
 
+// Whether the dX kernel's 32-bit lane offsets fall short: 36 bytes a reduction index of W, 124 bytes an output of dY.
+bool wide_rows(int D_in, int D_out, int K) { return (long)D_in * K > (1L << 26) || D_out > (1 << 25); }
+
 struct BwdPlan {
   int SG, MB, groups, NS;
+  bool wide;
   int splits_w, splits_x;
   size_t ws_floats;
+  bool fits;  // a grid holds the workgroups of one feature tile
 };
+
+// Workgroups of one launch: a grid holds fewer than 2^32 threads along x.
+constexpr long kBwdMaxGrid = 1L << 22;
 
 // Workspace cap of the split partial sums (floats).
 constexpr size_t kBwdWsFloats = size_t(64) << 20;
@@ -581,12 +595,15 @@ constexpr size_t kBwdWsFloats = size_t(64) << 20;
 BwdPlan plan_backward(int B, int D_in, int D_out, int K, int has_base, bool may_split) {
   BwdPlan p{};
   p.NS = K - 1 + has_base;
-  p.groups = std::max(1, (p.NS + kBwdMaxSG - 1) / kBwdMaxSG);
+  // (wide rows: one instantiation of the dX kernel, slot by slot)
+  p.wide = wide_rows(D_in, D_out, K);
+  p.groups = p.wide ? std::max(1, p.NS) : std::max(1, (p.NS + kBwdMaxSG - 1) / kBwdMaxSG);
   p.SG = std::max(1, (p.NS + p.groups - 1) / p.groups);
   p.MB = p.SG <= 5 ? 2 : 1;
   const int M = 4 * p.MB * 32;
   const long f_tiles = (D_in + kBwdF - 1) / kBwdF;
   const long per_w = (long)D_out * ((long)p.NS * D_in + 1), per_x = (long)B * D_in;
+  p.fits = ((long)D_out + M - 1) / M * p.groups <= kBwdMaxGrid && ((long)B + M - 1) / M <= kBwdMaxGrid;
   const long cap = may_split ? (long)kBwdWsFloats : 0;
   p.splits_w = choose_splits(((D_out + M - 1) / M) * f_tiles * p.groups, (B + kBwdStep - 1) / kBwdStep, cap / per_w);
   p.splits_x = choose_splits(((B + M - 1) / M) * f_tiles, (D_out + kBwdStep - 1) / kBwdStep, cap / per_x);
@@ -595,11 +612,21 @@ BwdPlan plan_backward(int B, int D_in, int D_out, int K, int has_base, bool may_
   return p;
 }
 
-template <typename T, int SG, int MB>
+template <typename T, int SG, int MB, bool kWide = false>
 hipError_t launch_bwd(BwdArgs<T> A, const BwdPlan& p, float* ws, hipStream_t st) {
   constexpr int M = 4 * MB * 32;
   A.groups = p.groups;
-  A.f_tiles = (A.D_in + kBwdF - 1) / kBwdF;
+  const int f_tiles = (A.D_in + kBwdF - 1) / kBwdF;
+  // launch(first feature tile, feature tiles) in parts of at most kBwdMaxGrid workgroups, `per` to a feature tile
+  auto parts = [&](long per, auto launch) {
+    const int n = (int)std::min<long>(f_tiles, std::max(1L, kBwdMaxGrid / per));
+    hipError_t e = hipSuccess;
+    for (int f = 0; f < f_tiles && e == hipSuccess; f += n) {
+      launch(f, std::min(n, f_tiles - f));
+      e = hipGetLastError();
+    }
+    return e;
+  };
   // dW: outputs x (slot, feature), contraction over the batch
   BwdArgs<T> W = A;
   W.m_tiles = (A.D_out + M - 1) / M;
@@ -608,9 +635,11 @@ hipError_t launch_bwd(BwdArgs<T> A, const BwdPlan& p, float* ws, hipStream_t st)
   const int splits_w = (W.steps + W.steps_per_split - 1) / W.steps_per_split;
   W.part = splits_w > 1 ? ws : nullptr;
   W.dbp = splits_w > 1 ? ws + (size_t)splits_w * A.D_out * A.NS * A.D_in : nullptr;
-  hipLaunchKernelGGL((k_cheby_bwd_dw<T, SG, MB>), dim3(W.m_tiles * A.f_tiles * A.groups, splits_w), dim3(kBwdThreads), 0,
-                     st, W);
-  hipError_t e = hipGetLastError();
+  hipError_t e = parts((long)W.m_tiles * A.groups, [&](int f0, int n) {
+    W.f0 = f0;
+    W.f_tiles = n;
+    hipLaunchKernelGGL((k_cheby_bwd_dw<T, SG, MB>), dim3(W.m_tiles * n * A.groups, splits_w), dim3(kBwdThreads), 0, st, W);
+  });
   if (e != hipSuccess) return e;
   if (splits_w > 1) {
     hipLaunchKernelGGL((k_cheby_bwd_dw_reduce<T>), dim3(reduce_blocks((long)A.D_out * A.NS * A.D_in)), dim3(256), 0, st, W,
@@ -625,8 +654,12 @@ hipError_t launch_bwd(BwdArgs<T> A, const BwdPlan& p, float* ws, hipStream_t st)
   const int splits_x = (X.steps + X.steps_per_split - 1) / X.steps_per_split;
   X.part = splits_x > 1 ? ws : nullptr;
   X.vec = A.D_out % (16 / (int)sizeof(T)) == 0 && ((uintptr_t)A.dY & 15) == 0;
-  hipLaunchKernelGGL((k_cheby_bwd_dx<T, SG, MB>), dim3(X.m_tiles * A.f_tiles, splits_x), dim3(kBwdThreads), 0, st, X);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  e = parts(X.m_tiles, [&](int f0, int n) {
+    X.f0 = f0;
+    X.f_tiles = n;
+    hipLaunchKernelGGL((k_cheby_bwd_dx<T, SG, MB, kWide>), dim3(X.m_tiles * n, splits_x), dim3(kBwdThreads), 0, st, X);
+  });
+  if (e != hipSuccess) return e;
   if (splits_x > 1) {
     const long n = (long)A.B * A.D_in;
     hipLaunchKernelGGL((k_sum_splits<T>), dim3(reduce_blocks(n)), dim3(256), 0, st, ws, A.dX, splits_x, n);
@@ -638,6 +671,9 @@ hipError_t launch_bwd(BwdArgs<T> A, const BwdPlan& p, float* ws, hipStream_t st)
 
 template <typename T>
 hipError_t launch_slots(const BwdArgs<T>& A, const BwdPlan& p, float* ws, hipStream_t st) {
+  if constexpr (sizeof(T) == 4) {
+    if (p.wide) return launch_bwd<T, 1, 2, true>(A, p, ws, st);
+  }
   switch (p.SG) {
     case 1: return launch_bwd<T, 1, 2>(A, p, ws, st);
     case 2: return launch_bwd<T, 2, 2>(A, p, ws, st);
@@ -683,13 +719,16 @@ using namespace kans;
 namespace {
 
 // The plan of one backward and the stream's workspace for its partial sums; without one the plan without splits.
-void acquire_ws(int B, int D_in, int D_out, int K, int has_base, bool may_split, hipStream_t st, BwdPlan* plan,
+int acquire_ws(int B, int D_in, int D_out, int K, int has_base, bool may_split, hipStream_t st, BwdPlan* plan,
                 float** ws) {
   *ws = nullptr;
   *plan = plan_backward(B, D_in, D_out, K, has_base, may_split);
-  if (plan->ws_floats == 0) return;
+  if (!plan->fits)
+    return kans_fail(KANS_ERR_UNSUPPORTED, "B=%d or D_out=%d at K=%d: more tiles than a grid holds", B, D_out, K);
+  if (plan->ws_floats == 0) return 0;
   *ws = kans_stream_workspace(st, plan->ws_floats * sizeof(float));
   if (!*ws) *plan = plan_backward(B, D_in, D_out, K, has_base, false);
+  return 0;
 }
 
 int check_bwd(const void* dY, const void* X, const void* W, const void* Wb, const void* dW, const void* dWb,
@@ -699,9 +738,6 @@ int check_bwd(const void* dY, const void* X, const void* W, const void* Wb, cons
     return kans_fail(KANS_ERR_ARG, "bad dims B=%d D_in=%d D_out=%d K=%d (1 <= K <= %d)", B, D_in, D_out, K, kMaxK);
   if ((has_base != 0 && has_base != 1) || (has_bias != 0 && has_bias != 1))
     return kans_fail(KANS_ERR_ARG, "has_base / has_bias must be 0 or 1");
-  // the dX kernel's lane offsets are 32 bits: 36 bytes a reduction index of W, 124 bytes an output of dY
-  if ((long)D_in * K > (1L << 26) || D_out > (1 << 25))
-    return kans_fail(KANS_ERR_UNSUPPORTED, "D_in * K = %ld above 2^26 or D_out = %d above 2^25", (long)D_in * K, D_out);
   if (has_base && (!Wb || !dWb)) return kans_fail(KANS_ERR_ARG, "has_base=1 but W_base or dW_base is null");
   return 0;
 }
@@ -729,7 +765,7 @@ int backward_host(const float* dY, const float* X, const float* W, const float* 
   if (has_base) HIP_TRY(hipMemcpyAsync(d_Wb, Wb, nWb * 4, hipMemcpyHostToDevice, st));
   BwdPlan plan;
   float* ws;
-  acquire_ws(B, D_in, D_out, K, has_base, true, st, &plan, &ws);
+  if ((rc = acquire_ws(B, D_in, D_out, K, has_base, true, st, &plan, &ws))) return rc;
   HIP_TRY(launch_cheby_backward<float>(d_dY, d_X, d_W, has_base ? d_Wb : nullptr, d_dW, has_base ? d_dWb : nullptr,
                                 has_bias ? d_db : nullptr, d_dX, B, D_in, D_out, K, has_base, plan, ws, st));
   HIP_TRY(hipMemcpyAsync(dW, d_dW, nW * 4, hipMemcpyDeviceToHost, st));
@@ -751,9 +787,10 @@ int kans_cheby_backward_ex(int dtype, const void* dY, const void* X, const void*
   if (rc) return rc;
   if (dtype != DT_F32 && dtype != DT_F16 && dtype != DT_BF16) return kans_fail(KANS_ERR_ARG, "unknown dtype %d", dtype);
   // partial gradients of several slot groups are added up in the output, which has to hold fp32
-  if (dtype != DT_F32 && (K - 1 + has_base < 1 || K - 1 + has_base > kBwdMaxSG))
-    return kans_fail(KANS_ERR_UNSUPPORTED, "16-bit backward takes 1 to %d slots (K - 1 + has_base = %d)", kBwdMaxSG,
-                     K - 1 + has_base);
+  if (dtype != DT_F32 && (K - 1 + has_base < 1 || K - 1 + has_base > kBwdMaxSG || wide_rows(D_in, D_out, K)))
+    return kans_fail(KANS_ERR_UNSUPPORTED,
+                     "16-bit backward takes 1 to %d slots, D_in * K <= 2^26 and D_out <= 2^25 (K - 1 + has_base = %d, "
+                     "D_in = %d, D_out = %d)", kBwdMaxSG, K - 1 + has_base, D_in, D_out);
   std::lock_guard<std::mutex> lk(kans_mutex());
   if ((rc = kans_ensure_init())) return rc;
   hipStream_t st = kans_caller_stream(stream);
@@ -762,7 +799,7 @@ int kans_cheby_backward_ex(int dtype, const void* dY, const void* X, const void*
   HIP_TRY(kans_capturing(st, &capturing));
   BwdPlan plan;
   float* ws;
-  acquire_ws(B, D_in, D_out, K, has_base, !capturing, st, &plan, &ws);
+  if ((rc = acquire_ws(B, D_in, D_out, K, has_base, !capturing, st, &plan, &ws))) return rc;
   auto* go = dtype == DT_F16 ? launch_cheby_backward<_Float16>
              : dtype == DT_BF16 ? launch_cheby_backward<__bf16>
                                 : launch_cheby_backward<float>;

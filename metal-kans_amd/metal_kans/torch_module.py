@@ -196,11 +196,13 @@ class TorchMetalKANLinear(nn.Module):
 
     def _backward_device(self, grad_out, x, weight, base_weight, bias):
         B = grad_out.numel() // self.out_features
-        # 16-bit arrays as they are where the kernels take them (all of one dtype, 1 to 10 slots), else in fp32
+        # 16-bit arrays as they are where kans_cheby_backward_ex takes them (all of one dtype, 1 to 10 slots, rows
+        # within its offsets), else in fp32
         dt = weight.dtype
         slots = self._K - 1 + int(base_weight is not None)
         given = [t for t in (x, grad_out, base_weight, bias) if t is not None]
-        if dt not in _DT or any(t.dtype != dt for t in given) or not 1 <= slots <= 10:
+        if (dt not in _DT or any(t.dtype != dt for t in given) or not 1 <= slots <= 10
+                or self.in_features * self._K > 1 << 26 or self.out_features > 1 << 25):
             dt = torch.float32
         as_dt = lambda t: None if t is None else t.detach().to(dt).contiguous()  # noqa: E731
         dy = as_dt(grad_out).reshape(B, self.out_features)

@@ -353,3 +353,41 @@ def test_backward_largest_values_and_products_of_infinities(gpu):
     keep = np.delete(np.arange(D_out), 11)
     assert np.isfinite(dWb[np.ix_(keep, np.delete(np.arange(D_in), 2))]).all()
     np.testing.assert_array_equal(dWb[keep, 2], np.sign(dY[7, keep]) * np.inf)
+
+
+@pytest.mark.parametrize("D_in,D_out,K,base", [(1, (1 << 25) + 5, 2, False),      # rows of dY
+                                               ((1 << 24) + 3, 2, 5, True),       # rows of W
+                                               ((1 << 24) + 3, 1, 20, True)])     # and more workgroups than a launch takes
+def test_backward_rows_beyond_32_bit_offsets(gpu, D_in, D_out, K, base):
+    """Shapes whose rows the dX kernel's 32-bit lane offsets do not reach over."""
+    B = 2
+    rng = np.random.default_rng(D_out)
+    X = rng.uniform(-1.2, 1.2, (B, D_in)).astype(np.float32)
+    W = (rng.random((D_out, D_in * K), dtype=np.float32) - 0.5) / np.float32(K)
+    Wb = rng.random((D_out, D_in), dtype=np.float32) - 0.5 if base else None
+    dY = (rng.random((B, D_out), dtype=np.float32) - 0.5)
+    dW, dWb, db, dX = run_host(gpu, gpu.metal_kan_cheby_backward_fused, dY, X, W, Wb, True)
+    x, g = X.astype(np.float64), dY.astype(np.float64)
+    t, inside = np.clip(x, -1, 1), np.abs(X) <= 1
+    # the largest sum here has 2^25 terms of both signs: 32768 partial steps, a random walk of half units (2^-24)
+    tol = 1e-5 if D_out < 1 << 20 else 4 * np.sqrt(6 * D_out / 64 / 16) * 2.0 ** -24
+
+    def close(got, want, name):
+        assert np.abs(got - want).max() <= tol * max(np.abs(want).max(), 1e-3), name
+    close(db, g.sum(0), "dbias")
+    T, D = [np.ones_like(t), t], [np.zeros_like(x), np.ones_like(x)]
+    dx = np.zeros_like(x)
+    W3, dW3 = W.reshape(D_out, D_in, K), dW.reshape(D_out, D_in, K)
+    for k in range(K):
+        if k >= 2:
+            T = [T[1], 2 * t * T[1] - T[0]]
+            D = [D[1], 2 * T[0] + 2 * t * D[1] - D[0]]
+        Tk, Dk = (T[k], D[k]) if k < 2 else (T[1], D[1])
+        close(dW3[:, :, k], g.T @ Tk, f"dW {k}")
+        if k:
+            dx += (g @ W3[:, :, k].astype(np.float64)) * Dk * inside
+    if base:
+        sg = 1 / (1 + np.exp(-x))
+        close(dWb, g.T @ (x * sg), "dW_base")
+        dx += (g @ Wb.astype(np.float64)) * sg * (1 + x * (1 - sg))
+    close(dX, dx, "dX")
