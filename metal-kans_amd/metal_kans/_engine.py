@@ -176,18 +176,20 @@ class LayerEngine:
             self.params = params
 
     def prepare_device(self, dt: int, W_ptr: int, W_base_ptr: Optional[int], bias_ptr: Optional[int],
-                       params: tuple, key: tuple, stream=None) -> None:
+                       params: tuple, key: tuple, stream=None) -> bool:
         """Make the device copy current from device arrays in dtype ``dt`` (e.g. torch tensors); ``key``
         identifies their contents (pointers and version counters): equal keys skip the re-tiling, which is
-        enqueued on ``stream`` behind whatever wrote the arrays there."""
+        enqueued on ``stream`` behind whatever wrote the arrays there.  True when it was: the arrays are read
+        until the stream has passed it."""
         lib = self._ensure_handle(dt)
         self._set_params(lib, params)
         if self.snaps is None and self.dev_key == key:
-            return
+            return False
         device.check(lib.kans_layer_load_weights_stream(self.handle, W_ptr, W_base_ptr, bias_ptr, stream),
                      "kans_layer_load_weights_stream")
         self.snaps = None
         self.dev_key = key
+        return True
 
     def prepare(self, dt: int, W: np.ndarray, W_base: Optional[np.ndarray], bias: Optional[np.ndarray],
                 params: tuple, src_f32: bool = False, verify: bool = True) -> None:

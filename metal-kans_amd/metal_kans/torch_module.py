@@ -61,9 +61,8 @@ _LEGACY_STREAM = 1
 _kept = {0}
 
 
-def _stream_of(dev: torch.device) -> ctypes.c_void_p:
-    """Handle of torch's current stream on ``dev``."""
-    s = torch.cuda.current_stream(dev)
+def _stream_of(s: torch.cuda.Stream) -> ctypes.c_void_p:
+    """The library's handle of a torch stream."""
     h = s.cuda_stream
     if h not in _kept and s.stream_id != h:  # (an external stream has its handle for id)
         device.check(device.get_metal_bridge().kans_stream_keep(h), "kans_stream_keep")
@@ -177,10 +176,14 @@ class TorchMetalKANLinear(nn.Module):
                    bias.contiguous() if bias is not None else None]
         key = tuple((p.data_ptr(), p._version) if p is not None else None for p in params)
         eng = self.metal_layer._engine()
-        stream = _stream_of(x.device)
-        eng.prepare_device(dt, params[0].data_ptr(), params[1].data_ptr() if params[1] is not None else None,
-                           params[2].data_ptr() if params[2] is not None else None,
-                           self.metal_layer._basis_params(), key, stream)
+        current = torch.cuda.current_stream(x.device)
+        stream = _stream_of(current)
+        if eng.prepare_device(dt, params[0].data_ptr(), params[1].data_ptr() if params[1] is not None else None,
+                              params[2].data_ptr() if params[2] is not None else None,
+                              self.metal_layer._basis_params(), key, stream):
+            for p in params:   # the re-tiling is queued: memory that the caller gives back is not to be reused before it
+                if p is not None:
+                    p.record_stream(current)
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
         if x2.shape[0] == 0:
@@ -214,7 +217,7 @@ class TorchMetalKANLinear(nn.Module):
         db = torch.empty((self.out_features,), dtype=dt, device=dev) if bias is not None else None
         dX = torch.empty((B, self.in_features), dtype=dt, device=dev)
         ptr = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
-        stream = _stream_of(dev)
+        stream = _stream_of(torch.cuda.current_stream(dev))
         device.check(device.get_metal_bridge().kans_cheby_backward_ex(
             _DT[dt], ptr(dy), ptr(xs), ptr(W), ptr(Wb), ptr(dW), ptr(dWb), ptr(db), ptr(dX), B, self.in_features,
             self.out_features, self._K, int(Wb is not None), int(db is not None), stream), "kans_cheby_backward_ex")

@@ -345,3 +345,27 @@ def test_per_thread_stream(gpu, cuda):
     for a, b in zip(outs, grads):
         assert (a - b).abs().max() <= 1e-5 * b.abs().max()
     assert gpu.kans_stream_keep(per_thread) < 0
+
+
+def test_parameters_given_back_while_their_retiling_is_queued(cuda):
+    """Parameters replaced right after a forward on a held stream: their memory is not reused before the re-tiling
+    has read it."""
+    m = module(512, 640, degree=4, use_base=False, bias=False)
+    x = torch.rand(128, 512, device=cuda) * 2 - 1
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        want = alone(m, x)
+        for fill in (float("nan"), 0.0):
+            m.weight = torch.nn.Parameter(m.weight.detach().clone())   # another version of the same values
+            torch.cuda.synchronize()
+            with torch.cuda.stream(side):
+                torch.cuda._sleep(HOLD)
+                y = m(x)
+            kept = m.weight.detach().cpu()
+            shape = m.weight.shape
+            m.weight = None
+            reuse = [torch.full(shape, fill, device=cuda) for _ in range(3)]
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
+            del reuse
+            m.weight = torch.nn.Parameter(kept.to(cuda))
