@@ -12,7 +12,7 @@ Unlike the reference, which copies every tensor to a NumPy array and back
 * the forward hands ``data_ptr()`` of x, of the parameters and of a new output
   tensor to the library and runs the fused kernel on torch's current stream;
   the parameters are re-tiled on the device only when one of them changed (its
-  pointer or version counter);
+  pointer, strides or version counter; an edit through ``.data`` moves neither);
 * the backward (Chebyshev basis) runs the fused backward kernels on device
   arrays and returns gradients for x **and** for the parameters (``weight``,
   ``base_weight``, ``bias_param``); the reference returns dx only.
@@ -174,7 +174,10 @@ class TorchMetalKANLinear(nn.Module):
         params = [weight.contiguous()]
         params += [base_weight.contiguous() if base_weight is not None else None,
                    bias.contiguous() if bias is not None else None]
-        key = tuple((p.data_ptr(), p._version) if p is not None else None for p in params)
+        # (of the parameters themselves: the contiguous copy of a strided one has a new version count each time, at an
+        # address that comes back)
+        key = tuple(None if p is None else (p.data_ptr(), p._version) if p.is_contiguous()
+                    else (p.data_ptr(), p._version, p.stride()) for p in (weight, base_weight, bias))
         eng = self.metal_layer._engine()
         current = torch.cuda.current_stream(x.device)
         stream = _stream_of(current)

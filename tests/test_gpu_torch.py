@@ -219,3 +219,28 @@ def test_weights_loaded_under_capture_are_refused(cuda):
             want = m(x)
             side.synchronize()
             assert torch.equal(y, want), n
+
+
+def test_strided_parameters_are_retiled_after_a_change(cuda):
+    """A parameter that is not contiguous goes through a copy; a change in place, and another stride of the same
+    memory, still re-tile it."""
+    import metal_kans as mk
+    np.random.seed(4)
+    m = mk.TorchMetalKANLinear(16, 64, degree=4, bias=False, use_base=False).to(cuda)
+    W = m.weight.detach()
+    assert W.shape == (64, 64)
+    x = torch.rand(33, 16, device=cuda) * 2 - 1
+    with torch.no_grad():
+        y, yt = m(x).clone(), None
+        m.weight = torch.nn.Parameter(W.t().contiguous().t())
+        assert torch.equal(m(x), y)
+        for n in range(1, 4):
+            m.weight.mul_(2.0)
+            assert torch.equal(m(x), y * 2.0 ** n)      # powers of two scale exactly
+        m.weight.mul_(0.125)
+        yt = m(x).clone()
+        assert torch.equal(yt, y)
+        m.weight = torch.nn.Parameter(m.weight.detach().t())   # same memory and version, transposed
+        flipped = m(x)
+    ref = O.kan_forward("cheby", x.double().cpu().numpy(), m.weight.detach().double().cpu().numpy(), None, None, {"K": 4})
+    assert O.rel_err(flipped.cpu().numpy(), ref) <= 1e-4
