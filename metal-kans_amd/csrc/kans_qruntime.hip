@@ -32,7 +32,7 @@ struct kans_qlayer {
   int nrb_pad;               // 16-row blocks, padded to a multiple of nw
   bool decode = false;       // decode records built (INT4 / ternary)
   DevBuf R, bias;            // re-tiled records (codes + group parameters), bias (bias_dtype)
-  DevBuf cbias;              // fp32 bias + sum_i W[o, i*K]: the Chebyshev constant term (qp_fold)
+  DevBuf cbias;              // fp32 bias + sum_i W[o, i*K]: the Chebyshev prefill's constant term (qp_fold)
   int bias_dtype = DT_F32;
   // decode workspace: activation basis, its group sums, split-K partials
   DevBuf Phi, S, part;
@@ -723,7 +723,7 @@ int create_affine(int bits, int D_in, int D_out, int K, int has_base, int has_bi
     if (L->prefill &&
         (r = build_ptiles(L, seg, tq.p, rowbytes, (const float*)ts.p, (const float*)tb.p, (int)gpr, st)))
       return r;
-    if (seg == 0) {
+    if (seg == 0 && L->prefill && prefill_fold(L, BASIS_CHEBY)) {
       if ((r = L->cbias.reserve((size_t)D_out * sizeof(float)))) return r;
       HIP_TRY(q_fold_affine(bits, (const unsigned char*)tq.p, rowbytes, (const float*)ts.p, (const float*)tb.p,
                             (int)gpr, D_out, D_in, K, has_bias ? L->bias.p : nullptr, bias_dtype,
@@ -907,7 +907,7 @@ int kans_qlayer_create_ternary(int D_in, int D_out, int K, int has_base, int has
                               seg ? L->Cw : L->Cb, seg ? L->Cb : 0, L->C_tot, L->R.p, st);
     if (e != hipSuccess) return kans_fail(KANS_ERR_HIP, "ternary re-tiling failed: %s", hipGetErrorString(e));
     if (L->prefill && (r = build_ptiles(L, seg, tw.p, wpr, (const float*)ts.p, nullptr, gpr, st))) return r;
-    if (seg == 0) {
+    if (seg == 0 && L->prefill && prefill_fold(L, BASIS_CHEBY)) {
       if ((r = L->cbias.reserve((size_t)D_out * sizeof(float)))) return r;
       HIP_TRY(q_fold_tern((const unsigned*)tw.p, wpr, (const float*)ts.p, gpr, D_out, D_in, K,
                           has_bias ? L->bias.p : nullptr, bias_dtype, (float*)L->cbias.p, st));
