@@ -171,22 +171,20 @@ class TorchMetalKANLinear(nn.Module):
             if p is not None and (p.dtype != pdt or not p.is_cuda):
                 raise TypeError("all parameters must share one dtype and live on the GPU")
         dt = _DT[pdt]
-        params = [weight.contiguous()]
-        params += [base_weight.contiguous() if base_weight is not None else None,
-                   bias.contiguous() if bias is not None else None]
+        given = (weight, base_weight, bias)
+        params = tuple(None if p is None else p.contiguous() for p in given)
+        ptrs = tuple(None if c is None else c.data_ptr() for c in params)
         # (of the parameters themselves: the contiguous copy of a strided one has a new version count each time, at an
         # address that comes back)
-        key = tuple(None if p is None else (p.data_ptr(), p._version) if p.is_contiguous()
-                    else (p.data_ptr(), p._version, p.stride()) for p in (weight, base_weight, bias))
+        key = tuple(None if p is None else (q, p._version) if c is p else (p.data_ptr(), p._version, p.stride())
+                    for p, c, q in zip(given, params, ptrs))
         eng = self.metal_layer._engine()
         current = torch.cuda.current_stream(x.device)
         stream = _stream_of(current)
-        if eng.prepare_device(dt, params[0].data_ptr(), params[1].data_ptr() if params[1] is not None else None,
-                              params[2].data_ptr() if params[2] is not None else None,
-                              self.metal_layer._basis_params(), key, stream):
-            for p in params:   # the re-tiling is queued: memory that the caller gives back is not to be reused before it
-                if p is not None:
-                    p.record_stream(current)
+        if eng.prepare_device(dt, *ptrs, self.metal_layer._basis_params(), key, stream):
+            for c in params:   # the re-tiling is queued: memory that the caller gives back is not to be reused before it
+                if c is not None:
+                    c.record_stream(current)
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
         if x2.shape[0] == 0:
