@@ -547,62 +547,67 @@ int kans_layer_load_weights_stream(kans_layer* L, const void* W, const void* W_b
 
 // Tile, feature splits and wave groups of one forward: those with the least
 // estimated time.  A configuration's estimate is, with n workgroups on the
-// fullest of the 256 CUs, F feature blocks per workgroup (per wave group) and
-// S slots per block,
+// fullest of the 256 CUs, F feature blocks per workgroup (per wave group), S
+// slots per block and y MB of output,
 //   n = 1:  F S alone + F block + wg                   one workgroup on a CU
 //   n > 1:  n (F S shared + F block + wg)              (rate with neighbours)
-//   + launch + (splits > 1: split_us + split_mb * MB of partial sums)
+//   + launch + y out_mb
+//   + (splits > 1: split_us + split_mb * MB of partial sums + split_8 * splits / 8)
 // in us.  The coefficients are non-negative least-squares fits (relative error
-// 5 to 14 %) to 11 500 timings: three bases, K = 4 to 9, fp16 and fp32, rows
-// 256 to 8192, widths 10 to 2048, 1 to 16 splits.  Choosing by them came within
-// 2 % of the fastest configuration on average (18 % at most); the earlier rule
-// (a preference order, first shape whose tiles fill the chip) took 1.47 times
-// the fastest on average and up to 5.5 times: it preferred 32-column tiles
-// without a split, which generate every basis value anew for each 32 columns,
-// to larger tiles with one.  4096 x 1024 -> 1024, K = 8 + base, fp16, us: RBF
-// 273 -> 94, B-spline 413 -> 95; fp32 738 -> 374 and 655 -> 262.
+// 5 to 17 %) to 37 000 timings (kans_layer_time_forward of the configurations that
+// kans_layer_set_tiling forces) of 1440 layers drawn over three bases, K = 3 to
+// 10, fp16 and fp32, rows 64 to 16384, D_in 16 to 2048, D_out 10 to 4096.  On
+// layers that the fit has not seen, the choice is 1.024 times the fastest
+// configuration on average, more than 1.1 times for 39 of 480, 1.38 times at most.
+// Without the output and split_8 terms, fitted to rows from 256 and long
+// contractions only, it was 1.07, 88 of 480 and 2.1 times: it took 256 x 256 tiles
+// for one or two feature blocks (114 x 16 -> 798 B-spline fp16: 12.5 us, now 5.9).
+// A rule before that (a preference order, first shape whose tiles fill the chip)
+// took 32-column tiles without a split, which generate every basis value anew for
+// each 32 columns: 4096 x 1024 -> 1024, K = 8 + base, fp16, us: RBF 273, now 94;
+// B-spline 413, 95; fp32 738, 374 and 655, 262.
 struct TileCost {
   int wm, nb, ks;
-  float alone, shared, wg, block, split_us, split_mb, launch;
+  float alone, shared, wg, block, split_us, split_mb, launch, out_mb, split_8;
 };
 
 // 16-bit Chebyshev (block kernels)
 static const TileCost kCostCheby16[] = {
-    {32, 8, 1, 0.286f, 0.285f, 0.0f, 0.581f, 2.88f, 0.194f, 3.42f},
-    {64, 4, 1, 0.179f, 0.105f, 0.0f, 0.66f, 2.0f, 0.187f, 4.76f},
-    {32, 4, 1, 0.117f, 0.0723f, 0.0f, 0.353f, 2.17f, 0.172f, 3.85f},
-    {32, 4, 2, 0.181f, 0.178f, 0.0f, 0.642f, 1.74f, 0.249f, 4.52f},
-    {32, 1, 1, 0.0823f, 0.0321f, 0.0f, 0.257f, 2.35f, 0.106f, 3.98f},
-    {32, 1, 2, 0.102f, 0.0609f, 0.0f, 0.5f, 2.59f, 0.118f, 3.79f},
-    {32, 1, 4, 0.13f, 0.123f, 0.747f, 1.11f, 2.22f, 0.151f, 3.48f}};
+    {32, 8, 1, 0.285f, 0.303f, 0.0f, 0.452f, 1.72f, 0.168f, 4.4f, 0.727f, 0.484f},
+    {64, 4, 1, 0.178f, 0.113f, 0.0f, 0.585f, 1.52f, 0.165f, 5.2f, 0.666f, 0.465f},
+    {32, 4, 1, 0.11f, 0.0683f, 0.0f, 0.351f, 1.73f, 0.155f, 3.82f, 0.561f, 0.523f},
+    {32, 4, 2, 0.175f, 0.194f, 0.0f, 0.562f, 1.25f, 0.216f, 4.4f, 0.679f, 0.692f},
+    {32, 1, 1, 0.0848f, 0.0329f, 0.0f, 0.253f, 1.84f, 0.108f, 3.37f, 0.304f, 0.577f},
+    {32, 1, 2, 0.102f, 0.0671f, 0.0f, 0.45f, 1.75f, 0.109f, 3.69f, 0.443f, 0.502f},
+    {32, 1, 4, 0.138f, 0.149f, 0.212f, 0.942f, 1.33f, 0.196f, 3.65f, 0.841f, 0.682f}};
 // 16-bit RBF, and the per-slot kernel of any basis whose slots exceed the block
 // kernels' (its (32, 8) tile has 128 rows: about the (64, 4) one's work)
 static const TileCost kCostRbf16[] = {
-    {32, 8, 1, 0.352f, 0.36f, 0.0f, 0.0f, 3.25f, 0.197f, 2.8f},
-    {64, 4, 1, 0.462f, 0.268f, 0.0f, 0.0f, 1.97f, 0.195f, 4.89f},
-    {32, 4, 1, 0.35f, 0.164f, 0.0f, 0.0f, 2.94f, 0.163f, 3.39f},
-    {32, 1, 1, 0.244f, 0.0964f, 0.0f, 0.0f, 1.8f, 0.0901f, 5.2f}};
+    {32, 8, 1, 0.341f, 0.327f, 0.0f, 0.225f, 1.7f, 0.179f, 3.93f, 0.62f, 0.753f},
+    {64, 4, 1, 0.42f, 0.217f, 0.0f, 0.346f, 1.42f, 0.178f, 5.17f, 0.439f, 0.604f},
+    {32, 4, 1, 0.326f, 0.139f, 0.0f, 0.145f, 2.06f, 0.153f, 3.66f, 0.448f, 0.558f},
+    {32, 1, 1, 0.231f, 0.0807f, 0.0f, 0.192f, 2.13f, 0.0856f, 3.23f, 0.366f, 0.759f}};
 static const TileCost kCostBspline16[] = {
-    {32, 8, 1, 0.369f, 0.369f, 0.0f, 0.0f, 3.22f, 0.193f, 3.49f},
-    {64, 4, 1, 0.741f, 0.465f, 0.0f, 0.0f, 2.71f, 0.17f, 4.65f},
-    {32, 4, 1, 0.423f, 0.205f, 0.0f, 0.0f, 2.74f, 0.154f, 3.96f},
-    {32, 1, 1, 0.335f, 0.156f, 0.0f, 0.0f, 1.59f, 0.0826f, 5.57f}};
+    {32, 8, 1, 0.468f, 0.42f, 0.779f, 0.0f, 1.97f, 0.18f, 4.36f, 0.747f, 0.516f},
+    {64, 4, 1, 0.62f, 0.328f, 0.0f, 1.06f, 1.82f, 0.163f, 5.42f, 0.408f, 0.428f},
+    {32, 4, 1, 0.366f, 0.145f, 0.0f, 0.525f, 2.31f, 0.146f, 3.71f, 0.37f, 0.458f},
+    {32, 1, 1, 0.319f, 0.132f, 0.0f, 0.313f, 2.47f, 0.066f, 3.14f, 0.401f, 0.617f}};
 // fp32 (kan_fused_split, B-spline K >= 5 kan_fused_split_sparse)
 static const TileCost kCostCheby32[] = {
-    {32, 8, 1, 1.91f, 1.93f, 1.42f, 0.53f, 5.05f, 0.284f, 2.59f},
-    {64, 4, 1, 1.0f, 1.04f, 0.0f, 0.292f, 2.7f, 0.242f, 4.34f},
-    {32, 4, 1, 0.775f, 0.555f, 0.0f, 0.265f, 2.75f, 0.191f, 4.38f},
-    {32, 1, 1, 0.363f, 0.238f, 0.0f, 0.196f, 2.39f, 0.171f, 4.27f}};
+    {32, 8, 1, 1.84f, 1.83f, 0.0f, 0.582f, 0.0f, 0.307f, 9.71f, 0.403f, 0.626f},
+    {64, 4, 1, 1.01f, 1.04f, 0.0f, 0.35f, 1.05f, 0.249f, 4.85f, 0.32f, 0.687f},
+    {32, 4, 1, 0.805f, 0.519f, 0.0f, 0.303f, 1.13f, 0.223f, 4.77f, 0.333f, 0.674f},
+    {32, 1, 1, 0.35f, 0.206f, 0.0f, 0.295f, 1.51f, 0.167f, 3.48f, 0.345f, 0.797f}};
 static const TileCost kCostRbf32[] = {
-    {32, 8, 1, 1.96f, 2.0f, 2.42f, 0.0f, 6.81f, 0.294f, 0.0f},
-    {64, 4, 1, 1.09f, 1.11f, 0.0f, 0.0f, 3.66f, 0.248f, 3.26f},
-    {32, 4, 1, 0.873f, 0.618f, 0.0f, 0.0f, 3.5f, 0.189f, 3.58f},
-    {32, 1, 1, 0.443f, 0.285f, 0.0f, 0.0f, 2.35f, 0.162f, 4.46f}};
+    {32, 8, 1, 1.97f, 1.89f, 1.38f, 0.0f, 1.78f, 0.3f, 6.17f, 0.519f, 0.546f},
+    {64, 4, 1, 1.07f, 1.08f, 0.813f, 0.076f, 1.75f, 0.237f, 3.15f, 0.431f, 0.751f},
+    {32, 4, 1, 0.88f, 0.574f, 0.0f, 0.0903f, 1.73f, 0.212f, 4.07f, 0.391f, 0.726f},
+    {32, 1, 1, 0.404f, 0.258f, 0.0f, 0.109f, 1.51f, 0.156f, 3.68f, 0.342f, 0.924f}};
 static const TileCost kCostSparse32[] = {
-    {32, 8, 1, 1.32f, 1.34f, 2.99f, 0.0f, 4.02f, 0.247f, 0.0f},
-    {64, 4, 1, 0.838f, 0.827f, 0.0f, 0.0f, 3.27f, 0.233f, 3.33f},
-    {32, 4, 1, 0.709f, 0.482f, 0.0f, 0.0f, 3.01f, 0.182f, 3.82f},
-    {32, 1, 1, 0.357f, 0.252f, 0.0f, 0.0f, 2.51f, 0.147f, 4.01f}};
+    {32, 8, 1, 1.24f, 1.27f, 0.363f, 0.096f, 1.74f, 0.261f, 4.32f, 0.523f, 0.764f},
+    {64, 4, 1, 0.733f, 0.742f, 0.0f, 0.475f, 1.58f, 0.239f, 3.92f, 0.471f, 0.879f},
+    {32, 4, 1, 0.678f, 0.442f, 0.0f, 0.11f, 1.7f, 0.189f, 3.83f, 0.365f, 0.851f},
+    {32, 1, 1, 0.339f, 0.226f, 0.0f, 0.0946f, 1.65f, 0.134f, 2.95f, 0.442f, 1.04f}};
 
 // Rows of a workgroup's tile.
 static int tile_rows(const kans_layer* L, int wm, int nb) {
@@ -615,8 +620,9 @@ static bool tile_groups_ok(const kans_layer* L, int wm, int nb, int ks) {
                      block_wave_groups_ok(wm, nb, ks));
 }
 
-// Partial sums of a split forward are kept below this.
+// Partial sums of a split forward are kept below this, and the splits.
 constexpr double kMaxPartMB = 256.0;
+constexpr int kMaxSplits = 128;
 
 // unsplit: one split whatever is forced.
 static TileCfg choose_tiling(const kans_layer* L, int B, bool unsplit = false) {
@@ -633,6 +639,7 @@ static TileCfg choose_tiling(const kans_layer* L, int B, bool unsplit = false) {
   }
   const bool per_slot8 = L->dtype != DT_F32 && block_waves(true, L->basis, 32, 8, L->slots) == 0;
   const int nob = (L->D_out + 31) / 32;
+  const double out = 1e-6 * B * L->D_out * dtype_size(L->dtype);
   TileCfg best{32, 1, 1, 1};
   double best_t = 0.0;
   bool any = false;
@@ -642,22 +649,23 @@ static TileCfg choose_tiling(const kans_layer* L, int B, bool unsplit = false) {
     if (L->forced_wm && (wm != L->forced_wm || nb != L->forced_nb || ks != 1)) continue;
     const int tr = tile_rows(L, wm, nb);
     const long tiles = (long)((B + tr - 1) / tr) * ((nob + nb - 1) / nb);
-    int last = 0;  // splits that come to the same feature blocks each are looked at once
-    for (int s = 1; s <= std::min(L->nfb, 32); ++s) {
-      const int fbps = forced_splits ? (L->nfb + forced_splits - 1) / forced_splits : (L->nfb + s - 1) / s;
-      if (fbps == last || (ks > 1 && fbps < 2 * ks)) continue;
-      last = fbps;
+    // every number of feature blocks a split that divides them differently
+    int fbps = L->nfb;
+    for (int s = 1; s <= kMaxSplits; s = fbps > 1 ? (L->nfb + fbps - 2) / (fbps - 1) : kMaxSplits + 1) {
+      fbps = forced_splits ? (L->nfb + forced_splits - 1) / forced_splits : (L->nfb + s - 1) / s;
+      if (ks > 1 && fbps < 2 * ks) break;
       const int splits = (L->nfb + fbps - 1) / fbps;
       const double mb = splits > 1 ? 8e-6 * splits * B * L->D_out : 0.0;
       if (splits > 1 && mb > 2.0 * kMaxPartMB && !forced_splits) break;
       const double n = (double)((tiles * splits + 255) / 256), F = (fbps + ks - 1) / ks;
-      double t = n * (F * L->slots * (n > 1 ? c.shared : c.alone) + F * c.block + c.wg) + c.launch;
-      if (splits > 1) t += c.split_us + mb * c.split_mb;
+      double t = n * (F * L->slots * (n > 1 ? c.shared : c.alone) + F * c.block + c.wg) + c.launch + out * c.out_mb;
+      if (splits > 1) t += c.split_us + mb * c.split_mb + (splits + 7) / 8 * c.split_8;
       if (!any || t < best_t) {
         any = true;
         best_t = t;
         best = TileCfg{wm, nb, forced_splits ? forced_splits : splits, ks};
       }
+      if (forced_splits) break;
     }
   }
   if (L->forced_wm) {

@@ -5,6 +5,8 @@ device-tensor path (no NumPy round trip) against the float64 oracle: forward at 
 fp32 / fp16 bars (1e-4 / 2e-2), gradients of x and of every parameter at 1e-4,
 re-tiling after an in-place optimizer step, padded input rows.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -205,7 +207,7 @@ def test_weights_loaded_under_capture_are_refused(cuda):
         for p in m.parameters():
             p.mul_(2.0)
         side.synchronize()
-        with pytest.raises(Exception):
+        with pytest.raises(mk.device.KansError, match="under graph capture"):
             with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=side):
                 m(x)
         refs.append(m(x).clone())
@@ -244,3 +246,32 @@ def test_strided_parameters_are_retiled_after_a_change(cuda):
         flipped = m(x)
     ref = O.kan_forward("cheby", x.double().cpu().numpy(), m.weight.detach().double().cpu().numpy(), None, None, {"K": 4})
     assert O.rel_err(flipped.cpu().numpy(), ref) <= 1e-4
+
+
+@pytest.mark.parametrize("basis,B,d_in,d_out,degree", [("bspline", 114, 16, 798, 4), ("bspline", 97, 32, 555, 4),
+                                                       ("rbf", 3814, 24, 3286, 8), ("bspline", 627, 24, 2183, 2)])
+def test_tile_choice_on_short_contractions(gpu, cuda, basis, B, d_in, d_out, degree):
+    """One or two feature blocks: the chosen configuration is near the fastest of the unsplit tiles (a 256 x 256
+    tile, which writes as much as it computes there, took 1.5 to 2.1 times as long)."""
+    import metal_kans as mk
+    m = mk.TorchMetalKANLinear(d_in, d_out, basis=basis, degree=degree).to(cuda).half()
+    x = (torch.rand(B, d_in, device=cuda) * 2 - 1).half()
+    y = torch.empty(B, d_out, device=cuda, dtype=torch.float16)
+    with torch.no_grad():
+        m(x)
+    torch.cuda.synchronize()
+    eng, ms = m.metal_layer._engine(), ctypes.c_float()
+
+    def best():
+        times = []
+        for _ in range(7):
+            assert gpu.kans_layer_time_forward(eng.handle, x.data_ptr(), d_in, y.data_ptr(), d_out, B, 5, 40,
+                                               ctypes.byref(ms)) == 0, gpu.kans_last_error()
+            times.append(ms.value)
+        return min(times)
+    chosen = best()
+    forced = []
+    for wm, nb in ((32, 1), (32, 4), (64, 4), (32, 8)):
+        eng.set_tiling(wm, nb, 1)
+        forced.append(best())
+    assert chosen <= 1.35 * min(forced), (chosen, forced)
