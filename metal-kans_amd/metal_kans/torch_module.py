@@ -24,7 +24,6 @@ and the ReLU-KAN family is outside this build.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import Any, Optional, Sequence
 
 import numpy as np
@@ -61,13 +60,13 @@ _LEGACY_STREAM = 1
 _kept = {0}
 
 
-def _stream_of(s: torch.cuda.Stream) -> ctypes.c_void_p:
+def _stream_of(s: torch.cuda.Stream) -> int:
     """The library's handle of a torch stream."""
     h = s.cuda_stream
     if h not in _kept and s.stream_id != h:  # (an external stream has its handle for id)
         device.check(device.get_metal_bridge().kans_stream_keep(h), "kans_stream_keep")
         _kept.add(h)
-    return ctypes.c_void_p(h or _LEGACY_STREAM)
+    return h or _LEGACY_STREAM
 
 
 class _KANFunction(torch.autograd.Function):
@@ -193,8 +192,7 @@ class TorchMetalKANLinear(nn.Module):
         xa, ldx = _aligned_rows(x2, self.in_features, 32)
         y = torch.empty((x2.shape[0], self.out_features), dtype=x.dtype, device=x.device)
         lib = device.get_metal_bridge()
-        device.check(lib.kans_layer_forward_ex(eng.handle, ctypes.c_void_p(xa.data_ptr()), xdt, ldx,
-                                               ctypes.c_void_p(y.data_ptr()), xdt, self.out_features,
+        device.check(lib.kans_layer_forward_ex(eng.handle, xa.data_ptr(), xdt, ldx, y.data_ptr(), xdt, self.out_features,
                                                x2.shape[0], stream), "kans_layer_forward_ex")
         return y.reshape(*shape[:-1], self.out_features)
 
@@ -217,7 +215,7 @@ class TorchMetalKANLinear(nn.Module):
         dWb = torch.empty_like(Wb) if Wb is not None else None
         db = torch.empty((self.out_features,), dtype=dt, device=dev) if bias is not None else None
         dX = torch.empty((B, self.in_features), dtype=dt, device=dev)
-        ptr = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
+        ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
         stream = _stream_of(torch.cuda.current_stream(dev))
         device.check(device.get_metal_bridge().kans_cheby_backward_ex(
             _DT[dt], ptr(dy), ptr(xs), ptr(W), ptr(Wb), ptr(dW), ptr(dWb), ptr(db), ptr(dX), B, self.in_features,
