@@ -208,9 +208,12 @@ int kans_layer_kernel_ex(const kans_layer* layer, int B, int x_dtype, int y_dtyp
 int kans_layer_load_weights(kans_layer* layer, const void* W, const void* W_base, const void* bias);
 int kans_layer_load_weights_device(kans_layer* layer, const void* W, const void* W_base, const void* bias);
 /* as kans_layer_load_weights_device, enqueued on `stream` (NULL = kans_stream()) and not waited for: forwards
- * on this stream run behind it, forwards on other streams wait for it on the device; the arrays stay as they
- * are until the stream has passed the call (a training step re-tiles its weights before every forward).
- * Refused (KANS_ERR_UNSUPPORTED) on a stream under graph capture. */
+ * on this stream run behind it, forwards and the library's graph replays on other streams wait for it on the
+ * device, and it runs behind every forward that still reads the old weights; the arrays stay as they are until
+ * the stream has passed the call (a training step re-tiles its weights before every forward).
+ * Refused (KANS_ERR_UNSUPPORTED) on a stream under graph capture.  A graph that a caller captures reads the
+ * weights of its layers at each replay; ordering its replays with later loads is the caller's part, and a graph
+ * captured on the stream that loaded the weights is to be launched behind that stream's work. */
 int kans_layer_load_weights_stream(kans_layer* layer, const void* W, const void* W_base, const void* bias,
                                    void* stream);
 /* host fp32 weights converted on the device to the layer dtype (round to nearest even) */

@@ -44,10 +44,10 @@
 // VALU instructions.
 //
 // The bound is the matrix pipe at 6 x 2 * B * D_in * D_out * NS operations: at
-// 8192 x 1024 -> 1024, K = 4 with the base branch, dW takes 350 us and dX 341 us
-// (1.18 and 1.21 PFLOP/s of bf16 MFMA, the rate a large bf16 matrix product
-// reaches on the same card), where the fp32 VALU kernels this replaces took 3203
-// and 2753 us.  Without the waves' turns 364 and 346 us.
+// 8192 x 1024 -> 1024, K = 4 with the base branch, dW takes 346 us and dX 335 us
+// (1.19 and 1.23 PFLOP/s of bf16 MFMA; an 8192^3 bf16 product reaches 1.12 on the
+// same card), where the fp32 VALU kernels this replaces took 3203 and 2753 us.
+// Without the waves' turns 364 and 346 us.
 // Grids that leave CUs idle split the contraction (choose_splits) into partial
 // sums that a second kernel adds in order: 64 workgroups of dW at that shape
 // become 256, and the sums cost 27 us.
@@ -56,8 +56,8 @@
 // its fp32 sum: a dX product is one MFMA, a bf16 dW product four (BwdTerms).
 // The steps are too short there for the matrix pipe to be the bound; the loads'
 // latency and, in dW, the 43 MB of partial sums are.  2000 x 300 -> 500, K = 6,
-// bf16: dW 36 us (41 us with the loads converted as they arrive), its sum 13 us,
-// dX 28 us; through fp32 copies of the arrays and back the training step took
+// bf16: dW 33 us (41 us with the loads converted as they arrive), its sum 13 us,
+// dX 27 us; through fp32 copies of the arrays and back the training step took
 // 245 us, now 203 us.
 #include "kans_common.h"
 #include "kans_api_internal.h"

@@ -13,10 +13,13 @@
 // Per wave and step: 6 NB MFMAs (1536 cycles at NB = 8) against 3 NB
 // B-fragment reads and about 110 VALU instructions (basis value, split) for
 // the next step, a quarter to a half of what the 16-bit kernel spends per MFMA.
-// The bound is the MFMA rate on dense mantissas, about 1.2 PFLOP/s of bf16 on this
-// card, i.e. 200 TFLOP/s of fp32 products; the fp32 MFMA (157 TFLOP/s peak)
-// reached 127.  8192 x 1024 -> 1024, Chebyshev K = 4 with the base branch: 582 us
-// on the fp32 MFMA, 333 us here (206 TFLOP/s).
+// The bound is the MFMA rate that dense mantissas leave: an 8192^3 bf16 product
+// reaches 1.12 PFLOP/s on the same card, this kernel 1.24 (six times 206 TFLOP/s
+// of fp32 products; the fp32 MFMA's peak is 157).  8192 x 1024 -> 1024, Chebyshev
+// K = 4 with the base branch, the four slots left without T_0: 333 us, 582 on the
+// fp32 MFMA (118 TFLOP/s).  Layers of about 10 us are up to 2 us slower than on the
+// fp32 MFMA (96 x 456 -> 89, K = 6: 10.9 and 9.5): one wave per SIMD waits for the
+// split of each step and for 1.5 times the weights.
 #include "kans_common.h"
 #include "kans_api_internal.h"
 #include "kans_split.h"
