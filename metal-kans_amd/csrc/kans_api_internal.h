@@ -115,8 +115,8 @@ hipError_t kans_capturing(hipStream_t st, bool* capturing);
 // calls on the stream share, since their kernels run one after the other (library lock held; st not under
 // capture by a caller).  Null where there is none -- no memory for it, or hipStreamPerThread, one handle
 // for several streams: the caller then runs unsplit.  It grows with the calls and stays until the next
-// larger request, until kMaxWorkspaces other streams have asked since, or until the library's last object
-// is destroyed (WorkspaceUser).
+// larger request or until kMaxWorkspaces other streams have asked since; the library's last object frees all
+// but a few MB (WorkspaceUser).
 float* kans_stream_workspace(hipStream_t st, size_t bytes);
 struct WorkspaceUser {
   WorkspaceUser();
