@@ -212,8 +212,8 @@ int kans_layer_load_weights_device(kans_layer* layer, const void* W, const void*
  * device, and it runs behind every forward that still reads the old weights; the arrays stay as they are until
  * the stream has passed the call (a training step re-tiles its weights before every forward).
  * Refused (KANS_ERR_UNSUPPORTED) on a stream under graph capture.  A graph that a caller captures reads the
- * weights of its layers at each replay; ordering its replays with later loads is the caller's part, and a graph
- * captured on the stream that loaded the weights is to be launched behind that stream's work. */
+ * weights of its layers at each replay: the capture waits for a load that is still queued, and ordering the
+ * replays with later loads is the caller's part. */
 int kans_layer_load_weights_stream(kans_layer* layer, const void* W, const void* W_base, const void* bias,
                                    void* stream);
 /* host fp32 weights converted on the device to the layer dtype (round to nearest even) */

@@ -418,6 +418,28 @@ int kans_layer_set_block_pairs(kans_layer* L, int on) {
   return 0;
 }
 
+// The host waits for the device's work.  hipFree does so too while some stream is
+// being captured, where hipDeviceSynchronize fails and breaks the capture off.
+static int device_wait() {
+  CaptureRelaxed relaxed;
+  void* p = nullptr;
+  HIP_TRY(hipMalloc(&p, 64));
+  HIP_TRY(hipFree(p));
+  return 0;
+}
+
+// Stream st waits for event ev.  Where ev's stream is being captured by now no
+// other stream can, and the host waits for the device.
+static int wait_for_event(hipStream_t st, hipEvent_t ev) {
+  const hipError_t e = hipStreamWaitEvent(st, ev, 0);
+  if (e != hipErrorStreamCaptureIsolation) {
+    HIP_TRY(e);
+    return 0;
+  }
+  (void)hipGetLastError();
+  return device_wait();
+}
+
 // Before the tiles are written on stream st (not under capture): behind the last
 // re-tiling and behind every forward that may still read them.  A reader's event
 // is recorded now, not behind each forward, where it costs 3.5 us of GPU time (a
@@ -426,7 +448,8 @@ int kans_layer_set_block_pairs(kans_layer* L, int on) {
 // with the device.
 static int layer_claim_weights(kans_layer* L, hipStream_t st) {
   CaptureRelaxed relaxed;
-  if (L->w_pending && L->w_stream != st) HIP_TRY(hipStreamWaitEvent(st, L->w_done, 0));
+  int rc;
+  if (L->w_pending && L->w_stream != st && (rc = wait_for_event(st, L->w_done))) return rc;
   bool sync = L->unnamed_reader;
   for (hipStream_t r : L->readers) {
     if (r == st) continue;
@@ -440,8 +463,7 @@ static int layer_claim_weights(kans_layer* L, hipStream_t st) {
     HIP_TRY(hipEventRecord(L->r_done, r));
     HIP_TRY(hipStreamWaitEvent(st, L->r_done, 0));
   }
-  if (sync) HIP_TRY(hipDeviceSynchronize());
-  return 0;
+  return sync ? device_wait() : 0;
 }
 
 // Upload weights (host or device memory) whose element type is src_dtype (the
@@ -720,28 +742,24 @@ static int layer_plan_locked(kans_layer* L, int B, hipStream_t st, FwdPlan* p) {
 // Before a kernel on stream st reads the layer's tiles: behind a re-tiling that
 // may still run.  Each stream waits once per re-tiling; after that the forward
 // makes no call here but the capture query (0.05 us).  A stream under capture
-// cannot wait for an event from outside, so the host waits for it, and the graph's
-// replays are the caller's to order.  Captured on the stream that loaded the
-// weights, the graph is to be launched behind that stream's work, as any graph is:
-// the event cannot be asked for while its stream is captured.
+// cannot wait for an event from outside, and the event cannot be asked for where
+// its own stream is the captured one, so the host waits for the device; replays
+// behind later loads are the caller's to order.
 static int layer_use_weights(kans_layer* L, hipStream_t st) {
   const bool known = std::find(L->readers.begin(), L->readers.end(), st) != L->readers.end();
   if (known && !L->w_pending) return 0;
   bool capturing = false;
   HIP_TRY(kans_capturing(st, &capturing));
-  const bool behind = L->w_pending && (st == hipStreamPerThread || L->w_stream != st);
-  if (capturing || st == hipStreamPerThread) {
-    if (behind) {
-      CaptureRelaxed relaxed;
-      HIP_TRY(hipEventSynchronize(L->w_done));
-      L->w_pending = false;
-    }
-    if (!capturing) L->unnamed_reader = true;
+  int rc;
+  if (capturing) {
+    if (L->w_pending && (rc = device_wait())) return rc;
+    L->w_pending = false;
     return 0;
   }
   if (known) return 0;
-  if (behind) HIP_TRY(hipStreamWaitEvent(st, L->w_done, 0));
-  if (L->readers.size() < kMaxReaders) L->readers.push_back(st);
+  const bool behind = L->w_pending && (st == hipStreamPerThread || L->w_stream != st);
+  if (behind && (rc = wait_for_event(st, L->w_done))) return rc;
+  if (st != hipStreamPerThread && L->readers.size() < kMaxReaders) L->readers.push_back(st);
   else L->unnamed_reader = true;
   return 0;
 }

@@ -369,3 +369,73 @@ def test_parameters_given_back_while_their_retiling_is_queued(cuda):
             assert torch.equal(y, want)
             del reuse
             m.weight = torch.nn.Parameter(kept.to(cuda))
+
+
+def test_capture_while_a_load_is_queued(gpu, cuda):
+    """Weights loaded on a held stream that is then captured: the captured forward waits for them (its replay runs on
+    another stream at once), and a first forward on a third stream meanwhile neither fails nor breaks the capture."""
+    import metal_kans as mk
+    m = module(64, 72, degree=4)
+    side, other, third = (torch.cuda.Stream() for _ in range(3))
+    x = torch.rand(96, 64, device=cuda) * 2 - 1
+    y3 = torch.empty(96, 72, device=cuda)
+    with torch.no_grad():
+        for third_first in (False, True):
+            old = alone(m, x)
+            scale(m, 2.0)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(side):
+                torch.cuda._sleep(HOLD)
+                m(x)                          # the load waits on the held stream
+                graph = torch.cuda.CUDAGraph()
+                graph.capture_begin()
+                if third_first:
+                    mk.device.check(gpu.kans_layer_forward_ex(m.metal_layer._engine().handle, x.data_ptr(), 0, 64,
+                                                              y3.data_ptr(), 0, 72, 96, third.cuda_stream), "forward")
+                y = m(x)
+                graph.capture_end()
+            with torch.cuda.stream(other):
+                graph.replay()
+                got = y.clone()
+            torch.cuda.synchronize()
+            want = alone(m, x)
+            assert torch.equal(got, want) and not torch.equal(got, old)
+            assert not third_first or torch.equal(y3, want)
+
+
+def test_load_while_a_readers_stream_is_captured(gpu, cuda):
+    """A load behind a forward whose stream is captured by then: the old forward keeps its weights, the capture
+    survives."""
+    import metal_kans as mk
+    m = module(512, 512, degree=5)
+    x = torch.rand(256, 512, device=cuda) * 2 - 1
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.no_grad():
+        old = alone(m, x)
+        scale(m, 2.0)
+        new = alone(m, x)
+        scale(m, 0.5)
+        torch.cuda.synchronize()
+        doubled = [(p.detach() * 2.0).contiguous() for p in (m.weight, m.base_weight, m.bias_param)]
+        with torch.cuda.stream(other):
+            m(x)                              # the old weights, loaded
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(HOLD)
+            y = m(x)                          # reads the old tiles, held
+            z = torch.zeros(8, device=cuda)
+            graph = torch.cuda.CUDAGraph()
+            graph.capture_begin()
+            mk.device.check(gpu.kans_layer_load_weights_stream(m.metal_layer._engine().handle,
+                                                               *[w.data_ptr() for w in doubled], other.cuda_stream), "load")
+            z.add_(1.0)
+            graph.capture_end()
+        torch.cuda.synchronize()
+        assert torch.equal(y, old)
+        graph.replay()
+        torch.cuda.synchronize()
+        y2 = torch.empty_like(new)
+        mk.device.check(gpu.kans_layer_forward_ex(m.metal_layer._engine().handle, x.data_ptr(), 0, 512, y2.data_ptr(), 0,
+                                                  512, 256, other.cuda_stream), "forward")
+        torch.cuda.synchronize()
+        assert torch.equal(y2, new) and z[0].item() == 1.0
